@@ -74,12 +74,24 @@ def kernel_name(variant, real):
     return f"k_rk_stage<{real}, {variant}> (CSR, {variant} lanes per row)"
 
 
+def step_bytes(A, rows):
+    """bytes the FP32 sliced layout of A has to move per RK4 step in nested form:
+    4 x (stored values + slot metadata), 16 B per slot more for the FP64 values the
+    last stage reads, and 14 vector passes of 8 B per row (the gathered input and
+    the output of each stage, the state's high word in stages 2-4 and its low word
+    in stages 3 and 4, the low word written); and the layout statistics"""
+    kept, layout = format_step_bytes(A, rows)
+    last = 16 * layout["slots"] if layout["kind"].startswith("row-pair") else 8 * layout["slots"]
+    return kept - 6 * rows * 8 + last, layout
+
+
 def format_step_bytes(A, rows):
-    """bytes the FP32 sliced layout of A has to move per RK4 step: 4 x (stored
-    values + slot metadata) + 20 vector passes of 8 B per row (stages 1-3: the
-    gathered stage input, the state's high word for Y, the K and Y writes;
-    stage 4: the gathered input, the state's high and low words, K1..K3, and the
-    new high and low words written); and the layout statistics"""
+    """bytes of an RK4 step of the form that keeps the stage derivatives (the
+    time-dependent stages): 4 x (stored values + slot metadata) + 20 vector passes
+    of 8 B per row (stages 1-3: the gathered stage input, the state's high word for
+    Y, the K and Y writes; stage 4: the gathered input, the state's high and low
+    words, K1..K3, and the new high and low words written); and the layout
+    statistics"""
     lanes = A.lanes()
     if lanes[1] in (140, 141, 142, 143, 144):  # row-pair layout: 40-byte slot metadata, values per lane pair
         layout = dict(A.pair_layout_info(), kind="row-pair (128 rows per wavefront)")
@@ -127,7 +139,7 @@ def roofline_obj(kname, workload, fmt_bytes, launch_ms, ev_ms, traffic, traffic_
     out = {"bound": "hbm", "achieved": round(ach, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
            "frac": round(ach / HBM_PEAK_GBS, 4), "traffic": traffic, "kernel": kname, "workload": workload,
            "bytes_per_launch": fmt_bytes, "bytes_basis": "bytes the sliced format moves per launch (stored values "
-                                                         "+ slot metadata + 20/4 vector passes of 8 B per row)",
+                                                         "+ slot metadata + 14/4 vector passes of 8 B per row)",
            "launch_ms": round(launch_ms, 5), "launch_ms_per_kernel_events": round(ev_ms, 5),
            "csr_model": {"bytes_per_launch": csr_bytes,
                          "gbs": round(csr_bytes / (launch_ms * 1e-3) / 1e9, 1),
@@ -176,7 +188,7 @@ def run_sweep(qa, recipes, build_system, subsystem_layout, K, W, n_inst, renorm)
     el32 = time.perf_counter() - t
     pops32 = b.populations(subs)
     lanes = bA.lanes()
-    fmt_step, layout = format_step_bytes(bA, rows)
+    fmt_step, layout = step_bytes(bA, rows)
     nprof = min(20, max(K, 1))
     ev_ms = qa.rk4_device(bA, bx, dt, nprof, timed=True)   # per-launch events (state advanced past the check)
     launch_ms = tm32.ms / (4 * K) if K > 0 else ev_ms
@@ -249,7 +261,7 @@ def run_chain(qa, recipes, build_system, subsystem_layout, K, W, renorm, nq=10, 
     spmv32 = qa.bench_spmv(A, qa.FP32, 30)
     spmv64 = qa.bench_spmv(A, qa.FP64, 30)
     lanes = A.lanes()
-    fmt_step, layout = format_step_bytes(A, rows)
+    fmt_step, layout = step_bytes(A, rows)
     qs.destroy()
     el64, dev64, p64, tr64 = res[qa.FP64]
     el32, dev32, p32, tr32 = res[qa.FP32]

@@ -667,6 +667,7 @@ extern "C" int qh_mat_destroy(qh_mat *m) {
   qh_free_ptr(m->ks2_emid);
   qh_free_ptr(m->ks2_cmid);
   qh_free_ptr(m->ks2_meta);
+  qh_free_ptr(m->ks2_metad);
   qh_free_ptr(m->ks2_val);
   qh_free_ptr(m->ks2_sval);
   qh_free_ptr(m->ks2_sval1);

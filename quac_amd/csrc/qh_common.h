@@ -78,6 +78,13 @@ struct qh_kmeta2 {
   uint32_t ad8, base;
   float v0re, v0im, v1re, v1im;
 };
+// The same slot with the uniform values (or the 1, 0 multipliers of a scalar slot)
+// in FP64, read by the stage whose products are formed in FP64.
+struct qh_kmeta2d {
+  uint64_t mask, sign;
+  uint32_t ad8, base;
+  double v0re, v0im, v1re, v1im;
+};
 // empty slots after the last one, so that a pass of up to 8 slots may read
 // its metadata without a bounds check
 #define QH_KS_PAD 16
@@ -133,6 +140,7 @@ struct qh_mat {
   int32_t *ks2_emid = nullptr;  // end of each slice's scalar slots with a value per row
   int32_t *ks2_cmid = nullptr;  // end of each slice's scalar slots (equal-scalar slots included)
   qh_kmeta2 *ks2_meta = nullptr;
+  qh_kmeta2d *ks2_metad = nullptr;  // the same slots with FP64 values
   float4 *ks2_val = nullptr;    // complex slots: (row 2l, row 2l+1) complex64 pairs
   float2 *ks2_sval = nullptr;   // scalar slots: (row 2l, row 2l+1) real pairs
   float *ks2_sval1 = nullptr;   // equal-scalar slots: one real value for both rows of a lane
@@ -164,13 +172,14 @@ struct qh_vec {
 };
 
 // FP32 row-pair sliced layout (qh_ks2.hip): build once per matrix, launch one
-// stage (mode 0 SpMV, 1 stages 1-3, 2 stage 4) with variant G = 140 .. 144; td
+// stage (a MODE of qh_ks.h: SpMV, AXPY, LAST, STAGE, FINAL) with variant G = 140 ..
+// 144; td
 // (may be null): the merged A_k of a time-dependent RHS summed in the same kernel
 // (variants 140, 142, 143)
 struct qh_td_ell;
 int ks2_build(qh_mat *A);
-int ks2_launch(int G, int mode, hipStream_t s, const qh_mat *A, const void *xin, void *kout, void *ynext, float cn,
-               const void *x, const void *k1, const void *k2, const void *k3, void *xout, float h, float2 *xlo,
+int ks2_launch(int G, int mode, hipStream_t s, const qh_mat *A, const void *xin, void *kout, void *ynext, double cn,
+               const void *x, const void *k1, const void *k2, const void *k3, void *xout, double h, float2 *xlo,
                const qh_td_ell *td = nullptr);
 
 // the Bogacki-Shampine trial step of qh_rk3bs_step with the merged

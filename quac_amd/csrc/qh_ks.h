@@ -9,10 +9,21 @@
 
 namespace {
 
-// stage epilogues: SpMV only; RK4 stages 1-3; RK4 stage 4; Bogacki-Shampine
-// stage 3 (k3 and the 3rd-order candidate); Bogacki-Shampine error stage (k4 and
-// the weighted error norm)
-enum { MODE_SPMV = 0, MODE_STAGE = 1, MODE_FINAL = 2, MODE_BS3 = 3, MODE_BS3E = 4 };
+// stage epilogues: SpMV only; RK4 stages 1-3 and stage 4 of the form that keeps
+// the stage derivatives (time-dependent terms); Bogacki-Shampine stage 3 (k3 and
+// the 3rd-order candidate); Bogacki-Shampine error stage (k4 and the weighted
+// error norm); a stage of the nested RK4 polynomial of a constant generator
+// (y = x + c A y'); its last stage on an FP32 state (hi + lo updated, products in
+// FP64)
+enum {
+  MODE_SPMV = 0,
+  MODE_STAGE = 1,
+  MODE_FINAL = 2,
+  MODE_BS3 = 3,
+  MODE_BS3E = 4,
+  MODE_AXPY = 5,
+  MODE_LAST = 6
+};
 
 // Raw buffer resource over n elements (gfx9 descriptor word 3: 32-bit data
 // format).  A buffer load whose byte offset is at or beyond n * sizeof(T)

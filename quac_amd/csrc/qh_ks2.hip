@@ -52,7 +52,7 @@ __global__ void __launch_bounds__(64) k_ks2_build(int32_t n, const int32_t *__re
                                                   const int32_t *__restrict__ col, const double2 *__restrict__ val,
                                                   int32_t *cnt, int32_t ns, const int32_t *moff, const int32_t *voff,
                                                   const int32_t *svoff, const int32_t *s1off, qh_kmeta2 *meta,
-                                                  float4 *kval, float2 *sval, float *sval1,
+                                                  qh_kmeta2d *metad, float4 *kval, float2 *sval, float *sval1,
                                                   const int32_t *__restrict__ slice_blk, int *overflow) {
   // per lane up to 2 * KS2_MAXROW pair loads: key << 12 | e0 << 6 | e1 (63 = no entry)
   __shared__ uint64_t keys[64][2 * KS2_MAXROW];
@@ -206,8 +206,19 @@ __global__ void __launch_bounds__(64) k_ks2_build(int32_t n, const int32_t *__re
           md.v0re = md.v1re = sca ? (isre ? 1.f : 0.f) : 0.f;
           md.v0im = md.v1im = sca ? (isre ? 0.f : 1.f) : 0.f;
         }
-        meta[uni ? (win ? mo + uwin : inorder ? mw + (ustr - uwin) : mu2 + (uslot - ustr))
-                 : sep ? mx + xslot : eq1 ? ms1 + s1slot : sca ? ms + sslot : mc + cslot] = md;
+        const int32_t at = uni ? (win ? mo + uwin : inorder ? mw + (ustr - uwin) : mu2 + (uslot - ustr))
+                               : sep ? mx + xslot : eq1 ? ms1 + s1slot : sca ? ms + sslot : mc + cslot;
+        meta[at] = md;
+        qh_kmeta2d dd;
+        dd.mask = md.mask;
+        dd.sign = md.sign;
+        dd.ad8 = md.ad8;
+        dd.base = md.base;
+        dd.v0re = uni ? f0r : (double)md.v0re;
+        dd.v0im = uni ? f0i : (double)md.v0im;
+        dd.v1re = uni ? f1r : (double)md.v1re;
+        dd.v1im = uni ? f1i : (double)md.v1im;
+        metad[at] = dd;
       }
       if (act && eq1)
         sval1[s1base + rank] = part(v0);
@@ -262,28 +273,75 @@ struct KsAcc2 {
   float p0r, p0i, p1r, p1i;
 };
 
-template <int KIND, int W>
+// the metadata of a slot and the type of its uniform values: FP32, or FP64 (D) for
+// the stage whose products are formed in FP64
+template <bool D>
+struct Ks2Meta {
+  typedef qh_kmeta2 M;
+  typedef float U;
+};
+template <>
+struct Ks2Meta<true> {
+  typedef qh_kmeta2d M;
+  typedef double U;
+};
+
+template <int KIND, int W, bool D>
 struct Ks2Buf {
+  typedef typename Ks2Meta<D>::U U;
   float4 xv[W], vv[W];
   float2 sv[W];
   float s1[W];
-  float u0r[W], u0i[W], u1r[W], u1i[W];
+  U u0r[W], u0i[W], u1r[W], u1i[W];
   uint32_t h[W];
 };
 
+// rows 2l, 2l+1 += the products of one slot (a: values, x: the two rows' entries);
+// FP32: into the partial sums, D: into the FP64 sums
+template <bool D>
+__device__ __forceinline__ void ks2_mul(KsAcc2 &acc, typename Ks2Meta<D>::U a0r, typename Ks2Meta<D>::U a0i,
+                                        typename Ks2Meta<D>::U a1r, typename Ks2Meta<D>::U a1i, float x0r, float x0i,
+                                        float x1r, float x1i) {
+  if constexpr (D) {
+    const double y0r = (double)x0r, y0i = (double)x0i, y1r = (double)x1r, y1i = (double)x1i;
+    acc.r0 = fma(a0r, y0r, fma(-a0i, y0i, acc.r0));
+    acc.i0 = fma(a0r, y0i, fma(a0i, y0r, acc.i0));
+    acc.r1 = fma(a1r, y1r, fma(-a1i, y1i, acc.r1));
+    acc.i1 = fma(a1r, y1i, fma(a1i, y1r, acc.i1));
+  } else {
+    acc.p0r = fmaf(a0r, x0r, fmaf(-a0i, x0i, acc.p0r));
+    acc.p0i = fmaf(a0r, x0i, fmaf(a0i, x0r, acc.p0i));
+    acc.p1r = fmaf(a1r, x1r, fmaf(-a1i, x1i, acc.p1r));
+    acc.p1i = fmaf(a1r, x1i, fmaf(a1i, x1r, acc.p1i));
+  }
+}
+
+template <bool D>
+__device__ __forceinline__ void ks2_flush(KsAcc2 &acc) {
+  if constexpr (!D) {
+    acc.r0 += (double)acc.p0r;
+    acc.i0 += (double)acc.p0i;
+    acc.r1 += (double)acc.p1r;
+    acc.i1 += (double)acc.p1i;
+    acc.p0r = acc.p0i = acc.p1r = acc.p1i = 0.f;
+  }
+}
+
 // INORDER: every slot of the group has row 2l on half 0 and row 2l+1 on half 1
 // (known at compile time, no selects)
-template <int KIND, bool INORDER = false, int AUX = 0>
+template <int KIND, bool D, bool INORDER = false, int AUX = 0>
 struct Ks2Ops {
   typedef KsAcc2 Acc;
+  typedef typename Ks2Meta<D>::M Meta;
+  typedef typename Ks2Meta<D>::U U;
   template <int W>
-  using Buf = Ks2Buf<KIND, W>;
-  const qh_kmeta2 *mp;
+  using Buf = Ks2Buf<KIND, W, D>;
+  const Meta *mp;
   uint32_t r8;  // byte offset of x[2l] within the stage input
   __amdgpu_buffer_rsrc_t xr, vr;
   template <int W>
   __device__ __forceinline__ void issue(Buf<W> &b) {
-    qh_kmeta2 m[W];
+    Meta m[W];
 #pragma unroll
     for (int j = 0; j < W; j++) {
       m[j] = mp[j];
@@ -319,7 +377,6 @@ struct Ks2Ops {
   }
   template <int W>
   __device__ __forceinline__ void fma(const Buf<W> &b, Acc &acc) {
-    float p0r = acc.p0r, p0i = acc.p0i, p1r = acc.p1r, p1i = acc.p1i;
 #pragma unroll
     for (int j = 0; j < W; j++) {
       const float4 xv = b.xv[j];
@@ -336,58 +393,47 @@ struct Ks2Ops {
         x1r = h1 ? xv.z : xv.x;
         x1i = h1 ? xv.w : xv.y;
       }
-      float a0r, a0i, a1r, a1i;
+      U a0r, a0i, a1r, a1i;
       if (KIND == KS_CPX) {
-        a0r = b.vv[j].x;
-        a0i = b.vv[j].y;
-        a1r = b.vv[j].z;
-        a1i = b.vv[j].w;
+        a0r = (U)b.vv[j].x;
+        a0i = (U)b.vv[j].y;
+        a1r = (U)b.vv[j].z;
+        a1i = (U)b.vv[j].w;
       } else if (KIND == KS_SC1) {
-        a0r = a1r = b.s1[j] * b.u0r[j];
-        a0i = a1i = b.s1[j] * b.u0i[j];
+        a0r = a1r = (U)b.s1[j] * b.u0r[j];
+        a0i = a1i = (U)b.s1[j] * b.u0i[j];
       } else if (KIND == KS_SCA) {
-        a0r = b.sv[j].x * b.u0r[j];
-        a0i = b.sv[j].x * b.u0i[j];
-        a1r = b.sv[j].y * b.u0r[j];
-        a1i = b.sv[j].y * b.u0i[j];
+        a0r = (U)b.sv[j].x * b.u0r[j];
+        a0i = (U)b.sv[j].x * b.u0i[j];
+        a1r = (U)b.sv[j].y * b.u0r[j];
+        a1i = (U)b.sv[j].y * b.u0i[j];
       } else {
         a0r = b.u0r[j];
         a0i = b.u0i[j];
         a1r = b.u1r[j];
         a1i = b.u1i[j];
       }
-      p0r = fmaf(a0r, x0r, fmaf(-a0i, x0i, p0r));
-      p0i = fmaf(a0r, x0i, fmaf(a0i, x0r, p0i));
-      p1r = fmaf(a1r, x1r, fmaf(-a1i, x1i, p1r));
-      p1i = fmaf(a1r, x1i, fmaf(a1i, x1r, p1i));
+      ks2_mul<D>(acc, a0r, a0i, a1r, a1i, x0r, x0i, x1r, x1i);
     }
-    acc.p0r = p0r;
-    acc.p0i = p0i;
-    acc.p1r = p1r;
-    acc.p1i = p1i;
   }
-  __device__ __forceinline__ void flush(Acc &acc) {
-    acc.r0 += (double)acc.p0r;
-    acc.i0 += (double)acc.p0i;
-    acc.r1 += (double)acc.p1r;
-    acc.i1 += (double)acc.p1i;
-    acc.p0r = acc.p0i = acc.p1r = acc.p1i = 0.f;
-  }
+  __device__ __forceinline__ void flush(Acc &acc) { ks2_flush<D>(acc); }
 };
 
 // In-order uniform slots whose loads all stay inside the workgroup's window of
 // KS2_WIN rows: the pair is read from the LDS copy of the window (xs, KS2_WIN + 2
 // complex64, the last two zero for inactive lanes) instead of global memory.
+template <bool D>
 struct Ks2OpsWin {
   typedef KsAcc2 Acc;
+  typedef typename Ks2Meta<D>::M Meta;
   template <int W>
-  using Buf = Ks2Buf<KS_UNI, W>;
-  const qh_kmeta2 *mp;
+  using Buf = Ks2Buf<KS_UNI, W, D>;
+  const Meta *mp;
   uint32_t w8;  // byte offset of row 2l within the window
   const float2 *xs;
   template <int W>
   __device__ __forceinline__ void issue(Buf<W> &b) {
-    qh_kmeta2 m[W];
+    Meta m[W];
 #pragma unroll
     for (int j = 0; j < W; j++) {
       m[j] = mp[j];
@@ -413,23 +459,27 @@ struct Ks2OpsWin {
   }
   template <int W>
   __device__ __forceinline__ void fma(const Buf<W> &b, Acc &acc) {
-    Ks2Ops<KS_UNI, true>{}.fma(b, acc);
+    Ks2Ops<KS_UNI, D, true>{}.fma(b, acc);
   }
-  __device__ __forceinline__ void flush(Acc &acc) { Ks2Ops<KS_UNI, true>{}.flush(acc); }
+  __device__ __forceinline__ void flush(Acc &acc) { ks2_flush<D>(acc); }
 };
 
 // Separable-diagonal slots (at most one per slice): the lane's own pair x[2l],
 // x[2l+1] times the diagonal entries g_i + h_j and g_(i+1) + h_j, formed in FP64
 // from the block's g and h (t = 2l - off, j = t / N, i = t - j N; i is even, so
-// i + 1 stays in the column) and rounded to FP32 as the stored diagonal would be.
+// i + 1 stays in the column) and, without D, rounded to FP32 as the stored diagonal
+// would be.
+template <bool D>
 struct Ks2OpsSep {
   typedef KsAcc2 Acc;
+  typedef typename Ks2Meta<D>::M Meta;
+  typedef typename Ks2Meta<D>::U U;
   template <int W>
   struct Buf {
     float4 xv[W];
     double2 g0[W], g1[W], h[W];
   };
-  const qh_kmeta2 *mp;
+  const Meta *mp;
   uint32_t r8;  // byte offset of x[2l] within the stage input
   int64_t r;    // row 2l
   __amdgpu_buffer_rsrc_t xr, ghr;
@@ -438,7 +488,7 @@ struct Ks2OpsSep {
   __device__ __forceinline__ void issue(Buf<W> &b) {
 #pragma unroll
     for (int j = 0; j < W; j++) {
-      const qh_kmeta2 m = mp[j];
+      const Meta m = mp[j];
       const bool on = __builtin_amdgcn_inverse_ballot_w64(m.mask);
       b.xv[j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xr, on ? r8 : QH_KS_OOB, 0, 0));
       const qh_sepblk q = bp[m.base];
@@ -454,23 +504,14 @@ struct Ks2OpsSep {
   }
   template <int W>
   __device__ __forceinline__ void fma(const Buf<W> &b, Acc &acc) {
-    float p0r = acc.p0r, p0i = acc.p0i, p1r = acc.p1r, p1i = acc.p1i;
 #pragma unroll
     for (int j = 0; j < W; j++) {
-      const float a0r = (float)(b.g0[j].x + b.h[j].x), a0i = (float)(b.g0[j].y + b.h[j].y);
-      const float a1r = (float)(b.g1[j].x + b.h[j].x), a1i = (float)(b.g1[j].y + b.h[j].y);
       const float4 xv = b.xv[j];
-      p0r = fmaf(a0r, xv.x, fmaf(-a0i, xv.y, p0r));
-      p0i = fmaf(a0r, xv.y, fmaf(a0i, xv.x, p0i));
-      p1r = fmaf(a1r, xv.z, fmaf(-a1i, xv.w, p1r));
-      p1i = fmaf(a1r, xv.w, fmaf(a1i, xv.z, p1i));
+      ks2_mul<D>(acc, (U)(b.g0[j].x + b.h[j].x), (U)(b.g0[j].y + b.h[j].y), (U)(b.g1[j].x + b.h[j].x),
+                 (U)(b.g1[j].y + b.h[j].y), xv.x, xv.y, xv.z, xv.w);
     }
-    acc.p0r = p0r;
-    acc.p0i = p0i;
-    acc.p1r = p1r;
-    acc.p1i = p1i;
   }
-  __device__ __forceinline__ void flush(Acc &acc) { Ks2Ops<KS_UNI, true>{}.flush(acc); }
+  __device__ __forceinline__ void flush(Acc &acc) { ks2_flush<D>(acc); }
 };
 
 // the two complex64 of rows (r, r+1) at byte offset o of a vector; the second is
@@ -495,6 +536,9 @@ __device__ inline void st_pair(__amdgpu_buffer_rsrc_t rs, uint32_t o, bool two, 
 }
 
 //   MODE_SPMV : kout = A xin
+//   MODE_AXPY : ynext = x + cn A xin (x = hi, or hi + lo where xlo is given)
+//   MODE_LAST : hi + lo = x + cn A xin in place (ynext = x, xlo), the products in
+//               FP64 from the FP64 slot metadata
 //   MODE_STAGE: kout = A xin;  ynext = x + cn * kout          (stages 1-3)
 //   MODE_FINAL: xout = x + h/6 (K1 + 2 K2 + 2 K3 + A xin)    (stage 4)
 // with the FP32 state x = hi + lo updated in FP64 and split again.
@@ -513,12 +557,12 @@ __global__ void __launch_bounds__(WIN ? KS2_WIN / 2 : 256, WIN ? 8 : 1) k_ks2_st
     int32_t n, int32_t nslices, const int32_t *__restrict__ moff, const int32_t *__restrict__ wmid,
     const int32_t *__restrict__ smid, const int32_t *__restrict__ umid, const int32_t *__restrict__ emid,
     const int32_t *__restrict__ cmid, const int32_t *__restrict__ xmid, const qh_sepblk *__restrict__ sepb,
-    int32_t ngh, const double2 *__restrict__ gh, const qh_kmeta2 *__restrict__ meta, int32_t nval,
+    int32_t ngh, const double2 *__restrict__ gh, const void *__restrict__ metap, int32_t nval,
                                                    const float4 *__restrict__ val, int32_t nsval,
                                                    const float2 *__restrict__ sval, int32_t nsval1,
                                                    const float *__restrict__ sval1, const float2 *xin, float2 *kout,
-                                                   float2 *ynext, float cn, const float2 *x, const float2 *k1,
-                                                   const float2 *k2, const float2 *k3, float2 *xout, float h,
+                                                   float2 *ynext, double cn, const float2 *x, const float2 *k1,
+                                                   const float2 *k2, const float2 *k3, float2 *xout, double h,
                                                    float2 *xlo, qh_td_ell td) {
   const unsigned b = qh_xcd_block(blockIdx.x, gridDim.x);
   const int s = (int)(b * (WIN ? KS2_WIN / 128 : 4) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
@@ -551,19 +595,24 @@ __global__ void __launch_bounds__(WIN ? KS2_WIN / 2 : 256, WIN ? 8 : 1) k_ks2_st
   const __amdgpu_buffer_rsrc_t s1r = ks_rsrc(sval1, (int64_t)nsval1 * 4);
   const uint32_t r8 = (uint32_t)r * 8u;
   KsAcc2 acc{0.0, 0.0, 0.0, 0.0, 0.f, 0.f, 0.f, 0.f};
+  // FP64 slot metadata for the stage with FP64 products (untyped in the kernel's
+  // signature: a type that depends on MODE would put the unnamed enum into its
+  // symbol, which the host and the device pass number differently)
+  constexpr bool D = MODE == MODE_LAST;
+  const typename Ks2Meta<D>::M *const meta = (const typename Ks2Meta<D>::M *)metap;
   // (a wavefront past the last slice has empty slot ranges: k0 = ... = kend = 0)
-  ks_run<U, true>(Ks2Ops<KS_UNI, true>{meta + kw, r8, xr, vr}, ku - kw, acc);
-  if (!WIN) ks_run<U, true>(Ks2Ops<KS_UNI, true>{meta + k0, r8, xr, vr}, kw - k0, acc);
+  ks_run<U, true>(Ks2Ops<KS_UNI, D, true>{meta + kw, r8, xr, vr}, ku - kw, acc);
+  if (!WIN) ks_run<U, true>(Ks2Ops<KS_UNI, D, true>{meta + k0, r8, xr, vr}, kw - k0, acc);
   constexpr int AUX = NT ? 2 : 0;
-  ks_run<U, true>(Ks2Ops<KS_UNI>{meta + ku, r8, xr, vr}, km - ku, acc);
-  ks_run<U, true>(Ks2Ops<KS_SCA, false, AUX>{meta + km, r8, xr, sr}, ke - km, acc);
-  ks_run<U, true>(Ks2Ops<KS_SC1, false, AUX>{meta + ke, r8, xr, s1r}, kc - ke, acc);
-  ks_run<U, true>(Ks2Ops<KS_CPX, false, AUX>{meta + kc, r8, xr, vr}, kx - kc, acc);
+  ks_run<U, true>(Ks2Ops<KS_UNI, D>{meta + ku, r8, xr, vr}, km - ku, acc);
+  ks_run<U, true>(Ks2Ops<KS_SCA, D, false, AUX>{meta + km, r8, xr, sr}, ke - km, acc);
+  ks_run<U, true>(Ks2Ops<KS_SC1, D, false, AUX>{meta + ke, r8, xr, s1r}, kc - ke, acc);
+  ks_run<U, true>(Ks2Ops<KS_CPX, D, false, AUX>{meta + kc, r8, xr, vr}, kx - kc, acc);
   if (SEP && kend > kx) {  // the one separable-diagonal slot of the slice, after the pipelined groups
-    Ks2OpsSep op{meta + kx, r8, (int64_t)r, xr, ks_rsrc(gh, (int64_t)ngh * 16), sepb};
-    Ks2OpsSep::Buf<1> sb;
-    op.issue<1>(sb);
-    op.fma<1>(sb, acc);
+    Ks2OpsSep<D> op{meta + kx, r8, (int64_t)r, xr, ks_rsrc(gh, (int64_t)ngh * 16), sepb};
+    typename Ks2OpsSep<D>::template Buf<1> sb;
+    op.template issue<1>(sb);
+    op.template fma<1>(sb, acc);
     op.flush(acc);
   }
   if (WIN) {
@@ -571,7 +620,7 @@ __global__ void __launch_bounds__(WIN ? KS2_WIN / 2 : 256, WIN ? 8 : 1) k_ks2_st
     xs[2 * threadIdx.x + 1] = make_float2(wv.z, wv.w);
     if (threadIdx.x == 0) xs[KS2_WIN] = xs[KS2_WIN + 1] = make_float2(0.f, 0.f);
     __syncthreads();
-    ks_run<U, true>(Ks2OpsWin{meta + k0, (uint32_t)(r - (int32_t)b * KS2_WIN) * 8u, xs}, kw - k0, acc);
+    ks_run<U, true>(Ks2OpsWin<D>{meta + k0, (uint32_t)(r - (int32_t)b * KS2_WIN) * 8u, xs}, kw - k0, acc);
   }
   if (!live) return;
   if (r >= n) return;
@@ -603,13 +652,27 @@ __global__ void __launch_bounds__(WIN ? KS2_WIN / 2 : 256, WIN ? 8 : 1) k_ks2_st
     return;
   }
   const float4 xo = ld_pair<AUX>(ks_rsrc(x, vb), r8, two);
+  if constexpr (MODE == MODE_AXPY || MODE == MODE_LAST) {
+    const __amdgpu_buffer_rsrc_t lr = ks_rsrc(xlo, vb);
+    const float4 lo = (MODE == MODE_LAST || xlo) ? ld_pair<AUX>(lr, r8, two) : make_float4(0.f, 0.f, 0.f, 0.f);
+    const double c = cn;
+    const double n0r = ((double)xo.x + (double)lo.x) + c * a0r, n0i = ((double)xo.y + (double)lo.y) + c * a0i;
+    const double n1r = ((double)xo.z + (double)lo.z) + c * a1r, n1i = ((double)xo.w + (double)lo.w) + c * a1i;
+    const float4 o = make_float4((float)n0r, (float)n0i, (float)n1r, (float)n1i);
+    st_pair(ks_rsrc(ynext, vb), r8, two, o);
+    if (MODE == MODE_LAST)
+      st_pair<AUX>(lr, r8, two,
+                   make_float4((float)(n0r - (double)o.x), (float)(n0i - (double)o.y), (float)(n1r - (double)o.z),
+                               (float)(n1i - (double)o.w)));
+    return;
+  }
   if (MODE == MODE_STAGE) {
     // the next stage input is stored in complex64: the low word of the state
     // (below half an ulp of the high word) would change it by at most one
     // rounding, so only the high word is read here (the update in stage 4
     // uses both)
     st_pair<AUX>(ks_rsrc(kout, vb), r8, two, y);
-    const double c = (double)cn;
+    const double c = cn;
     const float4 yn = make_float4((float)((double)xo.x + c * a0r), (float)((double)xo.y + c * a0i),
                                   (float)((double)xo.z + c * a1r), (float)((double)xo.w + c * a1i));
     st_pair(ks_rsrc(ynext, vb), r8, two, yn);
@@ -619,7 +682,7 @@ __global__ void __launch_bounds__(WIN ? KS2_WIN / 2 : 256, WIN ? 8 : 1) k_ks2_st
   const float4 lo = ld_pair<AUX>(lr, r8, two);
   const float4 a = ld_pair<AUX>(ks_rsrc(k1, vb), r8, two), bq = ld_pair<AUX>(ks_rsrc(k2, vb), r8, two),
                cq = ld_pair<AUX>(ks_rsrc(k3, vb), r8, two);
-  const double s6 = (double)h * (1.0 / 6.0), s3 = (double)h * (1.0 / 3.0);
+  const double s6 = h * (1.0 / 6.0), s3 = h * (1.0 / 3.0);
   const double n0r = ((double)xo.x + (double)lo.x) + (s6 * (double)a.x + s3 * (double)bq.x + s3 * (double)cq.x + s6 * a0r);
   const double n0i = ((double)xo.y + (double)lo.y) + (s6 * (double)a.y + s3 * (double)bq.y + s3 * (double)cq.y + s6 * a0i);
   const double n1r = ((double)xo.z + (double)lo.z) + (s6 * (double)a.z + s3 * (double)bq.z + s3 * (double)cq.z + s6 * a1r);
@@ -846,7 +909,8 @@ int ks2_build(qh_mat *A) {
   QH_HIP(hipMemcpyAsync(sblk, hsb.data(), sizeof(int32_t) * ns, hipMemcpyHostToDevice, s));
   QH_HIP(hipMemsetAsync(ovf, 0, sizeof(int), s));
   hipLaunchKernelGGL((k_ks2_build<false>), dim3(ns), dim3(64), 0, s, (int32_t)A->rows, A->rowptr, A->col, A->val,
-                     cnt, ns, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, sblk, ovf);
+                     cnt, ns, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, sblk,
+                     ovf);
   QH_HIP(hipGetLastError());
   int hovf = 0;
   std::vector<int32_t> hc((size_t)NC * ns);
@@ -902,6 +966,7 @@ int ks2_build(qh_mat *A) {
     }
   }
   if (!rc) rc = qh_alloc_t(&A->ks2_meta, (size_t)(tot > 0 ? tot : 1));
+  if (!rc) rc = qh_alloc_t(&A->ks2_metad, (size_t)(tot > 0 ? tot : 1));
   if (!rc) rc = qh_alloc_t(&A->ks2_val, (size_t)(totv > 0 ? totv : 1));
   if (!rc) rc = qh_alloc_t(&A->ks2_sval, (size_t)(tots > 0 ? tots : 1));
   if (!rc) rc = qh_alloc_t(&A->ks2_sval1, (size_t)(tots1 > 0 ? tots1 : 1));
@@ -922,8 +987,8 @@ int ks2_build(qh_mat *A) {
   QH_HIP(hipMemcpyAsync(svoff, hso.data(), sizeof(int32_t) * (ns + 1), hipMemcpyHostToDevice, s));
   QH_HIP(hipMemcpyAsync(s1off, hs1o.data(), sizeof(int32_t) * (ns + 1), hipMemcpyHostToDevice, s));
   hipLaunchKernelGGL((k_ks2_build<true>), dim3(ns), dim3(64), 0, s, (int32_t)A->rows, A->rowptr, A->col, A->val,
-                     cnt, ns, A->ks2_moff, voff, svoff, s1off, A->ks2_meta, A->ks2_val, A->ks2_sval, A->ks2_sval1,
-                     sblk, ovf);
+                     cnt, ns, A->ks2_moff, voff, svoff, s1off, A->ks2_meta, A->ks2_metad, A->ks2_val, A->ks2_sval,
+                     A->ks2_sval1, sblk, ovf);
   QH_HIP(hipGetLastError());
   QH_HIP(hipStreamSynchronize(s));
   cleanup();
@@ -943,8 +1008,8 @@ int ks2_build(qh_mat *A) {
 // 142: 2 slots per pass, window slots read from LDS; 143 / 144: 140 / 142 with
 // the non-temporal cache policy on the streamed data);
 // mode as in the one-row-per-lane kernels.
-int ks2_launch(int G, int mode, hipStream_t s, const qh_mat *A, const void *xin, void *kout, void *ynext, float cn,
-               const void *x, const void *k1, const void *k2, const void *k3, void *xout, float h, float2 *xlo,
+int ks2_launch(int G, int mode, hipStream_t s, const qh_mat *A, const void *xin, void *kout, void *ynext, double cn,
+               const void *x, const void *k1, const void *k2, const void *k3, void *xout, double h, float2 *xlo,
                const qh_td_ell *td) {
   if (A->ks2_state != 1) {
     qh_set_error("row-pair sliced layout not built for this matrix");
@@ -959,7 +1024,7 @@ int ks2_launch(int G, int mode, hipStream_t s, const qh_mat *A, const void *xin,
                      A->ks2_smid,                                                                                \
                      A->ks2_umid, A->ks2_emid, A->ks2_cmid, A->ks2_xmid, A->ks2_sep,                               \
                      (int32_t)A->ks2_ngh,                                                                        \
-                     A->ks2_gh, A->ks2_meta, (int32_t)A->ks2_nval, A->ks2_val,                                    \
+                     A->ks2_gh, MM == MODE_LAST ? (const void *)A->ks2_metad : (const void *)A->ks2_meta, (int32_t)A->ks2_nval, A->ks2_val,                                    \
                      (int32_t)A->ks2_nsval, A->ks2_sval, (int32_t)A->ks2_nsval1, A->ks2_sval1,                  \
                      (const float2 *)xin, (float2 *)kout, (float2 *)ynext, cn, (const float2 *)x,                \
                      (const float2 *)k1, (const float2 *)k2, (const float2 *)k3, (float2 *)xout, h, xlo, TD)
@@ -971,7 +1036,8 @@ int ks2_launch(int G, int mode, hipStream_t s, const qh_mat *A, const void *xin,
     else                                  \
       QH_LK2S(MM, UU, WW, NN, false);     \
   } while (0)
-  if (!QH_IS_KS2(G) || mode < MODE_SPMV || mode > MODE_FINAL) {
+  const bool known = mode == MODE_SPMV || mode == MODE_STAGE || mode == MODE_FINAL || mode == MODE_AXPY || mode == MODE_LAST;
+  if (!QH_IS_KS2(G) || !known || (td && (mode == MODE_AXPY || mode == MODE_LAST))) {
     qh_set_error("unsupported row-pair variant %d / mode %d", G, mode);
     return QH_EINVAL;
   }
@@ -1013,6 +1079,10 @@ int ks2_launch(int G, int mode, hipStream_t s, const qh_mat *A, const void *xin,
   }
   if (mode == MODE_SPMV) {
     QH_LK2G(MODE_SPMV)
+  } else if (mode == MODE_AXPY) {
+    QH_LK2G(MODE_AXPY)
+  } else if (mode == MODE_LAST) {
+    QH_LK2G(MODE_LAST)
   } else if (mode == MODE_STAGE) {
     QH_LK2G(MODE_STAGE)
   } else {

@@ -1,25 +1,29 @@
 // qh_spmv.hip -- the hot path: complex CSR SpMV fused with the RK4 stage updates.
 //
-// Each RK4 step of dx/dt = A x is four launches of one kernel template:
-//   S1: K1 = A x
-//   S2: K2 = A (x + h/2 K1)        (stage input formed on the fly in the gather)
-//   S3: K3 = A (x + h/2 K2)
-//   S4: x' = x + h/6 (K1 + 2 K2 + 2 K3 + A (x + h K3))   (update fused in the epilogue)
-// so the stage vectors Y_s are never materialised: per step the matrix is
-// streamed 4 times and 14 vector passes are made (4 gathers of x, 3 of K, 3 K
-// writes, 3 K reads + x read + x' write in the epilogue).
+// One classic RK4 step of dx/dt = A x with a constant A is the polynomial
+// x + hA x + (hA)^2 x / 2 + (hA)^3 x / 6 + (hA)^4 x / 24, evaluated in nested form:
+//   y = x + h/4 A x;  y = x + h/3 A y;  y = x + h/2 A y;  x = x + h A y
+// -- four launches of one kernel that gathers one vector, reads x and writes one
+// vector.  No stage derivative is kept: per step 11 vector passes (the first stage
+// gathers x itself) where K1..K3 take 18, and 2 work vectors where they take 6.
+// Measured per launch: 10-qubit chain FP64 31.2 -> 28.2 us, 12-qubit circuit FP64
+// (268 MB vectors) 308 -> 243 us, FP32 sweep of 512 instances 219.8 -> 202.2 us.
 //
-// Layout and mapping (gfx950, wave64): a group of G lanes owns one row (64/G rows
-// per wavefront, G autotuned per matrix); lanes stride through the row so every
-// load instruction of a wave reads contiguous col/val bytes; the matrix streams
-// use non-temporal loads so they do not evict x from L2/MALL; the group reduces
-// with cross-lane shuffles and lane 0 runs the fused epilogue.  Block indices
-// are remapped so each XCD sweeps one contiguous band of rows.
+// Layout and mapping (gfx950, wave64) of the CSR kernel: a group of G lanes owns
+// one row (64/G rows per wavefront, G autotuned per matrix); lanes stride through
+// the row so every load instruction of a wave reads contiguous col/val bytes; the
+// matrix streams use non-temporal loads so they do not evict x from L2/MALL; the
+// group reduces with cross-lane shuffles and lane 0 runs the fused epilogue.
+// Block indices are remapped so each XCD sweeps one contiguous band of rows.
 //
 // FP64 path: complex128 values, FP64 accumulation (the drop-in path).
-// FP32 path: complex64 values and vectors; each lane accumulates with TwoSum
-// compensation, the state carries a complex64 compensation word (x = hi + lo)
-// so that the RK update does not lose the low bits of x.
+// FP32 path: complex64 values and stage vectors, the state x = hi + lo (complex64
+// pair).  The last stage enters x' at first order in h, so its products are formed
+// in FP64 (from the FP64 values of the uniform slots and of the CSR), and the
+// third stage starts from hi + lo; the first two reach x' only at order h^2 and
+// h^3.  With K1..K3 the four products were averaged instead; the error of this form
+// against 64 bits is no larger (chain, 40 steps: 1.8e-8 of the state against 4.1e-8;
+// sweep, 20 steps: 1.6e-9 against 2.3e-9).
 #include <algorithm>
 #include <cstddef>
 #include <cstdlib>
@@ -106,14 +110,20 @@ struct Acc<float> {
   __device__ inline float2 value() const { return make_float2(re + cre, im + cim); }
 };
 
+//   MODE_SPMV: out = A xin
+//   MODE_AXPY: out = x + c A xin  (FP32: x = hi, or hi + lo where xlo is given)
+//   MODE_LAST: hi + lo = x + c A xin in place (FP32 state; FP64 products with the
+//              FP64 values)
+// out may be x (every row reads and writes its own entry of x only); xin is
+// another vector
 template <typename R, int G, int MODE>
-__global__ void __launch_bounds__(256) k_rk_stage(
-    int32_t nrows, const int32_t *__restrict__ rp, const int32_t *__restrict__ col,
-    const typename C2<R>::T *__restrict__ val, const typename C2<R>::T *__restrict__ x,
-    const typename C2<R>::T *__restrict__ kin, R ck, typename C2<R>::T *__restrict__ kout,
-    const typename C2<R>::T *__restrict__ k1, const typename C2<R>::T *__restrict__ k2,
-    const typename C2<R>::T *__restrict__ k3, typename C2<R>::T *__restrict__ xout, R h,
-    float2 *__restrict__ xlo) {
+__global__ void __launch_bounds__(256) k_rk_stage(int32_t nrows, const int32_t *__restrict__ rp,
+                                                  const int32_t *__restrict__ col,
+                                                  const typename C2<R>::T *__restrict__ val,
+                                                  const double2 *__restrict__ val64,
+                                                  const typename C2<R>::T *__restrict__ xin,
+                                                  typename C2<R>::T *out, const typename C2<R>::T *x, double c,
+                                                  float2 *xlo) {
   typedef typename C2<R>::T T;
   const unsigned b = qh_xcd_block(blockIdx.x, gridDim.x);
   const int64_t tid = (int64_t)b * 256 + threadIdx.x;
@@ -121,70 +131,62 @@ __global__ void __launch_bounds__(256) k_rk_stage(
   const int lane = (int)(tid % G);
   if (row >= nrows) return;  // G divides 256: a group never straddles the bound
   const int32_t beg = rp[row], end = rp[row + 1];
-  Acc<R> acc;
-  int32_t k = beg + lane;
-  // two independent loads in flight per lane
-  for (; k + G < end; k += 2 * G) {
-    const int32_t c0 = __builtin_nontemporal_load(col + k);
-    const int32_t c1 = __builtin_nontemporal_load(col + k + G);
-    const T a0 = ld_stream<R>(val + k);
-    const T a1 = ld_stream<R>(val + k + G);
-    T x0 = x[c0], x1 = x[c1];
-    if (MODE != MODE_SPMV) {
-      const T q0 = kin[c0], q1 = kin[c1];
-      x0.x += ck * q0.x;
-      x0.y += ck * q0.y;
-      x1.x += ck * q1.x;
-      x1.y += ck * q1.y;
+  double yr, yi;
+  if constexpr (MODE == MODE_LAST) {
+    Acc<double> acc;
+    for (int32_t k = beg + lane; k < end; k += G) {
+      const double2 a = ld_stream<double>(val64 + k);
+      const T v = xin[__builtin_nontemporal_load(col + k)];
+      acc.add(a.x * (double)v.x - a.y * (double)v.y, a.x * (double)v.y + a.y * (double)v.x);
     }
-    acc.add(a0.x * x0.x - a0.y * x0.y, a0.x * x0.y + a0.y * x0.x);
-    acc.add(a1.x * x1.x - a1.y * x1.y, a1.x * x1.y + a1.y * x1.x);
-  }
-  if (k < end) {
-    const int32_t c0 = __builtin_nontemporal_load(col + k);
-    const T a0 = ld_stream<R>(val + k);
-    T x0 = x[c0];
-    if (MODE != MODE_SPMV) {
-      const T q0 = kin[c0];
-      x0.x += ck * q0.x;
-      x0.y += ck * q0.y;
+    acc.template reduce<G>();
+    yr = acc.re;
+    yi = acc.im;
+  } else {
+    Acc<R> acc;
+    int32_t k = beg + lane;
+    // two independent loads in flight per lane
+    for (; k + G < end; k += 2 * G) {
+      const int32_t c0 = __builtin_nontemporal_load(col + k);
+      const int32_t c1 = __builtin_nontemporal_load(col + k + G);
+      const T a0 = ld_stream<R>(val + k);
+      const T a1 = ld_stream<R>(val + k + G);
+      const T x0 = xin[c0], x1 = xin[c1];
+      acc.add(a0.x * x0.x - a0.y * x0.y, a0.x * x0.y + a0.y * x0.x);
+      acc.add(a1.x * x1.x - a1.y * x1.y, a1.x * x1.y + a1.y * x1.x);
     }
-    acc.add(a0.x * x0.x - a0.y * x0.y, a0.x * x0.y + a0.y * x0.x);
+    if (k < end) {
+      const int32_t c0 = __builtin_nontemporal_load(col + k);
+      const T a0 = ld_stream<R>(val + k);
+      const T x0 = xin[c0];
+      acc.add(a0.x * x0.x - a0.y * x0.y, a0.x * x0.y + a0.y * x0.x);
+    }
+    acc.template reduce<G>();
+    const auto y = acc.value();
+    yr = (double)y.x;
+    yi = (double)y.y;
   }
-  acc.template reduce<G>();
   if (lane != 0) return;
-  const T y = acc.value();
-  if (MODE != MODE_FINAL) {
-    kout[row] = y;
+  if (MODE == MODE_SPMV) {
+    T o;
+    o.x = (R)yr;
+    o.y = (R)yi;
+    out[row] = o;
     return;
   }
-  // x' = x + h/6 (K1 + 2K2 + 2K3 + K4)
-  const T a = k1[row], bq = k2[row], cq = k3[row];
-  const R s6 = h * (R)(1.0 / 6.0), s3 = h * (R)(1.0 / 3.0);
-  const R dre = s6 * a.x + s3 * bq.x + s3 * cq.x + s6 * y.x;
-  const R dim = s6 * a.y + s3 * bq.y + s3 * cq.y + s6 * y.y;
   const T xo = x[row];
-  if (sizeof(R) == 8) {
-    T r;
-    r.x = xo.x + dre;
-    r.y = xo.y + dim;
-    xout[row] = r;
-  } else {
-    // compensated update of (hi, lo): hi' + lo' = hi + lo + d to ~2^-48
-    float2 lo = xlo[row];
-    float sr, er, si, ei;
-    two_sum((float)xo.x, (float)dre, sr, er);
-    two_sum((float)xo.y, (float)dim, si, ei);
-    float lr = lo.x + er, li = lo.y + ei;
-    float hr = sr + lr, hi = si + li;
-    lr = lr - (hr - sr);
-    li = li - (hi - si);
-    T r;
-    r.x = hr;
-    r.y = hi;
-    xout[row] = r;
-    xlo[row] = make_float2(lr, li);
+  double xr = (double)xo.x, xi = (double)xo.y;
+  if (sizeof(R) == 4 && xlo) {
+    const float2 lo = xlo[row];
+    xr += (double)lo.x;
+    xi += (double)lo.y;
   }
+  const double nr = xr + c * yr, ni = xi + c * yi;
+  T o;
+  o.x = (R)nr;
+  o.y = (R)ni;
+  out[row] = o;
+  if (MODE == MODE_LAST) xlo[row] = make_float2((float)(nr - (double)o.x), (float)(ni - (double)o.y));
 }
 
 // ------------------------------------------------- slot-aligned sliced ELL
@@ -434,10 +436,13 @@ __device__ __forceinline__ void ks_group(const qh_kmeta *__restrict__ meta, int3
   ks_run<U, PIPE>(ops, kend - k, acc);
 }
 
-// Stage kernel on the sliced layout.  The stage input Y_s = x + c_s K_{s-1} is
-// materialised by the previous stage's epilogue, so every stage gathers one
-// vector:
+// Stage kernel on the sliced layout: every stage gathers one vector.
 //   MODE_SPMV : kout = A xin
+//   MODE_AXPY : ynext = x + cn A xin      (a stage of the nested RK4 polynomial;
+//               FP32: x = hi, or hi + lo where xlo is given; ynext may be x)
+//   MODE_LAST : hi + lo = x + cn A xin in place (its last stage on an FP32 state,
+//               with FP64 products and FP64 uniform values)
+// and, where the generator changes within the step (time-dependent terms),
 //   MODE_STAGE: kout = A xin;  ynext = x + cn * kout          (stages 1-3)
 //   MODE_FINAL: xout = x + h/6 (K1 + 2 K2 + 2 K3 + A xin)    (stage 4)
 // U slots are processed per pass (all metadata loads, then all gathers, then
@@ -483,11 +488,10 @@ __global__ void __launch_bounds__(256) k_ks_stage(
     const int32_t *__restrict__ cmid, const qh_kmeta *__restrict__ meta, const qh_kmeta32 *__restrict__ meta32,
     int32_t nmeta, int32_t nval, const typename C2<R>::T *__restrict__ val, int32_t nsval,
     const R *__restrict__ sval,
-    const typename C2<R>::T *__restrict__ xin, typename C2<R>::T *__restrict__ kout,
-    typename C2<R>::T *__restrict__ ynext, R cn, const typename C2<R>::T *__restrict__ x,
-    const typename C2<R>::T *__restrict__ k1, const typename C2<R>::T *__restrict__ k2,
-    const typename C2<R>::T *__restrict__ k3, typename C2<R>::T *__restrict__ xout, R h,
-    float2 *__restrict__ xlo, double atol, double rtol, double *__restrict__ eacc, qh_td_ell td) {
+    const typename C2<R>::T *__restrict__ xin, typename C2<R>::T *__restrict__ kout, typename C2<R>::T *ynext, double cn,
+    const typename C2<R>::T *x, const typename C2<R>::T *__restrict__ k1, const typename C2<R>::T *__restrict__ k2,
+    const typename C2<R>::T *__restrict__ k3, typename C2<R>::T *xout, double h, float2 *__restrict__ xlo, double atol,
+    double rtol, double *__restrict__ eacc, qh_td_ell td) {
   typedef typename C2<R>::T T;
   const unsigned b = qh_xcd_block(blockIdx.x, gridDim.x);
   const int s = (int)(b * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
@@ -502,7 +506,7 @@ __global__ void __launch_bounds__(256) k_ks_stage(
   const uint32_t r8 = (uint32_t)r * (uint32_t)sizeof(T);
   KsAcc acc{0.0, 0.0};
   constexpr int AUX = NT ? 2 : 0;
-  if (sizeof(R) == 4 && !VV) {
+  if (sizeof(R) == 4 && !VV && MODE != MODE_LAST) {
     ks_group32<KS_UNI, U, PIPE>(meta32, k0, km, r8, xr, vr, acc);
     ks_group32<KS_SCA, U, PIPE, AUX>(meta32, km, kc, r8, xr, sr, acc);
     ks_group32<KS_CPX, U, PIPE, AUX>(meta32, kc, kend, r8, xr, vr, acc);
@@ -534,7 +538,7 @@ __global__ void __launch_bounds__(256) k_ks_stage(
       const double c1 = 2.0 / 9.0 - 7.0 / 24.0, c2 = 1.0 / 3.0 - 1.0 / 4.0, c3 = 4.0 / 9.0 - 1.0 / 3.0,
                    c4 = -1.0 / 8.0;
       const T a = k1[r], bq = k2[r], cq = k3[r], xo = x[r], xn = xin[r];
-      const double hh = (double)h;
+      const double hh = h;
       const double er = hh * (c1 * a.x + c2 * bq.x + c3 * cq.x + c4 * are);
       const double ei = hh * (c1 * a.y + c2 * bq.y + c3 * cq.y + c4 * aim);
       const double ax = sqrt((double)xo.x * xo.x + (double)xo.y * xo.y);
@@ -563,7 +567,7 @@ __global__ void __launch_bounds__(256) k_ks_stage(
     // Bogacki-Shampine stage 3: k3 = A Y3 and x_n = x + h (2/9 k1 + 1/3 k2 + 4/9 k3)
     kout[r] = y;
     const T xo = x[r], a = k1[r], bq = k2[r];
-    const double hh = (double)h;
+    const double hh = h;
     T o;
     o.x = (R)((double)xo.x + hh * (2.0 / 9.0) * a.x + hh / 3.0 * bq.x + hh * (4.0 / 9.0) * are);
     o.y = (R)((double)xo.y + hh * (2.0 / 9.0) * a.y + hh / 3.0 * bq.y + hh * (4.0 / 9.0) * aim);
@@ -571,6 +575,22 @@ __global__ void __launch_bounds__(256) k_ks_stage(
     return;
   }
   const T xo = ld_nt<NT, R>(x, r);
+  if constexpr (MODE == MODE_AXPY || MODE == MODE_LAST) {
+    double xr = (double)xo.x, xi = (double)xo.y;
+    if (sizeof(R) == 4 && xlo) {
+      const float2 lo = ld_nt<NT, float>(xlo, r);
+      xr += (double)lo.x;
+      xi += (double)lo.y;
+    }
+    const double nr = xr + cn * are, ni = xi + cn * aim;
+    T o;
+    o.x = (R)nr;
+    o.y = (R)ni;
+    ynext[r] = o;
+    if (MODE == MODE_LAST)
+      st_nt<NT, float>(xlo, r, make_float2((float)(nr - (double)o.x), (float)(ni - (double)o.y)));
+    return;
+  }
   if (MODE == MODE_STAGE) {
     st_nt<NT, R>(kout, r, y);
     T yn;
@@ -580,8 +600,8 @@ __global__ void __launch_bounds__(256) k_ks_stage(
     } else {
       // the complex64 stage input does not need the low word of the state (it
       // would change it by at most one rounding); stage 4 uses both words
-      yn.x = (R)((double)xo.x + (double)cn * are);
-      yn.y = (R)((double)xo.y + (double)cn * aim);
+      yn.x = (R)((double)xo.x + cn * are);
+      yn.y = (R)((double)xo.y + cn * aim);
     }
     ynext[r] = yn;
     return;
@@ -597,7 +617,7 @@ __global__ void __launch_bounds__(256) k_ks_stage(
     xout[r] = o;
   } else {
     // x' = hi + lo + d in FP64, split again into (hi', lo')
-    const double s6 = (double)h * (1.0 / 6.0), s3 = (double)h * (1.0 / 3.0);
+    const double s6 = h * (1.0 / 6.0), s3 = h * (1.0 / 3.0);
     const double dre = s6 * (double)a.x + s3 * (double)bq.x + s3 * (double)cq.x + s6 * are;
     const double dim = s6 * (double)a.y + s3 * (double)bq.y + s3 * (double)cq.y + s6 * aim;
     const float2 lo = ld_nt<NT, float>(xlo, r);
@@ -877,8 +897,8 @@ int ks_make_fp32(qh_mat *A) {
 
 // launch the sliced-layout kernel with the slot unroll encoded in the variant code G
 template <typename R, int MODE>
-int launch_ks(int G, hipStream_t s, const qh_mat *A, const void *xin, void *kout, void *ynext, R cn, const void *x,
-              const void *k1, const void *k2, const void *k3, void *xout, R h, float2 *xlo, double atol = 0.0,
+int launch_ks(int G, hipStream_t s, const qh_mat *A, const void *xin, void *kout, void *ynext, double cn,
+              const void *x, const void *k1, const void *k2, const void *k3, void *xout, double h, float2 *xlo, double atol = 0.0,
               double rtol = 0.0, double *eacc = nullptr, const qh_td_ell *td = nullptr) {
   typedef typename C2<R>::T T;
   const T *kv = sizeof(R) == 8 ? (const T *)A->ks_val : (const T *)A->ks_val32;
@@ -930,37 +950,35 @@ int launch_ks(int G, hipStream_t s, const qh_mat *A, const void *xin, void *kout
 
 // a stage on either sliced layout (the row-pair one is FP32 only)
 template <typename R, int MODE>
-int launch_sliced(int G, hipStream_t s, const qh_mat *A, const void *xin, void *kout, void *ynext, R cn,
-                  const void *x, const void *k1, const void *k2, const void *k3, void *xout, R h, float2 *xlo) {
+int launch_sliced(int G, hipStream_t s, const qh_mat *A, const void *xin, void *kout, void *ynext, double cn,
+                  const void *x, const void *k1, const void *k2, const void *k3, void *xout, double h, float2 *xlo) {
   if (QH_IS_KS2(G)) {
     if (sizeof(R) != 4) {
       qh_set_error("the row-pair sliced layout (variant %d) is FP32 only", G);
       return QH_EINVAL;
     }
-    return ks2_launch(G, MODE, s, A, xin, kout, ynext, (float)cn, x, k1, k2, k3, xout, (float)h, xlo);
+    return ks2_launch(G, MODE, s, A, xin, kout, ynext, cn, x, k1, k2, k3, xout, h, xlo);
   }
   return launch_ks<R, MODE>(G, s, A, xin, kout, ynext, cn, x, k1, k2, k3, xout, h, xlo);
 }
 
+// one launch of the CSR kernel (G lanes per row) or, for MODE_SPMV, MODE_AXPY and
+// MODE_LAST, of the sliced-layout kernel that variant G names: out = A xin or
+// out = x + c A xin
 template <typename R, int MODE>
-int launch_stage_g(int G, hipStream_t s, const qh_mat *A, const typename C2<R>::T *val, const void *x,
-                   const void *kin, R ck, void *kout, const void *k1, const void *k2, const void *k3, void *xout,
-                   R h, float2 *xlo) {
+int launch_stage(int G, hipStream_t s, const qh_mat *A, const void *xin, void *out, const void *x, double c,
+                 float2 *xlo) {
+  static_assert(MODE == MODE_SPMV || MODE == MODE_AXPY || (MODE == MODE_LAST && sizeof(R) == 4), "stage form");
   typedef typename C2<R>::T T;
   const int32_t n = (int32_t)A->rows;
-  if (QH_IS_KSELL(G) || QH_IS_KS2(G)) {  // plain y = A x on a sliced layout (stages go through launch_sliced)
-    if (MODE != MODE_SPMV) {
-      qh_set_error("sliced-layout stages go through launch_sliced");
-      return QH_EINVAL;
-    }
-    return launch_sliced<R, MODE_SPMV>(G, s, A, x, kout, nullptr, (R)0, nullptr, nullptr, nullptr, nullptr, nullptr,
-                                       (R)0, nullptr);
-  }
+  if (QH_IS_KSELL(G) || QH_IS_KS2(G))
+    return launch_sliced<R, MODE>(G, s, A, xin, MODE == MODE_SPMV ? out : nullptr, MODE == MODE_SPMV ? nullptr : out,
+                                  c, x, nullptr, nullptr, nullptr, nullptr, 0.0, xlo);
+  const T *val = sizeof(R) == 8 ? (const T *)A->val : (const T *)A->val32;
   const unsigned grid = qh_blocks((int64_t)n * G, 256);
-#define QH_L(GG)                                                                                                 \
-  hipLaunchKernelGGL((k_rk_stage<R, GG, MODE>), dim3(grid), dim3(256), 0, s, n, A->rowptr, A->col, val,          \
-                     (const T *)x, (const T *)kin, ck, (T *)kout, (const T *)k1, (const T *)k2, (const T *)k3,   \
-                     (T *)xout, h, xlo)
+#define QH_L(GG)                                                                                              \
+  hipLaunchKernelGGL((k_rk_stage<R, GG, MODE>), dim3(grid), dim3(256), 0, s, n, A->rowptr, A->col, val, A->val, \
+                     (const T *)xin, (T *)out, (const T *)x, c, xlo)
   switch (G) {
     case 1: QH_L(1); break;
     case 2: QH_L(2); break;
@@ -977,30 +995,50 @@ int launch_stage_g(int G, hipStream_t s, const qh_mat *A, const typename C2<R>::
   return QH_OK;
 }
 
+// One RK4 step of size h of x (and, FP32, its low word xlo) in place, launched on
+// stream s; ya, yb: work vectors.  ev (may be null): five events around the four
+// launches.
+template <typename R>
+int rk4_step(hipStream_t s, const qh_mat *A, int G, void *x, float2 *xlo, void *ya, void *yb, double h,
+             hipEvent_t *ev) {
+  const void *ins[4] = {x, ya, yb, ya};
+  void *outs[4] = {ya, yb, ya, x};
+  const double c[4] = {h / 4.0, h / 3.0, h / 2.0, h};
+  int rc = QH_OK;
+  for (int st = 0; st < 4 && !rc; st++) {
+    if (ev) QH_HIP(hipEventRecord(ev[st], s));
+    if constexpr (sizeof(R) == 4) {
+      if (st == 3)
+        rc = launch_stage<R, MODE_LAST>(G, s, A, ins[st], outs[st], x, c[st], xlo);
+      else
+        rc = launch_stage<R, MODE_AXPY>(G, s, A, ins[st], outs[st], x, c[st], st == 2 ? xlo : nullptr);
+    } else {
+      rc = launch_stage<R, MODE_AXPY>(G, s, A, ins[st], outs[st], x, c[st], nullptr);
+    }
+  }
+  if (ev) QH_HIP(hipEventRecord(ev[4], s));
+  return rc;
+}
+
 // ------------------------------------------------------------ autotuner
 // Time each variant (CSR lanes per row, sliced layouts) on the real matrix with
-// one plain SpMV launch plus one RK stage launch (the stage epilogue's vector
-// traffic and registers are part of what the stepping runs) and keep the fastest.
+// whole RK4 steps (the stage epilogues' vector traffic and registers are part of
+// what the stepping runs) and keep the fastest.
 template <typename R>
 int autotune(qh_mat *A, int *out_g) {
   typedef typename C2<R>::T T;
-  const typename C2<R>::T *val = sizeof(R) == 8 ? (const T *)A->val : (const T *)A->val32;
-  // the buffers of one RK4 step: state, K1..K3, the two stage inputs, the new state
-  void *x = nullptr, *kk[3] = {nullptr, nullptr, nullptr}, *ya = nullptr, *yb = nullptr, *xb = nullptr;
+  // the buffers of one RK4 step: the state and the two stage vectors
+  void *x = nullptr, *ya = nullptr, *yb = nullptr;
   float2 *lo = nullptr;
   const size_t vb = (size_t)A->rows * sizeof(T);
   int rc = qh_alloc(&x, vb);
-  for (int i = 0; i < 3 && !rc; i++) rc = qh_alloc(&kk[i], vb);
   if (!rc) rc = qh_alloc(&ya, vb);
   if (!rc) rc = qh_alloc(&yb, vb);
-  if (!rc) rc = qh_alloc(&xb, vb);
   if (!rc && sizeof(R) == 4) rc = qh_alloc_t(&lo, (size_t)A->rows);
   auto release = [&]() {
     qh_free_ptr(x);
-    for (void *p : kk) qh_free_ptr(p);
     qh_free_ptr(ya);
     qh_free_ptr(yb);
-    qh_free_ptr(xb);
     qh_free_ptr(lo);
   };
   if (rc) {
@@ -1010,29 +1048,8 @@ int autotune(qh_mat *A, int *out_g) {
   hipStream_t s = qh_stream();
   QH_HIP(hipMemsetAsync(x, 0, vb, s));
   if (lo) QH_HIP(hipMemsetAsync(lo, 0, (size_t)A->rows * sizeof(float2), s));
-  // one whole RK4 step with the launch sequence of rk4_step (three stage
-  // launches and the final one; the final stage moves the most data), so the
-  // choice reflects the mix a step runs
-  const R h = (R)0.01;
-  auto run = [&](int g) {
-    if (QH_IS_KSELL(g) || QH_IS_KS2(g)) {
-      const void *ins[4] = {x, ya, yb, ya};
-      void *outs[3] = {ya, yb, ya};
-      const R cns[3] = {h / 2, h / 2, h};
-      for (int st = 0; st < 3; st++)
-        launch_sliced<R, MODE_STAGE>(g, s, A, ins[st], kk[st], outs[st], cns[st], x, nullptr, nullptr, nullptr,
-                                     nullptr, h, lo);
-      launch_sliced<R, MODE_FINAL>(g, s, A, ins[3], nullptr, nullptr, (R)0, x, kk[0], kk[1], kk[2], xb, h, lo);
-    } else {
-      launch_stage_g<R, MODE_SPMV>(g, s, A, val, x, nullptr, (R)0, kk[0], nullptr, nullptr, nullptr, nullptr, h,
-                                   lo);
-      launch_stage_g<R, MODE_STAGE>(g, s, A, val, x, kk[0], h / 2, kk[1], nullptr, nullptr, nullptr, nullptr, h,
-                                    lo);
-      launch_stage_g<R, MODE_STAGE>(g, s, A, val, x, kk[1], h / 2, kk[2], nullptr, nullptr, nullptr, nullptr, h,
-                                    lo);
-      launch_stage_g<R, MODE_FINAL>(g, s, A, val, x, kk[2], h, nullptr, kk[0], kk[1], kk[2], xb, h, lo);
-    }
-  };
+  // one whole RK4 step, so the choice reflects the mix a step runs
+  auto run = [&](int g) { rk4_step<R>(s, A, g, x, lo, ya, yb, 0.01, nullptr); };
   hipEvent_t e0, e1;
   QH_HIP(hipEventCreate(&e0));
   QH_HIP(hipEventCreate(&e1));
@@ -1186,9 +1203,7 @@ struct Stepper {
   uint64_t Auid = 0;  // A's serial number: a new matrix may reuse a destroyed one's address
   int prec = 0;
   int64_t n = 0;
-  void *k[3] = {nullptr, nullptr, nullptr};
-  void *y[2] = {nullptr, nullptr};  // materialised stage inputs (sliced-layout path)
-  void *xalt = nullptr;  // double buffer for the state (hi part for FP32)
+  void *y[2] = {nullptr, nullptr};  // stage vectors
   double *partial = nullptr, *inv = nullptr;
   hipGraphExec_t exec = nullptr;
   hipGraph_t graph = nullptr;
@@ -1208,25 +1223,20 @@ static int64_t g_last_launches = 0;
 static void stepper_release() {
   if (g_st.exec) (void)hipGraphExecDestroy(g_st.exec);
   if (g_st.graph) (void)hipGraphDestroy(g_st.graph);
-  for (auto &p : g_st.k) qh_free_ptr(p);
   for (auto &p : g_st.y) qh_free_ptr(p);
-  qh_free_ptr(g_st.xalt);
   qh_free_ptr(g_st.partial);
   qh_free_ptr(g_st.inv);
   g_st = Stepper();
 }
 
 static int stepper_prepare(const qh_mat *A, int prec, int64_t n) {
-  if (g_st.A == A && g_st.Auid == A->uid && g_st.prec == prec && g_st.n == n && g_st.k[0]) return QH_OK;
+  if (g_st.A == A && g_st.Auid == A->uid && g_st.prec == prec && g_st.n == n && g_st.y[0]) return QH_OK;
   (void)hipStreamSynchronize(qh_stream());
   stepper_release();
   size_t es = prec == QH_FP64 ? 16 : 8;
   int rc = QH_OK;
-  for (auto &p : g_st.k)
-    if (!rc) rc = qh_alloc(&p, (size_t)n * es);
   for (auto &p : g_st.y)
     if (!rc) rc = qh_alloc(&p, (size_t)n * es);
-  if (!rc) rc = qh_alloc(&g_st.xalt, (size_t)n * es);
   if (!rc) rc = qh_alloc_t(&g_st.partial, 1024);
   if (!rc) rc = qh_alloc_t(&g_st.inv, 1);
   if (rc) {
@@ -1240,47 +1250,10 @@ static int stepper_prepare(const qh_mat *A, int prec, int64_t n) {
   return QH_OK;
 }
 
-// one RK4 step from xa into xb (xb != xa), launched on stream s
-template <typename R>
-static int rk4_step(hipStream_t s, const qh_mat *A, int G, const void *xa, void *xb, float2 *xlo, R h,
-                    hipEvent_t *ev) {
-  typedef typename C2<R>::T T;
-  const T *val = sizeof(R) == 8 ? (const T *)A->val : (const T *)A->val32;
-  void **k = g_st.k;
-  int rc;
-  if (QH_IS_KSELL(G) || QH_IS_KS2(G)) {
-    // stage inputs materialised in the epilogues: x -> Ya -> Yb -> Ya
-    void *Ya = g_st.y[0], *Yb = g_st.y[1];
-    const void *ins[4] = {xa, Ya, Yb, Ya};
-    void *outs[3] = {Ya, Yb, Ya};
-    const R cns[3] = {h / 2, h / 2, h};
-    for (int st = 0; st < 3; st++) {
-      if (ev) QH_HIP(hipEventRecord(ev[st], s));
-      rc = launch_sliced<R, MODE_STAGE>(G, s, A, ins[st], k[st], outs[st], cns[st], xa, nullptr, nullptr, nullptr,
-                                        nullptr, h, xlo);
-      if (rc) return rc;
-    }
-    if (ev) QH_HIP(hipEventRecord(ev[3], s));
-    rc = launch_sliced<R, MODE_FINAL>(G, s, A, ins[3], nullptr, nullptr, (R)0, xa, k[0], k[1], k[2], xb, h, xlo);
-    if (ev) QH_HIP(hipEventRecord(ev[4], s));
-    return rc;
-  }
-  if (ev) QH_HIP(hipEventRecord(ev[0], s));
-  rc = launch_stage_g<R, MODE_SPMV>(G, s, A, val, xa, nullptr, (R)0, k[0], nullptr, nullptr, nullptr, nullptr, h,
-                                    xlo);
-  if (ev) QH_HIP(hipEventRecord(ev[1], s));
-  if (!rc)
-    rc = launch_stage_g<R, MODE_STAGE>(G, s, A, val, xa, k[0], h / 2, k[1], nullptr, nullptr, nullptr, nullptr, h,
-                                       xlo);
-  if (ev) QH_HIP(hipEventRecord(ev[2], s));
-  if (!rc)
-    rc = launch_stage_g<R, MODE_STAGE>(G, s, A, val, xa, k[1], h / 2, k[2], nullptr, nullptr, nullptr, nullptr, h,
-                                       xlo);
-  if (ev) QH_HIP(hipEventRecord(ev[3], s));
-  if (!rc)
-    rc = launch_stage_g<R, MODE_FINAL>(G, s, A, val, xa, k[2], h, nullptr, k[0], k[1], k[2], xb, h, xlo);
-  if (ev) QH_HIP(hipEventRecord(ev[4], s));
-  return rc;
+// one RK4 step of x in place with the stepper's stage vectors
+static int step_x(hipStream_t s, const qh_mat *A, int G, qh_vec *x, double h, hipEvent_t *ev) {
+  return x->prec == QH_FP64 ? rk4_step<double>(s, A, G, x->d, nullptr, g_st.y[0], g_st.y[1], h, ev)
+                            : rk4_step<float>(s, A, G, x->d, x->lo, g_st.y[0], g_st.y[1], h, ev);
 }
 
 static int renorm_launch(hipStream_t s, qh_vec *x, void *hi, int64_t tot, int64_t base) {
@@ -1306,8 +1279,6 @@ extern "C" int qh_last_stage_ms(double *spmv_ms, int64_t *launches) {
   return QH_OK;
 }
 
-// Advance x in place by nsteps RK4 steps.  Steps are grouped in pairs (x -> alt
-// -> x) so a captured graph always starts and ends on the caller's buffer.
 // ------------------------------------------------ small systems in one workgroup
 // For a generator of at most QH_SMALL_ROWS rows the whole RK4 integration runs
 // in one workgroup with the state and the three stage vectors in LDS (5 x 16 B
@@ -1688,23 +1659,18 @@ static int rk4_small(qh_mat *A, qh_vec *x, double dt, int64_t nsteps, int64_t to
   return QH_OK;
 }
 
-// steps per captured graph: pairs of steps (the state ping-pongs back into the
-// caller's buffer), exactly renorm_every (rounded up to a pair) when the trace
-// is renormalised
-static int graph_pair_steps(int renorm_every) {
-  int pair_steps = g_graph_steps & ~1;
-  if (pair_steps < 2) pair_steps = 2;
-  if (renorm_every > 0) pair_steps = renorm_every + (renorm_every & 1);
-  return pair_steps;
+// steps per captured graph: renorm_every (rounded up to an even number) when the
+// trace is renormalised
+static int graph_len(int renorm_every) {
+  return renorm_every > 0 ? renorm_every + (renorm_every & 1) : g_graph_steps;
 }
 
-// capture and instantiate the graph of pair_steps steps of x under A, unless the
-// one held was captured with the same parameters
-static int graph_prepare(const qh_mat *A, qh_vec *x, double dt, int64_t tot, int renorm_every, int G,
-                         int pair_steps) {
+// capture and instantiate the graph of len steps of x under A, unless the one
+// held was captured with the same parameters
+static int graph_prepare(const qh_mat *A, qh_vec *x, double dt, int64_t tot, int renorm_every, int G, int len) {
   hipStream_t s = qh_stream();
   const bool recapture = !g_st.exec || g_st.gx != x->d || g_st.glo != x->lo || g_st.gdt != dt ||
-                         g_st.gsteps != pair_steps || g_st.grenorm != renorm_every || g_st.gG != G ||
+                         g_st.gsteps != len || g_st.grenorm != renorm_every || g_st.gG != G ||
                          g_st.gtot != tot;
   if (!recapture) return QH_OK;
   if (g_st.exec) (void)hipGraphExecDestroy(g_st.exec);
@@ -1713,11 +1679,7 @@ static int graph_prepare(const qh_mat *A, qh_vec *x, double dt, int64_t tot, int
   g_st.graph = nullptr;
   QH_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
   int crc = QH_OK;
-  for (int st = 0; st < pair_steps && !crc; st++) {
-    void *xa = (st & 1) ? g_st.xalt : x->d, *xb = (st & 1) ? x->d : g_st.xalt;
-    crc = x->prec == QH_FP64 ? rk4_step<double>(s, A, G, xa, xb, x->lo, dt, nullptr)
-                             : rk4_step<float>(s, A, G, xa, xb, x->lo, (float)dt, nullptr);
-  }
+  for (int st = 0; st < len && !crc; st++) crc = step_x(s, A, G, x, dt, nullptr);
   if (!crc && renorm_every > 0) crc = renorm_launch(s, x, x->d, tot, 0);
   hipGraph_t g = nullptr;
   hipError_t ce = hipStreamEndCapture(s, &g);
@@ -1731,7 +1693,7 @@ static int graph_prepare(const qh_mat *A, qh_vec *x, double dt, int64_t tot, int
   g_st.gx = x->d;
   g_st.glo = x->lo;
   g_st.gdt = dt;
-  g_st.gsteps = pair_steps;
+  g_st.gsteps = len;
   g_st.grenorm = renorm_every;
   g_st.gG = G;
   g_st.gtot = tot;
@@ -1763,16 +1725,11 @@ static int rk4_impl(qh_mat *A, qh_vec *x, double dt, int64_t nsteps, int64_t tot
     // eager launches with events around every stage kernel: per-launch durations
     std::vector<hipEvent_t> ev(5 * nsteps);
     for (auto &e : ev) QH_HIP(hipEventCreate(&e));
-    void *bufs[2] = {x->d, g_st.xalt};
     for (int64_t st = 0; st < nsteps; st++) {
-      void *xa = bufs[st & 1], *xb = bufs[(st + 1) & 1];
-      rc = x->prec == QH_FP64 ? rk4_step<double>(s, A, G, xa, xb, x->lo, dt, &ev[5 * st])
-                              : rk4_step<float>(s, A, G, xa, xb, x->lo, (float)dt, &ev[5 * st]);
+      rc = step_x(s, A, G, x, dt, &ev[5 * st]);
       if (rc) return rc;
-      if (renorm_every > 0 && (st + 1) % renorm_every == 0) renorm_launch(s, x, xb, tot, 0);
+      if (renorm_every > 0 && (st + 1) % renorm_every == 0) renorm_launch(s, x, x->d, tot, 0);
     }
-    if (nsteps & 1) QH_HIP(hipMemcpyAsync(x->d, g_st.xalt, x->n * (x->prec == QH_FP64 ? 16 : 8),
-                                          hipMemcpyDeviceToDevice, s));
     QH_HIP(hipStreamSynchronize(s));
     double tot_ms = 0.0;
     for (int64_t st = 0; st < nsteps; st++)
@@ -1787,24 +1744,20 @@ static int rk4_impl(qh_mat *A, qh_vec *x, double dt, int64_t nsteps, int64_t tot
     return QH_OK;
   }
 
-  // graph path: capture 2*P steps (P pairs) once, replay
-  const int pair_steps = graph_pair_steps(renorm_every);
-  const int64_t full = nsteps / pair_steps;
+  // graph path: capture len steps once, replay
+  const int len = graph_len(renorm_every);
+  const int64_t full = nsteps / len;
   if (full > 0) {
-    rc = graph_prepare(A, x, dt, tot, renorm_every, G, pair_steps);
+    rc = graph_prepare(A, x, dt, tot, renorm_every, G, len);
     if (rc) return rc;
     for (int64_t r = 0; r < full; r++) QH_HIP(hipGraphLaunch(g_st.exec, s));
   }
   // remainder: eager launches
-  const int64_t rem = nsteps - full * pair_steps;
+  const int64_t rem = nsteps - full * len;
   for (int64_t st = 0; st < rem; st++) {
-    void *xa = (st & 1) ? g_st.xalt : x->d, *xb = (st & 1) ? x->d : g_st.xalt;
-    rc = x->prec == QH_FP64 ? rk4_step<double>(s, A, G, xa, xb, x->lo, dt, nullptr)
-                            : rk4_step<float>(s, A, G, xa, xb, x->lo, (float)dt, nullptr);
+    rc = step_x(s, A, G, x, dt, nullptr);
     if (rc) return rc;
   }
-  if (rem & 1)
-    QH_HIP(hipMemcpyAsync(x->d, g_st.xalt, x->n * (x->prec == QH_FP64 ? 16 : 8), hipMemcpyDeviceToDevice, s));
   QH_HIP(hipGetLastError());
   return QH_OK;
 }
@@ -1831,7 +1784,7 @@ extern "C" int qh_rk4_prepare(qh_mat *A, qh_vec *x, double dt, int64_t tot, int 
   int G = 0;
   rc = lanes_for(A, x->prec, &G);
   if (!rc) rc = stepper_prepare(A, x->prec, x->n);
-  if (!rc) rc = graph_prepare(A, x, dt, tot, renorm_every, G, graph_pair_steps(renorm_every));
+  if (!rc) rc = graph_prepare(A, x, dt, tot, renorm_every, G, graph_len(renorm_every));
   if (!rc) QH_HIP(hipStreamSynchronize(qh_stream()));
   return rc;
 }
@@ -1914,10 +1867,8 @@ extern "C" int qh_bench_spmv(qh_mat *A, int prec, int reps, double *avg_ms) {
   for (auto &e : ev) QH_HIP(hipEventCreate(&e));
   for (int r = 0; r < reps && !rc; r++) {
     QH_HIP(hipEventRecord(ev[r], s));
-    rc = prec == QH_FP64 ? launch_stage_g<double, MODE_SPMV>(G, s, A, A->val, x, nullptr, 0.0, y, nullptr, nullptr,
-                                                             nullptr, nullptr, 0.0, nullptr)
-                         : launch_stage_g<float, MODE_SPMV>(G, s, A, A->val32, x, nullptr, 0.f, y, nullptr, nullptr,
-                                                            nullptr, nullptr, 0.f, nullptr);
+    rc = prec == QH_FP64 ? launch_stage<double, MODE_SPMV>(G, s, A, x, y, nullptr, 0.0, nullptr)
+                         : launch_stage<float, MODE_SPMV>(G, s, A, x, y, nullptr, 0.0, nullptr);
   }
   QH_HIP(hipEventRecord(ev[reps], s));
   QH_HIP(hipEventSynchronize(ev[reps]));
@@ -1943,11 +1894,9 @@ extern "C" int qh_spmv(const qh_mat *A_, const qh_vec *x, qh_vec *y) {
   if (rc) return rc;
   hipStream_t s = qh_stream();
   if (x->prec == QH_FP64)
-    rc = launch_stage_g<double, MODE_SPMV>(G, s, A, A->val, x->d, nullptr, 0.0, y->d, nullptr, nullptr, nullptr,
-                                           nullptr, 0.0, nullptr);
+    rc = launch_stage<double, MODE_SPMV>(G, s, A, x->d, y->d, nullptr, 0.0, nullptr);
   else {
-    rc = launch_stage_g<float, MODE_SPMV>(G, s, A, A->val32, x->d, nullptr, 0.f, y->d, nullptr, nullptr, nullptr,
-                                          nullptr, 0.f, nullptr);
+    rc = launch_stage<float, MODE_SPMV>(G, s, A, x->d, y->d, nullptr, 0.0, nullptr);
     if (!rc) QH_HIP(hipMemsetAsync(y->lo, 0, (size_t)y->n * 8, s));
   }
   QH_HIP(hipGetLastError());
@@ -2369,11 +2318,11 @@ int qh_td_sliced_stage(int G, const qh_mat *A, int prec, int mode, const void *x
   int rc;
   if (td && prec == QH_FP32 && (G == 140 || G == 142 || G == 143) && A->ks2_state == 1) {
     *fused = 1;
-    rc = ks2_launch(G, mode, s, A, xin, kout, ynext, (float)cn, x, k1, k2, k3, xout, (float)h, xlo, td);
+    rc = ks2_launch(G, mode, s, A, xin, kout, ynext, cn, x, k1, k2, k3, xout, h, xlo, td);
   } else if (td && (G == 128 || G == 134 || G == 136) && A->ks_state == 1) {
     *fused = 1;
 #define QH_TF(R, M) \
-  launch_ks<R, M>(G, s, A, xin, kout, ynext, (R)cn, x, k1, k2, k3, xout, (R)h, xlo, 0.0, 0.0, nullptr, td)
+  launch_ks<R, M>(G, s, A, xin, kout, ynext, cn, x, k1, k2, k3, xout, h, xlo, 0.0, 0.0, nullptr, td)
     if (prec == QH_FP64)
       rc = mode == MODE_SPMV ? QH_TF(double, MODE_SPMV) : mode == MODE_STAGE ? QH_TF(double, MODE_STAGE)
                                                                             : QH_TF(double, MODE_FINAL);
@@ -2383,7 +2332,7 @@ int qh_td_sliced_stage(int G, const qh_mat *A, int prec, int mode, const void *x
 #undef QH_TF
   } else {
 #define QH_TS(R, M) \
-  launch_sliced<R, M>(G, s, A, xin, kout, ynext, (R)cn, x, k1, k2, k3, xout, (R)h, xlo)
+  launch_sliced<R, M>(G, s, A, xin, kout, ynext, cn, x, k1, k2, k3, xout, h, xlo)
     if (prec == QH_FP64)
       rc = mode == MODE_SPMV ? QH_TS(double, MODE_SPMV) : mode == MODE_STAGE ? QH_TS(double, MODE_STAGE)
                                                                             : QH_TS(double, MODE_FINAL);
