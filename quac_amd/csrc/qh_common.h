@@ -128,6 +128,7 @@ struct qh_mat {
   float *ks_sval32 = nullptr;
   qh_kmeta32 *ks_meta32 = nullptr;  // FP32 metadata (ks_slots + QH_KS_PAD entries)
   int64_t ks_slots = 0;
+  int32_t ks_maxslots = 0;     // most slots of a slice
   int64_t ks_nval = 0;         // stored complex values
   int64_t ks_nsval = 0;        // stored scalar values
   // FP32 row-pair sliced layout (built on demand from the CSR)
@@ -147,6 +148,7 @@ struct qh_mat {
   int32_t *ks2_xmid = nullptr;  // end of each slice's complex slots (separable-diagonal slots follow)
   qh_sepblk *ks2_sep = nullptr; // blocks with a separable diagonal
   double2 *ks2_gh = nullptr;    // their g and h vectors
+  int32_t ks2_maxslots = 0;    // most slots of a slice
   int64_t ks2_slots = 0, ks2_nval = 0, ks2_nsval = 0, ks2_nsval1 = 0, ks2_nsep = 0, ks2_ngh = 0, ks2_nsepblk = 0;
   std::vector<int64_t> blk_off;  // row offsets of the blocks of a block-diagonal matrix (and its row count)
   qh_td_cache *td_cache = nullptr;  // built by the first time-dependent RHS on this matrix
@@ -154,7 +156,8 @@ struct qh_mat {
 // variant codes selecting the sliced-ELL kernel: 128 / 129 / 130 process 2 / 4 / 8
 // slots per pass; 131 / 132 process 4 / 8 slots per pass and read the uniform
 // slot values with vector loads; 133 / 134 process 2 / 4 slots per pass with the
-// loads of the next pass in flight during the products of the current one
+// loads of the next pass in flight during the products of the current one and the
+// slice's metadata in registers (slices of at most 64 slots)
 #define QH_KSELL 128
 // 135 / 136: 129 / 131 with the streamed data under the non-temporal cache policy
 #define QH_IS_KSELL(g) ((g) >= 128 && (g) <= 136)

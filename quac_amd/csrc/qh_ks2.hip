@@ -329,14 +329,14 @@ __device__ __forceinline__ void ks2_flush(KsAcc2 &acc) {
 
 // INORDER: every slot of the group has row 2l on half 0 and row 2l+1 on half 1
 // (known at compile time, no selects)
-template <int KIND, bool D, bool INORDER = false, int AUX = 0>
+template <int KIND, bool D, bool RL, bool INORDER = false, int AUX = 0>
 struct Ks2Ops {
   typedef KsAcc2 Acc;
   typedef typename Ks2Meta<D>::M Meta;
   typedef typename Ks2Meta<D>::U U;
   template <int W>
   using Buf = Ks2Buf<KIND, W, D>;
-  const Meta *mp;
+  KsSrc<Meta, RL> src;
   uint32_t r8;  // byte offset of x[2l] within the stage input
   __amdgpu_buffer_rsrc_t xr, vr;
   template <int W>
@@ -344,7 +344,7 @@ struct Ks2Ops {
     Meta m[W];
 #pragma unroll
     for (int j = 0; j < W; j++) {
-      m[j] = mp[j];
+      m[j] = src.get(j);
       b.h[j] = m[j].ad8 & 3u;
       b.u0r[j] = m[j].v0re;
       b.u0i[j] = m[j].v0im;
@@ -373,7 +373,7 @@ struct Ks2Ops {
               __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(vr, (m[j].base + rank) * 16u, 0, AUX));
       }
     }
-    mp += W;
+    src.skip(W);
   }
   template <int W>
   __device__ __forceinline__ void fma(const Buf<W> &b, Acc &acc) {
@@ -422,13 +422,13 @@ struct Ks2Ops {
 // In-order uniform slots whose loads all stay inside the workgroup's window of
 // KS2_WIN rows: the pair is read from the LDS copy of the window (xs, KS2_WIN + 2
 // complex64, the last two zero for inactive lanes) instead of global memory.
-template <bool D>
+template <bool D, bool RL>
 struct Ks2OpsWin {
   typedef KsAcc2 Acc;
   typedef typename Ks2Meta<D>::M Meta;
   template <int W>
   using Buf = Ks2Buf<KS_UNI, W, D>;
-  const Meta *mp;
+  KsSrc<Meta, RL> src;
   uint32_t w8;  // byte offset of row 2l within the window
   const float2 *xs;
   template <int W>
@@ -436,7 +436,7 @@ struct Ks2OpsWin {
     Meta m[W];
 #pragma unroll
     for (int j = 0; j < W; j++) {
-      m[j] = mp[j];
+      m[j] = src.get(j);
       b.h[j] = 0u;
       b.u0r[j] = m[j].v0re;
       b.u0i[j] = m[j].v0im;
@@ -455,11 +455,13 @@ struct Ks2OpsWin {
       const float2 lo = q[0], hi = q[1];
       b.xv[j] = make_float4(lo.x, lo.y, hi.x, hi.y);
     }
-    mp += W;
+    src.skip(W);
   }
   template <int W>
   __device__ __forceinline__ void fma(const Buf<W> &b, Acc &acc) {
-    Ks2Ops<KS_UNI, D, true>{}.fma(b, acc);
+#pragma unroll
+    for (int j = 0; j < W; j++)
+      ks2_mul<D>(acc, b.u0r[j], b.u0i[j], b.u1r[j], b.u1i[j], b.xv[j].x, b.xv[j].y, b.xv[j].z, b.xv[j].w);
   }
   __device__ __forceinline__ void flush(Acc &acc) { ks2_flush<D>(acc); }
 };
@@ -469,7 +471,7 @@ struct Ks2OpsWin {
 // from the block's g and h (t = 2l - off, j = t / N, i = t - j N; i is even, so
 // i + 1 stays in the column) and, without D, rounded to FP32 as the stored diagonal
 // would be.
-template <bool D>
+template <bool D, bool RL>
 struct Ks2OpsSep {
   typedef KsAcc2 Acc;
   typedef typename Ks2Meta<D>::M Meta;
@@ -479,7 +481,7 @@ struct Ks2OpsSep {
     float4 xv[W];
     double2 g0[W], g1[W], h[W];
   };
-  const Meta *mp;
+  KsSrc<Meta, RL> src;
   uint32_t r8;  // byte offset of x[2l] within the stage input
   int64_t r;    // row 2l
   __amdgpu_buffer_rsrc_t xr, ghr;
@@ -488,7 +490,7 @@ struct Ks2OpsSep {
   __device__ __forceinline__ void issue(Buf<W> &b) {
 #pragma unroll
     for (int j = 0; j < W; j++) {
-      const Meta m = mp[j];
+      const Meta m = src.get(j);
       const bool on = __builtin_amdgcn_inverse_ballot_w64(m.mask);
       b.xv[j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xr, on ? r8 : QH_KS_OOB, 0, 0));
       const qh_sepblk q = bp[m.base];
@@ -500,7 +502,7 @@ struct Ks2OpsSep {
       b.g1[j] = __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(ghr, on ? go + 16u : go, 0, 0));
       b.h[j] = __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(ghr, ho, 0, 0));
     }
-    mp += W;
+    src.skip(W);
   }
   template <int W>
   __device__ __forceinline__ void fma(const Buf<W> &b, Acc &acc) {
@@ -552,7 +554,10 @@ __device__ inline void st_pair(__amdgpu_buffer_rsrc_t rs, uint32_t o, bool two, 
 // TDP: each row also sums its merged A_k entries of a time-dependent RHS (the
 // sliced form over 64-row slices: a lane's two rows are adjacent entries of one
 // slice), before the epilogue
-template <int MODE, int U, bool WIN, bool NT = false, bool SEP = false, bool TDP = false>
+// RL: the slice's metadata held in registers (at most 64 slots); not with WIN, whose
+// 16-wavefront workgroups need the kernel within 64 VGPRs to run two on a CU
+// (10-qubit chain with RL: 68 VGPRs, 23.0 us a launch against 17.1 us)
+template <int MODE, int U, bool WIN, bool NT, bool SEP, bool TDP, bool RL>
 __global__ void __launch_bounds__(WIN ? KS2_WIN / 2 : 256, WIN ? 8 : 1) k_ks2_stage(
     int32_t n, int32_t nslices, const int32_t *__restrict__ moff, const int32_t *__restrict__ wmid,
     const int32_t *__restrict__ smid, const int32_t *__restrict__ umid, const int32_t *__restrict__ emid,
@@ -601,16 +606,24 @@ __global__ void __launch_bounds__(WIN ? KS2_WIN / 2 : 256, WIN ? 8 : 1) k_ks2_st
   constexpr bool D = MODE == MODE_LAST;
   const typename Ks2Meta<D>::M *const meta = (const typename Ks2Meta<D>::M *)metap;
   // (a wavefront past the last slice has empty slot ranges: k0 = ... = kend = 0)
-  ks_run<U, true>(Ks2Ops<KS_UNI, D, true>{meta + kw, r8, xr, vr}, ku - kw, acc);
-  if (!WIN) ks_run<U, true>(Ks2Ops<KS_UNI, D, true>{meta + k0, r8, xr, vr}, kw - k0, acc);
+  KsRegs<typename Ks2Meta<D>::M> regs;
+  if (RL) regs.load(meta + k0, kend - k0, lane);
+  auto src = [&](int32_t k) {
+    if constexpr (RL)
+      return KsSrc<typename Ks2Meta<D>::M, true>{regs, k - k0};
+    else
+      return KsSrc<typename Ks2Meta<D>::M, false>{meta + k};
+  };
+  ks_run<U, true>(Ks2Ops<KS_UNI, D, RL, true>{src(kw), r8, xr, vr}, ku - kw, acc);
+  if (!WIN) ks_run<U, true>(Ks2Ops<KS_UNI, D, RL, true>{src(k0), r8, xr, vr}, kw - k0, acc);
   constexpr int AUX = NT ? 2 : 0;
-  ks_run<U, true>(Ks2Ops<KS_UNI, D>{meta + ku, r8, xr, vr}, km - ku, acc);
-  ks_run<U, true>(Ks2Ops<KS_SCA, D, false, AUX>{meta + km, r8, xr, sr}, ke - km, acc);
-  ks_run<U, true>(Ks2Ops<KS_SC1, D, false, AUX>{meta + ke, r8, xr, s1r}, kc - ke, acc);
-  ks_run<U, true>(Ks2Ops<KS_CPX, D, false, AUX>{meta + kc, r8, xr, vr}, kx - kc, acc);
+  ks_run<U, true>(Ks2Ops<KS_UNI, D, RL>{src(ku), r8, xr, vr}, km - ku, acc);
+  ks_run<U, true>(Ks2Ops<KS_SCA, D, RL, false, AUX>{src(km), r8, xr, sr}, ke - km, acc);
+  ks_run<U, true>(Ks2Ops<KS_SC1, D, RL, false, AUX>{src(ke), r8, xr, s1r}, kc - ke, acc);
+  ks_run<U, true>(Ks2Ops<KS_CPX, D, RL, false, AUX>{src(kc), r8, xr, vr}, kx - kc, acc);
   if (SEP && kend > kx) {  // the one separable-diagonal slot of the slice, after the pipelined groups
-    Ks2OpsSep<D> op{meta + kx, r8, (int64_t)r, xr, ks_rsrc(gh, (int64_t)ngh * 16), sepb};
-    typename Ks2OpsSep<D>::template Buf<1> sb;
+    Ks2OpsSep<D, RL> op{src(kx), r8, (int64_t)r, xr, ks_rsrc(gh, (int64_t)ngh * 16), sepb};
+    typename Ks2OpsSep<D, RL>::template Buf<1> sb;
     op.template issue<1>(sb);
     op.template fma<1>(sb, acc);
     op.flush(acc);
@@ -620,7 +633,7 @@ __global__ void __launch_bounds__(WIN ? KS2_WIN / 2 : 256, WIN ? 8 : 1) k_ks2_st
     xs[2 * threadIdx.x + 1] = make_float2(wv.z, wv.w);
     if (threadIdx.x == 0) xs[KS2_WIN] = xs[KS2_WIN + 1] = make_float2(0.f, 0.f);
     __syncthreads();
-    ks_run<U, true>(Ks2OpsWin<D>{meta + k0, (uint32_t)(r - (int32_t)b * KS2_WIN) * 8u, xs}, kw - k0, acc);
+    ks_run<U, true>(Ks2OpsWin<D, RL>{src(k0), (uint32_t)(r - (int32_t)b * KS2_WIN) * 8u, xs}, kw - k0, acc);
   }
   if (!live) return;
   if (r >= n) return;
@@ -922,7 +935,9 @@ int ks2_build(qh_mat *A) {
   std::vector<int32_t> ho(ns + 1), hv(ns + 1), hso(ns + 1), hs1o(ns + 1), hm(ns), hem(ns), hcm(ns), hsm(ns), hwm(ns),
       hxm(ns);
   int64_t tot = 0, totv = 0, tots = 0, tots1 = 0, totx = 0;
+  int32_t most = 0;
   for (int32_t i = 0; i < ns; i++) {
+    most = std::max(most, hw[i]);
     ho[i] = (int32_t)tot;
     hv[i] = (int32_t)totv;
     hso[i] = (int32_t)tots;
@@ -994,6 +1009,7 @@ int ks2_build(qh_mat *A) {
   cleanup();
   A->ks2_nslices = ns;
   A->ks2_slots = tot;
+  A->ks2_maxslots = most;
   A->ks2_nval = totv;
   A->ks2_nsval = tots;
   A->ks2_nsval1 = tots1;
@@ -1019,8 +1035,8 @@ int ks2_launch(int G, int mode, hipStream_t s, const qh_mat *A, const void *xin,
   const bool win = G == 142 || G == 144;
   const dim3 grid(qh_blocks(ns, win ? KS2_WIN / 128 : 4)), blk(win ? KS2_WIN / 2 : 256);
   const qh_td_ell none{nullptr, nullptr, nullptr, nullptr, nullptr};
-#define QH_LK2T(MM, UU, WW, NN, SS, TT, TD)                                                                      \
-  hipLaunchKernelGGL((k_ks2_stage<MM, UU, WW, NN, SS, TT>), grid, blk, 0, s, n, ns, A->ks2_moff, A->ks2_wmid,       \
+#define QH_LK2T(MM, UU, WW, NN, SS, TT, RR, TD)                                                                      \
+  hipLaunchKernelGGL((k_ks2_stage<MM, UU, WW, NN, SS, TT, RR>), grid, blk, 0, s, n, ns, A->ks2_moff, A->ks2_wmid,       \
                      A->ks2_smid,                                                                                \
                      A->ks2_umid, A->ks2_emid, A->ks2_cmid, A->ks2_xmid, A->ks2_sep,                               \
                      (int32_t)A->ks2_ngh,                                                                        \
@@ -1028,32 +1044,36 @@ int ks2_launch(int G, int mode, hipStream_t s, const qh_mat *A, const void *xin,
                      (int32_t)A->ks2_nsval, A->ks2_sval, (int32_t)A->ks2_nsval1, A->ks2_sval1,                  \
                      (const float2 *)xin, (float2 *)kout, (float2 *)ynext, cn, (const float2 *)x,                \
                      (const float2 *)k1, (const float2 *)k2, (const float2 *)k3, (float2 *)xout, h, xlo, TD)
-#define QH_LK2S(MM, UU, WW, NN, SS) QH_LK2T(MM, UU, WW, NN, SS, false, none)
-#define QH_LK2(MM, UU, WW, NN)            \
+#define QH_LK2S(MM, UU, WW, NN, SS, RR) QH_LK2T(MM, UU, WW, NN, SS, false, RR, none)
+#define QH_LK2(MM, UU, WW, NN, RR)        \
   do {                                    \
     if (A->ks2_nsep)                      \
-      QH_LK2S(MM, UU, WW, NN, true);      \
+      QH_LK2S(MM, UU, WW, NN, true, RR);  \
     else                                  \
-      QH_LK2S(MM, UU, WW, NN, false);     \
+      QH_LK2S(MM, UU, WW, NN, false, RR); \
   } while (0)
   const bool known = mode == MODE_SPMV || mode == MODE_STAGE || mode == MODE_FINAL || mode == MODE_AXPY || mode == MODE_LAST;
   if (!QH_IS_KS2(G) || !known || (td && (mode == MODE_AXPY || mode == MODE_LAST))) {
     qh_set_error("unsupported row-pair variant %d / mode %d", G, mode);
     return QH_EINVAL;
   }
+  // a slice of more than 64 slots: the metadata read from memory slot by slot
+  const int QH_KS2_LONG = 0;
+  if (A->ks2_maxslots > 64 && !win && !(td && G == 141)) G = QH_KS2_LONG;
   if (td) {  // the time-dependent entries summed in the same kernel (variants 140, 142, 143)
-#define QH_LK2D(MM, UU, WW, NN)                                                             \
+#define QH_LK2D(MM, UU, WW, NN, RR)                                                             \
   do {                                                                                      \
     if (A->ks2_nsep)                                                                        \
-      QH_LK2T(MM, UU, WW, NN, true, true, *td);                                            \
+      QH_LK2T(MM, UU, WW, NN, true, true, RR, *td);                                            \
     else                                                                                    \
-      QH_LK2T(MM, UU, WW, NN, false, true, *td);                                           \
+      QH_LK2T(MM, UU, WW, NN, false, true, RR, *td);                                           \
   } while (0)
 #define QH_LK2DG(MM)                                                                        \
   switch (G) {                                                                              \
-    case 140: QH_LK2D(MM, 2, false, false); break;                                          \
-    case 142: QH_LK2D(MM, 2, true, false); break;                                           \
-    case 143: QH_LK2D(MM, 2, false, true); break;                                           \
+    case QH_KS2_LONG: QH_LK2D(MM, 2, false, false, false); break;                           \
+    case 140: QH_LK2D(MM, 2, false, false, true); break;                                    \
+    case 142: QH_LK2D(MM, 2, true, false, false); break;                                    \
+    case 143: QH_LK2D(MM, 2, false, true, true); break;                                     \
     default:                                                                                \
       qh_set_error("row-pair variant %d has no time-dependent form", G);                    \
       return QH_EINVAL;                                                                     \
@@ -1071,11 +1091,12 @@ int ks2_launch(int G, int mode, hipStream_t s, const qh_mat *A, const void *xin,
   }
 #define QH_LK2G(MM)                      \
   switch (G) {                           \
-    case 140: QH_LK2(MM, 2, false, false); break; \
-    case 141: QH_LK2(MM, 4, false, false); break; \
-    case 142: QH_LK2(MM, 2, true, false); break;  \
-    case 143: QH_LK2(MM, 2, false, true); break;  \
-    default: QH_LK2(MM, 2, true, true); break;    \
+    case QH_KS2_LONG: QH_LK2(MM, 2, false, false, false); break; \
+    case 140: QH_LK2(MM, 2, false, false, true); break; \
+    case 141: QH_LK2(MM, 4, false, false, true); break; \
+    case 142: QH_LK2(MM, 2, true, false, false); break;  \
+    case 143: QH_LK2(MM, 2, false, true, true); break;  \
+    default: QH_LK2(MM, 2, true, true, false); break;    \
   }
   if (mode == MODE_SPMV) {
     QH_LK2G(MODE_SPMV)

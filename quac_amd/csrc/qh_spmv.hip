@@ -219,7 +219,7 @@ __device__ inline R ks_load_real(__amdgpu_buffer_rsrc_t rs, uint32_t off) {
     return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, off, 0, AUX));
 }
 
-// One pass over U slots of a slice starting at mp, split into the issue of its
+// One pass over U slots of a slice from src, split into the issue of its
 // loads (ks_issue*) and the products of the loaded values (ks_fma*), so that a
 // group can keep the loads of the next pass in flight while it multiplies the
 // current one.  cnt valid slots when TAIL (the metadata array carries
@@ -231,7 +231,7 @@ __device__ inline R ks_load_real(__amdgpu_buffer_rsrc_t rs, uint32_t off) {
 // VV: the uniform value of a slot is read with a vector load (broadcast to all
 // lanes) instead of a scalar load, which keeps the metadata held in SGPRs at six
 // dwords per slot and lets a pass carry 8 slots; mr covers the metadata array
-// and k is the slot index of mp[0].
+// and k is the index of the pass's first slot there.
 template <typename R, int KIND, int U, bool VV>
 struct KsBuf {
   typename C2<R>::T xv[U], vv[U];
@@ -239,8 +239,8 @@ struct KsBuf {
   double ur[U], ui[U];  // uniform value, or the (1, 0) / (0, 1) multiplier of a scalar slot
 };
 
-template <typename R, int KIND, bool TAIL, int U, bool VV, int AUX = 0>
-__device__ __forceinline__ void ks_issue(const qh_kmeta *__restrict__ mp, int32_t cnt, uint32_t r8,
+template <typename R, int KIND, bool TAIL, int U, bool VV, int AUX = 0, typename Src>
+__device__ __forceinline__ void ks_issue(const Src &src, int32_t cnt, uint32_t r8,
                                          __amdgpu_buffer_rsrc_t xr, __amdgpu_buffer_rsrc_t vr,
                                          __amdgpu_buffer_rsrc_t mr, int32_t k, KsBuf<R, KIND, U, VV> &b) {
   typedef typename C2<R>::T T;
@@ -248,7 +248,7 @@ __device__ __forceinline__ void ks_issue(const qh_kmeta *__restrict__ mp, int32_
   uint64_t mask[U];
 #pragma unroll
   for (int j = 0; j < U; j++) {
-    m[j] = mp[j];
+    m[j] = src.get(j);
     mask[j] = (!TAIL || j < cnt) ? m[j].mask : 0ull;
   }
   if (KIND == KS_UNI && VV) {
@@ -318,15 +318,15 @@ struct KsBuf32 {
   float ur[U], ui[U];
 };
 
-template <int KIND, bool TAIL, int U, int AUX = 0>
-__device__ __forceinline__ void ks_issue32(const qh_kmeta32 *__restrict__ mp, int32_t cnt, uint32_t r8,
+template <int KIND, bool TAIL, int U, int AUX = 0, typename Src>
+__device__ __forceinline__ void ks_issue32(const Src &src, int32_t cnt, uint32_t r8,
                                            __amdgpu_buffer_rsrc_t xr, __amdgpu_buffer_rsrc_t vr,
                                            KsBuf32<KIND, U> &b) {
   qh_kmeta32 m[U];
   uint64_t mask[U];
 #pragma unroll
   for (int j = 0; j < U; j++) {
-    m[j] = mp[j];
+    m[j] = src.get(j);
     mask[j] = (!TAIL || j < cnt) ? m[j].mask : 0ull;
     b.ur[j] = m[j].vre;
     b.ui[j] = m[j].vim;
@@ -378,18 +378,18 @@ __device__ __forceinline__ void ks_fma32(const KsBuf32<KIND, U> &b, double &are,
 
 // Issue / multiply policies over the two metadata layouts, so that one group
 // driver serves both; W is the number of slots of a pass.
-template <int KIND, int AUX = 0>
+template <int KIND, bool RL, int AUX = 0>
 struct KsOps32 {
   typedef KsAcc Acc;
   template <int W>
   using Buf = KsBuf32<KIND, W>;
-  const qh_kmeta32 *mp;
+  KsSrc<qh_kmeta32, RL> src;
   uint32_t r8;
   __amdgpu_buffer_rsrc_t xr, vr;
   template <int W, bool TAIL = false>
   __device__ __forceinline__ void issue(Buf<W> &b, int32_t cnt = W) {
-    ks_issue32<KIND, TAIL, W, AUX>(mp, cnt, r8, xr, vr, b);
-    mp += W;
+    ks_issue32<KIND, TAIL, W, AUX>(src, cnt, r8, xr, vr, b);
+    src.skip(W);
   }
   template <int W>
   __device__ __forceinline__ void fma(const Buf<W> &b, Acc &a) {
@@ -398,19 +398,19 @@ struct KsOps32 {
   __device__ __forceinline__ void flush(Acc &) {}
 };
 
-template <typename R, int KIND, bool VV, int AUX = 0>
+template <typename R, int KIND, bool VV, bool RL, int AUX = 0>
 struct KsOps {
   typedef KsAcc Acc;
   template <int W>
   using Buf = KsBuf<R, KIND, W, VV>;
-  const qh_kmeta *mp;
+  KsSrc<qh_kmeta, RL> src;
   uint32_t r8;
   __amdgpu_buffer_rsrc_t xr, vr, mr;
   int32_t k;
   template <int W, bool TAIL = false>
   __device__ __forceinline__ void issue(Buf<W> &b, int32_t cnt = W) {
-    ks_issue<R, KIND, TAIL, W, VV, AUX>(mp, cnt, r8, xr, vr, mr, k, b);
-    mp += W;
+    ks_issue<R, KIND, TAIL, W, VV, AUX>(src, cnt, r8, xr, vr, mr, k, b);
+    src.skip(W);
     k += W;
   }
   template <int W>
@@ -419,22 +419,6 @@ struct KsOps {
   }
   __device__ __forceinline__ void flush(Acc &) {}
 };
-
-template <int KIND, int U, bool PIPE, int AUX = 0>
-__device__ __forceinline__ void ks_group32(const qh_kmeta32 *__restrict__ meta, int32_t k, int32_t kend,
-                                           uint32_t r8, __amdgpu_buffer_rsrc_t xr, __amdgpu_buffer_rsrc_t vr,
-                                           KsAcc &acc) {
-  KsOps32<KIND, AUX> ops{meta + k, r8, xr, vr};
-  ks_run<U, PIPE>(ops, kend - k, acc);
-}
-
-template <typename R, int KIND, int U, bool VV, bool PIPE, int AUX = 0>
-__device__ __forceinline__ void ks_group(const qh_kmeta *__restrict__ meta, int32_t k, int32_t kend, uint32_t r8,
-                                         __amdgpu_buffer_rsrc_t xr, __amdgpu_buffer_rsrc_t vr,
-                                         __amdgpu_buffer_rsrc_t mr, KsAcc &acc) {
-  KsOps<R, KIND, VV, AUX> ops{meta + k, r8, xr, vr, mr, k};
-  ks_run<U, PIPE>(ops, kend - k, acc);
-}
 
 // Stage kernel on the sliced layout: every stage gathers one vector.
 //   MODE_SPMV : kout = A xin
@@ -506,14 +490,33 @@ __global__ void __launch_bounds__(256) k_ks_stage(
   const uint32_t r8 = (uint32_t)r * (uint32_t)sizeof(T);
   KsAcc acc{0.0, 0.0};
   constexpr int AUX = NT ? 2 : 0;
-  if (sizeof(R) == 4 && !VV && MODE != MODE_LAST) {
-    ks_group32<KS_UNI, U, PIPE>(meta32, k0, km, r8, xr, vr, acc);
-    ks_group32<KS_SCA, U, PIPE, AUX>(meta32, km, kc, r8, xr, sr, acc);
-    ks_group32<KS_CPX, U, PIPE, AUX>(meta32, kc, kend, r8, xr, vr, acc);
+  // the pipelined kernels hold the slice's metadata in registers (at most 64
+  // slots: launch_ks chooses another kernel beyond)
+  constexpr bool RL = PIPE;
+  if constexpr (sizeof(R) == 4 && !VV && MODE != MODE_LAST) {
+    KsRegs<qh_kmeta32> regs;
+    if (RL) regs.load(meta32 + k0, kend - k0, lane);
+    auto src = [&](int32_t k) {
+      if constexpr (RL)
+        return KsSrc<qh_kmeta32, true>{regs, k - k0};
+      else
+        return KsSrc<qh_kmeta32, false>{meta32 + k};
+    };
+    ks_run<U, PIPE>(KsOps32<KS_UNI, RL>{src(k0), r8, xr, vr}, km - k0, acc);
+    ks_run<U, PIPE>(KsOps32<KS_SCA, RL, AUX>{src(km), r8, xr, sr}, kc - km, acc);
+    ks_run<U, PIPE>(KsOps32<KS_CPX, RL, AUX>{src(kc), r8, xr, vr}, kend - kc, acc);
   } else {
-    ks_group<R, KS_UNI, U, VV, PIPE>(meta, k0, km, r8, xr, vr, mr, acc);
-    ks_group<R, KS_SCA, U, VV, PIPE, AUX>(meta, km, kc, r8, xr, sr, mr, acc);
-    ks_group<R, KS_CPX, U, VV, PIPE, AUX>(meta, kc, kend, r8, xr, vr, mr, acc);
+    KsRegs<qh_kmeta> regs;
+    if (RL) regs.load(meta + k0, kend - k0, lane);
+    auto src = [&](int32_t k) {
+      if constexpr (RL)
+        return KsSrc<qh_kmeta, true>{regs, k - k0};
+      else
+        return KsSrc<qh_kmeta, false>{meta + k};
+    };
+    ks_run<U, PIPE>(KsOps<R, KS_UNI, VV, RL>{src(k0), r8, xr, vr, mr, k0}, km - k0, acc);
+    ks_run<U, PIPE>(KsOps<R, KS_SCA, VV, RL, AUX>{src(km), r8, xr, sr, mr, km}, kc - km, acc);
+    ks_run<U, PIPE>(KsOps<R, KS_CPX, VV, RL, AUX>{src(kc), r8, xr, vr, mr, kc}, kend - kc, acc);
   }
   double are = acc.re, aim = acc.im;
   if constexpr (TDP) {
@@ -814,7 +817,9 @@ int ks_build(qh_mat *A) {
   }
   std::vector<int32_t> ho(ns + 1), hv(ns + 1), hsvo(ns + 1), hm(ns), hcm(ns);
   int64_t tot = 0, totv = 0, tots = 0;
+  int32_t most = 0;
   for (int32_t i = 0; i < ns; i++) {
+    most = std::max(most, hw[i]);
     ho[i] = (int32_t)tot;
     hv[i] = (int32_t)totv;
     hsvo[i] = (int32_t)tots;
@@ -847,6 +852,7 @@ int ks_build(qh_mat *A) {
   cleanup();
   A->nslices = ns;
   A->ks_slots = tot;
+  A->ks_maxslots = most;
   A->ks_nval = totv;
   A->ks_nsval = tots;
   A->ks_state = 1;
@@ -906,6 +912,8 @@ int launch_ks(int G, hipStream_t s, const qh_mat *A, const void *xin, void *kout
   const dim3 grid(qh_blocks(A->nslices, 4)), blk(256);
   const int32_t n = (int32_t)A->rows, ns = A->nslices;
   const qh_td_ell none{nullptr, nullptr, nullptr, nullptr, nullptr};
+  // the pipelined kernels hold a slice's metadata in registers, one slot a lane
+  if (A->ks_maxslots > 64) G = G == 133 ? 128 : G == 134 ? (td ? 128 : 129) : G;
 #define QH_LKT(UU, VV, PP, NN, TT, TD)                                                                             \
   hipLaunchKernelGGL((k_ks_stage<R, MODE, UU, VV, PP, NN, TT>), grid, blk, 0, s, n, ns, A->ks_moff, A->ks_umid,     \
                      A->ks_cmid,                                                                              \
@@ -2049,9 +2057,8 @@ int qh_rk3bs_td_sliced(qh_mat *A, const qh_vec *x, qh_vec *xn, qh_vec *k1, qh_ve
   *done = 0;
   int rc = rk3bs_check(A, x, xn, k1, k2, k3, k4, y, err, "qh_rk3bs_td_step");
   if (rc) return rc;
-  if (A->rows <= QH_SMALL_ROWS && !A->lanes_forced) return QH_OK;
   int G = 0;
-  rc = lanes_for(A, QH_FP64, &G);
+  rc = qh_td_sliced_prepare(A, QH_FP64, &G);
   if (rc) return rc;
   if (!(G == 128 || G == 134 || G == 136) || A->ks_state != 1) return QH_OK;
   *done = 1;
@@ -2306,6 +2313,15 @@ int qh_td_sliced_prepare(qh_mat *A, int prec, int *G) {
   int g = 0;
   const int rc = lanes_for(A, prec, &g);
   if (rc) return rc;
+  // the autotuner's choice holds for A alone; the same layout is read by the
+  // variant that sums the A_k entries in A's kernel, which saves the pass of their
+  // own (10-qubit chain, three drives, FP64: 37 us a stage against 55 us)
+  if (!A->lanes_forced) {
+    if (g == 135) g = 136;
+    else if (QH_IS_KSELL(g) && g != 128 && g != 136) g = 134;
+    else if (g == 141) g = 140;
+    else if (g == 144) g = 142;
+  }
   if (QH_IS_KSELL(g) || QH_IS_KS2(g)) *G = g;
   return QH_OK;
 }
