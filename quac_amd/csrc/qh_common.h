@@ -105,6 +105,10 @@ void qh_td_cache_free(qh_td_cache *c);
 // matrix compare it with the pointer, which a new matrix may reuse)
 uint64_t qh_next_mat_uid();
 
+// the plan of a generator that falls apart into small closed sets of rows (qh_comp.hip)
+struct qh_comp;
+void qh_comp_free(qh_comp *c);
+
 struct qh_mat {
   uint64_t uid = qh_next_mat_uid();
   int64_t rows = 0, nnz = 0;
@@ -151,6 +155,8 @@ struct qh_mat {
   int32_t ks2_maxslots = 0;    // most slots of a slice
   int64_t ks2_slots = 0, ks2_nval = 0, ks2_nsval = 0, ks2_nsval1 = 0, ks2_nsep = 0, ks2_ngh = 0, ks2_nsepblk = 0;
   std::vector<int64_t> blk_off;  // row offsets of the blocks of a block-diagonal matrix (and its row count)
+  int comp_state = 0;          // 0 not looked at, 1 plan in comp, -1 not worth it
+  qh_comp *comp = nullptr;
   qh_td_cache *td_cache = nullptr;  // built by the first time-dependent RHS on this matrix
 };
 // variant codes selecting the sliced-ELL kernel: 128 / 129 / 130 process 2 / 4 / 8
@@ -193,6 +199,15 @@ int ks2_launch(int G, int mode, hipStream_t s, const qh_mat *A, const void *xin,
 int qh_rk3bs_td_sliced(qh_mat *A, const qh_vec *x, qh_vec *xn, qh_vec *k1, qh_vec *k2, qh_vec *k3, qh_vec *k4,
                        qh_vec *y, double h, double atol, double rtol, int have_k1, double *err,
                        const qh_td_ell *td4, int *done);
+
+// RK4 steps of a generator whose rows fall apart into closed sets (qh_comp.hip):
+// *usable = 1 where the plan exists (built on the first call) and beats the stage
+// kernels; nsteps steps of x in place on the library stream; QH_COMP_TRACE doubles
+// of device memory that the trace renormalisation of x may use (kept with the plan)
+#define QH_COMP_TRACE 1024
+int qh_comp_prepare(qh_mat *A, int *usable);
+int qh_comp_rk4(qh_mat *A, qh_vec *x, double dt, int64_t nsteps);
+double *qh_comp_trace(const qh_mat *A);
 
 // longest row of A into A->max_row (computed once per matrix)
 int qh_mat_max_row(qh_mat *A);

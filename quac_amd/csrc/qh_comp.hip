@@ -1,0 +1,744 @@
+// qh_comp.hip -- RK4 of a constant generator, one closed set of rows per workgroup.
+//
+// Generators of open systems often fall apart: a jump and the coherent term that
+// goes with it move a row index of rho and its column index together, so a
+// conserved difference (excitation numbers, the bits in which the two indices
+// differ) splits the rows into sets that no entry connects.  Within such a set the
+// whole integration needs nobody else: a workgroup keeps the set's vector in LDS
+// and its matrix entries in registers and runs every step of a call, so a call
+// reads and writes the state once instead of three vector passes and a launch per
+// stage.
+//
+// Plan (once per matrix): connected components of the sparsity pattern (union
+// find), components packed into bins of whole components, rows sorted within a bin.
+// A bin's rows are stored in slices of 64 (one wavefront): the diagonal apart, and
+// every other entry as one or two real entries, first the imaginary parts (an even
+// number of slots a slice), then the real parts, each a value and the 16-bit index
+// of its column within the bin.
+//
+// What bounds it: at few bins the chain of LDS reads of one stage and its barrier
+// (0.3 to 1.5 us a stage, where a launch a stage takes 2.6 to 4.3 us), at many
+// the LDS reads, 16 B an entry.
+#include <algorithm>
+#include <vector>
+
+#include <hipcub/hipcub.hpp>
+
+#include "qh_common.h"
+
+namespace {
+
+const int CP_GRAN = 64;         // rows of a granule: the components that start in 64 consecutive sorted rows
+const int CP_REG_ROWS = 2048;   // largest bin with its entries in registers (1024 threads, two rows each)
+const int CP_MAX_ROWS = 5056;   // largest bin: two buffers of rows + 1 complex128 in 160 KB of LDS
+const int CP_PROBE_ROWS = 16384;  // rows looked at before a large matrix as a whole
+const int CP_STREAM_S = 5;      // rows a thread of the kernel that reads its entries from memory
+const int CP_PACK_ROWS = 512;   // bins of small components are filled to this size once they outnumber the CUs
+
+// -------------------------------------------------------------- components
+// Parents only ever decrease.  The loads are ordinary cached ones: a value read late
+// is still an ancestor, and only the device-scope exchange that hangs one root below
+// another has to see the present one, which it returns when it fails.  (With every
+// load at device scope the 16 M rows of a sweep of 512 systems took 20 ms.)
+__device__ inline int32_t cc_load(const int32_t *p, int32_t i) {
+  return __hip_atomic_load(p + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ inline void cc_store(int32_t *p, int32_t i, int32_t v) {
+  __hip_atomic_store(p + i, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ inline int32_t cc_find(int32_t *p, int32_t i) {
+  int32_t q = cc_load(p, i);
+  while (q != i) {
+    const int32_t g = cc_load(p, q);
+    if (g != q) cc_store(p, i, g);
+    i = q;
+    q = g;
+  }
+  return i;
+}
+
+__global__ void k_cc_init(int32_t *parent, int32_t *size, int32_t n) {
+  for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < n; r += (int64_t)gridDim.x * blockDim.x) {
+    parent[r] = (int32_t)r;
+    size[r] = 0;
+  }
+}
+
+// rows r0 .. r0 + n, and the entries between them (indices from r0)
+__global__ void __launch_bounds__(256) k_cc_hook(int32_t *parent, const int32_t *__restrict__ rp,
+                                                 const int32_t *__restrict__ col, int32_t r0, int32_t n) {
+  const int64_t r = blockIdx.x * (int64_t)256 + threadIdx.x;
+  if (r >= n) return;
+  int32_t a = (int32_t)r;
+  for (int32_t e = rp[r0 + r]; e < rp[r0 + r + 1]; e++) {
+    int32_t b = col[e] - r0;
+    if (b == (int32_t)r || b < 0 || b >= n) continue;
+    b = cc_load(parent, b);
+    if (b == a) continue;
+    for (;;) {  // the larger root below the smaller one; the larger index decreases every round
+      a = cc_find(parent, a);
+      b = cc_find(parent, b);
+      if (a == b) break;
+      const int32_t hi = a > b ? a : b, lo = a > b ? b : a;
+      const int32_t old = atomicCAS(parent + hi, hi, lo);
+      if (old == hi) {
+        a = lo;
+        break;
+      }
+      cc_store(parent, hi, old);  // what this die's cache still held as a root
+      a = lo;
+      b = old;
+    }
+  }
+}
+
+// the root of every row, and the rows of every root
+__global__ void __launch_bounds__(256) k_cc_label(int32_t *parent, int32_t *lab, int32_t *size, int32_t n) {
+  const int64_t r = blockIdx.x * (int64_t)256 + threadIdx.x;
+  const bool on = r < n;
+  const int32_t l = on ? cc_find(parent, (int32_t)r) : -1;
+  if (on) lab[r] = l;
+  // lanes that share the first lane's root count together (one component is the common large case)
+  const int32_t f = __builtin_amdgcn_readfirstlane(l);
+  const uint64_t m = __ballot(on && l == f);
+  if (!on) return;
+  if (l == f) {
+    if ((threadIdx.x & 63) == 0) atomicAdd(size + f, (int32_t)__popcll(m));
+  } else {
+    atomicAdd(size + l, 1);
+  }
+}
+
+__global__ void k_cc_largest(const int32_t *size, int32_t *out, int32_t n) {
+  int32_t m = 0;
+  for (int64_t r = blockIdx.x * (int64_t)256 + threadIdx.x; r < n; r += (int64_t)gridDim.x * 256) m = max(m, size[r]);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o, 64));
+  if ((threadIdx.x & 63) == 0) atomicMax(out, m);
+}
+
+__global__ void k_cc_granules(const int32_t *size, const int32_t *off, int32_t *gsize, int32_t n) {
+  const int64_t r = blockIdx.x * (int64_t)256 + threadIdx.x;
+  if (r < n && size[r]) atomicAdd(gsize + off[r] / CP_GRAN, size[r]);
+}
+
+// ------------------------------------------------------------------- plan
+__global__ void k_cp_keys(const int32_t *lab, const int32_t *off, const int32_t *gbin, int32_t *key, int32_t *row,
+                          int32_t n) {
+  const int64_t r = blockIdx.x * (int64_t)256 + threadIdx.x;
+  if (r >= n) return;
+  key[r] = gbin[off[lab[r]] / CP_GRAN];
+  row[r] = (int32_t)r;
+}
+
+__global__ void k_cp_fill_order(int32_t *order, int64_t n) {
+  const int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x;
+  if (i < n) order[i] = -1;
+}
+
+// sorted position q -> padded position, and the row's index within its bin
+__global__ void k_cp_place(const int32_t *key, const int32_t *row, const int32_t *brow, const int32_t *bslice,
+                           int32_t *order, int32_t *pos, int32_t n) {
+  const int64_t q = blockIdx.x * (int64_t)256 + threadIdx.x;
+  if (q >= n) return;
+  const int32_t b = key[q], at = (int32_t)q - brow[b];
+  order[(int64_t)bslice[b] * 64 + at] = row[q];
+  pos[row[q]] = at;
+}
+
+__device__ inline int32_t cp_wave_max(int32_t v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
+  return v;
+}
+
+// slots of every slice: imaginary parts (made even) and all
+__global__ void __launch_bounds__(256) k_cp_width(const int32_t *order, const int32_t *__restrict__ rp,
+                                                  const int32_t *__restrict__ col, const double2 *__restrict__ val,
+                                                  int32_t *width, int32_t *nim, int32_t nslices) {
+  const int32_t s = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (s >= nslices) return;
+  const int32_t r = order[(int64_t)s * 64 + lane];
+  int32_t ni = 0, nr = 0;
+  if (r >= 0)
+    for (int32_t e = rp[r]; e < rp[r + 1]; e++) {
+      if (col[e] == r) continue;
+      const double2 v = val[e];
+      ni += v.y != 0.0;
+      nr += v.x != 0.0;
+    }
+  ni = (cp_wave_max(ni) + 1) & ~1;
+  nr = cp_wave_max(nr);
+  if (lane == 0) {
+    width[s] = ni + nr;
+    nim[s] = ni;
+  }
+}
+
+// the entries of every slice; zc[s]: index of the bin's zero cell, read by the
+// slots that a row does not fill
+__global__ void __launch_bounds__(256) k_cp_fill(const int32_t *order, const int32_t *pos,
+                                                 const int32_t *__restrict__ rp, const int32_t *__restrict__ col,
+                                                 const double2 *__restrict__ val, const int32_t *soff,
+                                                 const int32_t *nim, const int32_t *zc, double2 *diag, double *ev,
+                                                 uint16_t *ec, int32_t nslices) {
+  const int32_t s = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (s >= nslices) return;
+  const int32_t r = order[(int64_t)s * 64 + lane];
+  const int64_t s0 = soff[s], s1 = soff[s + 1];
+  int64_t pi = s0, pr = s0 + nim[s];
+  double2 d = make_double2(0.0, 0.0);
+  auto put = [&](int64_t slot, double v, int32_t c) {
+    ev[slot * 64 + lane] = v;
+    ec[slot * 64 + lane] = (uint16_t)c;
+  };
+  if (r >= 0)
+    for (int32_t e = rp[r]; e < rp[r + 1]; e++) {
+      const double2 v = val[e];
+      if (col[e] == r) {
+        d = v;
+        continue;
+      }
+      const int32_t c = pos[col[e]];
+      if (v.y != 0.0) put(pi++, v.y, c);
+      if (v.x != 0.0) put(pr++, v.x, c);
+    }
+  for (; pi < s0 + nim[s]; pi++) put(pi, 0.0, zc[s]);
+  for (; pr < s1; pr++) put(pr, 0.0, zc[s]);
+  diag[(int64_t)s * 64 + lane] = d;
+}
+
+// ------------------------------------------------------------------ stepping
+struct CpArgs {
+  const int32_t *bins, *bslice;  // this launch's bins; first slice of every bin
+  const int32_t *soff, *nim, *order;
+  const double2 *diag;
+  const double *ev;
+  const uint16_t *ec;
+  void *x;
+  float2 *xlo;   // the low words of an FP32 state, else null
+  int32_t cells;  // complex128 of one LDS buffer
+  double h;
+  int64_t nsteps;
+};
+
+// A thread owns S rows of the bin, wavefront w the slices w, w + waves, ...  REG:
+// the W slots of a row live in registers (2.5 dwords each), so that a step reads
+// LDS only; otherwise they are read again at every stage (through the caches).
+// RK4 on a linear autonomous system in nested form, y <- x + c A y with c = h/4,
+// h/3, h/2, h, double buffered: one barrier a stage.
+template <int S, int W, bool REG>
+__global__ void __launch_bounds__(1024) k_comp_rk4(CpArgs a) {
+  extern __shared__ double2 sm[];
+  const int b = a.bins[blockIdx.x];
+  const int32_t sl0 = a.bslice[b], nsl = a.bslice[b + 1] - sl0;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+  double2 x[S], y[REG ? S : 1], d[REG ? S : 1];
+  int32_t row[S], nim[S], s0[S], wid[S];
+  double v[REG ? S * W : 1];
+  uint32_t c2[REG ? S * W / 2 : 1];
+#pragma unroll
+  for (int k = 0; k < S; k++) {
+    const int32_t sl = wave + k * waves;
+    row[k] = -1;
+    nim[k] = wid[k] = s0[k] = 0;
+    x[k] = make_double2(0.0, 0.0);
+    if (REG) d[k] = x[k];
+    if (sl < nsl) {
+      const int64_t p = (int64_t)(sl0 + sl) * 64 + lane;
+      row[k] = a.order[p];
+      s0[k] = a.soff[sl0 + sl];
+      wid[k] = a.soff[sl0 + sl + 1] - s0[k];
+      nim[k] = a.nim[sl0 + sl];
+      if (REG) d[k] = a.diag[p];
+      if (row[k] >= 0) {
+        if (a.xlo) {
+          const float2 hi = ((const float2 *)a.x)[row[k]], lo = a.xlo[row[k]];
+          x[k] = make_double2((double)hi.x + (double)lo.x, (double)hi.y + (double)lo.y);
+        } else {
+          x[k] = ((const double2 *)a.x)[row[k]];
+        }
+      }
+      sm[sl * 64 + lane] = x[k];
+    }
+    if constexpr (REG) {
+      y[k] = x[k];
+#pragma unroll
+      for (int e = 0; e < W; e += 2) {
+        const bool f = e < wid[k], g = e + 1 < wid[k];
+        const int64_t at = (int64_t)(s0[k] + e) * 64 + lane;
+        v[k * W + e] = f ? a.ev[at] : 0.0;
+        v[k * W + e + 1] = g ? a.ev[at + 64] : 0.0;
+        const uint32_t z = (uint32_t)nsl * 64u;
+        const uint32_t lo = f ? a.ec[at] : z, hi = g ? a.ec[at + 64] : z;
+        c2[(k * W + e) / 2] = lo | (hi << 16);
+      }
+    }
+  }
+  if (threadIdx.x == 0) sm[nsl * 64] = sm[a.cells + nsl * 64] = make_double2(0.0, 0.0);
+  __syncthreads();
+  const double cs[4] = {a.h / 4.0, a.h / 3.0, a.h / 2.0, a.h};
+  for (int64_t st = 0; st < a.nsteps; st++) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const char *in = (const char *)(sm + (q & 1 ? a.cells : 0));
+      double2 *out = sm + (q & 1 ? 0 : a.cells);
+#pragma unroll
+      for (int k = 0; k < S; k++) {
+        const int32_t sl = wave + k * waves;
+        if (sl < nsl) {
+          double p = 0.0, r = 0.0;
+          if constexpr (REG) {
+            // LDS reads in flight (a divisor of W; the registers allow fewer beside more slots)
+            constexpr int CH = S > 1 || W > 16 ? 4 : W % 8 == 0 ? 8 : W == 12 ? 6 : 4;
+            static_assert(W % CH == 0 && CH % 2 == 0, "whole chunks");
+#pragma unroll
+            for (int e0 = 0; e0 < W; e0 += CH) {
+              double2 t[CH];
+#pragma unroll
+              for (int j = 0; j < CH; j++) {
+                const uint32_t w = c2[(k * W + e0 + j) / 2];
+                const uint32_t at = j & 1 ? (w >> 12) & 0xFFFF0u : (w << 4) & 0xFFFF0u;
+                t[j] = *(const double2 *)(in + at);
+              }
+#pragma unroll
+              for (int j = 0; j < CH; j++) {
+                // the imaginary parts are summed: times i, and the real parts follow
+                if (!(j & 1) && nim[k] == e0 + j) {
+                  const double u = p;
+                  p = -r;
+                  r = u;
+                }
+                p = fma(v[k * W + e0 + j], t[j].x, p);
+                r = fma(v[k * W + e0 + j], t[j].y, r);
+              }
+            }
+            if (nim[k] == W) {
+              const double u = p;
+              p = -r;
+              r = u;
+            }
+          } else {
+            const double *ev = a.ev + (int64_t)s0[k] * 64 + lane;
+            const uint16_t *ec = a.ec + (int64_t)s0[k] * 64 + lane;
+#pragma unroll 4
+            for (int32_t e = 0; e < nim[k]; e++) {
+              const double2 t = *(const double2 *)(in + (uint32_t)ec[e * 64] * 16u);
+              p = fma(ev[e * 64], t.x, p);
+              r = fma(ev[e * 64], t.y, r);
+            }
+            const double u = p;
+            p = -r;
+            r = u;
+#pragma unroll 4
+            for (int32_t e = nim[k]; e < wid[k]; e++) {
+              const double2 t = *(const double2 *)(in + (uint32_t)ec[e * 64] * 16u);
+              p = fma(ev[e * 64], t.x, p);
+              r = fma(ev[e * 64], t.y, r);
+            }
+          }
+          double2 yk, dk;
+          if constexpr (REG) {
+            yk = y[k];
+            dk = d[k];
+          } else {
+            yk = ((const double2 *)in)[sl * 64 + lane];
+            dk = a.diag[(int64_t)(sl0 + sl) * 64 + lane];
+          }
+          p = fma(dk.x, yk.x, fma(-dk.y, yk.y, p));
+          r = fma(dk.x, yk.y, fma(dk.y, yk.x, r));
+          yk.x = fma(cs[q], p, x[k].x);
+          yk.y = fma(cs[q], r, x[k].y);
+          out[sl * 64 + lane] = yk;
+          if (REG) y[k] = yk;
+          else if (q == 3) x[k] = yk;
+        }
+      }
+      __syncthreads();
+    }
+    if constexpr (REG) {
+#pragma unroll
+      for (int k = 0; k < S; k++) x[k] = y[k];
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < S; k++) {
+    if (row[k] < 0) continue;
+    if (a.xlo) {
+      const float hr = (float)x[k].x, hm = (float)x[k].y;
+      ((float2 *)a.x)[row[k]] = make_float2(hr, hm);
+      a.xlo[row[k]] = make_float2((float)(x[k].x - (double)hr), (float)(x[k].y - (double)hm));
+    } else {
+      ((double2 *)a.x)[row[k]] = x[k];
+    }
+  }
+}
+
+// one launch: bins of one shape
+struct CpClass {
+  int threads, S, W;  // W 0: entries read from memory
+  int first, count;   // range of the plan's bin list
+  int cells;
+};
+
+template <int S, int W, bool REG>
+int cp_launch(const CpClass &c, const CpArgs &a, hipStream_t s) {
+  const size_t lds = (size_t)2 * c.cells * sizeof(double2);
+  if (lds > 64 * 1024)
+    QH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_comp_rk4<S, W, REG>),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  hipLaunchKernelGGL((k_comp_rk4<S, W, REG>), dim3(c.count), dim3(c.threads), lds, s, a);
+  QH_HIP(hipGetLastError());
+  return QH_OK;
+}
+
+}  // namespace
+
+struct qh_comp {
+  void *buf = nullptr, *slots = nullptr;  // the plan's arrays; its entries
+  CpArgs a{};
+  double *trace = nullptr;  // QH_COMP_TRACE doubles for the trace renormalisation
+  std::vector<CpClass> classes;
+};
+
+void qh_comp_free(qh_comp *c) {
+  if (!c) return;
+  qh_free_ptr(c->buf);
+  qh_free_ptr(c->slots);
+  delete c;
+}
+
+namespace {
+
+// a workspace handed out in 256-byte aligned pieces; two passes: sizes, then pointers
+struct Carve {
+  char *p = nullptr;
+  size_t n = 0;
+  template <typename T>
+  T *take(size_t count) {
+    T *q = reinterpret_cast<T *>(p + n);
+    n += (count * sizeof(T) + 255) & ~(size_t)255;
+    return q;
+  }
+};
+
+// time of a stage in clocks of a CU: a slot of a slice is 64 LDS reads of 16 B (8
+// clocks at 128 B a clock, 10 measured), with 64 entries of 10 B from the caches 32
+const double CP_CLK_REG = 10.0, CP_CLK_MEM = 32.0, CP_CLK_FIXED = 500.0;
+
+int cp_build(qh_mat *A) {
+  const int32_t n = (int32_t)A->rows;
+  hipStream_t s = qh_stream();
+  const unsigned nb256 = qh_blocks(n, 256);
+  const int32_t ngran = n / CP_GRAN + 1;
+  size_t scan_b = 0, sort_b = 0;
+  QH_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, scan_b, (int32_t *)nullptr, (int32_t *)nullptr, n, s));
+  int bits = 1;
+  while ((1 << bits) < ngran && bits < 31) bits++;
+  QH_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, sort_b, (int32_t *)nullptr, (int32_t *)nullptr,
+                                            (int32_t *)nullptr, (int32_t *)nullptr, n, 0, bits, s));
+  int32_t *parent, *size, *lab, *off, *gsize, *gbin, *key, *row, *pos, *brow;
+  char *tmp;
+  auto layout = [&](Carve &c) {
+    parent = c.take<int32_t>(n);
+    size = c.take<int32_t>(n);
+    lab = c.take<int32_t>(n);
+    off = c.take<int32_t>(n);
+    key = c.take<int32_t>(n);
+    row = c.take<int32_t>(n);
+    pos = c.take<int32_t>(n);
+    gsize = c.take<int32_t>(ngran);
+    gbin = c.take<int32_t>(ngran);
+    brow = c.take<int32_t>(ngran + 1);
+    tmp = c.take<char>(std::max(scan_b, sort_b) + 1);
+  };
+  Carve meas, work;
+  layout(meas);
+  void *wbuf = nullptr;
+  int rc = qh_alloc(&wbuf, meas.n);
+  if (rc) return rc;
+  work.p = (char *)wbuf;
+  layout(work);
+  qh_comp *c = new qh_comp();
+  auto fail = [&](int code) {
+    (void)hipStreamSynchronize(s);
+    qh_free_ptr(wbuf);
+    qh_comp_free(c);
+    return code;
+  };
+#define CP_HIP(call)                                                                             \
+  do {                                                                                           \
+    hipError_t e_ = (call);                                                                      \
+    if (e_ != hipSuccess) {                                                                      \
+      qh_set_error("%s:%d %s: %s", __FILE__, __LINE__, #call, hipGetErrorString(e_));            \
+      return fail(QH_EHIP);                                                                      \
+    }                                                                                            \
+  } while (0)
+  // A large matrix is probed first: the rows of its largest block, or its first
+  // CP_PROBE_ROWS ones.  Rows that hang together there do so in the whole (10-qubit
+  // chain, 1 M rows: 0.1 ms for the probe, 1.2 ms for all rows; 16 M rows of a sweep 10 ms).
+  if (n > 4 * CP_PROBE_ROWS) {
+    int32_t r0 = 0, m = CP_PROBE_ROWS;
+    if (A->blk_off.size() > 2) {
+      size_t big = 0;
+      for (size_t i = 0; i + 1 < A->blk_off.size(); i++)
+        if (A->blk_off[i + 1] - A->blk_off[i] > A->blk_off[big + 1] - A->blk_off[big]) big = i;
+      r0 = (int32_t)A->blk_off[big];
+      m = (int32_t)(A->blk_off[big + 1] - A->blk_off[big]);
+    }
+    const unsigned nbp = qh_blocks(m, 256);
+    int32_t most = 0;
+    hipLaunchKernelGGL(k_cc_init, dim3(std::min(nbp, 4096u)), dim3(256), 0, s, parent, size, m);
+    hipLaunchKernelGGL(k_cc_hook, dim3(nbp), dim3(256), 0, s, parent, A->rowptr, A->col, r0, m);
+    hipLaunchKernelGGL(k_cc_label, dim3(nbp), dim3(256), 0, s, parent, lab, size, m);
+    CP_HIP(hipMemsetAsync(off, 0, sizeof(int32_t), s));
+    hipLaunchKernelGGL(k_cc_largest, dim3(std::min(nbp, 256u)), dim3(256), 0, s, size, off, m);
+    CP_HIP(hipMemcpyAsync(&most, off, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+    CP_HIP(hipStreamSynchronize(s));
+    if (most > CP_MAX_ROWS) {
+      fail(0);
+      A->comp_state = -1;
+      return QH_OK;
+    }
+  }
+  // components, and the rows that start in each granule of the sorted order
+  CP_HIP(hipMemsetAsync(gsize, 0, sizeof(int32_t) * ngran, s));
+  hipLaunchKernelGGL(k_cc_init, dim3(std::min(nb256, 4096u)), dim3(256), 0, s, parent, size, n);
+  hipLaunchKernelGGL(k_cc_hook, dim3(nb256), dim3(256), 0, s, parent, A->rowptr, A->col, 0, n);
+  hipLaunchKernelGGL(k_cc_label, dim3(nb256), dim3(256), 0, s, parent, lab, size, n);
+  size_t tb = std::max(scan_b, sort_b);
+  CP_HIP(hipcub::DeviceScan::ExclusiveSum(tmp, tb, size, off, n, s));
+  hipLaunchKernelGGL(k_cc_granules, dim3(nb256), dim3(256), 0, s, size, off, gsize, n);
+  std::vector<int32_t> hg(ngran);
+  CP_HIP(hipMemcpyAsync(hg.data(), gsize, sizeof(int32_t) * ngran, hipMemcpyDeviceToHost, s));
+  CP_HIP(hipStreamSynchronize(s));
+  // bins: consecutive granules up to CP_PACK_ROWS where there are many, else one each
+  const int64_t cus = qh_num_cus();
+  const int32_t pack = (int64_t)n > 2 * cus * CP_PACK_ROWS ? CP_PACK_ROWS : 0;
+  std::vector<int32_t> hbin(ngran), hrow{0}, hslice{0};
+  int32_t cur = 0, largest = 0;
+  auto close = [&] {
+    if (!cur) return;
+    hrow.push_back(hrow.back() + cur);
+    hslice.push_back(hslice.back() + (cur + 63) / 64);
+    largest = std::max(largest, cur);
+    cur = 0;
+  };
+  for (int32_t g = 0; g < ngran; g++) {
+    if (!hg[g]) {
+      hbin[g] = 0;
+      continue;
+    }
+    if (cur && cur + hg[g] > pack) close();
+    hbin[g] = (int32_t)hrow.size() - 1;
+    cur += hg[g];
+  }
+  close();
+  if (largest > CP_MAX_ROWS) {
+    fail(0);
+    A->comp_state = -1;
+    return QH_OK;
+  }
+  const int32_t nbins = (int32_t)hrow.size() - 1, nsl = hslice.back();
+  // order the rows by bin
+  CP_HIP(hipMemcpyAsync(gbin, hbin.data(), sizeof(int32_t) * ngran, hipMemcpyHostToDevice, s));
+  CP_HIP(hipMemcpyAsync(brow, hrow.data(), sizeof(int32_t) * (nbins + 1), hipMemcpyHostToDevice, s));
+  // `parent` and `size` are free from here: the sort's second buffers
+  hipLaunchKernelGGL(k_cp_keys, dim3(nb256), dim3(256), 0, s, lab, off, gbin, key, row, n);
+  CP_HIP(hipcub::DeviceRadixSort::SortPairs(tmp, tb, key, parent, row, size, n, 0, bits, s));
+  int32_t *order, *bslice, *soff, *nim, *zc, *width, *bins;
+  double2 *diag;
+  double *trace;
+  auto head = [&](Carve &q) {
+    order = q.take<int32_t>((size_t)nsl * 64);
+    bslice = q.take<int32_t>(nbins + 1);
+    soff = q.take<int32_t>((size_t)nsl + 1);
+    nim = q.take<int32_t>(nsl);
+    zc = q.take<int32_t>(nsl);
+    width = q.take<int32_t>(nsl);
+    bins = q.take<int32_t>(nbins);
+    diag = q.take<double2>((size_t)nsl * 64);
+    trace = q.take<double>(QH_COMP_TRACE);
+  };
+  Carve hm;
+  head(hm);
+  void *hbuf = nullptr;
+  rc = qh_alloc(&hbuf, hm.n);
+  if (rc) return fail(rc);
+  Carve hw;
+  hw.p = (char *)hbuf;
+  head(hw);
+  c->buf = hbuf;
+  std::vector<int32_t> hzc(nsl);
+  for (int32_t b = 0; b < nbins; b++)
+    for (int32_t i = hslice[b]; i < hslice[b + 1]; i++) hzc[i] = (hslice[b + 1] - hslice[b]) * 64;
+  CP_HIP(hipMemcpyAsync(bslice, hslice.data(), sizeof(int32_t) * (nbins + 1), hipMemcpyHostToDevice, s));
+  CP_HIP(hipMemcpyAsync(zc, hzc.data(), sizeof(int32_t) * nsl, hipMemcpyHostToDevice, s));
+  hipLaunchKernelGGL(k_cp_fill_order, dim3(qh_blocks((int64_t)nsl * 64, 256)), dim3(256), 0, s, order,
+                     (int64_t)nsl * 64);
+  hipLaunchKernelGGL(k_cp_place, dim3(nb256), dim3(256), 0, s, parent, size, brow, bslice, order, pos, n);
+  hipLaunchKernelGGL(k_cp_width, dim3(qh_blocks(nsl, 4)), dim3(256), 0, s, order, A->rowptr, A->col, A->val, width,
+                     nim, nsl);
+  CP_HIP(hipGetLastError());
+  std::vector<int32_t> hwid(nsl), hoff(nsl + 1);
+  CP_HIP(hipMemcpyAsync(hwid.data(), width, sizeof(int32_t) * nsl, hipMemcpyDeviceToHost, s));
+  CP_HIP(hipStreamSynchronize(s));
+  int64_t slots = 0;
+  for (int32_t i = 0; i < nsl; i++) {
+    hoff[i] = (int32_t)slots;
+    slots += hwid[i];
+    if (slots > (int64_t)0x7fffffff) {
+      fail(0);
+      A->comp_state = -1;
+      return QH_OK;
+    }
+  }
+  hoff[nsl] = (int32_t)slots;
+  // the shape of every bin's launch, and what the largest bin and all of them take
+  auto rup = [](int w) { return w <= 4 ? 4 : w <= 8 ? 8 : w <= 12 ? 12 : w <= 16 ? 16 : w <= 24 ? 24 : w <= 32 ? 32 : 0; };
+  const bool few = nbins <= 2 * cus;  // the chip is not full: one launch, so that nothing waits for a launch before it
+  struct Shape {
+    int stream, rows, W;
+    int32_t bin;
+  };
+  std::vector<Shape> sh(nbins);
+  double most = 0.0, all = 0.0;
+  int few_rows = 0, few_w = 0;
+  for (int32_t b = 0; b < nbins; b++) {
+    int w = 0;
+    int64_t sum = 0;
+    for (int32_t i = hslice[b]; i < hslice[b + 1]; i++) {
+      w = std::max(w, (int)hwid[i]);
+      sum += hwid[i];
+    }
+    const int rows = (hslice[b + 1] - hslice[b]) * 64;
+    const int W = rup(w);
+    // two rows a thread: up to 12 slots each fit 128 registers
+    const bool reg = W && (rows <= 1024 || (rows <= CP_REG_ROWS && W <= 12));
+    sh[b] = Shape{!reg, rows <= 64 ? 64 : rows <= 128 ? 128 : rows <= 256 ? 256 : rows <= 512 ? 512 : rows <= 1024 ? 1024 : rows, W, b};
+    if (reg) {
+      few_rows = std::max(few_rows, sh[b].rows);
+      few_w = std::max(few_w, W);
+    }
+    const double clk = reg ? CP_CLK_REG * W * (rows / 64) : CP_CLK_MEM * (double)sum;
+    most = std::max(most, clk + CP_CLK_FIXED);
+    all += clk;
+  }
+  // Against the sliced stage kernels: 2.5 us a launch, and 11 us a million rows.
+  // Measured us a stage, here / there: Jaynes-Cummings 2 x 24 0.30 / 2.6, Tavis-Cummings
+  // 2^2 x 23 0.44 / 2.7, 2^3 x 17 1.00 / 3.5, 2^3 x 30 1.49 / 4.3, decay and dephasing of
+  // 7 qubits 0.34 / 2.8, 10 5.1 / 13.2, 12 46.7 / 243.  Refused: 2^4 x 8 (bins of 1768
+  // rows whose entries do not fit the registers) 5.0 / 3.3, 2^4 x 19 10.5 / 5.4, 6-qubit
+  // chain (one bin of 4096 rows) 10.9 / 3.0.
+  const double clk_us = 2400.0, comp_us = std::max(most, all / (double)cus + CP_CLK_FIXED) / clk_us;
+  const double stage_us = 2.5 + 1.1e-5 * (double)n;
+  if (comp_us > 0.9 * stage_us) {
+    fail(0);
+    A->comp_state = -1;
+    return QH_OK;
+  }
+  if (few && !(few_rows > 1024 && few_w > 12))
+    for (auto &q : sh)
+      if (!q.stream) {
+        q.rows = few_rows;
+        q.W = few_w;
+      }
+  std::stable_sort(sh.begin(), sh.end(), [](const Shape &p, const Shape &q) {
+    if (p.stream != q.stream) return p.stream > q.stream;
+    const int pr = p.stream || p.rows > 1024 ? 1 << 20 : p.rows, qr = q.stream || q.rows > 1024 ? 1 << 20 : q.rows;
+    if (pr != qr) return pr > qr;
+    return !p.stream && p.W > q.W;
+  });
+  std::vector<int32_t> hbins(nbins);
+  for (int32_t i = 0; i < nbins; i++) {
+    const Shape &q = sh[i];
+    hbins[i] = q.bin;
+    const int S = q.stream ? CP_STREAM_S : q.rows > 1024 ? 2 : 1, threads = q.stream || S == 2 ? 1024 : q.rows;
+    const int W = q.stream ? 0 : q.W;
+    if (c->classes.empty() || c->classes.back().threads != threads || c->classes.back().S != S ||
+        c->classes.back().W != W)
+      c->classes.push_back(CpClass{threads, S, W, i, 0, 0});
+    CpClass &k = c->classes.back();
+    k.count++;
+    k.cells = std::max(k.cells, (hslice[q.bin + 1] - hslice[q.bin]) * 64 + 1);
+  }
+  double *ev;
+  uint16_t *ec;
+  Carve tail;
+  tail.take<double>((size_t)std::max<int64_t>(slots, 1) * 64);
+  tail.take<uint16_t>((size_t)std::max<int64_t>(slots, 1) * 64);
+  rc = qh_alloc(&c->slots, tail.n);
+  if (rc) return fail(rc);
+  Carve tw;
+  tw.p = (char *)c->slots;
+  ev = tw.take<double>((size_t)std::max<int64_t>(slots, 1) * 64);
+  ec = tw.take<uint16_t>((size_t)std::max<int64_t>(slots, 1) * 64);
+  CP_HIP(hipMemcpyAsync(soff, hoff.data(), sizeof(int32_t) * (nsl + 1), hipMemcpyHostToDevice, s));
+  CP_HIP(hipMemcpyAsync(bins, hbins.data(), sizeof(int32_t) * nbins, hipMemcpyHostToDevice, s));
+  hipLaunchKernelGGL(k_cp_fill, dim3(qh_blocks(nsl, 4)), dim3(256), 0, s, order, pos, A->rowptr, A->col, A->val,
+                     soff, nim, zc, diag, ev, ec, nsl);
+  CP_HIP(hipGetLastError());
+  CP_HIP(hipStreamSynchronize(s));  // the host vectors and the workspace go
+#undef CP_HIP
+  qh_free_ptr(wbuf);
+  c->a.bslice = bslice;
+  c->a.bins = bins;
+  c->a.soff = soff;
+  c->a.nim = nim;
+  c->a.order = order;
+  c->a.diag = diag;
+  c->a.ev = ev;
+  c->a.ec = ec;
+  c->trace = trace;
+  A->comp = c;
+  A->comp_state = 1;
+  return QH_OK;
+}
+
+}  // namespace
+
+int qh_comp_prepare(qh_mat *A, int *usable) {
+  *usable = 0;
+  if (A->comp_state == 0) {
+    // row and slot numbers are 32-bit
+    if (A->rows < 1 || A->rows > (int64_t)1 << 30)
+      A->comp_state = -1;
+    else if (int rc = cp_build(A))
+      return rc;
+  }
+  *usable = A->comp_state == 1;
+  return QH_OK;
+}
+
+int qh_comp_rk4(qh_mat *A, qh_vec *x, double dt, int64_t nsteps) {
+  hipStream_t s = qh_stream();
+  for (const CpClass &k : A->comp->classes) {
+    CpArgs a = A->comp->a;
+    a.bins += k.first;
+    a.x = x->d;
+    a.xlo = x->prec == QH_FP32 ? x->lo : nullptr;
+    a.cells = k.cells;
+    a.h = dt;
+    a.nsteps = nsteps;
+    int rc = QH_EINVAL;
+    if (k.W == 0) {
+      rc = cp_launch<CP_STREAM_S, 2, false>(k, a, s);
+    } else if (k.S == 2) {
+      rc = k.W == 4 ? cp_launch<2, 4, true>(k, a, s) : k.W == 8 ? cp_launch<2, 8, true>(k, a, s)
+                                                                : cp_launch<2, 12, true>(k, a, s);
+    } else {
+      switch (k.W) {
+        case 4: rc = cp_launch<1, 4, true>(k, a, s); break;
+        case 8: rc = cp_launch<1, 8, true>(k, a, s); break;
+        case 12: rc = cp_launch<1, 12, true>(k, a, s); break;
+        case 16: rc = cp_launch<1, 16, true>(k, a, s); break;
+        case 24: rc = cp_launch<1, 24, true>(k, a, s); break;
+        default: rc = cp_launch<1, 32, true>(k, a, s); break;
+      }
+    }
+    if (rc) return rc;
+  }
+  return QH_OK;
+}
+
+double *qh_comp_trace(const qh_mat *A) { return A->comp->trace; }

@@ -1264,13 +1264,13 @@ static int step_x(hipStream_t s, const qh_mat *A, int G, qh_vec *x, double h, hi
                             : rk4_step<float>(s, A, G, x->d, x->lo, g_st.y[0], g_st.y[1], h, ev);
 }
 
-static int renorm_launch(hipStream_t s, qh_vec *x, void *hi, int64_t tot, int64_t base) {
+// partial: 512 doubles, inv: one, in device memory
+static int renorm_launch(hipStream_t s, qh_vec *x, void *hi, int64_t tot, int64_t base, double *partial, double *inv) {
   const int nb = 512;
-  hipLaunchKernelGGL(k_trace_partial_f32, dim3(nb), dim3(256), 0, s, (const float2 *)hi, x->lo, tot, base,
-                     g_st.partial);
-  hipLaunchKernelGGL(k_trace_final, dim3(1), dim3(256), 0, s, g_st.partial, nb, g_st.inv);
+  hipLaunchKernelGGL(k_trace_partial_f32, dim3(nb), dim3(256), 0, s, (const float2 *)hi, x->lo, tot, base, partial);
+  hipLaunchKernelGGL(k_trace_final, dim3(1), dim3(256), 0, s, partial, nb, inv);
   hipLaunchKernelGGL(k_scale_by_dev, dim3(std::min<int64_t>(qh_blocks(x->n, 256), 8192)), dim3(256), 0, s,
-                     (float2 *)hi, x->lo, x->n, g_st.inv);
+                     (float2 *)hi, x->lo, x->n, inv);
   QH_HIP(hipGetLastError());
   return QH_OK;
 }
@@ -1688,7 +1688,7 @@ static int graph_prepare(const qh_mat *A, qh_vec *x, double dt, int64_t tot, int
   QH_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
   int crc = QH_OK;
   for (int st = 0; st < len && !crc; st++) crc = step_x(s, A, G, x, dt, nullptr);
-  if (!crc && renorm_every > 0) crc = renorm_launch(s, x, x->d, tot, 0);
+  if (!crc && renorm_every > 0) crc = renorm_launch(s, x, x->d, tot, 0, g_st.partial, g_st.inv);
   hipGraph_t g = nullptr;
   hipError_t ce = hipStreamEndCapture(s, &g);
   if (crc) {
@@ -1721,12 +1721,27 @@ static int rk4_impl(qh_mat *A, qh_vec *x, double dt, int64_t nsteps, int64_t tot
     if (nsteps == 0) return QH_OK;
     return rk4_small(A, x, dt, nsteps, tot, renorm_every);
   }
+  hipStream_t s = qh_stream();
+  // generators that fall apart into small closed sets of rows
+  if (!timed && !A->lanes_forced) {
+    int usable = 0;
+    rc = qh_comp_prepare(A, &usable);
+    if (rc) return rc;
+    if (usable) {
+      const int64_t len = renorm_every > 0 ? graph_len(renorm_every) : nsteps;
+      for (int64_t st = 0; st < nsteps && !rc; st += len) {
+        rc = qh_comp_rk4(A, x, dt, std::min<int64_t>(len, nsteps - st));
+        if (!rc && renorm_every > 0 && st + len <= nsteps)
+          rc = renorm_launch(s, x, x->d, tot, 0, qh_comp_trace(A), qh_comp_trace(A) + 512);
+      }
+      return rc;
+    }
+  }
   int G = 0;
   rc = lanes_for(A, x->prec, &G);
   if (rc) return rc;
   rc = stepper_prepare(A, x->prec, x->n);
   if (rc) return rc;
-  hipStream_t s = qh_stream();
   if (nsteps == 0) return QH_OK;
 
   if (timed) {
@@ -1736,7 +1751,7 @@ static int rk4_impl(qh_mat *A, qh_vec *x, double dt, int64_t nsteps, int64_t tot
     for (int64_t st = 0; st < nsteps; st++) {
       rc = step_x(s, A, G, x, dt, &ev[5 * st]);
       if (rc) return rc;
-      if (renorm_every > 0 && (st + 1) % renorm_every == 0) renorm_launch(s, x, x->d, tot, 0);
+      if (renorm_every > 0 && (st + 1) % renorm_every == 0) renorm_launch(s, x, x->d, tot, 0, g_st.partial, g_st.inv);
     }
     QH_HIP(hipStreamSynchronize(s));
     double tot_ms = 0.0;
@@ -1789,6 +1804,11 @@ extern "C" int qh_rk4_prepare(qh_mat *A, qh_vec *x, double dt, int64_t tot, int 
   QH_REQUIRE(renorm_every == 0 || (x->prec == QH_FP32 && tot > 0 && tot * tot == x->n), QH_EINVAL,
              "qh_rk4_prepare: trace renormalisation needs an FP32 density matrix of dimension tot");
   if (A->rows <= QH_SMALL_ROWS && !A->lanes_forced) return QH_OK;  // one-workgroup path: nothing to capture
+  if (!A->lanes_forced) {
+    int usable = 0;
+    rc = qh_comp_prepare(A, &usable);
+    if (rc || usable) return rc;
+  }
   int G = 0;
   rc = lanes_for(A, x->prec, &G);
   if (!rc) rc = stepper_prepare(A, x->prec, x->n);

@@ -1,0 +1,134 @@
+"""RK4 of generators whose rows fall apart into closed sets (qh_comp.hip), one set or
+several per workgroup, against the oracle's classic RK4 in FP64 and against the stage
+kernels that a forced variant selects: one and two rows a thread, entries in
+registers and in memory, slices with a remainder, real, imaginary and complex
+entries, rows without entries, uneven blocks of a batch."""
+import numpy as np
+import pytest
+
+import oracle
+import quac_amd as qa
+import recipes
+from qbuild import build_system
+
+pytestmark = pytest.mark.gpu
+
+
+def _tc(qubits, levels):
+    """emitters and a cavity: excitation numbers split the rows"""
+    c, terms = qubits, [("ham", 0.3, [(qubits, "n")])]
+    for i in range(qubits):
+        terms += [("ham", 0.1 + 0.02 * i, [(i, "raise"), (c, "lower")]), ("ham", 0.1 + 0.02 * i, [(c, "raise"), (i, "lower")])]
+        terms += [("lin", 0.02, [(i, "lower")])]
+    return {"subs": [("op", 2)] * qubits + [("op", levels)], "terms": terms + [("lin", 0.01, [(c, "lower")])], "mcwf": False}
+
+
+def _noisy(qubits, extra=()):
+    terms = [("lin", 0.02 + 0.01 * i, [(i, "lower")]) for i in range(qubits)]
+    terms += [("lin", 0.03, [(i, "sz")]) for i in range(qubits)]
+    return {"subs": [("op", 2)] * qubits, "terms": terms + list(extra), "mcwf": False}
+
+
+def _diagonal(levels):
+    """no off-diagonal entry: every row is a set"""
+    return {"subs": [("op", levels)], "terms": [("ham", 0.7, [(0, "n")]), ("lin", 0.05, [(0, "n")])], "mcwf": False}
+
+
+CASES = [
+    _tc(1, 15),  # bins of 1 to 2 slices
+    _tc(2, 9),
+    _tc(3, 17),  # a component of 1028 rows: two rows a thread
+    _noisy(6),
+    _noisy(8),  # more bins than two a CU: bins of several components, a launch per shape
+    _noisy(5, [("ham", 0.3, [(0, "sx")]), ("ham", 0.2, [(1, "sy")])]),  # real and imaginary entries
+    _diagonal(31),
+]
+
+
+def _start(n):
+    rng = np.random.default_rng(5)
+    psi = rng.normal(size=n) + 1j * rng.normal(size=n)
+    return np.outer(psi.conj(), psi).reshape(-1) / np.linalg.norm(psi) ** 2
+
+
+def _steps(A, x0, prec, dt, steps, **kw):
+    v = qa.DeviceVec(len(x0), prec)
+    v.set(x0)
+    qa.rk4_device(A, v, dt, steps, **kw)
+    return v.get()
+
+
+@pytest.mark.parametrize("recipe", CASES, ids=[str([n for _, n in c["subs"]]) for c in CASES])
+def test_closed_sets_match_oracle(recipe):
+    qs, _, _ = build_system(recipe)
+    A = qs.matrix()
+    tot, terms = recipes.oracle_terms(recipe)
+    x0, dt = _start(tot), 0.02
+    m = oracle.construct(tot, terms, dm=True)
+    rp, _, val = A.export()
+    norm = np.add.reduceat(np.abs(np.append(val, 0)), rp[:-1]).max() if len(val) else 0.0
+    for steps in (1, 7):
+        ref = m.rk4(x0, dt, steps)
+        for prec in (qa.FP64, qa.FP32):
+            # a few roundings of the state and of h A times it per step; FP32: the state
+            # is kept as two words, the generator in 64 bits
+            eps = 2.0 ** -53 if prec == qa.FP64 else 2.0 ** -47
+            tol = steps * np.abs(x0).max() * (2 * dt * norm + 8) * eps + (2.0 ** -47 if prec == qa.FP32 else 0.0)
+            got = _steps(A, x0, prec, dt, steps)
+            assert np.abs(got - ref).max() <= tol, (steps, prec)
+    A.set_lanes(8, 8)  # the stage kernels
+    ref = _steps(A, x0, qa.FP64, dt, 7)
+    A.set_lanes(0, 0)
+    assert np.abs(_steps(A, x0, qa.FP64, dt, 7) - ref).max() <= 7 * np.abs(x0).max() * (2 * dt * norm + 8) * 2.0 ** -52
+    qs.destroy()
+
+
+def test_entries_read_from_memory():
+    """13 slots a row and a component of 2048 rows and more: the kernel that reads its
+    entries from memory, beside the ones that hold them"""
+    r = _noisy(11)
+    qs, _, _ = build_system(r)
+    A = qs.matrix()
+    x0 = _start(2048)
+    got = _steps(A, x0, qa.FP64, 0.02, 3)
+    A.set_lanes(8, 0)
+    ref = _steps(A, x0, qa.FP64, 0.02, 3)
+    # rows of h A sum to at most 0.02 * 2 * 11 * 0.2 here
+    assert np.abs(got - ref).max() <= 3 * np.abs(x0).max() * 16 * 2.0 ** -53
+    qs.destroy()
+
+
+def test_renormalised_and_split_calls():
+    """a call's steps are the same in one call or several, and the trace is restored
+    every renorm_every steps"""
+    r = _tc(2, 12)
+    qs, _, _ = build_system(r)
+    A = qs.matrix()
+    x0 = _start(48)
+    one = _steps(A, x0, qa.FP64, 0.01, 9)
+    v = qa.DeviceVec(len(x0), qa.FP64)
+    v.set(x0)
+    for k in (1, 3, 5):
+        qa.rk4_device(A, v, 0.01, k)
+    assert np.array_equal(v.get(), one)
+    f = _steps(A, 1.5 * x0, qa.FP32, 0.01, 10, tot=48, renorm_every=10)
+    assert abs(np.trace(f.reshape(48, 48)) - 1.0) < 1e-12
+    qs.destroy()
+
+
+def test_batch_of_uneven_blocks():
+    sizes = [(1, 7), (2, 11), (1, 2), (3, 9)]
+    systems = [build_system(_tc(*s))[0] for s in sizes]
+    tots = [2 ** q * n for q, n in sizes]
+    b = qa.Batch([s.matrix() for s in systems], tots, prec=qa.FP64)
+    starts = [_start(t) for t in tots]
+    for i, x0 in enumerate(starts):
+        b.set_state(i, x0)
+    b.rk4(0.01, 6)
+    for i, (s, x0) in enumerate(zip(sizes, starts)):
+        tot, terms = recipes.oracle_terms(_tc(*s))
+        ref = oracle.construct(tot, terms, dm=True).rk4(x0, 0.01, 6)
+        assert np.abs(b.get_state(i) - ref).max() <= 6 * 16 * 2.0 ** -53
+    b.destroy()
+    for s in systems:
+        s.destroy()
