@@ -18,7 +18,8 @@
 //
 // What bounds it: at few bins the chain of LDS reads of one stage and its barrier
 // (0.3 to 1.5 us a stage, where a launch a stage takes 2.6 to 4.3 us), at many
-// the LDS reads, 16 B an entry.
+// the LDS reads, 16 B an entry: 12-qubit circuit (decay and dephasing), 10 steps of
+// 16.8 M rows in 1.4 ms, four launches a step of 233 us before.
 #include <algorithm>
 #include <vector>
 
@@ -226,8 +227,10 @@ struct CpArgs {
 // the W slots of a row live in registers (2.5 dwords each), so that a step reads
 // LDS only; otherwise they are read again at every stage (through the caches).
 // RK4 on a linear autonomous system in nested form, y <- x + c A y with c = h/4,
-// h/3, h/2, h, double buffered: one barrier a stage.
-template <int S, int W, bool REG>
+// h/3, h/2, h, double buffered: one barrier a stage.  SKIP: pairs of slots that none
+// of the slice's rows fills are passed over, which pays where the LDS is the bound
+// (bins on every CU); without it more reads are in flight at once.
+template <int S, int W, bool REG, bool SKIP>
 __global__ void __launch_bounds__(1024) k_comp_rk4(CpArgs a) {
   extern __shared__ double2 sm[];
   const int b = a.bins[blockIdx.x];
@@ -290,10 +293,11 @@ __global__ void __launch_bounds__(1024) k_comp_rk4(CpArgs a) {
           double p = 0.0, r = 0.0;
           if constexpr (REG) {
             // LDS reads in flight (a divisor of W; the registers allow fewer beside more slots)
-            constexpr int CH = S > 1 || W > 16 ? 4 : W % 8 == 0 ? 8 : W == 12 ? 6 : 4;
+            constexpr int CH = SKIP ? 2 : S > 1 || W > 16 ? (W == 10 || W == 12 ? 2 : 4) : W == 12 || W == 16 ? W / 2 : W;
             static_assert(W % CH == 0 && CH % 2 == 0, "whole chunks");
 #pragma unroll
             for (int e0 = 0; e0 < W; e0 += CH) {
+              if (SKIP && e0 >= wid[k]) continue;
               double2 t[CH];
 #pragma unroll
               for (int j = 0; j < CH; j++) {
@@ -313,7 +317,7 @@ __global__ void __launch_bounds__(1024) k_comp_rk4(CpArgs a) {
                 r = fma(v[k * W + e0 + j], t[j].y, r);
               }
             }
-            if (nim[k] == W) {
+            if (nim[k] == W || (SKIP && nim[k] > 0 && nim[k] >= wid[k])) {
               const double u = p;
               p = -r;
               r = u;
@@ -377,17 +381,18 @@ __global__ void __launch_bounds__(1024) k_comp_rk4(CpArgs a) {
 // one launch: bins of one shape
 struct CpClass {
   int threads, S, W;  // W 0: entries read from memory
+  bool skip, side;    // side: few blocks, launched beside the others
   int first, count;   // range of the plan's bin list
   int cells;
 };
 
-template <int S, int W, bool REG>
+template <int S, int W, bool REG, bool SKIP>
 int cp_launch(const CpClass &c, const CpArgs &a, hipStream_t s) {
   const size_t lds = (size_t)2 * c.cells * sizeof(double2);
   if (lds > 64 * 1024)
-    QH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_comp_rk4<S, W, REG>),
+    QH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_comp_rk4<S, W, REG, SKIP>),
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  hipLaunchKernelGGL((k_comp_rk4<S, W, REG>), dim3(c.count), dim3(c.threads), lds, s, a);
+  hipLaunchKernelGGL((k_comp_rk4<S, W, REG, SKIP>), dim3(c.count), dim3(c.threads), lds, s, a);
   QH_HIP(hipGetLastError());
   return QH_OK;
 }
@@ -399,10 +404,18 @@ struct qh_comp {
   CpArgs a{};
   double *trace = nullptr;  // QH_COMP_TRACE doubles for the trace renormalisation
   std::vector<CpClass> classes;
+  // launches of fewer blocks than CUs run on a stream of their own beside the
+  // others (disjoint rows), between two events of the library stream
+  hipStream_t side = nullptr;
+  hipEvent_t ev[2] = {nullptr, nullptr};
 };
 
 void qh_comp_free(qh_comp *c) {
   if (!c) return;
+  if (c->side) (void)hipStreamSynchronize(c->side);
+  for (hipEvent_t e : c->ev)
+    if (e) (void)hipEventDestroy(e);
+  if (c->side) (void)hipStreamDestroy(c->side);
   qh_free_ptr(c->buf);
   qh_free_ptr(c->slots);
   delete c;
@@ -595,8 +608,12 @@ int cp_build(qh_mat *A) {
   }
   hoff[nsl] = (int32_t)slots;
   // the shape of every bin's launch, and what the largest bin and all of them take
-  auto rup = [](int w) { return w <= 4 ? 4 : w <= 8 ? 8 : w <= 12 ? 12 : w <= 16 ? 16 : w <= 24 ? 24 : w <= 32 ? 32 : 0; };
   const bool few = nbins <= 2 * cus;  // the chip is not full: one launch, so that nothing waits for a launch before it
+  auto rup = [few](int w) {
+    for (int u : {4, 8, 10, 12, 16, 24, 32})
+      if (w <= u && (few || u != 10)) return u;
+    return 0;
+  };
   struct Shape {
     int stream, rows, W;
     int32_t bin;
@@ -637,7 +654,8 @@ int cp_build(qh_mat *A) {
     A->comp_state = -1;
     return QH_OK;
   }
-  if (few && !(few_rows > 1024 && few_w > 12))
+  const bool merge = few && !(few_rows > 1024 && few_w > 12);
+  if (merge)
     for (auto &q : sh)
       if (!q.stream) {
         q.rows = few_rows;
@@ -657,11 +675,19 @@ int cp_build(qh_mat *A) {
     const int W = q.stream ? 0 : q.W;
     if (c->classes.empty() || c->classes.back().threads != threads || c->classes.back().S != S ||
         c->classes.back().W != W)
-      c->classes.push_back(CpClass{threads, S, W, i, 0, 0});
+      c->classes.push_back(CpClass{threads, S, W, !merge, false, i, 0, 0});
     CpClass &k = c->classes.back();
     k.count++;
     k.cells = std::max(k.cells, (hslice[q.bin + 1] - hslice[q.bin]) * 64 + 1);
   }
+  for (CpClass &k : c->classes)
+    if (c->classes.size() > 1 && k.count < cus && k.first + k.count < nbins) {
+      k.side = true;
+      if (!c->side) {
+        CP_HIP(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
+        for (hipEvent_t &e : c->ev) CP_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+      }
+    }
   double *ev;
   uint16_t *ec;
   Carve tail;
@@ -711,32 +737,55 @@ int qh_comp_prepare(qh_mat *A, int *usable) {
 }
 
 int qh_comp_rk4(qh_mat *A, qh_vec *x, double dt, int64_t nsteps) {
+  const qh_comp &c = *A->comp;
   hipStream_t s = qh_stream();
-  for (const CpClass &k : A->comp->classes) {
-    CpArgs a = A->comp->a;
+  if (c.side) {
+    QH_HIP(hipEventRecord(c.ev[0], s));
+    QH_HIP(hipStreamWaitEvent(c.side, c.ev[0], 0));
+  }
+  for (const CpClass &k : c.classes) {
+    CpArgs a = c.a;
     a.bins += k.first;
     a.x = x->d;
     a.xlo = x->prec == QH_FP32 ? x->lo : nullptr;
     a.cells = k.cells;
     a.h = dt;
     a.nsteps = nsteps;
+    hipStream_t ks = k.side ? c.side : s;
     int rc = QH_EINVAL;
-    if (k.W == 0) {
-      rc = cp_launch<CP_STREAM_S, 2, false>(k, a, s);
-    } else if (k.S == 2) {
-      rc = k.W == 4 ? cp_launch<2, 4, true>(k, a, s) : k.W == 8 ? cp_launch<2, 8, true>(k, a, s)
-                                                                : cp_launch<2, 12, true>(k, a, s);
-    } else {
-      switch (k.W) {
-        case 4: rc = cp_launch<1, 4, true>(k, a, s); break;
-        case 8: rc = cp_launch<1, 8, true>(k, a, s); break;
-        case 12: rc = cp_launch<1, 12, true>(k, a, s); break;
-        case 16: rc = cp_launch<1, 16, true>(k, a, s); break;
-        case 24: rc = cp_launch<1, 24, true>(k, a, s); break;
-        default: rc = cp_launch<1, 32, true>(k, a, s); break;
-      }
+#define CP_CASE(SS, WW, SK)                    \
+  if (k.S == SS && k.W == WW && k.skip == SK) \
+    rc = cp_launch<SS, WW, true, SK>(k, a, ks);
+    if (k.W == 0) rc = cp_launch<CP_STREAM_S, 2, false, false>(k, a, ks);
+    CP_CASE(1, 4, false)
+    CP_CASE(1, 8, false)
+    CP_CASE(1, 10, false)
+    CP_CASE(1, 12, false)
+    CP_CASE(1, 16, false)
+    CP_CASE(1, 24, false)
+    CP_CASE(1, 32, false)
+    CP_CASE(2, 4, false)
+    CP_CASE(2, 8, false)
+    CP_CASE(2, 10, false)
+    CP_CASE(2, 12, false)
+    CP_CASE(1, 4, true)
+    CP_CASE(1, 8, true)
+    CP_CASE(1, 12, true)
+    CP_CASE(1, 16, true)
+    CP_CASE(1, 24, true)
+    CP_CASE(1, 32, true)
+    CP_CASE(2, 4, true)
+    CP_CASE(2, 8, true)
+    CP_CASE(2, 12, true)
+#undef CP_CASE
+    if (rc) {
+      qh_set_error("no kernel for bins of %d rows a thread and %d slots", k.S, k.W);
+      return rc;
     }
-    if (rc) return rc;
+  }
+  if (c.side) {
+    QH_HIP(hipEventRecord(c.ev[1], c.side));
+    QH_HIP(hipStreamWaitEvent(s, c.ev[1], 0));
   }
   return QH_OK;
 }
