@@ -155,8 +155,8 @@ struct qh_mat {
   int32_t ks2_maxslots = 0;    // most slots of a slice
   int64_t ks2_slots = 0, ks2_nval = 0, ks2_nsval = 0, ks2_nsval1 = 0, ks2_nsep = 0, ks2_ngh = 0, ks2_nsepblk = 0;
   std::vector<int64_t> blk_off;  // row offsets of the blocks of a block-diagonal matrix (and its row count)
-  int comp_state = 0;          // 0 not looked at, 1 plan in comp, -1 not worth it
-  qh_comp *comp = nullptr;
+  int comp_state[2] = {0, 0};  // for FP64 and FP32 states: 0 not looked at, 1 plan in comp, -1 not worth it
+  qh_comp *comp[2] = {nullptr, nullptr};
   qh_td_cache *td_cache = nullptr;  // built by the first time-dependent RHS on this matrix
 };
 // variant codes selecting the sliced-ELL kernel: 128 / 129 / 130 process 2 / 4 / 8
@@ -205,9 +205,9 @@ int qh_rk3bs_td_sliced(qh_mat *A, const qh_vec *x, qh_vec *xn, qh_vec *k1, qh_ve
 // kernels; nsteps steps of x in place on the library stream; QH_COMP_TRACE doubles
 // of device memory that the trace renormalisation of x may use (kept with the plan)
 #define QH_COMP_TRACE 1024
-int qh_comp_prepare(qh_mat *A, int *usable);
+int qh_comp_prepare(qh_mat *A, int prec, int *usable);
 int qh_comp_rk4(qh_mat *A, qh_vec *x, double dt, int64_t nsteps);
-double *qh_comp_trace(const qh_mat *A);
+double *qh_comp_trace(const qh_mat *A, int prec);
 
 // longest row of A into A->max_row (computed once per matrix)
 int qh_mat_max_row(qh_mat *A);

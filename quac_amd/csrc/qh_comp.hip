@@ -16,10 +16,15 @@
 // number of slots a slice), then the real parts, each a value and the 16-bit index
 // of its column within the bin.
 //
+// A set too large for that keeps its vector in LDS and reads its entries at every
+// stage, as 32-bit words of a column and an index into the bin's table of distinct
+// values (an entry repeats a few products of couplings and square roots).
+//
 // What bounds it: at few bins the chain of LDS reads of one stage and its barrier
 // (0.3 to 1.5 us a stage, where a launch a stage takes 2.6 to 4.3 us), at many
 // the LDS reads, 16 B an entry: 12-qubit circuit (decay and dephasing), 10 steps of
-// 16.8 M rows in 1.4 ms, four launches a step of 233 us before.
+// 16.8 M rows in 1.4 ms, four launches a step of 233 us before; 512 systems of 100 to
+// 230 400 rows in FP32, 10 steps of 16 M rows in 3.7 ms, 8.4 ms before.
 #include <algorithm>
 #include <vector>
 
@@ -31,9 +36,12 @@ namespace {
 
 const int CP_GRAN = 64;         // rows of a granule: the components that start in 64 consecutive sorted rows
 const int CP_REG_ROWS = 2048;   // largest bin with its entries in registers (1024 threads, two rows each)
-const int CP_MAX_ROWS = 5056;   // largest bin: two buffers of rows + 1 complex128 in 160 KB of LDS
+const int CP_DICT = 1024;       // values of a bin's table, zero among them
+// largest bin: two buffers of rows + 1 entries (complex128, or complex64 for an FP32
+// state) and the table in 160 KB of LDS, 6 or 8 rows a thread
+const int CP_MAX_ROWS64 = 4800, CP_MAX_ROWS32 = 8128;
+const int CP_DICT_W = 12;       // words of a row fetched ahead
 const int CP_PROBE_ROWS = 16384;  // rows looked at before a large matrix as a whole
-const int CP_STREAM_S = 5;      // rows a thread of the kernel that reads its entries from memory
 const int CP_PACK_ROWS = 512;   // bins of small components are filled to this size once they outnumber the CUs
 
 // -------------------------------------------------------------- components
@@ -176,17 +184,19 @@ __global__ void __launch_bounds__(256) k_cp_width(const int32_t *order, const in
   }
 }
 
-// the entries of every slice; zc[s]: index of the bin's zero cell, read by the
-// slots that a row does not fill
+// the diagonal of every slice, and the entries of those whose bin holds them in
+// registers; zc[s]: index of the bin's zero cell, read by the slots that a row does
+// not fill, or -1 where the bin reads words
 __global__ void __launch_bounds__(256) k_cp_fill(const int32_t *order, const int32_t *pos,
                                                  const int32_t *__restrict__ rp, const int32_t *__restrict__ col,
                                                  const double2 *__restrict__ val, const int32_t *soff,
-                                                 const int32_t *nim, const int32_t *zc, double2 *diag, double *ev,
-                                                 uint16_t *ec, int32_t nslices) {
+                                                 const int32_t *width, const int32_t *nim, const int32_t *zc,
+                                                 double2 *diag, double *ev, uint16_t *ec, int32_t nslices) {
   const int32_t s = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (s >= nslices) return;
   const int32_t r = order[(int64_t)s * 64 + lane];
-  const int64_t s0 = soff[s], s1 = soff[s + 1];
+  const bool reg = zc[s] >= 0;
+  const int64_t s0 = soff[s], s1 = s0 + width[s];
   int64_t pi = s0, pr = s0 + nim[s];
   double2 d = make_double2(0.0, 0.0);
   auto put = [&](int64_t slot, double v, int32_t c) {
@@ -200,82 +210,179 @@ __global__ void __launch_bounds__(256) k_cp_fill(const int32_t *order, const int
         d = v;
         continue;
       }
+      if (!reg) continue;
       const int32_t c = pos[col[e]];
       if (v.y != 0.0) put(pi++, v.y, c);
       if (v.x != 0.0) put(pr++, v.x, c);
     }
+  diag[(int64_t)s * 64 + lane] = d;
+  if (!reg) return;
   for (; pi < s0 + nim[s]; pi++) put(pi, 0.0, zc[s]);
   for (; pr < s1; pr++) put(pr, 0.0, zc[s]);
-  diag[(int64_t)s * 64 + lane] = d;
+}
+
+// The table and the words of one bin a workgroup: every distinct value of an entry
+// goes through a hash table in LDS (open addressing; the host takes the plan back
+// when a bin has more than CP_DICT - 1).  A word is the column's index plus one
+// (cell 0 is the zero cell) and, above it, the byte offset of the value.
+__global__ void __launch_bounds__(1024) k_cp_dict(const int32_t *bins, const int32_t *bslice, const int32_t *order,
+                                                  const int32_t *pos, const int32_t *__restrict__ rp,
+                                                  const int32_t *__restrict__ col, const double2 *__restrict__ val,
+                                                  const int32_t *soff, const int32_t *width, const int32_t *nim,
+                                                  uint32_t *ew, double *dict, int32_t *overflow) {
+  const int CELLS = 4 * CP_DICT;
+  __shared__ unsigned long long key[CELLS];
+  __shared__ int32_t id[CELLS], count;
+  const int32_t sl0 = bslice[bins[blockIdx.x]], nsl = bslice[bins[blockIdx.x] + 1] - sl0;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  for (int i = threadIdx.x; i < CELLS; i += 1024) key[i] = 0ull;
+  if (threadIdx.x == 0) count = 0;
+  __syncthreads();
+  auto cell = [&](double v, bool insert) -> int {
+    const unsigned long long k = (unsigned long long)__double_as_longlong(v);
+    unsigned h = (unsigned)((k * 0x9E3779B97F4A7C15ull) >> 52) & (CELLS - 1);
+    for (int i = 0; i < CELLS; i++, h = (h + 1) & (CELLS - 1)) {
+      unsigned long long old = *(volatile unsigned long long *)&key[h];
+      if (old == 0ull && insert) {
+        old = atomicCAS(&key[h], 0ull, k);
+        if (old == 0ull) {
+          atomicAdd(&count, 1);
+          return (int)h;
+        }
+      }
+      if (old == k) return (int)h;
+    }
+    return 0;  // full: the bin overflows
+  };
+  // a bin over the limit stops taking values, long before the table is full
+  for (int32_t s = wave; s < nsl; s += 16) {
+    const int32_t r = order[(int64_t)(sl0 + s) * 64 + lane];
+    if (r < 0 || *(volatile int32_t *)&count >= CP_DICT) continue;
+    for (int32_t e = rp[r]; e < rp[r + 1]; e++) {
+      if (col[e] == r) continue;
+      const double2 v = val[e];
+      if (v.y != 0.0) cell(v.y, true);
+      if (v.x != 0.0) cell(v.x, true);
+    }
+  }
+  __syncthreads();
+  const bool over = count >= CP_DICT;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    if (over) overflow[0] = 1;
+    count = 1;
+    dict[(int64_t)blockIdx.x * CP_DICT] = 0.0;
+  }
+  if (over) return;  // the whole workgroup
+  __syncthreads();
+  for (int i = threadIdx.x; i < CELLS; i += 1024)
+    if (key[i]) {
+      id[i] = atomicAdd(&count, 1);
+      dict[(int64_t)blockIdx.x * CP_DICT + id[i]] = __longlong_as_double((long long)key[i]);
+    }
+  __syncthreads();
+  for (int32_t s = wave; s < nsl; s += 16) {
+    const int32_t r = order[(int64_t)(sl0 + s) * 64 + lane];
+    const int64_t s0 = soff[sl0 + s], s1 = s0 + width[sl0 + s];
+    int64_t pi = s0, pr = s0 + nim[sl0 + s];
+    const int64_t p1 = pr;
+    auto put = [&](int64_t slot, double v, int32_t c) {
+      ew[slot * 64 + lane] = (uint32_t)(pos[c] + 1) | ((uint32_t)id[cell(v, false)] * 8u) << 16;
+    };
+    if (r >= 0)
+      for (int32_t e = rp[r]; e < rp[r + 1]; e++) {
+        if (col[e] == r) continue;
+        const double2 v = val[e];
+        if (v.y != 0.0) put(pi++, v.y, col[e]);
+        if (v.x != 0.0) put(pr++, v.x, col[e]);
+      }
+    for (; pi < p1; pi++) ew[pi * 64 + lane] = 0u;
+    for (; pr < s1; pr++) ew[pr * 64 + lane] = 0u;
+  }
 }
 
 // ------------------------------------------------------------------ stepping
 struct CpArgs {
   const int32_t *bins, *bslice;  // this launch's bins; first slice of every bin
-  const int32_t *soff, *nim, *order;
+  const int32_t *soff, *width, *nim, *order;
   const double2 *diag;
-  const double *ev;
+  const double *ev;    // entries held in registers: values and columns
   const uint16_t *ec;
+  const uint32_t *ew;  // entries read as words, and this launch's first table
+  const double *dict;
   void *x;
   float2 *xlo;   // the low words of an FP32 state, else null
-  int32_t cells;  // complex128 of one LDS buffer
+  int32_t cells;  // entries of one LDS buffer
   double h;
   int64_t nsteps;
 };
 
-// A thread owns S rows of the bin, wavefront w the slices w, w + waves, ...  REG:
-// the W slots of a row live in registers (2.5 dwords each), so that a step reads
-// LDS only; otherwise they are read again at every stage (through the caches).
+// entry r of the state as complex128, and back (an FP32 state is the sum of two words)
+__device__ inline double2 cp_load(const CpArgs &a, int32_t r) {
+  if (!a.xlo) return ((const double2 *)a.x)[r];
+  const float2 hi = ((const float2 *)a.x)[r], lo = a.xlo[r];
+  return make_double2((double)hi.x + (double)lo.x, (double)hi.y + (double)lo.y);
+}
+__device__ inline void cp_store(const CpArgs &a, int32_t r, double2 v) {
+  if (!a.xlo) {
+    ((double2 *)a.x)[r] = v;
+    return;
+  }
+  const float hr = (float)v.x, hm = (float)v.y;
+  ((float2 *)a.x)[r] = make_float2(hr, hm);
+  a.xlo[r] = make_float2((float)(v.x - (double)hr), (float)(v.y - (double)hm));
+}
+// the imaginary parts of a row are summed first, then the sum is turned by i and the
+// real parts follow
+__device__ inline void cp_times_i(double &p, double &r) {
+  const double u = p;
+  p = -r;
+  r = u;
+}
+
+// A thread owns S rows of the bin, wavefront w the slices w, w + waves, ...; the W
+// slots of a row live in registers (2.5 dwords each), so that a step reads LDS only.
 // RK4 on a linear autonomous system in nested form, y <- x + c A y with c = h/4,
 // h/3, h/2, h, double buffered: one barrier a stage.  SKIP: pairs of slots that none
 // of the slice's rows fills are passed over, which pays where the LDS is the bound
 // (bins on every CU); without it more reads are in flight at once.
-template <int S, int W, bool REG, bool SKIP>
+template <int S, int W, bool SKIP>
 __global__ void __launch_bounds__(1024) k_comp_rk4(CpArgs a) {
   extern __shared__ double2 sm[];
   const int b = a.bins[blockIdx.x];
   const int32_t sl0 = a.bslice[b], nsl = a.bslice[b + 1] - sl0;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
-  double2 x[S], y[REG ? S : 1], d[REG ? S : 1];
-  int32_t row[S], nim[S], s0[S], wid[S];
-  double v[REG ? S * W : 1];
-  uint32_t c2[REG ? S * W / 2 : 1];
+  double2 x[S], y[S], d[S];
+  int32_t row[S], nim[S], wid[S];
+  double v[S * W];
+  uint32_t c2[S * W / 2];
 #pragma unroll
   for (int k = 0; k < S; k++) {
     const int32_t sl = wave + k * waves;
+    int32_t s0 = 0;
     row[k] = -1;
-    nim[k] = wid[k] = s0[k] = 0;
-    x[k] = make_double2(0.0, 0.0);
-    if (REG) d[k] = x[k];
+    nim[k] = wid[k] = 0;
+    x[k] = d[k] = make_double2(0.0, 0.0);
     if (sl < nsl) {
       const int64_t p = (int64_t)(sl0 + sl) * 64 + lane;
       row[k] = a.order[p];
-      s0[k] = a.soff[sl0 + sl];
-      wid[k] = a.soff[sl0 + sl + 1] - s0[k];
+      s0 = a.soff[sl0 + sl];
+      wid[k] = a.width[sl0 + sl];
       nim[k] = a.nim[sl0 + sl];
-      if (REG) d[k] = a.diag[p];
-      if (row[k] >= 0) {
-        if (a.xlo) {
-          const float2 hi = ((const float2 *)a.x)[row[k]], lo = a.xlo[row[k]];
-          x[k] = make_double2((double)hi.x + (double)lo.x, (double)hi.y + (double)lo.y);
-        } else {
-          x[k] = ((const double2 *)a.x)[row[k]];
-        }
-      }
+      d[k] = a.diag[p];
+      if (row[k] >= 0) x[k] = cp_load(a, row[k]);
       sm[sl * 64 + lane] = x[k];
     }
-    if constexpr (REG) {
-      y[k] = x[k];
+    y[k] = x[k];
 #pragma unroll
-      for (int e = 0; e < W; e += 2) {
-        const bool f = e < wid[k], g = e + 1 < wid[k];
-        const int64_t at = (int64_t)(s0[k] + e) * 64 + lane;
-        v[k * W + e] = f ? a.ev[at] : 0.0;
-        v[k * W + e + 1] = g ? a.ev[at + 64] : 0.0;
-        const uint32_t z = (uint32_t)nsl * 64u;
-        const uint32_t lo = f ? a.ec[at] : z, hi = g ? a.ec[at + 64] : z;
-        c2[(k * W + e) / 2] = lo | (hi << 16);
-      }
+    for (int e = 0; e < W; e += 2) {
+      const bool f = e < wid[k], g = e + 1 < wid[k];
+      const int64_t at = (int64_t)(s0 + e) * 64 + lane;
+      v[k * W + e] = f ? a.ev[at] : 0.0;
+      v[k * W + e + 1] = g ? a.ev[at + 64] : 0.0;
+      const uint32_t z = (uint32_t)nsl * 64u;
+      const uint32_t lo = f ? a.ec[at] : z, hi = g ? a.ec[at + 64] : z;
+      c2[(k * W + e) / 2] = lo | (hi << 16);
     }
   }
   if (threadIdx.x == 0) sm[nsl * 64] = sm[a.cells + nsl * 64] = make_double2(0.0, 0.0);
@@ -291,108 +398,177 @@ __global__ void __launch_bounds__(1024) k_comp_rk4(CpArgs a) {
         const int32_t sl = wave + k * waves;
         if (sl < nsl) {
           double p = 0.0, r = 0.0;
-          if constexpr (REG) {
-            // LDS reads in flight (a divisor of W; the registers allow fewer beside more slots)
-            constexpr int CH = SKIP ? 2 : S > 1 || W > 16 ? (W == 10 || W == 12 ? 2 : 4) : W == 12 || W == 16 ? W / 2 : W;
-            static_assert(W % CH == 0 && CH % 2 == 0, "whole chunks");
+          // LDS reads in flight (a divisor of W; the registers allow fewer beside more slots)
+          constexpr int CH = SKIP ? 2 : S > 1 || W > 16 ? (W == 10 || W == 12 ? 2 : 4) : W == 12 || W == 16 ? W / 2 : W;
+          static_assert(W % CH == 0 && CH % 2 == 0, "whole chunks");
 #pragma unroll
-            for (int e0 = 0; e0 < W; e0 += CH) {
-              if (SKIP && e0 >= wid[k]) continue;
-              double2 t[CH];
+          for (int e0 = 0; e0 < W; e0 += CH) {
+            if (SKIP && e0 >= wid[k]) continue;
+            double2 t[CH];
 #pragma unroll
-              for (int j = 0; j < CH; j++) {
-                const uint32_t w = c2[(k * W + e0 + j) / 2];
-                const uint32_t at = j & 1 ? (w >> 12) & 0xFFFF0u : (w << 4) & 0xFFFF0u;
-                t[j] = *(const double2 *)(in + at);
-              }
+            for (int j = 0; j < CH; j++) {
+              const uint32_t w = c2[(k * W + e0 + j) / 2];
+              const uint32_t at = j & 1 ? (w >> 12) & 0xFFFF0u : (w << 4) & 0xFFFF0u;
+              t[j] = *(const double2 *)(in + at);
+            }
 #pragma unroll
-              for (int j = 0; j < CH; j++) {
-                // the imaginary parts are summed: times i, and the real parts follow
-                if (!(j & 1) && nim[k] == e0 + j) {
-                  const double u = p;
-                  p = -r;
-                  r = u;
-                }
-                p = fma(v[k * W + e0 + j], t[j].x, p);
-                r = fma(v[k * W + e0 + j], t[j].y, r);
-              }
-            }
-            if (nim[k] == W || (SKIP && nim[k] > 0 && nim[k] >= wid[k])) {
-              const double u = p;
-              p = -r;
-              r = u;
-            }
-          } else {
-            const double *ev = a.ev + (int64_t)s0[k] * 64 + lane;
-            const uint16_t *ec = a.ec + (int64_t)s0[k] * 64 + lane;
-#pragma unroll 4
-            for (int32_t e = 0; e < nim[k]; e++) {
-              const double2 t = *(const double2 *)(in + (uint32_t)ec[e * 64] * 16u);
-              p = fma(ev[e * 64], t.x, p);
-              r = fma(ev[e * 64], t.y, r);
-            }
-            const double u = p;
-            p = -r;
-            r = u;
-#pragma unroll 4
-            for (int32_t e = nim[k]; e < wid[k]; e++) {
-              const double2 t = *(const double2 *)(in + (uint32_t)ec[e * 64] * 16u);
-              p = fma(ev[e * 64], t.x, p);
-              r = fma(ev[e * 64], t.y, r);
+            for (int j = 0; j < CH; j++) {
+              if (!(j & 1) && nim[k] == e0 + j) cp_times_i(p, r);
+              p = fma(v[k * W + e0 + j], t[j].x, p);
+              r = fma(v[k * W + e0 + j], t[j].y, r);
             }
           }
-          double2 yk, dk;
-          if constexpr (REG) {
-            yk = y[k];
-            dk = d[k];
-          } else {
-            yk = ((const double2 *)in)[sl * 64 + lane];
-            dk = a.diag[(int64_t)(sl0 + sl) * 64 + lane];
-          }
-          p = fma(dk.x, yk.x, fma(-dk.y, yk.y, p));
-          r = fma(dk.x, yk.y, fma(dk.y, yk.x, r));
-          yk.x = fma(cs[q], p, x[k].x);
-          yk.y = fma(cs[q], r, x[k].y);
-          out[sl * 64 + lane] = yk;
-          if (REG) y[k] = yk;
-          else if (q == 3) x[k] = yk;
+          if (nim[k] == W || (SKIP && nim[k] > 0 && nim[k] >= wid[k])) cp_times_i(p, r);
+          p = fma(d[k].x, y[k].x, fma(-d[k].y, y[k].y, p));
+          r = fma(d[k].x, y[k].y, fma(d[k].y, y[k].x, r));
+          y[k].x = fma(cs[q], p, x[k].x);
+          y[k].y = fma(cs[q], r, x[k].y);
+          out[sl * 64 + lane] = y[k];
         }
       }
       __syncthreads();
     }
-    if constexpr (REG) {
 #pragma unroll
-      for (int k = 0; k < S; k++) x[k] = y[k];
+    for (int k = 0; k < S; k++) x[k] = y[k];
+  }
+#pragma unroll
+  for (int k = 0; k < S; k++)
+    if (row[k] >= 0) cp_store(a, row[k], x[k]);
+}
+
+// a wavefront's scalar, kept from being expanded into one condition per slot ahead of
+// the step loop (they would spill)
+__device__ inline int32_t cp_opaque(int32_t v) {
+  asm volatile("" : "+s"(v));
+  return v;
+}
+
+// The same steps with the entries read as words at every stage, the next slice's
+// CP_DICT_W words in flight during the products of this one.  Y: the stage vectors
+// in LDS (complex64 for an FP32 state, whose x stays in 64 bits); products and sums
+// in 64 bits.  1024 threads, S rows each (even, so that the two word buffers keep
+// their parity from stage to stage).
+template <typename Y, int S>
+__global__ void __launch_bounds__(1024) k_comp_dict(CpArgs a) {
+  static_assert(S % 2 == 0, "two word buffers");
+  extern __shared__ double2 sm[];
+  constexpr int WC = CP_DICT_W;
+  Y *buf = (Y *)sm;
+  double *dict = (double *)(buf + 2 * a.cells);
+  const int b = a.bins[blockIdx.x];
+  const int32_t sl0 = a.bslice[b], nsl = a.bslice[b + 1] - sl0;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (int i = threadIdx.x; i < CP_DICT; i += 1024) dict[i] = a.dict[(int64_t)blockIdx.x * CP_DICT + i];
+  double2 x[S], d[S];
+  int32_t wn[S], s0[S];  // width << 16 | imaginary slots; first slot
+  uint32_t w[2][WC];
+#pragma unroll
+  for (int k = 0; k < S; k++) {
+    const int32_t sl = wave + k * 16;
+    wn[k] = s0[k] = 0;
+    x[k] = d[k] = make_double2(0.0, 0.0);
+    if (sl < nsl) {
+      const int64_t p = (int64_t)(sl0 + sl) * 64 + lane;
+      const int32_t row = a.order[p];
+      s0[k] = a.soff[sl0 + sl];
+      wn[k] = a.width[sl0 + sl] << 16 | a.nim[sl0 + sl];
+      d[k] = a.diag[p];
+      if (row >= 0) x[k] = cp_load(a, row);
+      Y t;
+      t.x = x[k].x;
+      t.y = x[k].y;
+      buf[sl * 64 + lane + 1] = t;
+    }
+  }
+  // words past a slice's last slot read as zero: the zero cell times zero
+  auto fetch = [&](int k, uint32_t(&to)[WC]) {
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint32_t *>(a.ew + (int64_t)cp_opaque(s0[k]) * 64), (short)0, (cp_opaque(wn[k]) >> 16) * 256,
+        0x00020000);
+#pragma unroll
+    for (int e = 0; e < WC; e++)
+      to[e] = __builtin_amdgcn_raw_buffer_load_b32(rs, (uint32_t)(lane * 4 + e * 256), 0, 0);
+  };
+  fetch(0, w[0]);
+  if (threadIdx.x == 0) {
+    Y z;
+    z.x = z.y = 0;
+    buf[0] = buf[a.cells] = z;
+  }
+  __syncthreads();
+  const double cs[4] = {a.h / 4.0, a.h / 3.0, a.h / 2.0, a.h};
+  for (int64_t st = 0; st < a.nsteps; st++) {
+#pragma unroll 1
+    for (int q = 0; q < 4; q++) {
+      const Y *in = buf + (q & 1 ? a.cells : 0);
+      Y *out = buf + (q & 1 ? 0 : a.cells);
+      const double c = q == 0 ? cs[0] : q == 1 ? cs[1] : q == 2 ? cs[2] : cs[3];
+#pragma unroll
+      for (int k = 0; k < S; k++) {
+        const int32_t sl = wave + k * 16;
+        if (k + 1 == S)
+          fetch(0, w[0]);
+        else if (sl + 16 < nsl)
+          fetch((k + 1) % S, w[(k + 1) & 1]);
+        __builtin_amdgcn_sched_barrier(0);  // issued before this slice's products
+        if (sl < nsl) {
+          const int32_t wnk = cp_opaque(wn[k]), wid = wnk >> 16, nim = wnk & 0xFFFF;
+          double p = 0.0, r = 0.0;
+          auto term = [&](uint32_t u) {
+            const Y t = in[u & 0xFFFFu];
+            const double v = *(const double *)((const char *)dict + (u >> 16));
+            p = fma(v, (double)t.x, p);
+            r = fma(v, (double)t.y, r);
+          };
+#pragma unroll
+          for (int e = 0; e < WC; e += 2) {
+            if (e >= wid) continue;
+            if (nim == e) cp_times_i(p, r);
+            term(w[k & 1][e]);
+            term(w[k & 1][e + 1]);
+          }
+          for (int32_t e = WC; e < wid; e++) {
+            if (nim == e) cp_times_i(p, r);
+            term(a.ew[(int64_t)(s0[k] + e) * 64 + lane]);
+          }
+          if (nim > 0 && nim >= wid) cp_times_i(p, r);
+          const Y own = in[sl * 64 + lane + 1];
+          p = fma(d[k].x, (double)own.x, fma(-d[k].y, (double)own.y, p));
+          r = fma(d[k].x, (double)own.y, fma(d[k].y, (double)own.x, r));
+          p = fma(c, p, x[k].x);
+          r = fma(c, r, x[k].y);
+          if (q == 3) x[k] = make_double2(p, r);
+          Y t;
+          t.x = p;
+          t.y = r;
+          out[sl * 64 + lane + 1] = t;
+        }
+      }
+      __syncthreads();
     }
   }
 #pragma unroll
   for (int k = 0; k < S; k++) {
-    if (row[k] < 0) continue;
-    if (a.xlo) {
-      const float hr = (float)x[k].x, hm = (float)x[k].y;
-      ((float2 *)a.x)[row[k]] = make_float2(hr, hm);
-      a.xlo[row[k]] = make_float2((float)(x[k].x - (double)hr), (float)(x[k].y - (double)hm));
-    } else {
-      ((double2 *)a.x)[row[k]] = x[k];
-    }
+    const int32_t sl = wave + k * 16;
+    if (sl >= nsl) continue;
+    const int32_t row = a.order[(int64_t)(sl0 + sl) * 64 + lane];
+    if (row >= 0) cp_store(a, row, x[k]);
   }
 }
 
 // one launch: bins of one shape
 struct CpClass {
-  int threads, S, W;  // W 0: entries read from memory
+  int threads, S, W;  // W 0: entries read as words
   bool skip, side;    // side: few blocks, launched beside the others
   int first, count;   // range of the plan's bin list
   int cells;
 };
 
-template <int S, int W, bool REG, bool SKIP>
-int cp_launch(const CpClass &c, const CpArgs &a, hipStream_t s) {
-  const size_t lds = (size_t)2 * c.cells * sizeof(double2);
+int cp_launch(void (*kernel)(CpArgs), const CpClass &c, const CpArgs &a, size_t lds, hipStream_t s) {
   if (lds > 64 * 1024)
-    QH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_comp_rk4<S, W, REG, SKIP>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  hipLaunchKernelGGL((k_comp_rk4<S, W, REG, SKIP>), dim3(c.count), dim3(c.threads), lds, s, a);
+    QH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)lds));
+  hipLaunchKernelGGL(kernel, dim3(c.count), dim3(c.threads), lds, s, a);
   QH_HIP(hipGetLastError());
   return QH_OK;
 }
@@ -436,10 +612,13 @@ struct Carve {
 };
 
 // time of a stage in clocks of a CU: a slot of a slice is 64 LDS reads of 16 B (8
-// clocks at 128 B a clock, 10 measured), with 64 entries of 10 B from the caches 32
-const double CP_CLK_REG = 10.0, CP_CLK_MEM = 32.0, CP_CLK_FIXED = 500.0;
+// clocks at 128 B a clock, 10 measured), as words 64 reads of the vector and of the
+// table
+const double CP_CLK_REG = 10.0, CP_CLK_WORD = 24.0, CP_CLK_FIXED = 500.0;
 
-int cp_build(qh_mat *A) {
+int cp_build(qh_mat *A, int f32) {
+  const int32_t max_rows = f32 ? CP_MAX_ROWS32 : CP_MAX_ROWS64;
+  int &state = A->comp_state[f32];
   const int32_t n = (int32_t)A->rows;
   hipStream_t s = qh_stream();
   const unsigned nb256 = qh_blocks(n, 256);
@@ -508,9 +687,9 @@ int cp_build(qh_mat *A) {
     hipLaunchKernelGGL(k_cc_largest, dim3(std::min(nbp, 256u)), dim3(256), 0, s, size, off, m);
     CP_HIP(hipMemcpyAsync(&most, off, sizeof(int32_t), hipMemcpyDeviceToHost, s));
     CP_HIP(hipStreamSynchronize(s));
-    if (most > CP_MAX_ROWS) {
+    if (most > max_rows) {
       fail(0);
-      A->comp_state = -1;
+      state = -1;
       return QH_OK;
     }
   }
@@ -547,9 +726,9 @@ int cp_build(qh_mat *A) {
     cur += hg[g];
   }
   close();
-  if (largest > CP_MAX_ROWS) {
+  if (largest > max_rows) {
     fail(0);
-    A->comp_state = -1;
+    state = -1;
     return QH_OK;
   }
   const int32_t nbins = (int32_t)hrow.size() - 1, nsl = hslice.back();
@@ -559,7 +738,7 @@ int cp_build(qh_mat *A) {
   // `parent` and `size` are free from here: the sort's second buffers
   hipLaunchKernelGGL(k_cp_keys, dim3(nb256), dim3(256), 0, s, lab, off, gbin, key, row, n);
   CP_HIP(hipcub::DeviceRadixSort::SortPairs(tmp, tb, key, parent, row, size, n, 0, bits, s));
-  int32_t *order, *bslice, *soff, *nim, *zc, *width, *bins;
+  int32_t *order, *bslice, *soff, *nim, *zc, *width, *bins, *over;
   double2 *diag;
   double *trace;
   auto head = [&](Carve &q) {
@@ -570,6 +749,7 @@ int cp_build(qh_mat *A) {
     zc = q.take<int32_t>(nsl);
     width = q.take<int32_t>(nsl);
     bins = q.take<int32_t>(nbins);
+    over = q.take<int32_t>(1);
     diag = q.take<double2>((size_t)nsl * 64);
     trace = q.take<double>(QH_COMP_TRACE);
   };
@@ -582,31 +762,16 @@ int cp_build(qh_mat *A) {
   hw.p = (char *)hbuf;
   head(hw);
   c->buf = hbuf;
-  std::vector<int32_t> hzc(nsl);
-  for (int32_t b = 0; b < nbins; b++)
-    for (int32_t i = hslice[b]; i < hslice[b + 1]; i++) hzc[i] = (hslice[b + 1] - hslice[b]) * 64;
   CP_HIP(hipMemcpyAsync(bslice, hslice.data(), sizeof(int32_t) * (nbins + 1), hipMemcpyHostToDevice, s));
-  CP_HIP(hipMemcpyAsync(zc, hzc.data(), sizeof(int32_t) * nsl, hipMemcpyHostToDevice, s));
   hipLaunchKernelGGL(k_cp_fill_order, dim3(qh_blocks((int64_t)nsl * 64, 256)), dim3(256), 0, s, order,
                      (int64_t)nsl * 64);
   hipLaunchKernelGGL(k_cp_place, dim3(nb256), dim3(256), 0, s, parent, size, brow, bslice, order, pos, n);
   hipLaunchKernelGGL(k_cp_width, dim3(qh_blocks(nsl, 4)), dim3(256), 0, s, order, A->rowptr, A->col, A->val, width,
                      nim, nsl);
   CP_HIP(hipGetLastError());
-  std::vector<int32_t> hwid(nsl), hoff(nsl + 1);
+  std::vector<int32_t> hwid(nsl), hoff(nsl), hzc(nsl);
   CP_HIP(hipMemcpyAsync(hwid.data(), width, sizeof(int32_t) * nsl, hipMemcpyDeviceToHost, s));
   CP_HIP(hipStreamSynchronize(s));
-  int64_t slots = 0;
-  for (int32_t i = 0; i < nsl; i++) {
-    hoff[i] = (int32_t)slots;
-    slots += hwid[i];
-    if (slots > (int64_t)0x7fffffff) {
-      fail(0);
-      A->comp_state = -1;
-      return QH_OK;
-    }
-  }
-  hoff[nsl] = (int32_t)slots;
   // the shape of every bin's launch, and what the largest bin and all of them take
   const bool few = nbins <= 2 * cus;  // the chip is not full: one launch, so that nothing waits for a launch before it
   auto rup = [few](int w) {
@@ -614,8 +779,9 @@ int cp_build(qh_mat *A) {
       if (w <= u && (few || u != 10)) return u;
     return 0;
   };
+  int64_t slots[2] = {0, 0};  // held in registers, read as words
   struct Shape {
-    int stream, rows, W;
+    int words, rows, W;
     int32_t bin;
   };
   std::vector<Shape> sh(nbins);
@@ -630,14 +796,24 @@ int cp_build(qh_mat *A) {
     }
     const int rows = (hslice[b + 1] - hslice[b]) * 64;
     const int W = rup(w);
-    // two rows a thread: up to 12 slots each fit 128 registers
+    // two rows a thread: up to 12 slots each fit the 128 registers
     const bool reg = W && (rows <= 1024 || (rows <= CP_REG_ROWS && W <= 12));
     sh[b] = Shape{!reg, rows <= 64 ? 64 : rows <= 128 ? 128 : rows <= 256 ? 256 : rows <= 512 ? 512 : rows <= 1024 ? 1024 : rows, W, b};
     if (reg) {
       few_rows = std::max(few_rows, sh[b].rows);
       few_w = std::max(few_w, W);
     }
-    const double clk = reg ? CP_CLK_REG * W * (rows / 64) : CP_CLK_MEM * (double)sum;
+    for (int32_t i = hslice[b]; i < hslice[b + 1]; i++) {
+      hoff[i] = (int32_t)slots[!reg];
+      slots[!reg] += hwid[i];
+      hzc[i] = reg ? rows : -1;
+    }
+    if (std::max(slots[0], slots[1]) > (int64_t)0x7fffffff) {
+      fail(0);
+      state = -1;
+      return QH_OK;
+    }
+    const double clk = reg ? CP_CLK_REG * W * (rows / 64) : CP_CLK_WORD * (double)sum;
     most = std::max(most, clk + CP_CLK_FIXED);
     all += clk;
   }
@@ -651,28 +827,28 @@ int cp_build(qh_mat *A) {
   const double stage_us = 2.5 + 1.1e-5 * (double)n;
   if (comp_us > 0.9 * stage_us) {
     fail(0);
-    A->comp_state = -1;
+    state = -1;
     return QH_OK;
   }
   const bool merge = few && !(few_rows > 1024 && few_w > 12);
   if (merge)
     for (auto &q : sh)
-      if (!q.stream) {
+      if (!q.words) {
         q.rows = few_rows;
         q.W = few_w;
       }
   std::stable_sort(sh.begin(), sh.end(), [](const Shape &p, const Shape &q) {
-    if (p.stream != q.stream) return p.stream > q.stream;
-    const int pr = p.stream || p.rows > 1024 ? 1 << 20 : p.rows, qr = q.stream || q.rows > 1024 ? 1 << 20 : q.rows;
+    if (p.words != q.words) return p.words > q.words;
+    const int pr = p.words || p.rows > 1024 ? 1 << 20 : p.rows, qr = q.words || q.rows > 1024 ? 1 << 20 : q.rows;
     if (pr != qr) return pr > qr;
-    return !p.stream && p.W > q.W;
+    return !p.words && p.W > q.W;
   });
   std::vector<int32_t> hbins(nbins);
   for (int32_t i = 0; i < nbins; i++) {
     const Shape &q = sh[i];
     hbins[i] = q.bin;
-    const int S = q.stream ? CP_STREAM_S : q.rows > 1024 ? 2 : 1, threads = q.stream || S == 2 ? 1024 : q.rows;
-    const int W = q.stream ? 0 : q.W;
+    const int S = q.words ? (f32 ? 8 : 6) : q.rows > 1024 ? 2 : 1, threads = q.words || S == 2 ? 1024 : q.rows;
+    const int W = q.words ? 0 : q.W;
     if (c->classes.empty() || c->classes.back().threads != threads || c->classes.back().S != S ||
         c->classes.back().W != W)
       c->classes.push_back(CpClass{threads, S, W, !merge, false, i, 0, 0});
@@ -688,56 +864,79 @@ int cp_build(qh_mat *A) {
         for (hipEvent_t &e : c->ev) CP_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
       }
     }
-  double *ev;
+  const int ndict = sh[0].words ? (c->classes[0].count) : 0;  // these bins come first
+  double *ev, *dict;
   uint16_t *ec;
-  Carve tail;
-  tail.take<double>((size_t)std::max<int64_t>(slots, 1) * 64);
-  tail.take<uint16_t>((size_t)std::max<int64_t>(slots, 1) * 64);
-  rc = qh_alloc(&c->slots, tail.n);
+  uint32_t *ew;
+  auto entries = [&](Carve &q) {
+    ev = q.take<double>((size_t)slots[0] * 64 + 1);
+    ec = q.take<uint16_t>((size_t)slots[0] * 64 + 1);
+    ew = q.take<uint32_t>((size_t)slots[1] * 64 + 1);
+    dict = q.take<double>((size_t)ndict * CP_DICT + 1);
+  };
+  Carve em, ep;
+  entries(em);
+  rc = qh_alloc(&c->slots, em.n);
   if (rc) return fail(rc);
-  Carve tw;
-  tw.p = (char *)c->slots;
-  ev = tw.take<double>((size_t)std::max<int64_t>(slots, 1) * 64);
-  ec = tw.take<uint16_t>((size_t)std::max<int64_t>(slots, 1) * 64);
-  CP_HIP(hipMemcpyAsync(soff, hoff.data(), sizeof(int32_t) * (nsl + 1), hipMemcpyHostToDevice, s));
+  ep.p = (char *)c->slots;
+  entries(ep);
+  CP_HIP(hipMemcpyAsync(zc, hzc.data(), sizeof(int32_t) * nsl, hipMemcpyHostToDevice, s));
+  CP_HIP(hipMemcpyAsync(soff, hoff.data(), sizeof(int32_t) * nsl, hipMemcpyHostToDevice, s));
   CP_HIP(hipMemcpyAsync(bins, hbins.data(), sizeof(int32_t) * nbins, hipMemcpyHostToDevice, s));
   hipLaunchKernelGGL(k_cp_fill, dim3(qh_blocks(nsl, 4)), dim3(256), 0, s, order, pos, A->rowptr, A->col, A->val,
-                     soff, nim, zc, diag, ev, ec, nsl);
+                     soff, width, nim, zc, diag, ev, ec, nsl);
+  int32_t hover = 0;
+  if (ndict) {
+    CP_HIP(hipMemsetAsync(over, 0, sizeof(int32_t), s));
+    hipLaunchKernelGGL(k_cp_dict, dim3(ndict), dim3(1024), 0, s, bins, bslice, order, pos, A->rowptr, A->col, A->val,
+                       soff, width, nim, ew, dict, over);
+    CP_HIP(hipMemcpyAsync(&hover, over, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+  }
   CP_HIP(hipGetLastError());
   CP_HIP(hipStreamSynchronize(s));  // the host vectors and the workspace go
+  if (hover) {  // more values than a table holds
+    fail(0);
+    state = -1;
+    return QH_OK;
+  }
 #undef CP_HIP
   qh_free_ptr(wbuf);
   c->a.bslice = bslice;
   c->a.bins = bins;
   c->a.soff = soff;
+  c->a.width = width;
+  c->a.ew = ew;
+  c->a.dict = dict;
   c->a.nim = nim;
   c->a.order = order;
   c->a.diag = diag;
   c->a.ev = ev;
   c->a.ec = ec;
   c->trace = trace;
-  A->comp = c;
-  A->comp_state = 1;
+  A->comp[f32] = c;
+  state = 1;
   return QH_OK;
 }
 
 }  // namespace
 
-int qh_comp_prepare(qh_mat *A, int *usable) {
+int qh_comp_prepare(qh_mat *A, int prec, int *usable) {
+  const int f32 = prec == QH_FP32;
   *usable = 0;
-  if (A->comp_state == 0) {
+  if (A->comp_state[f32] == 0) {
     // row and slot numbers are 32-bit
     if (A->rows < 1 || A->rows > (int64_t)1 << 30)
-      A->comp_state = -1;
-    else if (int rc = cp_build(A))
+      A->comp_state[f32] = -1;
+    else if (int rc = cp_build(A, f32))
       return rc;
   }
-  *usable = A->comp_state == 1;
+  *usable = A->comp_state[f32] == 1;
   return QH_OK;
 }
 
 int qh_comp_rk4(qh_mat *A, qh_vec *x, double dt, int64_t nsteps) {
-  const qh_comp &c = *A->comp;
+  const int f32 = x->prec == QH_FP32;
+  const qh_comp &c = *A->comp[f32];
   hipStream_t s = qh_stream();
   if (c.side) {
     QH_HIP(hipEventRecord(c.ev[0], s));
@@ -747,16 +946,21 @@ int qh_comp_rk4(qh_mat *A, qh_vec *x, double dt, int64_t nsteps) {
     CpArgs a = c.a;
     a.bins += k.first;
     a.x = x->d;
-    a.xlo = x->prec == QH_FP32 ? x->lo : nullptr;
+    a.xlo = f32 ? x->lo : nullptr;
     a.cells = k.cells;
     a.h = dt;
     a.nsteps = nsteps;
     hipStream_t ks = k.side ? c.side : s;
+    const size_t table = CP_DICT * sizeof(double);
     int rc = QH_EINVAL;
-#define CP_CASE(SS, WW, SK)                    \
+    qh_set_error("no kernel for bins of %d rows a thread and %d slots", k.S, k.W);
+    if (k.W == 0 && f32)
+      rc = cp_launch(k_comp_dict<float2, 8>, k, a, (size_t)2 * k.cells * sizeof(float2) + table, ks);
+    else if (k.W == 0)
+      rc = cp_launch(k_comp_dict<double2, 6>, k, a, (size_t)2 * k.cells * sizeof(double2) + table, ks);
+#define CP_CASE(SS, WW, SK)                   \
   if (k.S == SS && k.W == WW && k.skip == SK) \
-    rc = cp_launch<SS, WW, true, SK>(k, a, ks);
-    if (k.W == 0) rc = cp_launch<CP_STREAM_S, 2, false, false>(k, a, ks);
+    rc = cp_launch(k_comp_rk4<SS, WW, SK>, k, a, (size_t)2 * k.cells * sizeof(double2), ks);
     CP_CASE(1, 4, false)
     CP_CASE(1, 8, false)
     CP_CASE(1, 10, false)
@@ -778,10 +982,7 @@ int qh_comp_rk4(qh_mat *A, qh_vec *x, double dt, int64_t nsteps) {
     CP_CASE(2, 8, true)
     CP_CASE(2, 12, true)
 #undef CP_CASE
-    if (rc) {
-      qh_set_error("no kernel for bins of %d rows a thread and %d slots", k.S, k.W);
-      return rc;
-    }
+    if (rc) return rc;
   }
   if (c.side) {
     QH_HIP(hipEventRecord(c.ev[1], c.side));
@@ -790,4 +991,4 @@ int qh_comp_rk4(qh_mat *A, qh_vec *x, double dt, int64_t nsteps) {
   return QH_OK;
 }
 
-double *qh_comp_trace(const qh_mat *A) { return A->comp->trace; }
+double *qh_comp_trace(const qh_mat *A, int prec) { return A->comp[prec == QH_FP32]->trace; }

@@ -1725,14 +1725,17 @@ static int rk4_impl(qh_mat *A, qh_vec *x, double dt, int64_t nsteps, int64_t tot
   // generators that fall apart into small closed sets of rows
   if (!timed && !A->lanes_forced) {
     int usable = 0;
-    rc = qh_comp_prepare(A, &usable);
+    rc = qh_comp_prepare(A, x->prec, &usable);
     if (rc) return rc;
     if (usable) {
       const int64_t len = renorm_every > 0 ? graph_len(renorm_every) : nsteps;
       for (int64_t st = 0; st < nsteps && !rc; st += len) {
         rc = qh_comp_rk4(A, x, dt, std::min<int64_t>(len, nsteps - st));
         if (!rc && renorm_every > 0 && st + len <= nsteps)
-          rc = renorm_launch(s, x, x->d, tot, 0, qh_comp_trace(A), qh_comp_trace(A) + 512);
+          {
+          double *t = qh_comp_trace(A, x->prec);
+          rc = renorm_launch(s, x, x->d, tot, 0, t, t + 512);
+        }
       }
       return rc;
     }
@@ -1806,7 +1809,7 @@ extern "C" int qh_rk4_prepare(qh_mat *A, qh_vec *x, double dt, int64_t tot, int 
   if (A->rows <= QH_SMALL_ROWS && !A->lanes_forced) return QH_OK;  // one-workgroup path: nothing to capture
   if (!A->lanes_forced) {
     int usable = 0;
-    rc = qh_comp_prepare(A, &usable);
+    rc = qh_comp_prepare(A, x->prec, &usable);
     if (rc || usable) return rc;
   }
   int G = 0;

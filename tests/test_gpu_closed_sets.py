@@ -83,9 +83,9 @@ def test_closed_sets_match_oracle(recipe):
     qs.destroy()
 
 
-def test_entries_read_from_memory():
-    """13 slots a row and a component of 2048 rows and more: the kernel that reads its
-    entries from memory, beside the ones that hold them"""
+def test_entries_read_as_words():
+    """13 slots a row and a component of 2048 rows: the kernel that reads its entries
+    at every stage, beside the ones that hold them"""
     r = _noisy(11)
     qs, _, _ = build_system(r)
     A = qs.matrix()
@@ -96,6 +96,31 @@ def test_entries_read_from_memory():
     # rows of h A sum to at most 0.02 * 2 * 11 * 0.2 here
     assert np.abs(got - ref).max() <= 3 * np.abs(x0).max() * 16 * 2.0 ** -53
     qs.destroy()
+
+
+def test_entries_read_as_words_fp32():
+    """components of up to 2280 rows and 13 slots (more than are fetched ahead), enough
+    of them to fill the chip: complex64 stage vectors"""
+    recipe, count, dt, steps = _tc(4, 10), 20, 0.02, 3
+    systems = [build_system(recipe)[0] for _ in range(count)]
+    b = qa.Batch([s.matrix() for s in systems], [160] * count, prec=qa.FP32)
+    x0 = _start(160)
+    for i in range(count):
+        b.set_state(i, x0 if i % 2 else x0.conj())
+    b.rk4(dt, steps)
+    tot, terms = recipes.oracle_terms(recipe)
+    m = oracle.construct(tot, terms, dm=True)
+    rp, _, val = systems[0].matrix().export()
+    norm = np.add.reduceat(np.abs(val), rp[:-1]).max()
+    # per step: h |A| of a state rounded to 32 bits, and the two words' rounding
+    tol = steps * np.abs(x0).max() * (2 * dt * norm * 2.0 ** -24 + 8 * 2.0 ** -48)
+    for i in (0, 7, count - 1):
+        ref = m.rk4(x0 if i % 2 else x0.conj(), dt, steps)
+        assert np.abs(b.get_state(i) - ref).max() <= tol
+    assert np.array_equal(b.get_state(1), b.get_state(count - 1))
+    b.destroy()
+    for s in systems:
+        s.destroy()
 
 
 def test_renormalised_and_split_calls():
