@@ -1289,137 +1289,161 @@ extern "C" int qh_last_stage_ms(double *spmv_ms, int64_t *launches) {
 
 // ------------------------------------------------ small systems in one workgroup
 // For a generator of at most QH_SMALL_ROWS rows the whole RK4 integration runs
-// in one workgroup with the state and the three stage vectors in LDS (5 x 16 B
-// per row): every stage is one pass over the CSR rows followed by a barrier, so
-// a step costs four barriers instead of four kernel launches.  The state is kept
-// in FP64 in LDS for both storage precisions; the matrix values are FP64.
+// in one workgroup, a row per thread: the state and the row's entries in registers,
+// the stage vector in LDS (two buffers, 16 B per row each), so a stage is one LDS
+// read per entry and one barrier.  The state is kept in FP64 for both storage
+// precisions; the matrix values are FP64.
+// Bound by that chain: reads, dependent FMAs, barrier.  Jaynes-Cummings 2 x 10 (400
+// rows of at most 5 entries), 100 steps: 95 us, 180 us with the
+// stage derivatives in LDS (two reads an entry, no two in flight).
 #define QH_SMALL_ROWS 800
+// up to this many rows a thread has the registers for more than 8 entries
+#define QH_SMALL_WIDE_ROWS 640
 
-// MAXNZ > 0: every thread owns at most one row and keeps its (at most MAXNZ)
-// entries in registers; MAXNZ == 0: rows are read from the CSR in memory.
-template <bool F32, int MAXNZ>
-__global__ void __launch_bounds__(1024) k_rk4_small(int32_t n, const int32_t *__restrict__ rp,
-                                                    const int32_t *__restrict__ col, const double2 *__restrict__ val,
-                                                    void *xg, float2 *xlo, double h, int64_t nsteps, int64_t tot,
-                                                    int renorm_every) {
-  extern __shared__ double2 sm[];
-  double2 *xa = sm, *xb = sm + n, *k1 = sm + 2 * n, *k2 = sm + 3 * n, *k3 = sm + 4 * n;
-  __shared__ double2 scale;
-  const int tid = threadIdx.x, nt = blockDim.x;
-  for (int r = tid; r < n; r += nt) {
-    if (F32) {
-      const float2 hi = ((const float2 *)xg)[r], lo = xlo[r];
-      xa[r] = make_double2((double)hi.x + (double)lo.x, (double)hi.y + (double)lo.y);
-    } else {
-      xa[r] = ((const double2 *)xg)[r];
+// Row r of the generator: its (at most MAXNZ) entries in registers, filled up with
+// zeros times the zero cell n of the vector so that all reads are in flight
+// together; MAXNZ == 0: read from the CSR in memory.
+template <int MAXNZ>
+struct SmallRow {
+  int32_t c[MAXNZ > 0 ? MAXNZ : 1];
+  double2 v[MAXNZ > 0 ? MAXNZ : 1];
+  int32_t b = 0, e = 0;
+  __device__ __forceinline__ void load(int32_t n, int32_t r, const int32_t *rp, const int32_t *col, const double2 *val) {
+    if (r < n) {
+      b = rp[r];
+      e = rp[r + 1];
     }
-  }
-  __syncthreads();
-  // register copy of this thread's row (MAXNZ > 0: n <= blockDim.x, one row per thread)
-  int32_t rc_[MAXNZ > 0 ? MAXNZ : 1];
-  double2 rv_[MAXNZ > 0 ? MAXNZ : 1];
-  int rlen = 0;
-  if (MAXNZ > 0 && tid < n) {
-    const int32_t b = rp[tid];
-    rlen = rp[tid + 1] - b;
 #pragma unroll
-    for (int k = 0; k < (MAXNZ > 0 ? MAXNZ : 1); k++) {
-      rc_[k] = k < rlen ? col[b + k] : 0;
-      rv_[k] = k < rlen ? val[b + k] : make_double2(0.0, 0.0);
+    for (int k = 0; k < MAXNZ; k++) {
+      const bool on = b + k < e;
+      c[k] = on ? col[b + k] : n;
+      v[k] = on ? val[b + k] : make_double2(0.0, 0.0);
     }
   }
-  auto rowdot = [&](int r, const double2 *xs, const double2 *kin, double c) {
+  // the row times y
+  __device__ __forceinline__ double2 dot(const double2 *y, const int32_t *col, const double2 *val) const {
     double are = 0.0, aim = 0.0;
-    if (MAXNZ > 0) {
+    auto add = [&](double2 a, double2 x) {
+      are = fma(a.x, x.x, fma(-a.y, x.y, are));
+      aim = fma(a.x, x.y, fma(a.y, x.x, aim));
+    };
+    if constexpr (MAXNZ > 0) {
+      constexpr int CH = MAXNZ <= 8 ? MAXNZ : 4;  // reads in flight (the registers hold the entries as well)
 #pragma unroll
-      for (int k = 0; k < (MAXNZ > 0 ? MAXNZ : 1); k++) {
-        if (k < rlen) {
-          double2 v = xs[rc_[k]];
-          if (kin) {
-            v.x += c * kin[rc_[k]].x;
-            v.y += c * kin[rc_[k]].y;
-          }
-          const double2 a = rv_[k];
-          are = fma(a.x, v.x, fma(-a.y, v.y, are));
-          aim = fma(a.x, v.y, fma(a.y, v.x, aim));
-        }
+      for (int k0 = 0; k0 < MAXNZ; k0 += CH) {
+        double2 t[CH];
+#pragma unroll
+        for (int k = 0; k < CH; k++) t[k] = y[c[k0 + k]];
+#pragma unroll
+        for (int k = 0; k < CH; k++) add(v[k0 + k], t[k]);
+        if (CH < MAXNZ) __builtin_amdgcn_sched_barrier(0);
       }
-      return make_double2(are, aim);
-    }
-    for (int32_t k = rp[r]; k < rp[r + 1]; k++) {
-      const int32_t cc = col[k];
-      double2 v = xs[cc];
-      if (kin) {
-        v.x += c * kin[cc].x;
-        v.y += c * kin[cc].y;
-      }
-      const double2 a = val[k];
-      are = fma(a.x, v.x, fma(-a.y, v.y, are));
-      aim = fma(a.x, v.y, fma(a.y, v.x, aim));
+    } else {
+      for (int32_t k = b; k < e; k++) add(val[k], y[col[k]]);
     }
     return make_double2(are, aim);
-  };
-  const double s6 = h * (1.0 / 6.0), s3 = h * (1.0 / 3.0);
-  for (int64_t st = 0; st < nsteps; st++) {
-    for (int r = tid; r < n; r += nt) k1[r] = rowdot(r, xa, nullptr, 0.0);
-    __syncthreads();
-    for (int r = tid; r < n; r += nt) k2[r] = rowdot(r, xa, k1, 0.5 * h);
-    __syncthreads();
-    for (int r = tid; r < n; r += nt) k3[r] = rowdot(r, xa, k2, 0.5 * h);
-    __syncthreads();
-    for (int r = tid; r < n; r += nt) {
-      const double2 k4 = rowdot(r, xa, k3, h), a = k1[r], b = k2[r], c = k3[r], xo = xa[r];
-      xb[r] = make_double2(xo.x + s6 * a.x + s3 * b.x + s3 * c.x + s6 * k4.x,
-                           xo.y + s6 * a.y + s3 * b.y + s3 * c.y + s6 * k4.y);
+  }
+};
+
+template <bool F32, int MAXNZ>
+__global__ void __launch_bounds__(MAXNZ > 8 ? QH_SMALL_WIDE_ROWS : 832) k_rk4_small(int32_t n, const int32_t *__restrict__ rp,
+                                                   const int32_t *__restrict__ col, const double2 *__restrict__ val,
+                                                   void *xg, float2 *xlo, double h, int64_t nsteps, int64_t tot,
+                                                   int renorm_every) {
+  extern __shared__ double2 sm[];
+  __shared__ double2 scale;
+  double2 *const y0 = sm, *const y1 = sm + n + 1;
+  const int r = threadIdx.x;  // n <= blockDim.x
+  SmallRow<MAXNZ> row;
+  row.load(n, r, rp, col, val);
+  double2 x = make_double2(0.0, 0.0);
+  if (r < n) {
+    if (F32) {
+      const float2 hi = ((const float2 *)xg)[r], lo = xlo[r];
+      x = make_double2((double)hi.x + (double)lo.x, (double)hi.y + (double)lo.y);
+    } else {
+      x = ((const double2 *)xg)[r];
     }
-    __syncthreads();
-    double2 *t = xa;
-    xa = xb;
-    xb = t;
+    y0[r] = x;
+  }
+  if (r == 0) y0[n] = y1[n] = make_double2(0.0, 0.0);
+  __syncthreads();
+  const double cs[4] = {h / 4.0, h / 3.0, h / 2.0, h};
+  for (int64_t st = 0; st < nsteps; st++) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const double2 k = row.dot(q & 1 ? y1 : y0, col, val);
+      const double2 y = make_double2(fma(cs[q], k.x, x.x), fma(cs[q], k.y, x.y));
+      if (r < n) (q & 1 ? y0 : y1)[r] = y;
+      if (q == 3) x = y;
+      __syncthreads();
+    }
     if (renorm_every > 0 && (st + 1) % renorm_every == 0) {
-      if (tid == 0) {
+      if (r == 0) {
         double tr = 0.0, ti = 0.0;
         for (int64_t i = 0; i < tot; i++) {
-          tr += xa[i * (tot + 1)].x;
-          ti += xa[i * (tot + 1)].y;
+          tr += y0[i * (tot + 1)].x;
+          ti += y0[i * (tot + 1)].y;
         }
         const double d = tr * tr + ti * ti;
         scale = d > 0.0 ? make_double2(tr / d, -ti / d) : make_double2(1.0, 0.0);
       }
       __syncthreads();
       const double2 sc = scale;
-      for (int r = tid; r < n; r += nt) {
-        const double2 v = xa[r];
-        xa[r] = make_double2(sc.x * v.x - sc.y * v.y, sc.x * v.y + sc.y * v.x);
-      }
+      x = make_double2(sc.x * x.x - sc.y * x.y, sc.x * x.y + sc.y * x.x);
+      if (r < n) y0[r] = x;
       __syncthreads();
     }
   }
-  for (int r = tid; r < n; r += nt) {
-    const double2 v = xa[r];
-    if (F32) {
-      const float hr = (float)v.x, hm = (float)v.y;
-      ((float2 *)xg)[r] = make_float2(hr, hm);
-      xlo[r] = make_float2((float)(v.x - (double)hr), (float)(v.y - (double)hm));
-    } else {
-      ((double2 *)xg)[r] = v;
-    }
+  if (r >= n) return;
+  if (F32) {
+    const float hr = (float)x.x, hm = (float)x.y;
+    ((float2 *)xg)[r] = make_float2(hr, hm);
+    xlo[r] = make_float2((float)(x.x - (double)hr), (float)(x.y - (double)hm));
+  } else {
+    ((double2 *)xg)[r] = x;
   }
 }
 
 // The adaptive Bogacki-Shampine integration of time_step_sys (TSRK3BS with
 // TSAdapt basic, qsystem.c:995-1005) in one workgroup for a generator of at most
-// QH_SMALL_BS3_ROWS rows: x, the candidate and K1..K4 in LDS (6 x 16 B per row),
-// the step-size controller on the device (thread 0, broadcast through LDS), so a
-// trial step costs five barriers and no host round trip.  The same stage
-// formulas, error weights and controller as the host-driven loop: K2 = A(x +
-// h/2 K1), K3 = A(x + 3h/4 K2), xn = x + h(2/9 K1 + 1/3 K2 + 4/9 K3), K4 = A xn,
-// err = RMS of h sum (b_i - b^_i) K_i over atol + rtol max(|x|, |xn|);
-// fac = 0.9 err^(-1/3) in [0.1, 10], h' = h fac in [hmin, hmax]; accepted when
-// err <= 1 or h <= hmin (1 + 1e-12), with K1 of the next step = K4 (FSAL).
-// adaptive == 0: fixed steps of h0 (the last cut at tmax), K1 recomputed.
+// QH_SMALL_BS3_ROWS rows: a row per thread with x, K1..K4 and the row's entries in
+// registers, the stage vector in LDS (two buffers), the step-size controller in
+// every thread on the same numbers, so a trial step costs four barriers and no host
+// round trip.  The same stage formulas, error weights and controller as the
+// host-driven loop: K2 = A(x + h/2 K1), K3 = A(x + 3h/4 K2), xn = x + h(2/9 K1 +
+// 1/3 K2 + 4/9 K3), K4 = A xn, err = RMS of h sum (b_i - b^_i) K_i over atol + rtol
+// max(|x|, |xn|); fac = 0.9 err^(-1/3) in [0.1, 10], h' = h fac in [hmin, hmax];
+// accepted when err <= 1 or h <= hmin (1 + 1e-12), with K1 of the next step = K4
+// (FSAL).  adaptive == 0: fixed steps of h0 (the last cut at tmax), K1 recomputed.
 // out: final time, accepted steps, the next step size.
+// Bound by the chain of a trial: three stages, the weighted error, its sum over the
+// workgroup, the controller.  Jaynes-Cummings 2 x 10 (400 rows), t = 20: 1.05 ms,
+// 1.85 ms with everything in LDS, the controller on one thread and pow.
 #define QH_SMALL_BS3_ROWS 640
+
+// sum over the wavefront, in every lane
+__device__ inline double wave_sum(double v) {
+  auto add = [&](int lo, int hi) {
+    const unsigned long long u = (unsigned long long)(unsigned)hi << 32 | (unsigned)lo;
+    v += __longlong_as_double((long long)u);
+  };
+#define QH_DPP(ctrl)                                                                        \
+  add(__builtin_amdgcn_update_dpp(0, __double2loint(v), ctrl, 0xF, 0xF, false),             \
+      __builtin_amdgcn_update_dpp(0, __double2hiint(v), ctrl, 0xF, 0xF, false))
+  QH_DPP(0xB1);   // quad_perm 1 0 3 2
+  QH_DPP(0x4E);   // quad_perm 2 3 0 1
+  QH_DPP(0x141);  // row_half_mirror: the other four of eight lanes
+  QH_DPP(0x140);  // row_mirror: the other eight of sixteen
+#undef QH_DPP
+  // the four rows, from one lane of each
+  double s = 0.0;
+#pragma unroll
+  for (int l = 0; l < 64; l += 16)
+    s += __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                          __builtin_amdgcn_readlane(__double2loint(v), l));
+  return s;
+}
 
 template <int MAXNZ>
 __global__ void __launch_bounds__(QH_SMALL_BS3_ROWS) k_rk3bs_small(int32_t n, const int32_t *__restrict__ rp,
@@ -1429,62 +1453,20 @@ __global__ void __launch_bounds__(QH_SMALL_BS3_ROWS) k_rk3bs_small(int32_t n, co
                                                       double rtol, double hmin, double hmax, int adaptive, double eps,
                                                       double *out) {
   extern __shared__ double2 sm[];
-  double2 *xa = sm, *xn = sm + n, *k1 = sm + 2 * n, *k2 = sm + 3 * n, *k3 = sm + 4 * n, *k4 = sm + 5 * n;
   __shared__ double red[QH_SMALL_BS3_ROWS / 64];
-  __shared__ double s_hnew;
-  __shared__ int s_acc, s_bad;
-  const int tid = threadIdx.x, nt = blockDim.x;
-  for (int r = tid; r < n; r += nt) xa[r] = xg[r];
-  int32_t rc_[MAXNZ > 0 ? MAXNZ : 1];
-  double2 rv_[MAXNZ > 0 ? MAXNZ : 1];
-  int rlen = 0;
-  if (MAXNZ > 0 && tid < n) {
-    const int32_t b = rp[tid];
-    rlen = rp[tid + 1] - b;
-#pragma unroll
-    for (int k = 0; k < (MAXNZ > 0 ? MAXNZ : 1); k++) {
-      rc_[k] = k < rlen ? col[b + k] : 0;
-      rv_[k] = k < rlen ? val[b + k] : make_double2(0.0, 0.0);
-    }
-  }
+  double2 *const ya = sm, *const yb = sm + n + 1;
+  const int r = threadIdx.x, waves = blockDim.x >> 6;  // n <= blockDim.x
+  SmallRow<MAXNZ> row;
+  row.load(n, r, rp, col, val);
+  const double2 zero = make_double2(0.0, 0.0);
+  double2 x = r < n ? xg[r] : zero, k1 = zero;
+  if (r == 0) ya[n] = yb[n] = zero;
+  if (r < n) yb[r] = x;
   __syncthreads();
-  auto rowdot = [&](int r, const double2 *xs, const double2 *kin, double c) {
-    double are = 0.0, aim = 0.0;
-    if (MAXNZ > 0) {
-#pragma unroll
-      for (int k = 0; k < (MAXNZ > 0 ? MAXNZ : 1); k++) {
-        if (k < rlen) {
-          double2 v = xs[rc_[k]];
-          if (kin) {
-            v.x += c * kin[rc_[k]].x;
-            v.y += c * kin[rc_[k]].y;
-          }
-          const double2 a = rv_[k];
-          are = fma(a.x, v.x, fma(-a.y, v.y, are));
-          aim = fma(a.x, v.y, fma(a.y, v.x, aim));
-        }
-      }
-      return make_double2(are, aim);
-    }
-    for (int32_t k = rp[r]; k < rp[r + 1]; k++) {
-      const int32_t cc = col[k];
-      double2 v = xs[cc];
-      if (kin) {
-        v.x += c * kin[cc].x;
-        v.y += c * kin[cc].y;
-      }
-      const double2 a = val[k];
-      are = fma(a.x, v.x, fma(-a.y, v.y, are));
-      aim = fma(a.x, v.y, fma(a.y, v.x, aim));
-    }
-    return make_double2(are, aim);
-  };
   const double c1 = 2.0 / 9.0 - 7.0 / 24.0, c2 = 1.0 / 3.0 - 1.0 / 4.0, c3 = 4.0 / 9.0 - 1.0 / 3.0, c4 = -1.0 / 8.0;
   double t = t0, h = h0;
   int64_t step = 0;
-  bool have_k1 = false;
-  if (tid == 0) s_bad = 0;
-  __syncthreads();
+  bool have_k1 = false, bad = false;
   // a bound on the trial steps: a rejection shrinks the step by at least 0.9
   // and a step at hmin is always accepted, so fewer than 64 trials per accepted
   // step are possible while the state is finite; the loop ends in every case
@@ -1492,79 +1474,65 @@ __global__ void __launch_bounds__(QH_SMALL_BS3_ROWS) k_rk3bs_small(int32_t n, co
   int64_t trials = 0;
   while (t < tmax - eps && step < steps_max && trials++ < trial_cap) {
     const double hh = (t + h > tmax) ? tmax - t : h;
-    if (!have_k1) {
-      for (int r = tid; r < n; r += nt) k1[r] = rowdot(r, xa, nullptr, 0.0);
-      __syncthreads();
-    }
-    for (int r = tid; r < n; r += nt) k2[r] = rowdot(r, xa, k1, 0.5 * hh);
+    // yb holds x wherever K1 is still to be formed: at the start, and after every
+    // fixed step (its xn)
+    if (!have_k1) k1 = row.dot(yb, col, val);
+    if (r < n) ya[r] = make_double2(x.x + 0.5 * hh * k1.x, x.y + 0.5 * hh * k1.y);
     __syncthreads();
-    for (int r = tid; r < n; r += nt) k3[r] = rowdot(r, xa, k2, 0.75 * hh);
+    const double2 k2 = row.dot(ya, col, val);
+    if (r < n) yb[r] = make_double2(x.x + 0.75 * hh * k2.x, x.y + 0.75 * hh * k2.y);
     __syncthreads();
-    for (int r = tid; r < n; r += nt) {
-      const double2 xo = xa[r], a = k1[r], bq = k2[r], cq = k3[r];
-      xn[r] = make_double2(xo.x + hh * (2.0 / 9.0) * a.x + hh / 3.0 * bq.x + hh * (4.0 / 9.0) * cq.x,
-                           xo.y + hh * (2.0 / 9.0) * a.y + hh / 3.0 * bq.y + hh * (4.0 / 9.0) * cq.y);
-    }
+    const double2 k3 = row.dot(yb, col, val);
+    const double2 xn = make_double2(x.x + hh * (2.0 / 9.0) * k1.x + hh / 3.0 * k2.x + hh * (4.0 / 9.0) * k3.x,
+                                    x.y + hh * (2.0 / 9.0) * k1.y + hh / 3.0 * k2.y + hh * (4.0 / 9.0) * k3.y);
+    if (r < n) ya[r] = xn;
     __syncthreads();
+    const double2 k4 = row.dot(ya, col, val);
     double v = 0.0;
-    for (int r = tid; r < n; r += nt) {
-      const double2 d = rowdot(r, xn, nullptr, 0.0), a = k1[r], bq = k2[r], cq = k3[r], xo = xa[r], xw = xn[r];
-      k4[r] = d;
-      const double er = hh * (c1 * a.x + c2 * bq.x + c3 * cq.x + c4 * d.x);
-      const double ei = hh * (c1 * a.y + c2 * bq.y + c3 * cq.y + c4 * d.y);
-      const double ax = sqrt(xo.x * xo.x + xo.y * xo.y), an = sqrt(xw.x * xw.x + xw.y * xw.y);
-      const double sc = atol + rtol * (ax > an ? ax : an);
-      v += (er * er + ei * ei) / (sc * sc);
+    if (r < n) {
+      const double er = hh * (c1 * k1.x + c2 * k2.x + c3 * k3.x + c4 * k4.x);
+      const double ei = hh * (c1 * k1.y + c2 * k2.y + c3 * k3.y + c4 * k4.y);
+      const double ax = x.x * x.x + x.y * x.y, an = xn.x * xn.x + xn.y * xn.y;
+      const double sc = atol + rtol * sqrt(ax > an ? ax : an);
+      v = (er * er + ei * ei) / (sc * sc);
+      if (!adaptive) yb[r] = xn;  // read again only after the barrier below
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    if ((tid & 63) == 0) red[tid >> 6] = v;
+    v = wave_sum(v);
+    if ((r & 63) == 0) red[r >> 6] = v;
     __syncthreads();
-    if (tid == 0) {
-      double sum = 0.0;
-      for (int w = 0; w < (nt + 63) / 64; w++) sum += red[w];
-      const double err = sqrt(sum / (double)n);
-      // a non-finite error estimate (a NaN or infinite state) ends the
-      // integration: the controller could not leave the step otherwise
-      s_bad = !(err <= 1.7976931348623157e308);
-      double fac = 0.9 * pow(err > 1e-300 ? err : 1e-300, -1.0 / 3.0);
-      fac = fac < 0.1 ? 0.1 : (fac > 10.0 ? 10.0 : fac);
-      double hn = hh * fac;
-      hn = hn < hmin ? hmin : (hn > hmax ? hmax : hn);
-      s_hnew = hn;
-      s_acc = (!adaptive || err <= 1.0 || hh <= hmin * (1 + 1e-12)) ? 1 : 0;
+    double sum = 0.0;
+    for (int w = 0; w < waves; w++) sum += red[w];
+    const double err = sqrt(sum / (double)n);
+    // a non-finite error estimate (a NaN or infinite state) ends the
+    // integration: the controller could not leave the step otherwise
+    if (!(err <= 1.7976931348623157e308)) {
+      bad = true;
+      break;
     }
-    __syncthreads();
-    if (s_bad) break;
-    const int acc = s_acc;
+    double fac = 0.9 * rcbrt(err > 1e-300 ? err : 1e-300);
+    fac = fac < 0.1 ? 0.1 : (fac > 10.0 ? 10.0 : fac);
+    double hn = hh * fac;
+    hn = hn < hmin ? hmin : (hn > hmax ? hmax : hn);
+    const bool acc = !adaptive || err <= 1.0 || hh <= hmin * (1 + 1e-12);
     if (acc) {
-      double2 *tp = xa;
-      xa = xn;
-      xn = tp;
+      x = xn;
       t += hh;
       step++;
     }
     if (adaptive) {
-      if (acc) {
-        double2 *tk = k1;
-        k1 = k4;
-        k4 = tk;
-      }
+      if (acc) k1 = k4;
       have_k1 = true;
       // a step cut to land on tmax (the end, or an event the caller stops at)
       // leaves the step size as it was, as the host loop does after an event
-      if (!(acc && hh < h && t >= tmax - eps)) h = s_hnew;
+      if (!(acc && hh < h && t >= tmax - eps)) h = hn;
     }
-    // the next trial writes K2 (and K1 at fixed steps) only after every thread
-    // has read s_acc / s_hnew: the barrier after its first stage orders that
-    __syncthreads();
   }
-  for (int r = tid; r < n; r += nt) xg[r] = xa[r];
-  if (tid == 0) {
+  if (r < n) xg[r] = x;
+  if (r == 0) {
     out[0] = t;
     out[1] = (double)step;
     out[2] = h;
-    out[3] = s_bad ? 1.0 : 0.0;
+    out[3] = bad ? 1.0 : 0.0;
   }
 }
 
@@ -1583,20 +1551,21 @@ extern "C" int qh_rk3bs_small(qh_mat *A, qh_vec *x, double t0, double tmax, doub
   if (rc) return rc;
   const int32_t n = (int32_t)A->rows;
   int bt = ((n + 63) / 64) * 64;
-  const size_t lds = (size_t)6 * n * sizeof(double2);
+  const size_t lds = (size_t)2 * (n + 1) * sizeof(double2);
   const double eps = 1e-12 * (fabs(tmax) + fabs(h0) + 1.0);
   hipStream_t s = qh_stream();
-  // rows of at most 8 entries in registers (one row per thread); longer rows read
-  // from the CSR, which the caches hold for a generator this small (register
-  // copies of 16 or 32 entries would spill)
-  const int mz = A->max_row <= 8 ? 8 : 0;
+  // the least padding of the rows' registers; rows of more than 16 entries are read
+  // from the CSR, which the caches hold for a generator this small
+  const int mr = A->max_row;
 #define QH_LB(Z)                                                                                                \
   hipLaunchKernelGGL((k_rk3bs_small<Z>), dim3(1), dim3(bt), lds, s, n, A->rowptr, A->col, A->val,             \
                      (double2 *)x->d, t0, tmax, h0, steps_max, atol, rtol, hmin, hmax, adaptive, eps, dout)
-  if (mz == 8)
-    QH_LB(8);
-  else
-    QH_LB(0);
+  if (mr <= 4) QH_LB(4);
+  else if (mr <= 6) QH_LB(6);
+  else if (mr <= 8) QH_LB(8);
+  else if (mr <= 12) QH_LB(12);
+  else if (mr <= 16) QH_LB(16);
+  else QH_LB(0);
 #undef QH_LB
   QH_HIP(hipGetLastError());
   QH_HIP(hipMemcpyAsync(hout, dout, 4 * sizeof(double), hipMemcpyDeviceToHost, s));
@@ -1647,22 +1616,24 @@ static int rk4_small(qh_mat *A, qh_vec *x, double dt, int64_t nsteps, int64_t to
   int rc0 = qh_mat_max_row(A);
   if (rc0) return rc0;
   const int32_t n = (int32_t)A->rows;
-  int bt = ((n + 63) / 64) * 64;
-  if (bt > 1024) bt = 1024;
-  const size_t lds = (size_t)5 * n * sizeof(double2);
+  const int bt = ((n + 63) / 64) * 64;
+  const size_t lds = (size_t)2 * (n + 1) * sizeof(double2);
   hipStream_t s = qh_stream();
-  const int mz = A->max_row <= 8 ? 8 : A->max_row <= 16 ? 16 : A->max_row <= 32 ? 32 : 0;
-#define QH_LS(F, Z)                                                                                             \
+  const int mr = A->max_row;
+#define QH_LS1(F, Z)                                                                                            \
   hipLaunchKernelGGL((k_rk4_small<F, Z>), dim3(1), dim3(bt), lds, s, n, A->rowptr, A->col, A->val, x->d, x->lo, \
                      dt, nsteps, tot, renorm_every)
-  const bool f32 = x->prec == QH_FP32;
-  switch (mz) {
-    case 8: if (f32) QH_LS(true, 8); else QH_LS(false, 8); break;
-    case 16: if (f32) QH_LS(true, 16); else QH_LS(false, 16); break;
-    case 32: if (f32) QH_LS(true, 32); else QH_LS(false, 32); break;
-    default: if (f32) QH_LS(true, 0); else QH_LS(false, 0); break;
-  }
+#define QH_LS(Z)                      \
+  if (x->prec == QH_FP32) QH_LS1(true, Z); \
+  else QH_LS1(false, Z)
+  if (mr <= 4) { QH_LS(4); }
+  else if (mr <= 6) { QH_LS(6); }
+  else if (mr <= 8) { QH_LS(8); }
+  else if (mr <= 12 && n <= QH_SMALL_WIDE_ROWS) { QH_LS(12); }
+  else if (mr <= 16 && n <= QH_SMALL_WIDE_ROWS) { QH_LS(16); }
+  else { QH_LS(0); }
 #undef QH_LS
+#undef QH_LS1
   QH_HIP(hipGetLastError());
   return QH_OK;
 }
