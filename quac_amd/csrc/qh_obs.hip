@@ -2,6 +2,7 @@
 // the trace, and all subsystem populations in one pass over the diagonal.
 // qvec_utilities.c:322-392 (trace), :1197-1281 (DM expectation), :1682-2022
 // (bitstring probabilities = Re diag rho).
+#include <algorithm>
 #include <mutex>
 #include <vector>
 
@@ -16,6 +17,32 @@ __device__ inline double2 ld(const void *d, const float2 *lo, int64_t i) {
   if (!lo) return ((const double2 *)d)[i];
   float2 h = ((const float2 *)d)[i], l = lo[i];
   return make_double2((double)h.x + (double)l.x, (double)h.y + (double)l.y);
+}
+
+// An op chain that fits goes to its kernel as an argument: no copies to the device
+// before a reduction (two of them cost 10 us of the 25 us of an expectation value).
+const int ARG_OPS = 8, ARG_LEV = 96;
+struct ChainArg {
+  int nops;  // 0: the chain is in device memory
+  qh_op ops[ARG_OPS];
+  qh_level lev[ARG_LEV];
+};
+// the chain in LDS, where each lane reads its own level
+struct Chain {
+  const qh_op *ops;
+  const qh_level *tab;
+  int n;
+};
+__device__ inline Chain chain_of(const ChainArg &c, const qh_op *ops, int nops, const qh_level *tab) {
+  __shared__ qh_op so[ARG_OPS];
+  __shared__ qh_level sl[ARG_LEV];
+  if (c.nops == 0) return Chain{ops, tab, nops};
+  for (int i = threadIdx.x; i < ARG_LEV; i += blockDim.x) {
+    if (i < ARG_OPS) so[i] = c.ops[i];
+    sl[i] = c.lev[i];
+  }
+  __syncthreads();
+  return Chain{so, sl, c.nops};
 }
 
 // forward op chain on index i in [0, tot) (the TENSOR_IG rule of kron.c:294-538)
@@ -52,13 +79,15 @@ __device__ inline void block_sum2(double &a, double &b, double2 *partial) {
   if (threadIdx.x == 0) partial[blockIdx.x] = make_double2(sa[0], sb[0]);
 }
 
-__global__ void __launch_bounds__(256) k_expect_dm(const void *x, const float2 *lo, int64_t tot, const qh_op *ops,
-                                                   int nops, const qh_level *tab, double2 *partial) {
+__global__ void __launch_bounds__(256) k_expect_dm(const void *x, const float2 *lo, int64_t tot, ChainArg arg,
+                                                   const qh_op *ops, int nops, const qh_level *tab,
+                                                   double2 *partial) {
+  const Chain c = chain_of(arg, ops, nops, tab);
   double ar = 0.0, ai = 0.0;
   for (int64_t i = blockIdx.x * 256 + threadIdx.x; i < tot; i += (int64_t)gridDim.x * 256) {
     int64_t k;
     double2 v;
-    if (!chain_ig(ops, nops, tab, i, k, v)) continue;
+    if (!chain_ig(c.ops, c.n, c.tab, i, k, v)) continue;
     const double2 r = ld(x, lo, tot * i + k);  // rho[k, i]
     ar += v.x * r.x - v.y * r.y;
     ai += v.x * r.y + v.y * r.x;
@@ -66,13 +95,15 @@ __global__ void __launch_bounds__(256) k_expect_dm(const void *x, const float2 *
   block_sum2(ar, ai, partial);
 }
 
-__global__ void __launch_bounds__(256) k_expect_wf(const void *x, const float2 *lo, int64_t tot, const qh_op *ops,
-                                                   int nops, const qh_level *tab, double2 *partial) {
+__global__ void __launch_bounds__(256) k_expect_wf(const void *x, const float2 *lo, int64_t tot, ChainArg arg,
+                                                   const qh_op *ops, int nops, const qh_level *tab,
+                                                   double2 *partial) {
+  const Chain c = chain_of(arg, ops, nops, tab);
   double ar = 0.0, ai = 0.0;
   for (int64_t i = blockIdx.x * 256 + threadIdx.x; i < tot; i += (int64_t)gridDim.x * 256) {
     int64_t k;
     double2 v;
-    if (!chain_ig(ops, nops, tab, i, k, v)) continue;
+    if (!chain_ig(c.ops, c.n, c.tab, i, k, v)) continue;
     const double2 pk = ld(x, lo, k), pi = ld(x, lo, i);
     const double tr = v.x * pk.x - v.y * pk.y, ti = v.x * pk.y + v.y * pk.x;
     ar += pi.x * tr + pi.y * ti;  // conj(psi_i) * t
@@ -83,8 +114,9 @@ __global__ void __launch_bounds__(256) k_expect_wf(const void *x, const float2 *
 
 // ensemble of M wavefunctions (trajectory b at [b*tot, (b+1)*tot)): block b writes
 // <psi_b|O|psi_b> / <psi_b|psi_b> (qvec_utilities.c:1353-1420)
-__global__ void __launch_bounds__(256) k_expect_ens(const double2 *x, int64_t tot, const qh_op *ops, int nops,
-                                                    const qh_level *tab, double2 *out) {
+__global__ void __launch_bounds__(256) k_expect_ens(const double2 *x, int64_t tot, ChainArg arg, const qh_op *ops,
+                                                    int nops, const qh_level *tab, double2 *out) {
+  const Chain c = chain_of(arg, ops, nops, tab);
   const double2 *p = x + (int64_t)blockIdx.x * tot;
   double ar = 0.0, ai = 0.0, nn = 0.0;
   for (int64_t i = threadIdx.x; i < tot; i += 256) {
@@ -92,7 +124,7 @@ __global__ void __launch_bounds__(256) k_expect_ens(const double2 *x, int64_t to
     nn += pi.x * pi.x + pi.y * pi.y;
     int64_t k;
     double2 v;
-    if (!chain_ig(ops, nops, tab, i, k, v)) continue;
+    if (!chain_ig(c.ops, c.n, c.tab, i, k, v)) continue;
     const double2 pk = p[k];
     const double tr = v.x * pk.x - v.y * pk.y, ti = v.x * pk.y + v.y * pk.x;
     ar += pi.x * tr + pi.y * ti;
@@ -157,12 +189,7 @@ __global__ void __launch_bounds__(256) k_pops(const void *x, const float2 *lo, i
   }
 }
 
-int finish2(double2 *dpart, int nb, double *re, double *im) {
-  double2 *h = nullptr;
-  int rc = qh_scratch(0, nullptr, sizeof(double2) * nb, (void **)&h);
-  if (rc) return rc;
-  QH_HIP(hipMemcpyAsync(h, dpart, sizeof(double2) * nb, hipMemcpyDeviceToHost, qh_stream()));
-  QH_HIP(hipStreamSynchronize(qh_stream()));
+void sum2(const double2 *h, int nb, double *re, double *im) {
   double a = 0.0, b = 0.0;
   for (int i = 0; i < nb; i++) {
     a += h[i].x;
@@ -170,6 +197,15 @@ int finish2(double2 *dpart, int nb, double *re, double *im) {
   }
   *re = a;
   *im = b;
+}
+
+int finish2(double2 *dpart, int nb, double *re, double *im) {
+  double2 *h = nullptr;
+  int rc = qh_scratch(0, nullptr, sizeof(double2) * nb, (void **)&h);
+  if (rc) return rc;
+  QH_HIP(hipMemcpyAsync(h, dpart, sizeof(double2) * nb, hipMemcpyDeviceToHost, qh_stream()));
+  QH_HIP(hipStreamSynchronize(qh_stream()));
+  sum2(h, nb, re, im);
   return QH_OK;
 }
 
@@ -182,13 +218,25 @@ int blocks_for(int64_t n) {
 
 size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// The op chain and the NB partial sums of one reduction in the scratch buffer:
-// [ops | levels | partials], each part 256-byte aligned.
-int upload_chain(int nops, const qh_op *ops, int nlev, const qh_level *lev, qh_op **dops, qh_level **dlev,
-                 size_t part_bytes, void **part) {
+// The op chain of one reduction, as a kernel argument where it fits, else in the
+// scratch buffer, and part_bytes of that buffer: [ops | levels | part], each
+// 256-byte aligned.
+int place_chain(int nops, const qh_op *ops, int nlev, const qh_level *lev, ChainArg *arg, qh_op **dops,
+                qh_level **dlev, size_t part_bytes, void **part) {
   for (int k = 0; k < nops; k++)
     QH_REQUIRE(ops[k].levels > 0 && ops[k].stride > 0 && ops[k].tab >= 0 && ops[k].tab + ops[k].levels <= nlev,
                QH_EINVAL, "observable op %d out of range", k);
+  arg->nops = 0;
+  *dops = nullptr;
+  *dlev = nullptr;
+  if (nops > 0 && nops <= ARG_OPS && nlev <= ARG_LEV) {
+    std::fill_n(arg->ops, ARG_OPS, qh_op{});
+    std::fill_n(arg->lev, ARG_LEV, qh_level{});
+    std::copy_n(ops, nops, arg->ops);
+    std::copy_n(lev, nlev, arg->lev);
+    arg->nops = nops;
+    return part_bytes ? qh_scratch(part_bytes, part, 0, nullptr) : QH_OK;
+  }
   const size_t bo = align256(sizeof(qh_op) * (nops > 0 ? nops : 1)),
                bl = align256(sizeof(qh_level) * (nlev > 0 ? nlev : 1));
   char *d = nullptr;
@@ -196,7 +244,7 @@ int upload_chain(int nops, const qh_op *ops, int nlev, const qh_level *lev, qh_o
   if (rc) return rc;
   *dops = (qh_op *)d;
   *dlev = (qh_level *)(d + bo);
-  *part = d + bo + bl;
+  if (part_bytes) *part = d + bo + bl;
   if (nops) QH_HIP(hipMemcpyAsync(*dops, ops, sizeof(qh_op) * nops, hipMemcpyHostToDevice, qh_stream()));
   if (nlev) QH_HIP(hipMemcpyAsync(*dlev, lev, sizeof(qh_level) * nlev, hipMemcpyHostToDevice, qh_stream()));
   return QH_OK;
@@ -208,17 +256,22 @@ int expect_impl(int dm, const qh_vec *x, int64_t tot, int nops, const qh_op *ops
   QH_REQUIRE(dm ? (tot * tot == x->n) : (tot == x->n), QH_EINVAL, "expectation: vector size mismatch");
   qh_op *dops = nullptr;
   qh_level *dlev = nullptr;
+  // the blocks write their sums straight into pinned host memory
   double2 *part = nullptr;
-  int rc = upload_chain(nops, ops, nlev, lev, &dops, &dlev, sizeof(double2) * NB, (void **)&part);
+  const int nb = blocks_for(tot);
+  ChainArg arg;
+  int rc = place_chain(nops, ops, nlev, lev, &arg, &dops, &dlev, 0, nullptr);
+  if (!rc) rc = qh_scratch(0, nullptr, sizeof(double2) * nb, (void **)&part);
   if (!rc) {
-    const int nb = blocks_for(tot);
     if (dm)
-      hipLaunchKernelGGL(k_expect_dm, dim3(nb), dim3(256), 0, qh_stream(), (const void *)x->d, x->lo, tot, dops,
-                         nops, dlev, part);
+      hipLaunchKernelGGL(k_expect_dm, dim3(nb), dim3(256), 0, qh_stream(), (const void *)x->d, x->lo, tot, arg,
+                         dops, nops, dlev, part);
     else
-      hipLaunchKernelGGL(k_expect_wf, dim3(nb), dim3(256), 0, qh_stream(), (const void *)x->d, x->lo, tot, dops,
-                         nops, dlev, part);
-    rc = finish2(part, nb, re, im);
+      hipLaunchKernelGGL(k_expect_wf, dim3(nb), dim3(256), 0, qh_stream(), (const void *)x->d, x->lo, tot, arg,
+                         dops, nops, dlev, part);
+    QH_HIP(hipGetLastError());
+    QH_HIP(hipStreamSynchronize(qh_stream()));
+    sum2(part, nb, re, im);
   }
   return rc;
 }
@@ -367,12 +420,13 @@ extern "C" int qh_ens_expect(const qh_vec *ens, int64_t M, int64_t tot, int nops
   qh_op *dops = nullptr;
   qh_level *dlev = nullptr;
   double2 *out = nullptr;
-  rc = upload_chain(nops, ops, nlev, levels, &dops, &dlev, sizeof(double2) * (size_t)M, (void **)&out);
+  ChainArg arg;
+  rc = place_chain(nops, ops, nlev, levels, &arg, &dops, &dlev, sizeof(double2) * (size_t)M, (void **)&out);
   double2 *h = nullptr;
   if (!rc) rc = qh_scratch(0, nullptr, sizeof(double2) * (size_t)M, (void **)&h);
   if (!rc) {
     hipLaunchKernelGGL(k_expect_ens, dim3((unsigned)M), dim3(256), 0, qh_stream(), (const double2 *)ens->d, tot,
-                       dops, nops, dlev, out);
+                       arg, dops, nops, dlev, out);
     if (hipMemcpyAsync(h, out, sizeof(double2) * M, hipMemcpyDeviceToHost, qh_stream()) != hipSuccess ||
         hipStreamSynchronize(qh_stream()) != hipSuccess) {
       qh_set_error("qh_ens_expect: device copy failed");
@@ -472,7 +526,10 @@ extern "C" int qh_expect_dm_noalloc(const qh_vec *x, int64_t tot, int nops, cons
   if (nops) QH_HIP(hipMemcpyAsync(dops, ops, sizeof(qh_op) * nops, hipMemcpyHostToDevice, s));
   if (nlev) QH_HIP(hipMemcpyAsync(dlev, levels, sizeof(qh_level) * nlev, hipMemcpyHostToDevice, s));
   const int nb = blocks_for(tot);
-  hipLaunchKernelGGL(k_expect_dm, dim3(nb), dim3(256), 0, s, (const void *)x->d, x->lo, tot, dops, nops, dlev, part);
+  ChainArg arg;  // left empty: the chain is in the array
+  arg.nops = 0;
+  hipLaunchKernelGGL(k_expect_dm, dim3(nb), dim3(256), 0, s, (const void *)x->d, x->lo, tot, arg, dops, nops, dlev,
+                     part);
   hipLaunchKernelGGL(k_sum_partials_seq, dim3(1), dim3(1), 0, s, (const double2 *)part, nb, total);
   QH_HIP(hipGetLastError());
   double2 h;
