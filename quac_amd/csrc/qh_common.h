@@ -119,6 +119,7 @@ struct qh_mat {
   int lanes64 = 0, lanes32 = 0;  // SpMV variant: lanes per row of the CSR kernel, or QH_KSELL
   int lanes_forced = 0;          // set by qh_mat_set_lanes (not by the autotuner)
   int32_t max_row = 0;         // longest row
+  int32_t max_off = 0;         // most entries of a row off the diagonal (small matrices, with max_row)
   // slot-aligned sliced ELL (built on demand from the CSR)
   int ks_state = 0;            // 0 not built, 1 built, -1 not applicable (a row longer than 64)
   int32_t nslices = 0;

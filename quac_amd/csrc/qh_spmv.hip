@@ -1294,34 +1294,43 @@ extern "C" int qh_last_stage_ms(double *spmv_ms, int64_t *launches) {
 // read per entry and one barrier.  The state is kept in FP64 for both storage
 // precisions; the matrix values are FP64.
 // Bound by that chain: reads, dependent FMAs, barrier.  Jaynes-Cummings 2 x 10 (400
-// rows of at most 5 entries), 100 steps: 95 us, 180 us with the
+// rows of at most 5 entries), 100 steps: 75 us, 180 us with the
 // stage derivatives in LDS (two reads an entry, no two in flight).
 #define QH_SMALL_ROWS 800
 // up to this many rows a thread has the registers for more than 8 entries
 #define QH_SMALL_WIDE_ROWS 640
 
-// Row r of the generator: its (at most MAXNZ) entries in registers, filled up with
-// zeros times the zero cell n of the vector so that all reads are in flight
-// together; MAXNZ == 0: read from the CSR in memory.
+// Row r of the generator in registers: its diagonal entry, which multiplies the
+// thread's own value, and its (at most MAXNZ) other entries, filled up with zeros
+// times the zero cell n of the vector so that all reads are in flight together;
+// MAXNZ == 0: the row is read from the CSR in memory.
 template <int MAXNZ>
 struct SmallRow {
   int32_t c[MAXNZ > 0 ? MAXNZ : 1];
   double2 v[MAXNZ > 0 ? MAXNZ : 1];
+  double2 d = {0.0, 0.0};
   int32_t b = 0, e = 0;
   __device__ __forceinline__ void load(int32_t n, int32_t r, const int32_t *rp, const int32_t *col, const double2 *val) {
     if (r < n) {
       b = rp[r];
       e = rp[r + 1];
     }
+    if constexpr (MAXNZ > 0) {
+      int32_t at = e - b;  // position of the diagonal entry
+      for (int32_t k = b; k < e; k++)
+        if (col[k] == r) at = k - b;
+      if (at < e - b) d = val[b + at];
 #pragma unroll
-    for (int k = 0; k < MAXNZ; k++) {
-      const bool on = b + k < e;
-      c[k] = on ? col[b + k] : n;
-      v[k] = on ? val[b + k] : make_double2(0.0, 0.0);
+      for (int k = 0; k < MAXNZ; k++) {
+        const int32_t s = b + k + (k >= at ? 1 : 0);
+        const bool on = s < e;
+        c[k] = on ? col[s] : n;
+        v[k] = on ? val[s] : make_double2(0.0, 0.0);
+      }
     }
   }
-  // the row times y
-  __device__ __forceinline__ double2 dot(const double2 *y, const int32_t *col, const double2 *val) const {
+  // the row times y; own: y of the row itself
+  __device__ __forceinline__ double2 dot(const double2 *y, double2 own, const int32_t *col, const double2 *val) const {
     double are = 0.0, aim = 0.0;
     auto add = [&](double2 a, double2 x) {
       are = fma(a.x, x.x, fma(-a.y, x.y, are));
@@ -1329,6 +1338,7 @@ struct SmallRow {
     };
     if constexpr (MAXNZ > 0) {
       constexpr int CH = MAXNZ <= 8 ? MAXNZ : 4;  // reads in flight (the registers hold the entries as well)
+      add(d, own);
 #pragma unroll
       for (int k0 = 0; k0 < MAXNZ; k0 += CH) {
         double2 t[CH];
@@ -1370,10 +1380,11 @@ __global__ void __launch_bounds__(MAXNZ > 8 ? QH_SMALL_WIDE_ROWS : 832) k_rk4_sm
   __syncthreads();
   const double cs[4] = {h / 4.0, h / 3.0, h / 2.0, h};
   for (int64_t st = 0; st < nsteps; st++) {
+    double2 y = x;
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-      const double2 k = row.dot(q & 1 ? y1 : y0, col, val);
-      const double2 y = make_double2(fma(cs[q], k.x, x.x), fma(cs[q], k.y, x.y));
+      const double2 k = row.dot(q & 1 ? y1 : y0, y, col, val);
+      y = make_double2(fma(cs[q], k.x, x.x), fma(cs[q], k.y, x.y));
       if (r < n) (q & 1 ? y0 : y1)[r] = y;
       if (q == 3) x = y;
       __syncthreads();
@@ -1418,7 +1429,7 @@ __global__ void __launch_bounds__(MAXNZ > 8 ? QH_SMALL_WIDE_ROWS : 832) k_rk4_sm
 // (FSAL).  adaptive == 0: fixed steps of h0 (the last cut at tmax), K1 recomputed.
 // out: final time, accepted steps, the next step size.
 // Bound by the chain of a trial: three stages, the weighted error, its sum over the
-// workgroup, the controller.  Jaynes-Cummings 2 x 10 (400 rows), t = 20: 1.05 ms,
+// workgroup, the controller.  Jaynes-Cummings 2 x 10 (400 rows), t = 20: 1.0 ms,
 // 1.85 ms with everything in LDS, the controller on one thread and pow.
 #define QH_SMALL_BS3_ROWS 640
 
@@ -1453,14 +1464,16 @@ __global__ void __launch_bounds__(QH_SMALL_BS3_ROWS) k_rk3bs_small(int32_t n, co
                                                       double rtol, double hmin, double hmax, int adaptive, double eps,
                                                       double *out) {
   extern __shared__ double2 sm[];
-  __shared__ double red[QH_SMALL_BS3_ROWS / 64];
+  constexpr int WAVES = QH_SMALL_BS3_ROWS / 64;
+  __shared__ double red[WAVES];  // zero past the workgroup's wavefronts
   double2 *const ya = sm, *const yb = sm + n + 1;
-  const int r = threadIdx.x, waves = blockDim.x >> 6;  // n <= blockDim.x
+  const int r = threadIdx.x;  // n <= blockDim.x
   SmallRow<MAXNZ> row;
   row.load(n, r, rp, col, val);
   const double2 zero = make_double2(0.0, 0.0);
   double2 x = r < n ? xg[r] : zero, k1 = zero;
   if (r == 0) ya[n] = yb[n] = zero;
+  if (r < WAVES) red[r] = 0.0;
   if (r < n) yb[r] = x;
   __syncthreads();
   const double c1 = 2.0 / 9.0 - 7.0 / 24.0, c2 = 1.0 / 3.0 - 1.0 / 4.0, c3 = 4.0 / 9.0 - 1.0 / 3.0, c4 = -1.0 / 8.0;
@@ -1476,18 +1489,20 @@ __global__ void __launch_bounds__(QH_SMALL_BS3_ROWS) k_rk3bs_small(int32_t n, co
     const double hh = (t + h > tmax) ? tmax - t : h;
     // yb holds x wherever K1 is still to be formed: at the start, and after every
     // fixed step (its xn)
-    if (!have_k1) k1 = row.dot(yb, col, val);
-    if (r < n) ya[r] = make_double2(x.x + 0.5 * hh * k1.x, x.y + 0.5 * hh * k1.y);
+    if (!have_k1) k1 = row.dot(yb, x, col, val);
+    const double2 y2 = make_double2(x.x + 0.5 * hh * k1.x, x.y + 0.5 * hh * k1.y);
+    if (r < n) ya[r] = y2;
     __syncthreads();
-    const double2 k2 = row.dot(ya, col, val);
-    if (r < n) yb[r] = make_double2(x.x + 0.75 * hh * k2.x, x.y + 0.75 * hh * k2.y);
+    const double2 k2 = row.dot(ya, y2, col, val);
+    const double2 y3 = make_double2(x.x + 0.75 * hh * k2.x, x.y + 0.75 * hh * k2.y);
+    if (r < n) yb[r] = y3;
     __syncthreads();
-    const double2 k3 = row.dot(yb, col, val);
+    const double2 k3 = row.dot(yb, y3, col, val);
     const double2 xn = make_double2(x.x + hh * (2.0 / 9.0) * k1.x + hh / 3.0 * k2.x + hh * (4.0 / 9.0) * k3.x,
                                     x.y + hh * (2.0 / 9.0) * k1.y + hh / 3.0 * k2.y + hh * (4.0 / 9.0) * k3.y);
     if (r < n) ya[r] = xn;
     __syncthreads();
-    const double2 k4 = row.dot(ya, col, val);
+    const double2 k4 = row.dot(ya, xn, col, val);
     double v = 0.0;
     if (r < n) {
       const double er = hh * (c1 * k1.x + c2 * k2.x + c3 * k3.x + c4 * k4.x);
@@ -1500,8 +1515,11 @@ __global__ void __launch_bounds__(QH_SMALL_BS3_ROWS) k_rk3bs_small(int32_t n, co
     v = wave_sum(v);
     if ((r & 63) == 0) red[r >> 6] = v;
     __syncthreads();
-    double sum = 0.0;
-    for (int w = 0; w < waves; w++) sum += red[w];
+    double part[WAVES], sum = 0.0;
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) part[w] = red[w];
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) sum += part[w];
     const double err = sqrt(sum / (double)n);
     // a non-finite error estimate (a NaN or infinite state) ends the
     // integration: the controller could not leave the step otherwise
@@ -1554,9 +1572,9 @@ extern "C" int qh_rk3bs_small(qh_mat *A, qh_vec *x, double t0, double tmax, doub
   const size_t lds = (size_t)2 * (n + 1) * sizeof(double2);
   const double eps = 1e-12 * (fabs(tmax) + fabs(h0) + 1.0);
   hipStream_t s = qh_stream();
-  // the least padding of the rows' registers; rows of more than 16 entries are read
+  // the least padding of the rows' registers; rows of more than 16 entries off the diagonal are read
   // from the CSR, which the caches hold for a generator this small
-  const int mr = A->max_row;
+  const int mr = A->max_off;
 #define QH_LB(Z)                                                                                                \
   hipLaunchKernelGGL((k_rk3bs_small<Z>), dim3(1), dim3(bt), lds, s, n, A->rowptr, A->col, A->val,             \
                      (double2 *)x->d, t0, tmax, h0, steps_max, atol, rtol, hmin, hmax, adaptive, eps, dout)
@@ -1579,12 +1597,21 @@ extern "C" int qh_rk3bs_small(qh_mat *A, qh_vec *x, double t0, double tmax, doub
 }
 
 // longest row of a CSR: per-block maxima over a grid-stride range, combined
-// with an atomic max into out[0] (zeroed by the caller)
-__global__ void k_max_row(const int32_t *__restrict__ rp, int64_t n, int32_t *out) {
+// with an atomic max into out[0] (zeroed by the caller); with col (a small matrix)
+// also the most entries off the diagonal, into out[1]
+__global__ void k_max_row(const int32_t *__restrict__ rp, const int32_t *__restrict__ col, int64_t n, int32_t *out) {
   __shared__ int32_t red[256];
-  int32_t m = 0;
-  for (int64_t r = blockIdx.x * 256 + threadIdx.x; r < n; r += (int64_t)gridDim.x * 256)
-    m = max(m, rp[r + 1] - rp[r]);
+  int32_t m = 0, off = 0;
+  for (int64_t r = blockIdx.x * 256 + threadIdx.x; r < n; r += (int64_t)gridDim.x * 256) {
+    const int32_t len = rp[r + 1] - rp[r];
+    m = max(m, len);
+    if (col) {
+      int32_t own = 0;
+      for (int32_t k = rp[r]; k < rp[r + 1]; k++) own += col[k] == (int32_t)r;
+      off = max(off, len - own);
+    }
+  }
+  if (off) atomicMax(out + 1, off);
   red[threadIdx.x] = m;
   __syncthreads();
   for (int o = 128; o > 0; o >>= 1) {
@@ -1597,18 +1624,20 @@ __global__ void k_max_row(const int32_t *__restrict__ rp, int64_t n, int32_t *ou
 int qh_mat_max_row(qh_mat *A) {
   if (A->max_row > 0) return QH_OK;
   int32_t *d = nullptr;
-  int rc = qh_alloc_t(&d, 1);
+  int rc = qh_alloc_t(&d, 2);
   if (rc) return rc;
   hipStream_t s = qh_stream();
-  QH_HIP(hipMemsetAsync(d, 0, sizeof(int32_t), s));
+  QH_HIP(hipMemsetAsync(d, 0, 2 * sizeof(int32_t), s));
   const unsigned nb = (unsigned)std::min<int64_t>(qh_blocks(A->rows, 256), 1024);
-  hipLaunchKernelGGL(k_max_row, dim3(nb > 0 ? nb : 1), dim3(256), 0, s, A->rowptr, A->rows, d);
+  hipLaunchKernelGGL(k_max_row, dim3(nb > 0 ? nb : 1), dim3(256), 0, s, A->rowptr,
+                     A->rows <= QH_SMALL_ROWS ? A->col : nullptr, A->rows, d);
   QH_HIP(hipGetLastError());
-  int32_t h = 0;
-  QH_HIP(hipMemcpyAsync(&h, d, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+  int32_t h[2] = {0, 0};
+  QH_HIP(hipMemcpyAsync(h, d, sizeof(h), hipMemcpyDeviceToHost, s));
   QH_HIP(hipStreamSynchronize(s));
   qh_free_ptr(d);
-  A->max_row = h > 0 ? h : 1;
+  A->max_row = h[0] > 0 ? h[0] : 1;
+  A->max_off = h[1];
   return QH_OK;
 }
 
@@ -1619,7 +1648,7 @@ static int rk4_small(qh_mat *A, qh_vec *x, double dt, int64_t nsteps, int64_t to
   const int bt = ((n + 63) / 64) * 64;
   const size_t lds = (size_t)2 * (n + 1) * sizeof(double2);
   hipStream_t s = qh_stream();
-  const int mr = A->max_row;
+  const int mr = A->max_off;
 #define QH_LS1(F, Z)                                                                                            \
   hipLaunchKernelGGL((k_rk4_small<F, Z>), dim3(1), dim3(bt), lds, s, n, A->rowptr, A->col, A->val, x->d, x->lo, \
                      dt, nsteps, tot, renorm_every)
