@@ -327,6 +327,9 @@ int qh_ens_norms(const qh_vec *ens, int64_t M, double *norms2);
 /* mean over the trajectories of <psi|O|psi>/<psi|psi> (qvec_utilities.c:1353-1420) */
 int qh_ens_expect(const qh_vec *ens, int64_t M, int64_t tot, int nops, const qh_op *ops, int nlev,
                   const qh_level *levels, double *re, double *im);
+/* mean and variance (over M - 1) over the trajectories of |a_i|^2 / <psi|psi> for
+ * every level i, into host arrays of tot entries (qvec_utilities.c:1682-2022) */
+int qh_ens_probs(const qh_vec *ens, int64_t M, int64_t tot, double *mean, double *var);
 /* fits = 1 when the qh_mcwf_* calls below accept A and nj jump operators */
 int qh_mcwf_fits(const qh_mat *A, int nj, int *fits);
 /* Trajectories of at most 1024 amplitudes (rows of A with at most 16 entries):
