@@ -161,12 +161,14 @@ __device__ inline int32_t cp_wave_max(int32_t v) {
   return v;
 }
 
-// slots of every slice: imaginary parts (made even) and all
+// slots of every slice: imaginary parts (made even) and all (count: the slices'
+// number where only the device has it)
 __global__ void __launch_bounds__(256) k_cp_width(const int32_t *order, const int32_t *__restrict__ rp,
                                                   const int32_t *__restrict__ col, const double2 *__restrict__ val,
-                                                  int32_t *width, int32_t *nim, int32_t nslices) {
+                                                  int32_t *width, int32_t *nim, int32_t nslices,
+                                                  const int32_t *count) {
   const int32_t s = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (s >= nslices) return;
+  if (s >= (count ? *count : nslices)) return;
   const int32_t r = order[(int64_t)s * 64 + lane];
   int32_t ni = 0, nr = 0;
   if (r >= 0)
@@ -298,6 +300,188 @@ __global__ void __launch_bounds__(1024) k_cp_dict(const int32_t *bins, const int
       }
     for (; pi < p1; pi++) ew[pi * 64 + lane] = 0u;
     for (; pr < s1; pr++) ew[pr * 64 + lane] = 0u;
+  }
+}
+
+// ------------------------------------------------------- plan of a small matrix
+// A matrix of up to CP_SMALL_ROWS rows has its components, bins and order formed by
+// one workgroup in LDS and its offsets by another, so that a new parameter set waits
+// for the device once (four integers) and not for a dozen launches and three round
+// trips: 2^2 x 23 rows from its terms to its populations 0.56 -> 0.44 ms.
+const int CP_SMALL_ROWS = 16384, CP_SMALL_GRAN = CP_SMALL_ROWS / CP_GRAN + 1;
+enum { CPS_BINS = 0, CPS_SLICES, CPS_ROWS, CPS_WIDTH, CPS_SLOTS, CPS_N };  // rows: the largest bin's, whole slices
+
+// inclusive sum over the wavefront
+__device__ inline int32_t cp_wave_scan(int32_t v, int lane) {
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int32_t u = __shfl_up(v, o, 64);
+    if (lane >= o) v += u;
+  }
+  return v;
+}
+
+__global__ void __launch_bounds__(1024) k_cp_small(const int32_t *__restrict__ rp, const int32_t *__restrict__ col,
+                                                   int32_t n, int32_t *order, int32_t *pos, int32_t *bslice,
+                                                   int32_t *bins, int32_t *info) {
+  extern __shared__ int32_t ls[];
+  int32_t *parent = ls, *size = ls + n;  // size: rows of a root, then its offset in the sorted order
+  __shared__ int32_t hist[16][CP_SMALL_GRAN], gsize[CP_SMALL_GRAN], gbin[CP_SMALL_GRAN], first[CP_SMALL_GRAN + 1];
+  __shared__ int32_t part[16];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int32_t ngran = n / CP_GRAN + 1;
+  for (int32_t r = t; r < n; r += 1024) {
+    parent[r] = r;
+    size[r] = 0;
+  }
+  for (int32_t g = t; g < ngran; g += 1024) {
+    gsize[g] = 0;
+    for (int w = 0; w < 16; w++) hist[w][g] = 0;
+  }
+  __syncthreads();
+  volatile int32_t *vp = parent;
+  auto find = [&](int32_t i) {
+    int32_t q = vp[i];
+    while (q != i) {
+      const int32_t g = vp[q];
+      if (g != q) vp[i] = g;
+      i = q;
+      q = g;
+    }
+    return i;
+  };
+  for (int32_t r = t; r < n; r += 1024) {
+    int32_t a = r;
+    const int32_t end = rp[r + 1];
+    for (int32_t e0 = rp[r]; e0 < end; e0 += 8) {
+      int32_t c[8];  // in flight together
+#pragma unroll
+      for (int k = 0; k < 8; k++) c[k] = e0 + k < end ? col[e0 + k] : r;
+#pragma unroll 1
+      for (int k = 0; k < 8; k++) {
+        int32_t b = c[0];
+#pragma unroll
+        for (int q = 0; q < 7; q++) c[q] = c[q + 1];
+        if (b == r) continue;
+        for (;;) {
+          a = find(a);
+          b = find(b);
+          if (a == b) break;
+          const int32_t hi = a > b ? a : b, lo = a > b ? b : a;
+          const int32_t old = atomicCAS(parent + hi, hi, lo);
+          a = lo;
+          if (old == hi) break;
+          b = old;
+        }
+      }
+    }
+  }
+  __syncthreads();
+  for (int32_t r = t; r < n; r += 1024) {
+    const int32_t l = find(r);
+    vp[r] = l;
+    atomicAdd(size + l, 1);
+  }
+  __syncthreads();
+  // offsets of the components in the order of their roots, and the granules' rows
+  const int32_t per = (n + 1023) / 1024, b0 = min(t * per, n), b1 = min(b0 + per, n);
+  int32_t own = 0;
+  for (int32_t r = b0; r < b1; r++) own += size[r];
+  const int32_t inc = cp_wave_scan(own, lane);
+  if (lane == 63) part[wave] = inc;
+  __syncthreads();
+  int32_t run = inc - own;
+  for (int w = 0; w < wave; w++) run += part[w];
+  for (int32_t r = b0; r < b1; r++) {
+    const int32_t s = size[r];
+    if (s) atomicAdd(gsize + run / CP_GRAN, s);
+    size[r] = run;
+    run += s;
+  }
+  __syncthreads();
+  if (wave == 0) {  // a bin for every granule with rows
+    int32_t nb = 0, sl = 0, most = 0;
+    for (int32_t g0 = 0; g0 < ngran; g0 += 64) {
+      const int32_t v = g0 + lane < ngran ? gsize[g0 + lane] : 0;
+      const uint64_t m = __ballot(v > 0);
+      const int32_t b = nb + (int32_t)__popcll(m & ((1ull << lane) - 1ull)), k = (v + 63) / 64;
+      const int32_t at = sl + cp_wave_scan(k, lane) - k;
+      if (v > 0) {
+        gbin[g0 + lane] = b;
+        first[b] = at;
+        bslice[b] = at;
+        bins[b] = b;
+      }
+      most = max(most, cp_wave_max(k));
+      nb += (int32_t)__popcll(m);
+      sl = __shfl(at + k, 63, 64);
+    }
+    if (lane == 0) {
+      first[nb] = sl;
+      bslice[nb] = sl;
+      info[CPS_BINS] = nb;
+      info[CPS_SLICES] = sl;
+      info[CPS_ROWS] = most * 64;
+    }
+    part[0] = nb;
+  }
+  __syncthreads();
+  const int32_t nb = part[0];
+  for (int32_t p = t; p < first[nb] * 64; p += 1024) order[p] = -1;
+  for (int32_t r = t; r < n; r += 1024) parent[r] = gbin[size[parent[r]] / CP_GRAN];  // the row's bin
+  __syncthreads();
+  // rows in increasing order within a bin: wavefront w takes the w-th part of them
+  const int32_t c = ((n + 15) / 16 + 63) / 64 * 64, r0 = min(wave * c, n), r1 = min(r0 + c, n);
+  for (int32_t r = r0 + lane; r < r1; r += 64) atomicAdd(&hist[wave][parent[r]], 1);
+  __syncthreads();
+  for (int32_t b = t; b < nb; b += 1024) {
+    int32_t s = 0;
+    for (int w = 0; w < 16; w++) {
+      const int32_t v = hist[w][b];
+      hist[w][b] = s;
+      s += v;
+    }
+  }
+  __syncthreads();
+  for (int32_t rr = r0; rr < r1; rr += 64) {
+    const int32_t r = rr + lane;
+    const int32_t b = r < r1 ? parent[r] : -1;
+    uint64_t left = __ballot(b >= 0);
+    int32_t at = 0;
+    while (left) {
+      const int32_t f = __shfl(b, __ffsll((unsigned long long)left) - 1, 64);
+      const uint64_t m = __ballot(b == f);
+      if (b == f) at = hist[wave][f] + (int32_t)__popcll(m & ((1ull << lane) - 1ull));
+      __builtin_amdgcn_wave_barrier();
+      if (lane == 0) hist[wave][f] += (int32_t)__popcll(m);
+      __builtin_amdgcn_wave_barrier();
+      left &= ~m;
+    }
+    if (b >= 0) {
+      pos[r] = at;
+      order[(int64_t)first[b] * 64 + at] = r;
+    }
+  }
+}
+
+// offsets of the slices' slots, their bins' zero cells, the widest slice and all slots
+__global__ void __launch_bounds__(64) k_cp_small_offsets(const int32_t *width, const int32_t *bslice, int32_t *soff,
+                                                         int32_t *zc, int32_t *info) {
+  const int lane = threadIdx.x;
+  const int32_t nsl = info[CPS_SLICES], nb = info[CPS_BINS];
+  int32_t run = 0, most = 0;
+  for (int32_t s0 = 0; s0 < nsl; s0 += 64) {
+    const int32_t w = s0 + lane < nsl ? width[s0 + lane] : 0;
+    const int32_t inc = cp_wave_scan(w, lane);
+    if (s0 + lane < nsl) soff[s0 + lane] = run + inc - w;
+    most = max(most, cp_wave_max(w));
+    run += __shfl(inc, 63, 64);
+  }
+  for (int32_t b = lane; b < nb; b += 64)
+    for (int32_t s = bslice[b]; s < bslice[b + 1]; s++) zc[s] = (bslice[b + 1] - bslice[b]) * 64;
+  if (lane == 0) {
+    info[CPS_WIDTH] = most;
+    info[CPS_SLOTS] = run;
   }
 }
 
@@ -616,6 +800,129 @@ struct Carve {
 // table
 const double CP_CLK_REG = 10.0, CP_CLK_WORD = 24.0, CP_CLK_FIXED = 500.0;
 
+// Whether a stage of the plan (the largest bin's clocks, and all bins') beats the
+// sliced stage kernels: 2.5 us a launch, and 11 us a million rows.
+// Measured us a stage, here / there: Jaynes-Cummings 2 x 24 0.30 / 2.6, Tavis-Cummings
+// 2^2 x 23 0.44 / 2.7, 2^3 x 17 1.00 / 3.5, 2^3 x 30 1.49 / 4.3, decay and dephasing of
+// 7 qubits 0.34 / 2.8, 10 5.1 / 13.2, 12 46.7 / 243.  Refused: 2^4 x 8 (bins of 1768
+// rows whose entries do not fit the registers) 5.0 / 3.3, 2^4 x 19 10.5 / 5.4, 6-qubit
+// chain (one bin of 4096 rows) 10.9 / 3.0.
+bool cp_worth(double most, double all, int64_t n) {
+  const double comp_us = std::max(most, all / (double)qh_num_cus() + CP_CLK_FIXED) / 2400.0;
+  return comp_us <= 0.9 * (2.5 + 1.1e-5 * (double)n);
+}
+
+int cp_width_class(int w, bool few) {
+  for (int u : {4, 8, 10, 12, 16, 24, 32})
+    if (w <= u && (few || u != 10)) return u;
+  return 0;
+}
+
+int cp_threads(int rows) {
+  return rows <= 64 ? 64 : rows <= 128 ? 128 : rows <= 256 ? 256 : rows <= 512 ? 512 : 1024;
+}
+
+// two rows a thread: up to 12 slots each fit the 128 registers
+bool cp_fits_registers(int rows, int W) { return W && (rows <= 1024 || (rows <= CP_REG_ROWS && W <= 12)); }
+
+// The plan of a matrix of at most CP_SMALL_ROWS rows with one shape for all bins
+// (*done = 0 where it needs the general builder)
+int cp_build_small(qh_mat *A, int f32, int *done) {
+  *done = 0;
+  const int32_t n = (int32_t)A->rows;
+  hipStream_t s = qh_stream();
+  const int32_t ngran = n / CP_GRAN + 1, maxsl = n / 64 + ngran;
+  int32_t *order, *pos, *bslice, *bins, *soff, *nim, *zc, *width, *info;
+  double2 *diag;
+  double *trace;
+  auto arrays = [&](Carve &q) {
+    order = q.take<int32_t>((size_t)maxsl * 64);
+    pos = q.take<int32_t>(n);
+    bslice = q.take<int32_t>(ngran + 1);
+    bins = q.take<int32_t>(ngran);
+    soff = q.take<int32_t>(maxsl);
+    nim = q.take<int32_t>(maxsl);
+    zc = q.take<int32_t>(maxsl);
+    width = q.take<int32_t>(maxsl);
+    info = q.take<int32_t>(CPS_N);
+    diag = q.take<double2>((size_t)maxsl * 64);
+    trace = q.take<double>(QH_COMP_TRACE);
+  };
+  Carve size, at;
+  arrays(size);
+  qh_comp *c = new qh_comp();
+  auto fail = [&](int code) {
+    (void)hipStreamSynchronize(s);
+    qh_comp_free(c);
+    return code;
+  };
+  int32_t *h = nullptr;
+  int rc = qh_alloc(&c->buf, size.n);
+  if (!rc) rc = qh_scratch(0, nullptr, CPS_N * sizeof(int32_t), (void **)&h);
+  if (rc) return fail(rc);
+  at.p = (char *)c->buf;
+  arrays(at);
+#define CP_HIP(call)                                                                  \
+  do {                                                                                \
+    hipError_t e_ = (call);                                                           \
+    if (e_ != hipSuccess) {                                                           \
+      qh_set_error("%s:%d %s: %s", __FILE__, __LINE__, #call, hipGetErrorString(e_)); \
+      return fail(QH_EHIP);                                                           \
+    }                                                                                 \
+  } while (0)
+  const size_t lds = (size_t)2 * n * sizeof(int32_t);
+  if (lds > 40 * 1024)
+    CP_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_cp_small), hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)lds));
+  hipLaunchKernelGGL(k_cp_small, dim3(1), dim3(1024), lds, s, A->rowptr, A->col, n, order, pos, bslice, bins, info);
+  hipLaunchKernelGGL(k_cp_width, dim3(qh_blocks(maxsl, 4)), dim3(256), 0, s, order, A->rowptr, A->col, A->val, width,
+                     nim, maxsl, (const int32_t *)(info + CPS_SLICES));
+  hipLaunchKernelGGL(k_cp_small_offsets, dim3(1), dim3(64), 0, s, width, bslice, soff, zc, info);
+  CP_HIP(hipGetLastError());
+  CP_HIP(hipMemcpyAsync(h, info, CPS_N * sizeof(int32_t), hipMemcpyDeviceToHost, s));
+  CP_HIP(hipStreamSynchronize(s));
+  const int nb = h[CPS_BINS], nsl = h[CPS_SLICES], rows = h[CPS_ROWS], W = cp_width_class(h[CPS_WIDTH], true);
+  const int64_t slots = h[CPS_SLOTS];
+  if (!cp_fits_registers(rows, W)) return fail(QH_OK);
+  *done = 1;
+  if (!cp_worth(CP_CLK_REG * W * (rows / 64) + CP_CLK_FIXED, CP_CLK_REG * W * nsl, n)) {
+    A->comp_state[f32] = -1;
+    return fail(QH_OK);
+  }
+  double *ev;
+  uint16_t *ec;
+  auto entries = [&](Carve &q) {
+    ev = q.take<double>((size_t)slots * 64 + 1);
+    ec = q.take<uint16_t>((size_t)slots * 64 + 1);
+  };
+  Carve em, ep;
+  entries(em);
+  rc = qh_alloc(&c->slots, em.n);
+  if (rc) return fail(rc);
+  ep.p = (char *)c->slots;
+  entries(ep);
+  hipLaunchKernelGGL(k_cp_fill, dim3(qh_blocks(nsl, 4)), dim3(256), 0, s, order, pos, A->rowptr, A->col, A->val,
+                     soff, width, nim, zc, diag, ev, ec, nsl);
+  CP_HIP(hipGetLastError());
+#undef CP_HIP
+  const int S = rows > 1024 ? 2 : 1;
+  c->classes.push_back(CpClass{cp_threads(rows), S, W, false, false, 0, nb, rows + 1});
+  c->a = CpArgs{};
+  c->a.bins = bins;
+  c->a.bslice = bslice;
+  c->a.soff = soff;
+  c->a.width = width;
+  c->a.nim = nim;
+  c->a.order = order;
+  c->a.diag = diag;
+  c->a.ev = ev;
+  c->a.ec = ec;
+  c->trace = trace;
+  A->comp[f32] = c;
+  A->comp_state[f32] = 1;
+  return QH_OK;
+}
+
 int cp_build(qh_mat *A, int f32) {
   const int32_t max_rows = f32 ? CP_MAX_ROWS32 : CP_MAX_ROWS64;
   int &state = A->comp_state[f32];
@@ -767,18 +1074,13 @@ int cp_build(qh_mat *A, int f32) {
                      (int64_t)nsl * 64);
   hipLaunchKernelGGL(k_cp_place, dim3(nb256), dim3(256), 0, s, parent, size, brow, bslice, order, pos, n);
   hipLaunchKernelGGL(k_cp_width, dim3(qh_blocks(nsl, 4)), dim3(256), 0, s, order, A->rowptr, A->col, A->val, width,
-                     nim, nsl);
+                     nim, nsl, nullptr);
   CP_HIP(hipGetLastError());
   std::vector<int32_t> hwid(nsl), hoff(nsl), hzc(nsl);
   CP_HIP(hipMemcpyAsync(hwid.data(), width, sizeof(int32_t) * nsl, hipMemcpyDeviceToHost, s));
   CP_HIP(hipStreamSynchronize(s));
   // the shape of every bin's launch, and what the largest bin and all of them take
   const bool few = nbins <= 2 * cus;  // the chip is not full: one launch, so that nothing waits for a launch before it
-  auto rup = [few](int w) {
-    for (int u : {4, 8, 10, 12, 16, 24, 32})
-      if (w <= u && (few || u != 10)) return u;
-    return 0;
-  };
   int64_t slots[2] = {0, 0};  // held in registers, read as words
   struct Shape {
     int words, rows, W;
@@ -795,10 +1097,9 @@ int cp_build(qh_mat *A, int f32) {
       sum += hwid[i];
     }
     const int rows = (hslice[b + 1] - hslice[b]) * 64;
-    const int W = rup(w);
-    // two rows a thread: up to 12 slots each fit the 128 registers
-    const bool reg = W && (rows <= 1024 || (rows <= CP_REG_ROWS && W <= 12));
-    sh[b] = Shape{!reg, rows <= 64 ? 64 : rows <= 128 ? 128 : rows <= 256 ? 256 : rows <= 512 ? 512 : rows <= 1024 ? 1024 : rows, W, b};
+    const int W = cp_width_class(w, few);
+    const bool reg = cp_fits_registers(rows, W);
+    sh[b] = Shape{!reg, rows <= 1024 ? cp_threads(rows) : rows, W, b};
     if (reg) {
       few_rows = std::max(few_rows, sh[b].rows);
       few_w = std::max(few_w, W);
@@ -817,15 +1118,7 @@ int cp_build(qh_mat *A, int f32) {
     most = std::max(most, clk + CP_CLK_FIXED);
     all += clk;
   }
-  // Against the sliced stage kernels: 2.5 us a launch, and 11 us a million rows.
-  // Measured us a stage, here / there: Jaynes-Cummings 2 x 24 0.30 / 2.6, Tavis-Cummings
-  // 2^2 x 23 0.44 / 2.7, 2^3 x 17 1.00 / 3.5, 2^3 x 30 1.49 / 4.3, decay and dephasing of
-  // 7 qubits 0.34 / 2.8, 10 5.1 / 13.2, 12 46.7 / 243.  Refused: 2^4 x 8 (bins of 1768
-  // rows whose entries do not fit the registers) 5.0 / 3.3, 2^4 x 19 10.5 / 5.4, 6-qubit
-  // chain (one bin of 4096 rows) 10.9 / 3.0.
-  const double clk_us = 2400.0, comp_us = std::max(most, all / (double)cus + CP_CLK_FIXED) / clk_us;
-  const double stage_us = 2.5 + 1.1e-5 * (double)n;
-  if (comp_us > 0.9 * stage_us) {
+  if (!cp_worth(most, all, n)) {
     fail(0);
     state = -1;
     return QH_OK;
@@ -925,10 +1218,13 @@ int qh_comp_prepare(qh_mat *A, int prec, int *usable) {
   *usable = 0;
   if (A->comp_state[f32] == 0) {
     // row and slot numbers are 32-bit
+    int rc = QH_OK, done = 0;
     if (A->rows < 1 || A->rows > (int64_t)1 << 30)
       A->comp_state[f32] = -1;
-    else if (int rc = cp_build(A, f32))
-      return rc;
+    else if (A->rows <= CP_SMALL_ROWS)
+      rc = cp_build_small(A, f32, &done);
+    if (!rc && A->comp_state[f32] == 0 && !done) rc = cp_build(A, f32);
+    if (rc) return rc;
   }
   *usable = A->comp_state[f32] == 1;
   return QH_OK;

@@ -39,6 +39,7 @@ CASES = [
     _tc(2, 9),
     _tc(3, 17),  # a component of 1028 rows: two rows a thread
     _noisy(6),
+    _noisy(7),  # 16 384 rows, the most whose plan one workgroup forms
     _noisy(8),  # more bins than two a CU: bins of several components, a launch per shape
     _noisy(5, [("ham", 0.3, [(0, "sx")]), ("ham", 0.2, [(1, "sy")])]),  # real and imaginary entries
     _diagonal(31),
