@@ -222,6 +222,12 @@ struct qh_td_ell {
   const int32_t *col;
   const uint16_t *idx;
   const double2 *cf;
+  // variant 134, FP64: entries that every row of a uniform slot of A has in the same
+  // place and with the same value are not in the lists but added to the slot's value:
+  // their dictionary index per slot of A (-1: none), and the dictionary's size (at
+  // most 64); null: all entries are in the lists
+  const int16_t *fold = nullptr;
+  int32_t ncf = 0;
 };
 
 // A's part of the time-dependent RK stages on A's autotuned variant when that is

@@ -348,6 +348,12 @@ struct qh_td_cache {
   int32_t *sw = nullptr;            // entries per row of each slice,
   int32_t *ecol = nullptr;          // columns
   uint16_t *eidx = nullptr;         // and dictionary indices (the zero entry: index dv.size() - 1)
+  // the lists without the entries that A's uniform slots take over (td_fold): 0 not
+  // looked at, 1 built, -1 not applicable
+  int fold_state = 0;
+  int16_t *fslot = nullptr;         // dictionary index per slot of A, or -1
+  int32_t *fw = nullptr, *fcol = nullptr;
+  uint16_t *fidx = nullptr;
   std::vector<int> dk;              // the dictionary's terms
   std::vector<double2> dv;          // and values (host)
   double2 *s = nullptr;             // 4 stages x (TD_MAX coefficients, or the dictionary's s_k v)
@@ -385,6 +391,10 @@ void qh_td_cache_free(qh_td_cache *c) {
   qh_free_ptr(c->sw);
   qh_free_ptr(c->ecol);
   qh_free_ptr(c->eidx);
+  qh_free_ptr(c->fslot);
+  qh_free_ptr(c->fw);
+  qh_free_ptr(c->fcol);
+  qh_free_ptr(c->fidx);
   qh_free_ptr(c->s);
   qh_free_ptr(c->steps_cf);
   td_free_bufs(c);
@@ -689,11 +699,103 @@ static int td_add_launch(const qh_td_cache *c, int prec, const double2 *s, const
   return QH_OK;
 }
 
-// the sliced form of the merged A_k for A's stage kernel to sum in the same pass
-// (lanes 0: wherever A's variant has that form), or null
-static const qh_td_ell *td_fusable(const qh_td_cache *c, const double2 *cf, qh_td_ell *buf) {
+// One wavefront a slice: a uniform slot of A takes over a time-dependent entry that
+// each of its rows has in the slot's column with one dictionary index (a drive on an
+// operator that A itself holds); the others move up in their rows' lists.
+__global__ void __launch_bounds__(64) k_td_fold(int64_t nrows, const int32_t *__restrict__ moff,
+                                                const int32_t *__restrict__ umid, const qh_kmeta *__restrict__ meta,
+                                                const int64_t *__restrict__ soff, const int32_t *__restrict__ sw,
+                                                const int32_t *__restrict__ ecol, const uint16_t *__restrict__ eidx,
+                                                uint16_t zero, int16_t *fslot, int32_t *fw, int32_t *fcol,
+                                                uint16_t *fidx, unsigned long long *folded) {
+  const int64_t s = blockIdx.x, r = s * 64 + threadIdx.x, base = soff[s] + threadIdx.x;
+  const int lane = threadIdx.x;
+  const int32_t w = sw[s];
+  uint64_t used = 0;  // entries taken over (w <= 64)
+  unsigned long long n = 0;
+  for (int32_t k = moff[s]; k < moff[s + 1]; k++) {
+    int32_t f = -1;
+    if (k < umid[s]) {
+      const qh_kmeta m = meta[k];
+      const bool on = (m.mask >> lane) & 1u;
+      const int64_t c = (m.sign >> lane) & 1u ? r - (int64_t)m.ad : r + (int64_t)m.ad;
+      int32_t at = -1, id = -1;
+      if (on)
+        for (int32_t i = 0; i < w; i++) {
+          const int64_t e = base + 64 * (int64_t)i;
+          if (!((used >> i) & 1u) && eidx[e] != zero && ecol[e] == c) {
+            at = i;
+            id = eidx[e];
+            break;
+          }
+        }
+      const int32_t first = __shfl(id, __ffsll((unsigned long long)m.mask) - 1, 64);
+      if (first >= 0 && __ballot(on && id != first) == 0ull) {
+        f = first;
+        if (on) used |= 1ull << at;
+        n += __popcll(m.mask);
+      }
+    }
+    if (lane == 0) fslot[k] = (int16_t)f;
+  }
+  int32_t p = 0;
+  for (int32_t i = 0; i < w; i++) {
+    const int64_t e = base + 64 * (int64_t)i;
+    if (((used >> i) & 1u) || eidx[e] == zero) continue;
+    fcol[base + 64 * (int64_t)p] = ecol[e];
+    fidx[base + 64 * (int64_t)p] = eidx[e];
+    p++;
+  }
+  int32_t most = p;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) most = max(most, __shfl_xor(most, o, 64));
+  for (; p < most; p++) {
+    fcol[base + 64 * (int64_t)p] = (int32_t)(r < nrows ? r : 0);
+    fidx[base + 64 * (int64_t)p] = zero;
+  }
+  if (lane == 0) {
+    fw[s] = most;
+    if (n) atomicAdd(folded, n);
+  }
+}
+
+// builds the lists for variant 134 of A's sliced layout, once per cache
+static int td_fold(const qh_mat *A, qh_td_cache *c) {
+  if (c->fold_state) return QH_OK;
+  c->fold_state = -1;
+  if (!c->soff || c->dv.size() > 64 || c->max_row > 64 || A->ks_state != 1 || A->ks_maxslots > 64) return QH_OK;
+  hipStream_t s = qh_stream();
+  const size_t nsl = (size_t)A->nslices;
+  int64_t te = 0;
+  QH_HIP(hipMemcpyAsync(&te, c->soff + nsl, sizeof(te), hipMemcpyDeviceToHost, s));
+  QH_HIP(hipStreamSynchronize(s));
+  unsigned long long *n = nullptr, hn = 0;
+  int rc = qh_alloc_t(&c->fslot, (size_t)A->ks_slots + 1);
+  if (!rc) rc = qh_alloc_t(&c->fw, nsl);
+  if (!rc) rc = qh_alloc_t(&c->fcol, (size_t)te + 1);
+  if (!rc) rc = qh_alloc_t(&c->fidx, (size_t)te + 1);
+  if (!rc) rc = qh_alloc_t(&n, 1);
+  if (rc) return rc;
+  QH_HIP(hipMemsetAsync(n, 0, sizeof(*n), s));
+  hipLaunchKernelGGL(k_td_fold, dim3((unsigned)nsl), dim3(64), 0, s, A->rows, A->ks_moff, A->ks_umid, A->ks_meta,
+                     c->soff, c->sw, c->ecol, c->eidx, (uint16_t)(c->dv.size() - 1), c->fslot, c->fw, c->fcol, c->fidx,
+                     n);
+  QH_HIP(hipGetLastError());
+  QH_HIP(hipMemcpyAsync(&hn, n, sizeof(hn), hipMemcpyDeviceToHost, s));
+  QH_HIP(hipStreamSynchronize(s));
+  qh_free_ptr(n);
+  if (hn) c->fold_state = 1;
+  return QH_OK;
+}
+
+// the sliced form of the merged A_k for A's stage kernel (variant G) to sum in the
+// same pass (lanes 0: wherever A's variant has that form), or null
+static const qh_td_ell *td_fusable(const qh_td_cache *c, int G, int prec, const double2 *cf, qh_td_ell *buf) {
   if (!c->soff || g_td_lanes != 0) return nullptr;
-  *buf = qh_td_ell{c->soff, c->sw, c->ecol, c->eidx, cf};
+  if (G == 134 && prec == QH_FP64 && c->fold_state == 1)
+    *buf = qh_td_ell{c->soff, c->fw, c->fcol, c->fidx, cf, c->fslot, (int32_t)c->dv.size()};
+  else
+    *buf = qh_td_ell{c->soff, c->sw, c->ecol, c->eidx, cf, nullptr, 0};
   return buf;
 }
 
@@ -725,6 +827,7 @@ extern "C" int qh_spmv_td(const qh_mat *A, int ntd, qh_mat *const *Ak, const dou
   int G = 0;
   if (g_td_sliced) {
     rc = qh_td_sliced_prepare(Am, x->prec, &G);
+    if (!rc && G == 134 && x->prec == QH_FP64) rc = td_fold(A, c);
     if (rc) return rc;
   }
   std::vector<double2> hs((size_t)c->stride() + 1);
@@ -734,7 +837,7 @@ extern "C" int qh_spmv_td(const qh_mat *A, int ntd, qh_mat *const *Ak, const dou
     qh_td_ell tb;
     int fused = 0;
     rc = qh_td_sliced_stage(G, A, x->prec, MODE_SPMV, x->d, y->d, nullptr, 0.0, nullptr, nullptr, nullptr, nullptr,
-                            nullptr, 0.0, nullptr, td_fusable(c, c->s, &tb), &fused);
+                            nullptr, 0.0, nullptr, td_fusable(c, G, x->prec, c->s, &tb), &fused);
     if (rc || fused) return rc;
     return td_add_launch<MODE_SPMV>(c, x->prec, c->s, x->d, y->d, nullptr, 0.0, nullptr, nullptr, 0.0);
   }
@@ -757,6 +860,7 @@ extern "C" int qh_rk4_td_step(qh_mat *A, int ntd, qh_mat *const *Ak, const doubl
   int G = 0;
   if (g_td_sliced) {
     rc = qh_td_sliced_prepare(A, x->prec, &G);
+    if (!rc && G == 134 && x->prec == QH_FP64) rc = td_fold(A, c);
     if (rc) return rc;
   }
   if (c->prec != x->prec) {
@@ -792,14 +896,14 @@ extern "C" int qh_rk4_td_step(qh_mat *A, int ntd, qh_mat *const *Ak, const doubl
     for (int j = 0; j < 3 && !rc; j++) {
       const double2 *cf = c->s + (size_t)j * st;
       rc = qh_td_sliced_stage(G, A, x->prec, MODE_STAGE, ins[j], c->k[j], outs[j], cs[j], x->d, nullptr, nullptr,
-                              nullptr, nullptr, h, lo, td_fusable(c, cf, &tb), &fused);
+                              nullptr, nullptr, h, lo, td_fusable(c, G, x->prec, cf, &tb), &fused);
       if (!rc && !fused)
         rc = td_add_launch<MODE_STAGE>(c, x->prec, cf, ins[j], c->k[j], outs[j], cs[j], nullptr, nullptr, 0.0);
     }
     const double2 *cf = c->s + (size_t)3 * st;
     if (!rc)
       rc = qh_td_sliced_stage(G, A, x->prec, MODE_FINAL, c->y[0], nullptr, nullptr, 0.0, x->d, c->k[0], c->k[1],
-                              c->k[2], x->d, h, lo, td_fusable(c, cf, &tb), &fused);
+                              c->k[2], x->d, h, lo, td_fusable(c, G, x->prec, cf, &tb), &fused);
     if (!rc && !fused)
       rc = td_add_launch<MODE_FINAL>(c, x->prec, cf, c->y[0], nullptr, nullptr, 0.0, x->d, lo, h);
     return rc;
@@ -826,12 +930,16 @@ extern "C" int qh_rk3bs_td_step(qh_mat *A, int ntd, qh_mat *const *Ak, const dou
   if (rc) return rc;
   if (g_td_sliced && c->soff && g_td_lanes == 0) {
     // the four stage tables in one upload, the entries summed in A's stage kernels
+    int G = 0;
+    rc = qh_td_sliced_prepare(A, x->prec, &G);
+    if (!rc && G == 134) rc = td_fold(A, c);
+    if (rc) return rc;
     const int st = c->stride();
     std::vector<double2> hs((size_t)4 * st);
     for (int j = 0; j < 4; j++) td_table(c, ntd, s4_re_im + 2 * (size_t)j * ntd, hs.data() + (size_t)j * st);
     QH_HIP(hipMemcpyAsync(c->s, hs.data(), sizeof(double2) * 4 * st, hipMemcpyHostToDevice, qh_stream()));
     qh_td_ell t4[4];
-    for (int j = 0; j < 4; j++) t4[j] = qh_td_ell{c->soff, c->sw, c->ecol, c->eidx, c->s + (size_t)j * st};
+    for (int j = 0; j < 4; j++) td_fusable(c, G, x->prec, c->s + (size_t)j * st, &t4[j]);
     int done = 0;
     rc = qh_rk3bs_td_sliced(A, x, xn, k1, k2, k3, k4, y, h, atol, rtol, have_k1, err, t4, &done);
     if (rc || done) return rc;
