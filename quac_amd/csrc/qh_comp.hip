@@ -41,6 +41,7 @@ const int CP_DICT = 1024;       // values of a bin's table, zero among them
 // state) and the table in 160 KB of LDS, 6 or 8 rows a thread
 const int CP_MAX_ROWS64 = 4800, CP_MAX_ROWS32 = 8128;
 const int CP_DICT_W = 12;       // words of a row fetched ahead
+const size_t CP_SCRATCH = (size_t)64 << 20;  // workspace taken from the library's scratch
 const int CP_PROBE_ROWS = 16384;  // rows looked at before a large matrix as a whole
 const int CP_PACK_ROWS = 512;   // bins of small components are filled to this size once they outnumber the CUs
 
@@ -101,21 +102,33 @@ __global__ void __launch_bounds__(256) k_cc_hook(int32_t *parent, const int32_t 
   }
 }
 
-// the root of every row, and the rows of every root
+// The root of every row, and the rows of every root.  A block counts its 1024 rows by
+// root in an LDS table first: a few large components would otherwise queue a global
+// atomic per row (0.25 ms for 230 400 rows in 67 of them).
+const int CC_LABEL_ROWS = 1024;
 __global__ void __launch_bounds__(256) k_cc_label(int32_t *parent, int32_t *lab, int32_t *size, int32_t n) {
-  const int64_t r = blockIdx.x * (int64_t)256 + threadIdx.x;
-  const bool on = r < n;
-  const int32_t l = on ? cc_find(parent, (int32_t)r) : -1;
-  if (on) lab[r] = l;
-  // lanes that share the first lane's root count together (one component is the common large case)
-  const int32_t f = __builtin_amdgcn_readfirstlane(l);
-  const uint64_t m = __ballot(on && l == f);
-  if (!on) return;
-  if (l == f) {
-    if ((threadIdx.x & 63) == 0) atomicAdd(size + f, (int32_t)__popcll(m));
-  } else {
-    atomicAdd(size + l, 1);
+  __shared__ int32_t key[2 * CC_LABEL_ROWS], cnt[2 * CC_LABEL_ROWS];
+  for (int i = threadIdx.x; i < 2 * CC_LABEL_ROWS; i += 256) {
+    key[i] = -1;
+    cnt[i] = 0;
   }
+  __syncthreads();
+  for (int k = 0; k < CC_LABEL_ROWS; k += 256) {
+    const int64_t r = (int64_t)blockIdx.x * CC_LABEL_ROWS + k + threadIdx.x;
+    if (r >= n) break;
+    const int32_t l = cc_find(parent, (int32_t)r);
+    lab[r] = l;
+    unsigned h = ((unsigned)l * 2654435761u) >> 21;  // 11 bits: the table's size, half of it used at most
+    for (;;) {
+      const int32_t old = atomicCAS(&key[h], -1, l);
+      if (old == -1 || old == l) break;
+      h = (h + 1) & (2 * CC_LABEL_ROWS - 1);
+    }
+    atomicAdd(&cnt[h], 1);
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < 2 * CC_LABEL_ROWS; i += 256)
+    if (cnt[i]) atomicAdd(size + key[i], cnt[i]);
 }
 
 __global__ void k_cc_largest(const int32_t *size, int32_t *out, int32_t n) {
@@ -161,6 +174,34 @@ __device__ inline int32_t cp_wave_max(int32_t v) {
   return v;
 }
 
+// f(column, value) of row r's entries off the diagonal, the loads of four entries in
+// flight together; the diagonal entry (zero where there is none) is returned
+template <typename F>
+__device__ __forceinline__ double2 cp_entries(int32_t r, const int32_t *__restrict__ rp,
+                                              const int32_t *__restrict__ col, const double2 *__restrict__ val, F &&f) {
+  double2 d = make_double2(0.0, 0.0);
+  const int32_t end = rp[r + 1];
+  for (int32_t e = rp[r]; e < end; e += 4) {
+    int32_t c[4];
+    double2 v[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const int32_t q = min(e + k, end - 1);
+      c[k] = col[q];
+      v[k] = val[q];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      if (e + k >= end) break;
+      if (c[k] == r)
+        d = v[k];
+      else
+        f(c[k], v[k]);
+    }
+  }
+  return d;
+}
+
 // slots of every slice: imaginary parts (made even) and all (count: the slices'
 // number where only the device has it)
 __global__ void __launch_bounds__(256) k_cp_width(const int32_t *order, const int32_t *__restrict__ rp,
@@ -172,12 +213,10 @@ __global__ void __launch_bounds__(256) k_cp_width(const int32_t *order, const in
   const int32_t r = order[(int64_t)s * 64 + lane];
   int32_t ni = 0, nr = 0;
   if (r >= 0)
-    for (int32_t e = rp[r]; e < rp[r + 1]; e++) {
-      if (col[e] == r) continue;
-      const double2 v = val[e];
+    cp_entries(r, rp, col, val, [&](int32_t, double2 v) {
       ni += v.y != 0.0;
       nr += v.x != 0.0;
-    }
+    });
   ni = (cp_wave_max(ni) + 1) & ~1;
   nr = cp_wave_max(nr);
   if (lane == 0) {
@@ -206,17 +245,12 @@ __global__ void __launch_bounds__(256) k_cp_fill(const int32_t *order, const int
     ec[slot * 64 + lane] = (uint16_t)c;
   };
   if (r >= 0)
-    for (int32_t e = rp[r]; e < rp[r + 1]; e++) {
-      const double2 v = val[e];
-      if (col[e] == r) {
-        d = v;
-        continue;
-      }
-      if (!reg) continue;
-      const int32_t c = pos[col[e]];
+    d = cp_entries(r, rp, col, val, [&](int32_t q, double2 v) {
+      if (!reg) return;
+      const int32_t c = pos[q];
       if (v.y != 0.0) put(pi++, v.y, c);
       if (v.x != 0.0) put(pr++, v.x, c);
-    }
+    });
   diag[(int64_t)s * 64 + lane] = d;
   if (!reg) return;
   for (; pi < s0 + nim[s]; pi++) put(pi, 0.0, zc[s]);
@@ -260,12 +294,10 @@ __global__ void __launch_bounds__(1024) k_cp_dict(const int32_t *bins, const int
   for (int32_t s = wave; s < nsl; s += 16) {
     const int32_t r = order[(int64_t)(sl0 + s) * 64 + lane];
     if (r < 0 || *(volatile int32_t *)&count >= CP_DICT) continue;
-    for (int32_t e = rp[r]; e < rp[r + 1]; e++) {
-      if (col[e] == r) continue;
-      const double2 v = val[e];
+    cp_entries(r, rp, col, val, [&](int32_t, double2 v) {
       if (v.y != 0.0) cell(v.y, true);
       if (v.x != 0.0) cell(v.x, true);
-    }
+    });
   }
   __syncthreads();
   const bool over = count >= CP_DICT;
@@ -292,12 +324,10 @@ __global__ void __launch_bounds__(1024) k_cp_dict(const int32_t *bins, const int
       ew[slot * 64 + lane] = (uint32_t)(pos[c] + 1) | ((uint32_t)id[cell(v, false)] * 8u) << 16;
     };
     if (r >= 0)
-      for (int32_t e = rp[r]; e < rp[r + 1]; e++) {
-        if (col[e] == r) continue;
-        const double2 v = val[e];
-        if (v.y != 0.0) put(pi++, v.y, col[e]);
-        if (v.x != 0.0) put(pr++, v.x, col[e]);
-      }
+      cp_entries(r, rp, col, val, [&](int32_t c, double2 v) {
+        if (v.y != 0.0) put(pi++, v.y, c);
+        if (v.x != 0.0) put(pr++, v.x, c);
+      });
     for (; pi < p1; pi++) ew[pi * 64 + lane] = 0u;
     for (; pr < s1; pr++) ew[pr * 64 + lane] = 0u;
   }
@@ -825,6 +855,13 @@ int cp_threads(int rows) {
 // two rows a thread: up to 12 slots each fit the 128 registers
 bool cp_fits_registers(int rows, int W) { return W && (rows <= 1024 || (rows <= CP_REG_ROWS && W <= 12)); }
 
+// clocks of a stage of a bin of so many rows at the least: as many slots as the
+// matrix has entries off the diagonal a row on average
+double cp_least(int64_t rows, const qh_mat *A) {
+  const double w = std::max(0.0, (double)A->nnz / (double)A->rows - 1.0);
+  return (rows <= CP_REG_ROWS ? CP_CLK_REG : CP_CLK_WORD) * w * (double)rows / 64.0 + CP_CLK_FIXED;
+}
+
 // The plan of a matrix of at most CP_SMALL_ROWS rows with one shape for all bins
 // (*done = 0 where it needs the general builder)
 int cp_build_small(qh_mat *A, int f32, int *done) {
@@ -883,8 +920,12 @@ int cp_build_small(qh_mat *A, int f32, int *done) {
   CP_HIP(hipStreamSynchronize(s));
   const int nb = h[CPS_BINS], nsl = h[CPS_SLICES], rows = h[CPS_ROWS], W = cp_width_class(h[CPS_WIDTH], true);
   const int64_t slots = h[CPS_SLOTS];
-  if (!cp_fits_registers(rows, W)) return fail(QH_OK);
+  if (!cp_fits_registers(rows, W) && cp_worth(cp_least(rows, A), 0.0, n)) return fail(QH_OK);
   *done = 1;
+  if (!cp_fits_registers(rows, W)) {
+    A->comp_state[f32] = -1;
+    return fail(QH_OK);
+  }
   if (!cp_worth(CP_CLK_REG * W * (rows / 64) + CP_CLK_FIXED, CP_CLK_REG * W * nsl, n)) {
     A->comp_state[f32] = -1;
     return fail(QH_OK);
@@ -953,15 +994,18 @@ int cp_build(qh_mat *A, int f32) {
   };
   Carve meas, work;
   layout(meas);
-  void *wbuf = nullptr;
-  int rc = qh_alloc(&wbuf, meas.n);
+  // (an allocation of some MB and its release take up to a millisecond: the library's
+  // scratch, kept, up to CP_SCRATCH bytes)
+  void *wbuf = nullptr, *own = nullptr;
+  int rc = meas.n <= CP_SCRATCH ? qh_scratch(meas.n, &wbuf, 0, nullptr) : qh_alloc(&own, meas.n);
   if (rc) return rc;
+  if (own) wbuf = own;
   work.p = (char *)wbuf;
   layout(work);
   qh_comp *c = new qh_comp();
   auto fail = [&](int code) {
     (void)hipStreamSynchronize(s);
-    qh_free_ptr(wbuf);
+    qh_free_ptr(own);
     qh_comp_free(c);
     return code;
   };
@@ -989,12 +1033,12 @@ int cp_build(qh_mat *A, int f32) {
     int32_t most = 0;
     hipLaunchKernelGGL(k_cc_init, dim3(std::min(nbp, 4096u)), dim3(256), 0, s, parent, size, m);
     hipLaunchKernelGGL(k_cc_hook, dim3(nbp), dim3(256), 0, s, parent, A->rowptr, A->col, r0, m);
-    hipLaunchKernelGGL(k_cc_label, dim3(nbp), dim3(256), 0, s, parent, lab, size, m);
+    hipLaunchKernelGGL(k_cc_label, dim3(qh_blocks(m, CC_LABEL_ROWS)), dim3(256), 0, s, parent, lab, size, m);
     CP_HIP(hipMemsetAsync(off, 0, sizeof(int32_t), s));
     hipLaunchKernelGGL(k_cc_largest, dim3(std::min(nbp, 256u)), dim3(256), 0, s, size, off, m);
     CP_HIP(hipMemcpyAsync(&most, off, sizeof(int32_t), hipMemcpyDeviceToHost, s));
     CP_HIP(hipStreamSynchronize(s));
-    if (most > max_rows) {
+    if (most > max_rows || !cp_worth(cp_least(most, A), 0.0, n)) {
       fail(0);
       state = -1;
       return QH_OK;
@@ -1004,7 +1048,7 @@ int cp_build(qh_mat *A, int f32) {
   CP_HIP(hipMemsetAsync(gsize, 0, sizeof(int32_t) * ngran, s));
   hipLaunchKernelGGL(k_cc_init, dim3(std::min(nb256, 4096u)), dim3(256), 0, s, parent, size, n);
   hipLaunchKernelGGL(k_cc_hook, dim3(nb256), dim3(256), 0, s, parent, A->rowptr, A->col, 0, n);
-  hipLaunchKernelGGL(k_cc_label, dim3(nb256), dim3(256), 0, s, parent, lab, size, n);
+  hipLaunchKernelGGL(k_cc_label, dim3(qh_blocks(n, CC_LABEL_ROWS)), dim3(256), 0, s, parent, lab, size, n);
   size_t tb = std::max(scan_b, sort_b);
   CP_HIP(hipcub::DeviceScan::ExclusiveSum(tmp, tb, size, off, n, s));
   hipLaunchKernelGGL(k_cc_granules, dim3(nb256), dim3(256), 0, s, size, off, gsize, n);
@@ -1033,7 +1077,7 @@ int cp_build(qh_mat *A, int f32) {
     cur += hg[g];
   }
   close();
-  if (largest > max_rows) {
+  if (largest > max_rows || !cp_worth(cp_least(largest, A), 0.0, n)) {
     fail(0);
     state = -1;
     return QH_OK;
@@ -1193,7 +1237,7 @@ int cp_build(qh_mat *A, int f32) {
     return QH_OK;
   }
 #undef CP_HIP
-  qh_free_ptr(wbuf);
+  qh_free_ptr(own);
   c->a.bslice = bslice;
   c->a.bins = bins;
   c->a.soff = soff;
