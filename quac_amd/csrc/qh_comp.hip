@@ -80,24 +80,32 @@ __global__ void __launch_bounds__(256) k_cc_hook(int32_t *parent, const int32_t 
   const int64_t r = blockIdx.x * (int64_t)256 + threadIdx.x;
   if (r >= n) return;
   int32_t a = (int32_t)r;
-  for (int32_t e = rp[r0 + r]; e < rp[r0 + r + 1]; e++) {
-    int32_t b = col[e] - r0;
-    if (b == (int32_t)r || b < 0 || b >= n) continue;
-    b = cc_load(parent, b);
-    if (b == a) continue;
-    for (;;) {  // the larger root below the smaller one; the larger index decreases every round
-      a = cc_find(parent, a);
-      b = cc_find(parent, b);
-      if (a == b) break;
-      const int32_t hi = a > b ? a : b, lo = a > b ? b : a;
-      const int32_t old = atomicCAS(parent + hi, hi, lo);
-      if (old == hi) {
+  const int32_t end = rp[r0 + r + 1];
+  for (int32_t e = rp[r0 + r]; e < end; e += 4) {
+    int32_t c[4];  // four entries' columns and their parents in flight together
+#pragma unroll
+    for (int k = 0; k < 4; k++) c[k] = e + k < end ? col[e + k] - r0 : (int32_t)r;
+#pragma unroll
+    for (int k = 0; k < 4; k++) c[k] = c[k] < 0 || c[k] >= n ? (int32_t)r : c[k];
+#pragma unroll
+    for (int k = 0; k < 4; k++) c[k] = c[k] == (int32_t)r ? a : cc_load(parent, c[k]);
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      int32_t b = c[k];
+      while (b != a) {  // the larger root below the smaller one; the larger index decreases every round
+        a = cc_find(parent, a);
+        b = cc_find(parent, b);
+        if (a == b) break;
+        const int32_t hi = a > b ? a : b, lo = a > b ? b : a;
+        const int32_t old = atomicCAS(parent + hi, hi, lo);
+        if (old == hi) {
+          a = lo;
+          break;
+        }
+        cc_store(parent, hi, old);  // what this die's cache still held as a root
         a = lo;
-        break;
+        b = old;
       }
-      cc_store(parent, hi, old);  // what this die's cache still held as a root
-      a = lo;
-      b = old;
     }
   }
 }
