@@ -31,15 +31,11 @@
 #include <hipcub/hipcub.hpp>
 
 #include "qh_common.h"
+#include "qh_comp_plan.h"
 
 namespace {
 
 const int CP_GRAN = 64;         // rows of a granule: the components that start in 64 consecutive sorted rows
-const int CP_REG_ROWS = 2048;   // largest bin with its entries in registers (1024 threads, two rows each)
-const int CP_DICT = 1024;       // values of a bin's table, zero among them
-// largest bin: two buffers of rows + 1 entries (complex128, or complex64 for an FP32
-// state) and the table in 160 KB of LDS, 6 or 8 rows a thread
-const int CP_MAX_ROWS64 = 4800, CP_MAX_ROWS32 = 8128;
 const int CP_DICT_W = 12;       // words of a row fetched ahead
 const size_t CP_SCRATCH = (size_t)64 << 20;  // workspace taken from the library's scratch
 const int CP_PROBE_ROWS = 16384;  // rows looked at before a large matrix as a whole
@@ -778,14 +774,6 @@ __global__ void __launch_bounds__(1024) k_comp_dict(CpArgs a) {
   }
 }
 
-// one launch: bins of one shape
-struct CpClass {
-  int threads, S, W;  // W 0: entries read as words
-  bool skip, side;    // side: few blocks, launched beside the others
-  int first, count;   // range of the plan's bin list
-  int cells;
-};
-
 int cp_launch(void (*kernel)(CpArgs), const CpClass &c, const CpArgs &a, size_t lds, hipStream_t s) {
   if (lds > 64 * 1024)
     QH_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -833,42 +821,9 @@ struct Carve {
   }
 };
 
-// time of a stage in clocks of a CU: a slot of a slice is 64 LDS reads of 16 B (8
-// clocks at 128 B a clock, 10 measured), as words 64 reads of the vector and of the
-// table
-const double CP_CLK_REG = 10.0, CP_CLK_WORD = 24.0, CP_CLK_FIXED = 500.0;
-
-// Whether a stage of the plan (the largest bin's clocks, and all bins') beats the
-// sliced stage kernels: 2.5 us a launch, and 11 us a million rows.
-// Measured us a stage, here / there: Jaynes-Cummings 2 x 24 0.30 / 2.6, Tavis-Cummings
-// 2^2 x 23 0.44 / 2.7, 2^3 x 17 1.00 / 3.5, 2^3 x 30 1.49 / 4.3, decay and dephasing of
-// 7 qubits 0.34 / 2.8, 10 5.1 / 13.2, 12 46.7 / 243.  Refused: 2^4 x 8 (bins of 1768
-// rows whose entries do not fit the registers) 5.0 / 3.3, 2^4 x 19 10.5 / 5.4, 6-qubit
-// chain (one bin of 4096 rows) 10.9 / 3.0.
-bool cp_worth(double most, double all, int64_t n) {
-  const double comp_us = std::max(most, all / (double)qh_num_cus() + CP_CLK_FIXED) / 2400.0;
-  return comp_us <= 0.9 * (2.5 + 1.1e-5 * (double)n);
-}
-
-int cp_width_class(int w, bool few) {
-  for (int u : {4, 8, 10, 12, 16, 24, 32})
-    if (w <= u && (few || u != 10)) return u;
-  return 0;
-}
-
-int cp_threads(int rows) {
-  return rows <= 64 ? 64 : rows <= 128 ? 128 : rows <= 256 ? 256 : rows <= 512 ? 512 : 1024;
-}
-
-// two rows a thread: up to 12 slots each fit the 128 registers
-bool cp_fits_registers(int rows, int W) { return W && (rows <= 1024 || (rows <= CP_REG_ROWS && W <= 12)); }
-
-// clocks of a stage of a bin of so many rows at the least: as many slots as the
-// matrix has entries off the diagonal a row on average
-double cp_least(int64_t rows, const qh_mat *A) {
-  const double w = std::max(0.0, (double)A->nnz / (double)A->rows - 1.0);
-  return (rows <= CP_REG_ROWS ? CP_CLK_REG : CP_CLK_WORD) * w * (double)rows / 64.0 + CP_CLK_FIXED;
-}
+// the rules of qh_comp_plan.h on this device and matrix
+bool cp_worth(double most, double all, int64_t n) { return ::cp_worth(most, all, n, qh_num_cus()); }
+double cp_least(int64_t rows, const qh_mat *A) { return ::cp_least(rows, (double)A->nnz / (double)A->rows - 1.0); }
 
 // The plan of a matrix of at most CP_SMALL_ROWS rows with one shape for all bins
 // (*done = 0 where it needs the general builder)
@@ -926,7 +881,7 @@ int cp_build_small(qh_mat *A, int f32, int *done) {
   CP_HIP(hipGetLastError());
   CP_HIP(hipMemcpyAsync(h, info, CPS_N * sizeof(int32_t), hipMemcpyDeviceToHost, s));
   CP_HIP(hipStreamSynchronize(s));
-  const int nb = h[CPS_BINS], nsl = h[CPS_SLICES], rows = h[CPS_ROWS], W = cp_width_class(h[CPS_WIDTH], true);
+  const int nb = h[CPS_BINS], nsl = h[CPS_SLICES], rows = h[CPS_ROWS], W = cp_width_class(h[CPS_WIDTH], false);
   const int64_t slots = h[CPS_SLOTS];
   if (!cp_fits_registers(rows, W) && cp_worth(cp_least(rows, A), 0.0, n)) return fail(QH_OK);
   *done = 1;
@@ -1132,84 +1087,39 @@ int cp_build(qh_mat *A, int f32) {
   CP_HIP(hipMemcpyAsync(hwid.data(), width, sizeof(int32_t) * nsl, hipMemcpyDeviceToHost, s));
   CP_HIP(hipStreamSynchronize(s));
   // the shape of every bin's launch, and what the largest bin and all of them take
-  const bool few = nbins <= 2 * cus;  // the chip is not full: one launch, so that nothing waits for a launch before it
-  int64_t slots[2] = {0, 0};  // held in registers, read as words
-  struct Shape {
-    int words, rows, W;
-    int32_t bin;
-  };
-  std::vector<Shape> sh(nbins);
-  double most = 0.0, all = 0.0;
-  int few_rows = 0, few_w = 0;
+  std::vector<CpBin> hbn(nbins);
   for (int32_t b = 0; b < nbins; b++) {
-    int w = 0;
-    int64_t sum = 0;
+    hbn[b] = CpBin{(hslice[b + 1] - hslice[b]) * 64, 0, 0};
     for (int32_t i = hslice[b]; i < hslice[b + 1]; i++) {
-      w = std::max(w, (int)hwid[i]);
-      sum += hwid[i];
+      hbn[b].width = std::max(hbn[b].width, (int)hwid[i]);
+      hbn[b].slots += hwid[i];
     }
-    const int rows = (hslice[b + 1] - hslice[b]) * 64;
-    const int W = cp_width_class(w, few);
-    const bool reg = cp_fits_registers(rows, W);
-    sh[b] = Shape{!reg, rows <= 1024 ? cp_threads(rows) : rows, W, b};
-    if (reg) {
-      few_rows = std::max(few_rows, sh[b].rows);
-      few_w = std::max(few_w, W);
-    }
-    for (int32_t i = hslice[b]; i < hslice[b + 1]; i++) {
-      hoff[i] = (int32_t)slots[!reg];
-      slots[!reg] += hwid[i];
-      hzc[i] = reg ? rows : -1;
-    }
-    if (std::max(slots[0], slots[1]) > (int64_t)0x7fffffff) {
-      fail(0);
-      state = -1;
-      return QH_OK;
-    }
-    const double clk = reg ? CP_CLK_REG * W * (rows / 64) : CP_CLK_WORD * (double)sum;
-    most = std::max(most, clk + CP_CLK_FIXED);
-    all += clk;
   }
-  if (!cp_worth(most, all, n)) {
+  const CpShapes sh = cp_shapes(hbn, f32, (int)cus);
+  int64_t slots[2] = {0, 0};  // held in registers, read as words
+  for (int32_t b = 0; b < nbins; b++)
+    for (int32_t i = hslice[b]; i < hslice[b + 1]; i++) {
+      hoff[i] = (int32_t)slots[sh.words[b]];
+      slots[sh.words[b]] += hwid[i];
+      hzc[i] = sh.words[b] ? -1 : hbn[b].rows;
+      if (slots[sh.words[b]] > (int64_t)0x7fffffff) {
+        fail(0);
+        state = -1;
+        return QH_OK;
+      }
+    }
+  if (!sh.runnable || !cp_worth(sh.most, sh.all, n)) {
     fail(0);
     state = -1;
     return QH_OK;
   }
-  const bool merge = few && !(few_rows > 1024 && few_w > 12);
-  if (merge)
-    for (auto &q : sh)
-      if (!q.words) {
-        q.rows = few_rows;
-        q.W = few_w;
-      }
-  std::stable_sort(sh.begin(), sh.end(), [](const Shape &p, const Shape &q) {
-    if (p.words != q.words) return p.words > q.words;
-    const int pr = p.words || p.rows > 1024 ? 1 << 20 : p.rows, qr = q.words || q.rows > 1024 ? 1 << 20 : q.rows;
-    if (pr != qr) return pr > qr;
-    return !p.words && p.W > q.W;
-  });
-  std::vector<int32_t> hbins(nbins);
-  for (int32_t i = 0; i < nbins; i++) {
-    const Shape &q = sh[i];
-    hbins[i] = q.bin;
-    const int S = q.words ? (f32 ? 8 : 6) : q.rows > 1024 ? 2 : 1, threads = q.words || S == 2 ? 1024 : q.rows;
-    const int W = q.words ? 0 : q.W;
-    if (c->classes.empty() || c->classes.back().threads != threads || c->classes.back().S != S ||
-        c->classes.back().W != W)
-      c->classes.push_back(CpClass{threads, S, W, !merge, false, i, 0, 0});
-    CpClass &k = c->classes.back();
-    k.count++;
-    k.cells = std::max(k.cells, (hslice[q.bin + 1] - hslice[q.bin]) * 64 + 1);
-  }
-  for (CpClass &k : c->classes)
-    if (c->classes.size() > 1 && k.count < cus && k.first + k.count < nbins) {
-      k.side = true;
-      if (!c->side) {
-        CP_HIP(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
-        for (hipEvent_t &e : c->ev) CP_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-      }
+  c->classes = sh.classes;
+  for (const CpClass &k : c->classes)
+    if (k.side && !c->side) {
+      CP_HIP(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
+      for (hipEvent_t &e : c->ev) CP_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     }
-  const int ndict = sh[0].words ? (c->classes[0].count) : 0;  // these bins come first
+  const int ndict = c->classes[0].W == 0 ? c->classes[0].count : 0;  // these bins come first
   double *ev, *dict;
   uint16_t *ec;
   uint32_t *ew;
@@ -1227,7 +1137,7 @@ int cp_build(qh_mat *A, int f32) {
   entries(ep);
   CP_HIP(hipMemcpyAsync(zc, hzc.data(), sizeof(int32_t) * nsl, hipMemcpyHostToDevice, s));
   CP_HIP(hipMemcpyAsync(soff, hoff.data(), sizeof(int32_t) * nsl, hipMemcpyHostToDevice, s));
-  CP_HIP(hipMemcpyAsync(bins, hbins.data(), sizeof(int32_t) * nbins, hipMemcpyHostToDevice, s));
+  CP_HIP(hipMemcpyAsync(bins, sh.bins.data(), sizeof(int32_t) * nbins, hipMemcpyHostToDevice, s));
   hipLaunchKernelGGL(k_cp_fill, dim3(qh_blocks(nsl, 4)), dim3(256), 0, s, order, pos, A->rowptr, A->col, A->val,
                      soff, width, nim, zc, diag, ev, ec, nsl);
   int32_t hover = 0;
@@ -1309,26 +1219,7 @@ int qh_comp_rk4(qh_mat *A, qh_vec *x, double dt, int64_t nsteps) {
 #define CP_CASE(SS, WW, SK)                   \
   if (k.S == SS && k.W == WW && k.skip == SK) \
     rc = cp_launch(k_comp_rk4<SS, WW, SK>, k, a, (size_t)2 * k.cells * sizeof(double2), ks);
-    CP_CASE(1, 4, false)
-    CP_CASE(1, 8, false)
-    CP_CASE(1, 10, false)
-    CP_CASE(1, 12, false)
-    CP_CASE(1, 16, false)
-    CP_CASE(1, 24, false)
-    CP_CASE(1, 32, false)
-    CP_CASE(2, 4, false)
-    CP_CASE(2, 8, false)
-    CP_CASE(2, 10, false)
-    CP_CASE(2, 12, false)
-    CP_CASE(1, 4, true)
-    CP_CASE(1, 8, true)
-    CP_CASE(1, 12, true)
-    CP_CASE(1, 16, true)
-    CP_CASE(1, 24, true)
-    CP_CASE(1, 32, true)
-    CP_CASE(2, 4, true)
-    CP_CASE(2, 8, true)
-    CP_CASE(2, 12, true)
+    CP_REG_KERNELS(CP_CASE)
 #undef CP_CASE
     if (rc) return rc;
   }

@@ -1,0 +1,92 @@
+"""The host-side choices of a closed-set plan (quac_amd/csrc/qh_comp_plan.h), compiled
+with the host compiler: every launch that a plan can hold has a kernel whose thread
+count, rows a thread, slots and LDS take every bin of the launch, and every bin is in
+one launch."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CSRC = os.path.join(os.path.dirname(HERE), "quac_amd", "csrc")
+
+pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="needs a host C++ compiler")
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    """run(name, body): body's output, compiled behind the header with a main()"""
+    d = tmp_path_factory.mktemp("plan")
+
+    def _run(name, body):
+        src, exe = str(d / (name + ".cpp")), str(d / name)
+        with open(src, "w") as f:
+            f.write('#include <cstdio>\n#include <cstdlib>\n#include <random>\n#include "qh_comp_plan.h"\n' + body)
+        subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-fsanitize=address,undefined", "-I", CSRC, src,
+                        "-o", exe], check=True)
+        return subprocess.run([exe], check=True, capture_output=True, text=True).stdout
+
+    return _run
+
+
+CHECK = r"""
+#define NEED(x) do { if (!(x)) { printf("line %d: %s\n", __LINE__, #x); exit(1); } } while (0)
+static const int CUS = 256;
+static void check(const std::vector<CpBin> &bin, bool f32) {
+  const CpShapes s = cp_shapes(bin, f32, CUS);
+  NEED(s.runnable);
+  std::vector<int> seen(bin.size());
+  int at = 0;
+  for (const CpClass &k : s.classes) {
+    NEED(k.first == at && k.count > 0 && cp_has_kernel(k));
+    NEED(k.threads <= 1024 && k.threads % 64 == 0);
+    // two buffers of k.cells entries, and the table beside words
+    const size_t cell = k.W == 0 && f32 ? 8 : 16;
+    NEED(2 * cell * k.cells + (k.W == 0 ? 8 * CP_DICT : 0) <= 160 * 1024);
+    for (int i = 0; i < k.count; i++) {
+      const CpBin &b = bin[s.bins[at + i]];
+      seen[s.bins[at + i]]++;
+      NEED(s.words[s.bins[at + i]] == (k.W == 0));
+      NEED(b.rows <= k.threads * k.S && b.rows + 1 <= k.cells);
+      if (k.W) NEED(b.width <= k.W);
+    }
+    at += k.count;
+  }
+  NEED(at == (int)bin.size());
+  for (int n : seen) NEED(n == 1);
+  NEED(!s.classes.back().side);
+}
+"""
+
+
+def test_every_launch_has_a_kernel(run):
+    out = run("shapes", CHECK + r"""
+int main() {
+  // every pair of bins: up to one slice, up to one and two rows a thread, and words,
+  // beside every width of a slice
+  const int rows[] = {64, 128, 192, 512, 576, 1024, 1088, 2048, 2112, 4800};
+  const int widths[] = {0, 4, 5, 8, 9, 10, 11, 12, 13, 16, 24, 32, 33};
+  for (int few = 0; few < 2; few++)
+    for (int r1 : rows)
+      for (int r2 : rows)
+        for (int w1 : widths)
+          for (int w2 : widths) {
+            std::vector<CpBin> bin{{r1, w1, (int64_t)w1 * r1 / 64}, {r2, w2, (int64_t)w2 * r2 / 64}};
+            if (!few) bin.resize(2 * CUS + 1, bin[0]);
+            check(bin, (w1 + w2) & 1);
+          }
+  std::mt19937 rng(7);
+  for (int t = 0; t < 1000; t++) {
+    std::vector<CpBin> bin(1 + rng() % (t % 8 ? 24 : 900));
+    for (CpBin &b : bin) {
+      b.rows = 64 * (1 + rng() % (rng() % 4 ? 16 : 75));
+      b.width = rng() % (rng() % 3 ? 14 : 40);
+      b.slots = (int64_t)b.width * (b.rows / 64);
+    }
+    check(bin, t & 1);
+  }
+  printf("ok\n");
+}
+""")
+    assert out == "ok\n"

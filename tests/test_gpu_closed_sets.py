@@ -158,3 +158,32 @@ def test_batch_of_uneven_blocks():
     b.destroy()
     for s in systems:
         s.destroy()
+
+
+@pytest.mark.parametrize("prec", [qa.FP64, qa.FP32])
+@pytest.mark.parametrize("sizes", [[(3, 17), (4, 5)], [(3, 20), (4, 6), (2, 10)]])
+def test_batch_of_shapes_with_no_common_kernel(sizes, prec):
+    """three emitters of 17 or more levels (bins of more than 1024 rows and 10 slots)
+    beside four emitters (up to 16 slots): a launch for every shape, and in the second
+    batch bins that read their entries as words"""
+    dt, steps = 0.01, 4
+    systems = [build_system(_tc(*s))[0] for s in sizes]
+    tots = [2 ** q * n for q, n in sizes]
+    b = qa.Batch([s.matrix() for s in systems], tots, prec=prec)
+    starts = [_start(t) for t in tots]
+    for i, x0 in enumerate(starts):
+        b.set_state(i, x0)
+    b.rk4(dt, 1)
+    b.rk4(dt, steps - 1)
+    for i, (s, x0) in enumerate(zip(sizes, starts)):
+        tot, terms = recipes.oracle_terms(_tc(*s))
+        m = oracle.construct(tot, terms, dm=True)
+        rp, _, val = systems[i].matrix().export()
+        norm = np.add.reduceat(np.abs(val), rp[:-1]).max()
+        # per step: a few roundings of the state and of h A times it; FP32 words: h |A| of
+        # a state rounded to 32 bits, and the two words' rounding
+        eps = (2 * dt * norm + 8) * 2.0 ** -53 if prec == qa.FP64 else 2 * dt * norm * 2.0 ** -24 + 8 * 2.0 ** -48
+        assert np.abs(b.get_state(i) - m.rk4(x0, dt, steps)).max() <= steps * np.abs(x0).max() * eps
+    b.destroy()
+    for s in systems:
+        s.destroy()
