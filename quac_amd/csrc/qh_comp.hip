@@ -1196,11 +1196,17 @@ int qh_comp_rk4(qh_mat *A, qh_vec *x, double dt, int64_t nsteps) {
   const int f32 = x->prec == QH_FP32;
   const qh_comp &c = *A->comp[f32];
   hipStream_t s = qh_stream();
-  if (c.side) {
+  auto fork = [&]() -> int {
     QH_HIP(hipEventRecord(c.ev[0], s));
     QH_HIP(hipStreamWaitEvent(c.side, c.ev[0], 0));
-  }
-  for (const CpClass &k : c.classes) {
+    return QH_OK;
+  };
+  auto join = [&]() -> int {
+    if (hipEventRecord(c.ev[1], c.side) == hipSuccess && hipStreamWaitEvent(s, c.ev[1], 0) == hipSuccess) return QH_OK;
+    QH_HIP(hipStreamSynchronize(c.side));
+    return QH_OK;
+  };
+  auto launch = [&](const CpClass &k) -> int {
     CpArgs a = c.a;
     a.bins += k.first;
     a.x = x->d;
@@ -1221,13 +1227,9 @@ int qh_comp_rk4(qh_mat *A, qh_vec *x, double dt, int64_t nsteps) {
     rc = cp_launch(k_comp_rk4<SS, WW, SK>, k, a, (size_t)2 * k.cells * sizeof(double2), ks);
     CP_REG_KERNELS(CP_CASE)
 #undef CP_CASE
-    if (rc) return rc;
-  }
-  if (c.side) {
-    QH_HIP(hipEventRecord(c.ev[1], c.side));
-    QH_HIP(hipStreamWaitEvent(s, c.ev[1], 0));
-  }
-  return QH_OK;
+    return rc;
+  };
+  return cp_run(c.classes, launch, fork, join);
 }
 
 double *qh_comp_trace(const qh_mat *A, int prec) { return A->comp[prec == QH_FP32]->trace; }

@@ -149,4 +149,19 @@ inline CpShapes cp_shapes(const std::vector<CpBin> &bin, bool f32, int cus) {
   return out;
 }
 
+// All launches of a plan: fork() before the first where some run on the side stream,
+// launch(class) each, and join() after them, also when a launch fails: the caller's
+// stream never goes on while the side stream still writes the state.
+template <typename Launch, typename Fork, typename Join>
+int cp_run(const std::vector<CpClass> &classes, Launch &&launch, Fork &&fork, Join &&join) {
+  bool side = false;
+  int rc = 0;
+  for (const CpClass &k : classes) side = side || k.side;
+  if (side && (rc = fork())) return rc;
+  for (const CpClass &k : classes)
+    if ((rc = launch(k))) break;
+  const int jrc = side ? join() : 0;
+  return rc ? rc : jrc;
+}
+
 #endif

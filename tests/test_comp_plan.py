@@ -90,3 +90,32 @@ int main() {
 }
 """)
     assert out == "ok\n"
+
+
+def test_side_stream_is_joined_when_a_launch_fails(run):
+    """the order of fork, launches and join for every launch that may fail"""
+    out = run("order", CHECK + r"""
+int main() {
+  for (int sides = 0; sides < 2; sides++)
+    for (int bad = -1; bad < 4; bad++) {
+      std::vector<CpClass> c(4, CpClass{64, 1, 4, true, false, 0, 1, 65});
+      c[0].side = c[2].side = sides;
+      int forks = 0, joins = 0, launched = 0;
+      const int rc = cp_run(
+          c,
+          [&](const CpClass &k) {
+            NEED(!k.side || (forks == 1 && joins == 0));
+            return launched++ == bad ? -7 : 0;
+          },
+          [&] { return forks++, 0; }, [&] { return joins++, 0; });
+      NEED(rc == (bad < 0 ? 0 : -7) && launched == (bad < 0 ? 4 : bad + 1));
+      NEED(forks == sides && joins == sides);
+      NEED(cp_run(c, [](const CpClass &) { return 0; }, [] { return 0; }, [] { return -3; }) == (sides ? -3 : 0));
+      int n = 0;
+      NEED(cp_run(c, [&](const CpClass &) { return n++, 0; }, [] { return -5; }, [&] { return n++, 0; }) ==
+           (sides ? -5 : 0) && n == (sides ? 0 : 4));
+    }
+  printf("ok\n");
+}
+""")
+    assert out == "ok\n"
