@@ -32,8 +32,8 @@ def run(tmp_path_factory):
 
 CHECK = r"""
 #define NEED(x) do { if (!(x)) { printf("line %d: %s\n", __LINE__, #x); exit(1); } } while (0)
-static const int CUS = 256;
-static void check(const std::vector<CpBin> &bin, bool f32) {
+[[maybe_unused]] static const int CUS = 256;
+[[maybe_unused]] static void check(const std::vector<CpBin> &bin, bool f32) {
   const CpShapes s = cp_shapes(bin, f32, CUS);
   NEED(s.runnable);
   std::vector<int> seen(bin.size());
