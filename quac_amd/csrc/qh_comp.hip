@@ -1216,18 +1216,16 @@ int qh_comp_rk4(qh_mat *A, qh_vec *x, double dt, int64_t nsteps) {
     a.nsteps = nsteps;
     hipStream_t ks = k.side ? c.side : s;
     const size_t table = CP_DICT * sizeof(double);
-    int rc = QH_EINVAL;
-    qh_set_error("no kernel for bins of %d rows a thread and %d slots", k.S, k.W);
     if (k.W == 0 && f32)
-      rc = cp_launch(k_comp_dict<float2, 8>, k, a, (size_t)2 * k.cells * sizeof(float2) + table, ks);
-    else if (k.W == 0)
-      rc = cp_launch(k_comp_dict<double2, 6>, k, a, (size_t)2 * k.cells * sizeof(double2) + table, ks);
+      return cp_launch(k_comp_dict<float2, 8>, k, a, (size_t)2 * k.cells * sizeof(float2) + table, ks);
+    if (k.W == 0) return cp_launch(k_comp_dict<double2, 6>, k, a, (size_t)2 * k.cells * sizeof(double2) + table, ks);
 #define CP_CASE(SS, WW, SK)                   \
   if (k.S == SS && k.W == WW && k.skip == SK) \
-    rc = cp_launch(k_comp_rk4<SS, WW, SK>, k, a, (size_t)2 * k.cells * sizeof(double2), ks);
+    return cp_launch(k_comp_rk4<SS, WW, SK>, k, a, (size_t)2 * k.cells * sizeof(double2), ks);
     CP_REG_KERNELS(CP_CASE)
 #undef CP_CASE
-    return rc;
+    qh_set_error("no kernel for bins of %d rows a thread and %d slots", k.S, k.W);
+    return QH_EINVAL;
   };
   return cp_run(c.classes, launch, fork, join);
 }

@@ -187,3 +187,17 @@ def test_batch_of_shapes_with_no_common_kernel(sizes, prec):
     b.destroy()
     for s in systems:
         s.destroy()
+
+
+def test_success_leaves_the_error_text():
+    """qh_last_error() is the message of the last failure, not of steps that ran"""
+    qs, _, _ = build_system(_tc(2, 9))
+    A, x0 = qs.matrix(), _start(36)
+    v = qa.DeviceVec(len(x0), qa.FP64)
+    v.set(x0)
+    assert qa.lib().qh_mat_set_lanes(A.h, 3, 0) != 0
+    text = qa.lib().qh_last_error()
+    assert b"lanes" in text
+    qa.rk4_device(A, v, 0.01, 3)
+    assert qa.lib().qh_last_error() == text
+    qs.destroy()
