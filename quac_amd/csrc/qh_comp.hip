@@ -26,12 +26,15 @@
 // 16.8 M rows in 1.4 ms, four launches a step of 233 us before; 512 systems of 100 to
 // 230 400 rows in FP32, 10 steps of 16 M rows in 3.7 ms, 8.4 ms before.
 #include <algorithm>
+#include <memory>
+#include <string>
 #include <vector>
 
 #include <hipcub/hipcub.hpp>
 
 #include "qh_common.h"
 #include "qh_comp_plan.h"
+#include "qh_optional.h"
 
 namespace {
 
@@ -850,10 +853,10 @@ int cp_build_small(qh_mat *A, int f32, int *done) {
   };
   Carve size, at;
   arrays(size);
-  qh_comp *c = new qh_comp();
+  // freed on every return before it is handed to A (the free waits for the device)
+  std::unique_ptr<qh_comp, void (*)(qh_comp *)> c(new qh_comp(), qh_comp_free);
   auto fail = [&](int code) {
     (void)hipStreamSynchronize(s);
-    qh_comp_free(c);
     return code;
   };
   int32_t *h = nullptr;
@@ -922,7 +925,7 @@ int cp_build_small(qh_mat *A, int f32, int *done) {
   c->a.ev = ev;
   c->a.ec = ec;
   c->trace = trace;
-  A->comp[f32] = c;
+  A->comp[f32] = c.release();
   A->comp_state[f32] = 1;
   return QH_OK;
 }
@@ -965,11 +968,11 @@ int cp_build(qh_mat *A, int f32) {
   if (own) wbuf = own;
   work.p = (char *)wbuf;
   layout(work);
-  qh_comp *c = new qh_comp();
+  // freed on every return before it is handed to A (the frees wait for the device)
+  std::unique_ptr<void, void (*)(void *)> owned(own, qh_free_ptr);
+  std::unique_ptr<qh_comp, void (*)(qh_comp *)> c(new qh_comp(), qh_comp_free);
   auto fail = [&](int code) {
     (void)hipStreamSynchronize(s);
-    qh_free_ptr(own);
-    qh_comp_free(c);
     return code;
   };
 #define CP_HIP(call)                                                                             \
@@ -1155,7 +1158,6 @@ int cp_build(qh_mat *A, int f32) {
     return QH_OK;
   }
 #undef CP_HIP
-  qh_free_ptr(own);
   c->a.bslice = bslice;
   c->a.bins = bins;
   c->a.soff = soff;
@@ -1168,7 +1170,7 @@ int cp_build(qh_mat *A, int f32) {
   c->a.ev = ev;
   c->a.ec = ec;
   c->trace = trace;
-  A->comp[f32] = c;
+  A->comp[f32] = c.release();
   state = 1;
   return QH_OK;
 }
@@ -1180,12 +1182,22 @@ int qh_comp_prepare(qh_mat *A, int prec, int *usable) {
   *usable = 0;
   if (A->comp_state[f32] == 0) {
     // row and slot numbers are 32-bit
-    int rc = QH_OK, done = 0;
-    if (A->rows < 1 || A->rows > (int64_t)1 << 30)
-      A->comp_state[f32] = -1;
-    else if (A->rows <= CP_SMALL_ROWS)
-      rc = cp_build_small(A, f32, &done);
-    if (!rc && A->comp_state[f32] == 0 && !done) rc = cp_build(A, f32);
+    const std::string text = qh_last_error();
+    auto build = [&]() -> int {
+      int rc = QH_OK, done = 0;
+      if (A->rows < 1 || A->rows > (int64_t)1 << 30)
+        A->comp_state[f32] = -1;
+      else if (A->rows <= CP_SMALL_ROWS)
+        rc = cp_build_small(A, f32, &done);
+      if (!rc && A->comp_state[f32] == 0 && !done) rc = cp_build(A, f32);
+      return rc;
+    };
+    auto none = [&] {
+      (void)hipGetLastError();
+      qh_set_error("%s", text.c_str());
+      A->comp_state[f32] = -1;  // the stage kernels run without the plan
+    };
+    const int rc = qh_optional(QH_ENOMEM, build, none);
     if (rc) return rc;
   }
   *usable = A->comp_state[f32] == 1;

@@ -22,7 +22,7 @@ def run(tmp_path_factory):
     def _run(name, body):
         src, exe = str(d / (name + ".cpp")), str(d / name)
         with open(src, "w") as f:
-            f.write('#include <cstdio>\n#include <cstdlib>\n#include <random>\n#include "qh_comp_plan.h"\n' + body)
+            f.write('#include <cstdio>\n#include <cstdlib>\n#include <random>\n#include "qh_comp_plan.h"\n#include "qh_optional.h"\n' + body)
         subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-fsanitize=address,undefined", "-I", CSRC, src,
                         "-o", exe], check=True)
         return subprocess.run([exe], check=True, capture_output=True, text=True).stdout
@@ -115,6 +115,22 @@ int main() {
       NEED(cp_run(c, [&](const CpClass &) { return n++, 0; }, [] { return -5; }, [&] { return n++, 0; }) ==
            (sides ? -5 : 0) && n == (sides ? 0 : 4));
     }
+  printf("ok\n");
+}
+""")
+    assert out == "ok\n"
+
+
+def test_no_memory_for_a_plan_is_no_error(run):
+    """a plan or list that does not fit in memory is done without; other errors stay"""
+    out = run("optional", CHECK + r"""
+int main() {
+  int none = 0;
+  auto n = [&] { none++; };
+  NEED(qh_optional(-2, [] { return 0; }, n) == 0 && none == 0);
+  NEED(qh_optional(-2, [] { return -3; }, n) == -3 && none == 0);
+  NEED(qh_optional(-2, [] { return -2; }, n) == 0 && none == 1);
+  NEED(qh_optional(-2, []() -> int { throw std::bad_alloc(); }, n) == 0 && none == 2);
   printf("ok\n");
 }
 """)
