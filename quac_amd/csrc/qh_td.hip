@@ -23,11 +23,13 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <string>
 #include <unordered_map>
 #include <vector>
 
 #include "qh_common.h"
 #include "qh_ks.h"
+#include "qh_optional.h"
 
 namespace {
 
@@ -759,33 +761,53 @@ __global__ void __launch_bounds__(64) k_td_fold(int64_t nrows, const int32_t *__
   }
 }
 
-// builds the lists for variant 134 of A's sliced layout, once per cache
+// builds the lists for variant 134 of A's sliced layout, once per cache (without the
+// memory for them all entries stay in the full lists)
 static int td_fold(const qh_mat *A, qh_td_cache *c) {
   if (c->fold_state) return QH_OK;
   c->fold_state = -1;
   if (!c->soff || c->dv.size() > 64 || c->max_row > 64 || A->ks_state != 1 || A->ks_maxslots > 64) return QH_OK;
   hipStream_t s = qh_stream();
   const size_t nsl = (size_t)A->nslices;
-  int64_t te = 0;
-  QH_HIP(hipMemcpyAsync(&te, c->soff + nsl, sizeof(te), hipMemcpyDeviceToHost, s));
-  QH_HIP(hipStreamSynchronize(s));
   unsigned long long *n = nullptr, hn = 0;
-  int rc = qh_alloc_t(&c->fslot, (size_t)A->ks_slots + 1);
-  if (!rc) rc = qh_alloc_t(&c->fw, nsl);
-  if (!rc) rc = qh_alloc_t(&c->fcol, (size_t)te + 1);
-  if (!rc) rc = qh_alloc_t(&c->fidx, (size_t)te + 1);
-  if (!rc) rc = qh_alloc_t(&n, 1);
-  if (rc) return rc;
-  QH_HIP(hipMemsetAsync(n, 0, sizeof(*n), s));
-  hipLaunchKernelGGL(k_td_fold, dim3((unsigned)nsl), dim3(64), 0, s, A->rows, A->ks_moff, A->ks_umid, A->ks_meta,
-                     c->soff, c->sw, c->ecol, c->eidx, (uint16_t)(c->dv.size() - 1), c->fslot, c->fw, c->fcol, c->fidx,
-                     n);
-  QH_HIP(hipGetLastError());
-  QH_HIP(hipMemcpyAsync(&hn, n, sizeof(hn), hipMemcpyDeviceToHost, s));
-  QH_HIP(hipStreamSynchronize(s));
+  auto build = [&]() -> int {
+    int64_t te = 0;
+    QH_HIP(hipMemcpyAsync(&te, c->soff + nsl, sizeof(te), hipMemcpyDeviceToHost, s));
+    QH_HIP(hipStreamSynchronize(s));
+    int rc = qh_alloc_t(&c->fslot, (size_t)A->ks_slots + 1);
+    if (!rc) rc = qh_alloc_t(&c->fw, nsl);
+    if (!rc) rc = qh_alloc_t(&c->fcol, (size_t)te + 1);
+    if (!rc) rc = qh_alloc_t(&c->fidx, (size_t)te + 1);
+    if (!rc) rc = qh_alloc_t(&n, 1);
+    if (rc) return rc;
+    QH_HIP(hipMemsetAsync(n, 0, sizeof(*n), s));
+    hipLaunchKernelGGL(k_td_fold, dim3((unsigned)nsl), dim3(64), 0, s, A->rows, A->ks_moff, A->ks_umid, A->ks_meta,
+                       c->soff, c->sw, c->ecol, c->eidx, (uint16_t)(c->dv.size() - 1), c->fslot, c->fw, c->fcol,
+                       c->fidx, n);
+    QH_HIP(hipGetLastError());
+    QH_HIP(hipMemcpyAsync(&hn, n, sizeof(hn), hipMemcpyDeviceToHost, s));
+    QH_HIP(hipStreamSynchronize(s));
+    return QH_OK;
+  };
+  const std::string text = qh_last_error();
+  const int rc = qh_optional(QH_ENOMEM, build, [&] {
+    (void)hipGetLastError();
+    qh_set_error("%s", text.c_str());
+  });
   qh_free_ptr(n);
-  if (hn) c->fold_state = 1;
-  return QH_OK;
+  if (hn && !rc) {
+    c->fold_state = 1;
+    return QH_OK;
+  }
+  // nothing taken over: the lists go
+  qh_free_ptr(c->fslot);
+  qh_free_ptr(c->fw);
+  qh_free_ptr(c->fcol);
+  qh_free_ptr(c->fidx);
+  c->fslot = nullptr;
+  c->fw = c->fcol = nullptr;
+  c->fidx = nullptr;
+  return rc;
 }
 
 // the sliced form of the merged A_k for A's stage kernel (variant G) to sum in the
