@@ -1727,11 +1727,8 @@ static int rk4_small(qh_mat *A, qh_vec *x, double dt, int64_t nsteps, int64_t to
   return QH_OK;
 }
 
-// steps per captured graph: renorm_every (rounded up to an even number) when the
-// trace is renormalised
-static int graph_len(int renorm_every) {
-  return renorm_every > 0 ? renorm_every + (renorm_every & 1) : g_graph_steps;
-}
+// steps per captured graph: renorm_every when the trace is renormalised
+static int graph_len(int renorm_every) { return renorm_every > 0 ? renorm_every : g_graph_steps; }
 
 // capture and instantiate the graph of len steps of x under A, unless the one
 // held was captured with the same parameters
@@ -1788,14 +1785,11 @@ static int rk4_impl(qh_mat *A, qh_vec *x, double dt, int64_t nsteps, int64_t tot
     rc = qh_comp_prepare(A, x->prec, &usable);
     if (rc) return rc;
     if (usable) {
-      const int64_t len = renorm_every > 0 ? graph_len(renorm_every) : nsteps;
+      const int64_t len = renorm_every > 0 ? renorm_every : nsteps;
+      double *t = qh_comp_trace(A, x->prec);
       for (int64_t st = 0; st < nsteps && !rc; st += len) {
         rc = qh_comp_rk4(A, x, dt, std::min<int64_t>(len, nsteps - st));
-        if (!rc && renorm_every > 0 && st + len <= nsteps)
-          {
-          double *t = qh_comp_trace(A, x->prec);
-          rc = renorm_launch(s, x, x->d, tot, 0, t, t + 512);
-        }
+        if (!rc && renorm_every > 0 && st + len <= nsteps) rc = renorm_launch(s, x, x->d, tot, 0, t, t + 512);
       }
       return rc;
     }

@@ -201,3 +201,19 @@ def test_success_leaves_the_error_text():
     qa.rk4_device(A, v, 0.01, 3)
     assert qa.lib().qh_last_error() == text
     qs.destroy()
+
+
+@pytest.mark.parametrize("recipe", [_tc(2, 12), _noisy(5, [("ham", 0.3 + 0.1 * i, [(i, "sx")]) for i in range(5)])],
+                         ids=["closed sets", "stage kernels"])
+def test_renormalised_every_odd_number_of_steps(recipe):
+    """the trace is one after exactly renorm_every steps, and the steps after it leave it"""
+    qs, _, _ = build_system(recipe)
+    A, n = qs.matrix(), qs.total_levels
+    x0 = 1.5 * _start(n)
+    for every, steps in ((5, 5), (3, 9), (1, 4), (7, 16)):
+        f = _steps(A, x0, qa.FP32, 0.01, steps, tot=n, renorm_every=every)
+        # the two words' rounding of n entries, and of a step that keeps the trace
+        assert abs(np.trace(f.reshape(n, n)) - 1.0) < 1e-12 + (steps % every) * n * 2.0 ** -24, (every, steps)
+    f = _steps(A, x0, qa.FP32, 0.01, 4, tot=n, renorm_every=5)
+    assert abs(np.trace(f.reshape(n, n)) - 1.5) < 4 * n * 2.0 ** -24
+    qs.destroy()
