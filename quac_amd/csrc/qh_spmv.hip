@@ -1356,35 +1356,55 @@ extern "C" int qh_last_stage_ms(double *spmv_ms, int64_t *launches) {
 // Bound by that chain: reads, dependent FMAs, barrier.  Jaynes-Cummings 2 x 10 (400
 // rows of at most 5 entries), 100 steps: 75 us, 180 us with the
 // stage derivatives in LDS (two reads an entry, no two in flight).
+// Rows of up to 32 entries off the diagonal stay in registers, the last of them
+// spilled, which scratch memory interleaves by lane; rows read from the CSR are one
+// cache line a lane and entry.  50 steps from registers / the CSR: 784 rows of 14 off the
+// diagonal 190 / 1090 us, of 18 362 / 1427 us, of 28 1060 / 2590 us; 576 rows of 19
+// 213 / 1119 us.
 #define QH_SMALL_ROWS 800
-// up to this many rows a thread has the registers for more than 8 entries
+#define QH_SMALL_THREADS 832  // four wavefronts a SIMD, 128 registers a thread
+// up to this many rows three wavefronts a SIMD hold them: 168 registers a thread
 #define QH_SMALL_WIDE_ROWS 640
 
 // Row r of the generator in registers: its diagonal entry, which multiplies the
 // thread's own value, and its (at most MAXNZ) other entries, filled up with zeros
 // times the zero cell n of the vector so that all reads are in flight together;
 // MAXNZ == 0: the row is read from the CSR in memory.
-template <int MAXNZ>
+// PACK: two columns a register (of at most 800 rows), which costs an instruction an
+// entry and is for rows that would not fit otherwise.
+template <int MAXNZ, bool PACK = false>
 struct SmallRow {
-  int32_t c[MAXNZ > 0 ? MAXNZ : 1];
+  int32_t c[MAXNZ > 0 ? (PACK ? MAXNZ / 2 : MAXNZ) : 1];
   double2 v[MAXNZ > 0 ? MAXNZ : 1];
   double2 d = {0.0, 0.0};
   int32_t b = 0, e = 0;
+  __device__ __forceinline__ int32_t at(int k) const {
+    if constexpr (PACK) {
+      uint32_t w = c[k / 2];
+      asm volatile("" : "+v"(w));  // taken apart where it is used, not ahead of the step loop
+      return (int32_t)(k & 1 ? w >> 16 : w & 0xFFFFu);
+    }
+    return c[k];
+  }
   __device__ __forceinline__ void load(int32_t n, int32_t r, const int32_t *rp, const int32_t *col, const double2 *val) {
     if (r < n) {
       b = rp[r];
       e = rp[r + 1];
     }
     if constexpr (MAXNZ > 0) {
-      int32_t at = e - b;  // position of the diagonal entry
+      int32_t diag = e - b;  // position of the diagonal entry
       for (int32_t k = b; k < e; k++)
-        if (col[k] == r) at = k - b;
-      if (at < e - b) d = val[b + at];
+        if (col[k] == r) diag = k - b;
+      if (diag < e - b) d = val[b + diag];
 #pragma unroll
       for (int k = 0; k < MAXNZ; k++) {
-        const int32_t s = b + k + (k >= at ? 1 : 0);
+        const int32_t s = b + k + (k >= diag ? 1 : 0);
         const bool on = s < e;
-        c[k] = on ? col[s] : n;
+        const int32_t q = on ? col[s] : n;
+        if (!PACK)
+          c[k] = q;
+        else
+          c[k / 2] = k & 1 ? c[k / 2] | q << 16 : q;
         v[k] = on ? val[s] : make_double2(0.0, 0.0);
       }
     }
@@ -1403,7 +1423,7 @@ struct SmallRow {
       for (int k0 = 0; k0 < MAXNZ; k0 += CH) {
         double2 t[CH];
 #pragma unroll
-        for (int k = 0; k < CH; k++) t[k] = y[c[k0 + k]];
+        for (int k = 0; k < CH; k++) t[k] = y[at(k0 + k)];
 #pragma unroll
         for (int k = 0; k < CH; k++) add(v[k0 + k], t[k]);
         if (CH < MAXNZ) __builtin_amdgcn_sched_barrier(0);
@@ -1415,16 +1435,17 @@ struct SmallRow {
   }
 };
 
-template <bool F32, int MAXNZ>
-__global__ void __launch_bounds__(MAXNZ > 8 ? QH_SMALL_WIDE_ROWS : 832) k_rk4_small(int32_t n, const int32_t *__restrict__ rp,
-                                                   const int32_t *__restrict__ col, const double2 *__restrict__ val,
-                                                   void *xg, float2 *xlo, double h, int64_t nsteps, int64_t tot,
-                                                   int renorm_every) {
+template <bool F32, int MAXNZ, int THREADS>
+__global__ void __launch_bounds__(THREADS) k_rk4_small(int32_t n, const int32_t *__restrict__ rp,
+                                                       const int32_t *__restrict__ col,
+                                                       const double2 *__restrict__ val, void *xg, float2 *xlo,
+                                                       double h, int64_t nsteps, int64_t tot, int renorm_every) {
   extern __shared__ double2 sm[];
   __shared__ double2 scale;
   double2 *const y0 = sm, *const y1 = sm + n + 1;
   const int r = threadIdx.x;  // n <= blockDim.x
-  SmallRow<MAXNZ> row;
+  // up to 16 entries fit 168 registers with their columns apart, up to 12 fit 128
+  SmallRow<MAXNZ, (MAXNZ > (THREADS > QH_SMALL_WIDE_ROWS ? 12 : 16))> row;
   row.load(n, r, rp, col, val);
   double2 x = make_double2(0.0, 0.0);
   if (r < n) {
@@ -1709,20 +1730,24 @@ static int rk4_small(qh_mat *A, qh_vec *x, double dt, int64_t nsteps, int64_t to
   const size_t lds = (size_t)2 * (n + 1) * sizeof(double2);
   hipStream_t s = qh_stream();
   const int mr = A->max_off;
-#define QH_LS1(F, Z)                                                                                            \
-  hipLaunchKernelGGL((k_rk4_small<F, Z>), dim3(1), dim3(bt), lds, s, n, A->rowptr, A->col, A->val, x->d, x->lo, \
-                     dt, nsteps, tot, renorm_every)
-#define QH_LS(Z)                      \
-  if (x->prec == QH_FP32) QH_LS1(true, Z); \
-  else QH_LS1(false, Z)
-  if (mr <= 4) { QH_LS(4); }
-  else if (mr <= 6) { QH_LS(6); }
-  else if (mr <= 8) { QH_LS(8); }
-  else if (mr <= 12 && n <= QH_SMALL_WIDE_ROWS) { QH_LS(12); }
-  else if (mr <= 16 && n <= QH_SMALL_WIDE_ROWS) { QH_LS(16); }
-  else { QH_LS(0); }
+  auto run = [&](auto *k32, auto *k64) {
+    hipLaunchKernelGGL(x->prec == QH_FP32 ? k32 : k64, dim3(1), dim3(bt), lds, s, n, A->rowptr, A->col, A->val, x->d,
+                       x->lo, dt, nsteps, tot, renorm_every);
+  };
+#define QH_LS(Z, T) run(k_rk4_small<true, Z, T>, k_rk4_small<false, Z, T>)
+  const bool few = n <= QH_SMALL_WIDE_ROWS;
+  if (mr <= 4) QH_LS(4, QH_SMALL_THREADS);
+  else if (mr <= 6) QH_LS(6, QH_SMALL_THREADS);
+  else if (mr <= 8) QH_LS(8, QH_SMALL_THREADS);
+  else if (mr <= 12) QH_LS(12, QH_SMALL_THREADS);
+  else if (mr <= 16 && few) QH_LS(16, QH_SMALL_WIDE_ROWS);
+  else if (mr <= 16) QH_LS(16, QH_SMALL_THREADS);
+  else if (mr <= 24 && few) QH_LS(24, QH_SMALL_WIDE_ROWS);
+  else if (mr <= 24) QH_LS(24, QH_SMALL_THREADS);
+  else if (mr <= 32 && few) QH_LS(32, QH_SMALL_WIDE_ROWS);
+  else if (mr <= 32) QH_LS(32, QH_SMALL_THREADS);
+  else QH_LS(0, QH_SMALL_THREADS);
 #undef QH_LS
-#undef QH_LS1
   QH_HIP(hipGetLastError());
   return QH_OK;
 }

@@ -96,3 +96,42 @@ def test_small_adaptive_matches_numpy(dims):
     assert np.abs(x.get() - ref).max() <= steps * (4 * norm + 8) * np.abs(x0).max() * 2.0 ** -53
     x.destroy()
     qs.destroy()
+
+
+def _wide(dims, exchange, squeezed=()):
+    r = _coupled(dims)
+    for a, b in exchange:
+        r["terms"] += [("ham", 0.1, [(a, "raise"), (b, "lower")]), ("ham", 0.1, [(b, "raise"), (a, "lower")])]
+    for a, b in squeezed:
+        r["terms"] += [("ham", 0.07, [(a, "raise"), (b, "raise")]), ("ham", 0.07, [(a, "lower"), (b, "lower")])]
+    return r
+
+
+RING = [(0, 1), (1, 2), (0, 2)]
+
+
+# the entries off the diagonal of the longest row: every width of the kernels for up to
+# 640 rows and for up to 800
+@pytest.mark.parametrize("recipe,off", [
+    (_coupled((3, 9)), 10), (_wide((4, 6), [(0, 1)]), 14), (_wide((4, 7), [(0, 1)]), 14),
+    (_wide((4, 6), [(0, 1)], [(1, 1)]), 18), (_wide((4, 7), [(0, 1)], [(1, 1)]), 18),
+    (_wide((3, 3, 3), [(0, 1), (1, 2)]), 23), (_wide((2, 3, 4), RING, [(1, 2)]), 25),
+    (_wide((2, 3, 4), RING, RING), 29), (_wide((3, 3, 3), RING, [(0, 1)]), 31), (_wide((3, 3, 3), RING, RING), 39),
+])
+def test_wide_rows(recipe, off):
+    qs, _, _ = build_system(recipe)
+    A = qs.matrix()
+    tot, terms = recipes.oracle_terms(recipe)
+    x0, dt, steps = _start(tot), 0.02, 7
+    ref = oracle.construct(tot, terms, dm=True).rk4(x0, dt, steps)
+    rp, col, val = A.export()
+    rows = np.repeat(np.arange(tot * tot), np.diff(rp))
+    assert np.bincount(rows[col != rows]).max() == off
+    norm = np.add.reduceat(np.abs(val), rp[:-1]).max()
+    for prec, eps in ((qa.FP64, 2.0 ** -53), (qa.FP32, 2.0 ** -47)):
+        v = qa.DeviceVec(tot * tot, prec)
+        v.set(x0)
+        qa.rk4_device(A, v, dt, steps)
+        # a few roundings of the state and of h A times it per step
+        assert np.abs(v.get() - ref).max() <= (steps * (2 * dt * norm + 8) + 1) * np.abs(x0).max() * eps
+    qs.destroy()
