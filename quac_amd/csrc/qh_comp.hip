@@ -792,7 +792,8 @@ struct qh_comp {
   void *buf = nullptr, *slots = nullptr;  // the plan's arrays; its entries
   CpArgs a{};
   double *trace = nullptr;  // QH_COMP_TRACE doubles for the trace renormalisation
-  std::vector<CpClass> classes;
+  std::vector<CpClass> classes, brief;  // brief: of a call of up to brief_steps steps
+  int64_t brief_steps = 0;
   // launches of fewer blocks than CUs run on a stream of their own beside the
   // others (disjoint rows), between two events of the library stream
   hipStream_t side = nullptr;
@@ -1117,6 +1118,8 @@ int cp_build(qh_mat *A, int f32) {
     return QH_OK;
   }
   c->classes = sh.classes;
+  c->brief = sh.brief;
+  c->brief_steps = sh.brief_steps;
   for (const CpClass &k : c->classes)
     if (k.side && !c->side) {
       CP_HIP(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
@@ -1239,7 +1242,7 @@ int qh_comp_rk4(qh_mat *A, qh_vec *x, double dt, int64_t nsteps) {
     qh_set_error("no kernel for bins of %d rows a thread and %d slots", k.S, k.W);
     return QH_EINVAL;
   };
-  return cp_run(c.classes, launch, fork, join);
+  return cp_run(nsteps <= c.brief_steps ? c.brief : c.classes, launch, fork, join);
 }
 
 double *qh_comp_trace(const qh_mat *A, int prec) { return A->comp[prec == QH_FP32]->trace; }

@@ -84,7 +84,59 @@ struct CpShapes {
   std::vector<int32_t> bins;          // all bins in the order of the launches
   double most = 0.0, all = 0.0;       // clocks of a stage: the largest bin, all bins
   bool runnable = true;               // every launch has a kernel
+  // the launches of a call of up to brief_steps steps: words, and all other bins in one
+  std::vector<CpClass> brief;
+  int64_t brief_steps = 0;
 };
+
+// wavefronts that a CU holds of a class's kernel (its registers), as workgroups
+inline double cp_resident(const CpClass &c) {
+  const int waves = c.W == 0 || c.S > 1 || c.W > 12 ? 16 : c.W > 8 ? 20 : 32;
+  return (double)waves * 64.0 / c.threads;
+}
+
+// Bins of several shapes each have their launch, and launches run one after the other or
+// wait for a stream beside: 6 to 8 us each, whatever the steps.  In one launch of the
+// largest shape small bins hold more wavefronts than they need, and fewer bins run at a
+// time.  The line lies where that costs as much as 3 us a launch saved (half of what a
+// launch costs, so that a call of more steps is not slowed down where the estimate is off).
+// Measured us a call, several launches / one, for 1, 5 and 20 steps: decay and dephasing of
+// 8 qubits 45 / 8, 50 / 13, 94 / 30; 9 qubits 58 / 24, 62 / 47, 122 / 132; 10 qubits 80 / 42,
+// 124 / 85, 315 / 250; 11 qubits 180 / 192, 263 / 371, 764 / 1082 (several always).
+inline void cp_brief(CpShapes &s, const std::vector<CpBin> &bin, int cus) {
+  CpClass one{0, 0, 0, true, false, -1, 0, 0};
+  double apart = 0.0, together = 0.0, reads = 0.0;  // clocks of a stage of all CUs
+  for (const CpClass &k : s.classes) {
+    if (k.W == 0) {
+      s.brief.push_back(k);
+      s.brief.back().side = false;
+      continue;
+    }
+    if (one.first < 0) one.first = k.first;
+    one.threads = std::max(one.threads, k.threads);
+    one.S = std::max(one.S, k.S);
+    one.W = std::max(one.W, k.W);
+    one.cells = std::max(one.cells, k.cells);
+    one.count += k.count;
+  }
+  if (one.count == 0 || !cp_has_kernel(one) || s.brief.size() + 1 >= s.classes.size()) {
+    s.brief.clear();
+    return;
+  }
+  for (const CpClass &k : s.classes) {
+    if (k.W == 0) continue;
+    for (int i = 0; i < k.count; i++) {
+      const double clk = CP_CLK_REG * (double)bin[s.bins[k.first + i]].slots;
+      reads += clk;
+      apart += (clk + CP_CLK_FIXED) / cp_resident(k);
+      together += (clk + CP_CLK_FIXED) / cp_resident(one);
+    }
+  }
+  const double more_us = 4.0 * (std::max(together, reads) - std::max(apart, reads)) / cus / 2400.0;
+  const double saved_us = 3.0 * (double)(s.classes.size() - s.brief.size() - 1);
+  s.brief.push_back(one);
+  s.brief_steps = more_us <= 0.0 ? INT64_MAX : (int64_t)std::min(1e9, saved_us / more_us);
+}
 
 inline CpShapes cp_shapes(const std::vector<CpBin> &bin, bool f32, int cus) {
   CpShapes out;
@@ -146,6 +198,7 @@ inline CpShapes cp_shapes(const std::vector<CpBin> &bin, bool f32, int cus) {
     if (out.classes.size() > 1 && k.count < cus && k.first + k.count < n) k.side = true;
     if (!cp_has_kernel(k)) out.runnable = false;
   }
+  cp_brief(out, bin, cus);
   return out;
 }
 

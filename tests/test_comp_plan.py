@@ -22,7 +22,7 @@ def run(tmp_path_factory):
     def _run(name, body):
         src, exe = str(d / (name + ".cpp")), str(d / name)
         with open(src, "w") as f:
-            f.write('#include <cstdio>\n#include <cstdlib>\n#include <random>\n#include "qh_comp_plan.h"\n#include "qh_optional.h"\n' + body)
+            f.write('#include <array>\n#include <cstdio>\n#include <cstdlib>\n#include <random>\n#include "qh_comp_plan.h"\n#include "qh_optional.h"\n' + body)
         subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-fsanitize=address,undefined", "-I", CSRC, src,
                         "-o", exe], check=True)
         return subprocess.run([exe], check=True, capture_output=True, text=True).stdout
@@ -33,12 +33,10 @@ def run(tmp_path_factory):
 CHECK = r"""
 #define NEED(x) do { if (!(x)) { printf("line %d: %s\n", __LINE__, #x); exit(1); } } while (0)
 [[maybe_unused]] static const int CUS = 256;
-[[maybe_unused]] static void check(const std::vector<CpBin> &bin, bool f32) {
-  const CpShapes s = cp_shapes(bin, f32, CUS);
-  NEED(s.runnable);
+static void walk(const std::vector<CpBin> &bin, bool f32, const CpShapes &s, const std::vector<CpClass> &classes) {
   std::vector<int> seen(bin.size());
   int at = 0;
-  for (const CpClass &k : s.classes) {
+  for (const CpClass &k : classes) {
     NEED(k.first == at && k.count > 0 && cp_has_kernel(k));
     NEED(k.threads <= 1024 && k.threads % 64 == 0);
     // two buffers of k.cells entries, and the table beside words
@@ -55,7 +53,15 @@ CHECK = r"""
   }
   NEED(at == (int)bin.size());
   for (int n : seen) NEED(n == 1);
-  NEED(!s.classes.back().side);
+  NEED(!classes.back().side);
+}
+[[maybe_unused]] static void check(const std::vector<CpBin> &bin, bool f32) {
+  const CpShapes s = cp_shapes(bin, f32, CUS);
+  NEED(s.runnable);
+  walk(bin, f32, s, s.classes);
+  NEED(s.brief.empty() ? s.brief_steps == 0 : s.brief_steps >= 0 && s.brief.size() < s.classes.size());
+  if (!s.brief.empty()) walk(bin, f32, s, s.brief);
+  for (const CpClass &k : s.brief) NEED(!k.side);
 }
 """
 
@@ -86,6 +92,31 @@ int main() {
     }
     check(bin, t & 1);
   }
+  printf("ok\n");
+}
+""")
+    assert out == "ok\n"
+
+
+def test_short_calls_take_fewer_launches(run):
+    """many small bins go into one launch for a call of few steps, whatever the steps of
+    a larger one; bins of a launch of their own stay in it where the rest would idle"""
+    out = run("brief", CHECK + r"""
+static std::vector<CpBin> bins(std::vector<std::array<int, 3>> groups) {
+  std::vector<CpBin> b;
+  for (auto g : groups)
+    for (int i = 0; i < g[0]; i++) b.push_back({g[1], g[2], (int64_t)g[2] * g[1] / 64});
+  return b;
+}
+int main() {
+  // the bins of decay and dephasing of 8, 10 and 11 qubits
+  const CpShapes s8 = cp_shapes(bins({{9, 256, 8}, {233, 128, 7}, {128, 128, 4}, {266, 64, 6}, {369, 64, 4}}), false, CUS);
+  const CpShapes s10 = cp_shapes(bins({{9, 1024, 10}, {12, 512, 9}, {2156, 512, 7}, {16, 512, 4}, {9, 64, 4}}), false, CUS);
+  const CpShapes s11 = cp_shapes(
+      bins({{9, 2048, 11}, {102, 1024, 10}, {132, 512, 9}, {8458, 512, 8}, {22, 512, 4}, {57, 256, 8}, {13, 64, 8}}), false, CUS);
+  NEED(s8.classes.size() == 5 && s8.brief.size() == 1 && s8.brief_steps >= 20);
+  NEED(s10.brief.size() == 1 && s10.brief_steps >= 2 && s10.brief_steps <= 20);
+  NEED(s11.brief.size() == 1 && s11.brief_steps == 0);
   printf("ok\n");
 }
 """)

@@ -217,3 +217,27 @@ def test_renormalised_every_odd_number_of_steps(recipe):
     f = _steps(A, x0, qa.FP32, 0.01, 4, tot=n, renorm_every=5)
     assert abs(np.trace(f.reshape(n, n)) - 1.5) < 4 * n * 2.0 ** -24
     qs.destroy()
+
+
+@pytest.mark.parametrize("prec", [qa.FP64, qa.FP32])
+@pytest.mark.parametrize("recipe", [_noisy(8), _noisy(9)], ids=["8", "9"])
+def test_short_calls_step_the_same_state(recipe, prec):
+    """one step a call (all bins in one launch) and many (a launch a shape, some on the
+    side stream) are the same arithmetic"""
+    qs, _, _ = build_system(recipe)
+    A, n, dt, steps = qs.matrix(), qs.total_levels, 0.02, 200
+    x0 = _start(n)
+    one = _steps(A, x0, prec, dt, steps)
+    v = qa.DeviceVec(len(x0), prec)
+    v.set(x0)
+    for _ in range(steps):
+        qa.rk4_device(A, v, dt, 1)
+    # FP64: bitwise; FP32: the state is split into its two words between the calls
+    assert np.abs(v.get() - one).max() <= (0.0 if prec == qa.FP64 else steps * np.abs(x0).max() * 2.0 ** -48)
+    tot, terms = recipes.oracle_terms(recipe)
+    ref = oracle.construct(tot, terms, dm=True).rk4(x0, dt, 5)
+    rp, _, val = A.export()
+    norm = np.add.reduceat(np.abs(val), rp[:-1]).max()
+    tol = 5 * np.abs(x0).max() * (2 * dt * norm + 8) * (2.0 ** -53 if prec == qa.FP64 else 2.0 ** -47)
+    assert np.abs(_steps(A, x0, prec, dt, 5) - ref).max() <= tol + (2.0 ** -47 if prec == qa.FP32 else 0.0)
+    qs.destroy()
