@@ -96,6 +96,14 @@ int qh_mat_pair_layout_info(qh_mat *m, int64_t *slices, int64_t *slots, int64_t 
                             int64_t *stored_real_pairs, int64_t *meta_bytes, int64_t *stored_real_singles,
                             int64_t *sep_slots);
 
+/* the plan by which qh_rk4 steps states of precision prec where the rows of the
+ * generator fall apart into small closed sets: its workgroups (bins of whole sets),
+ * those that read their entries as 32-bit words at every stage, the launches of a
+ * call of many steps, and the 64-entry slots held in registers and as words; zeros
+ * where there is none (not formed yet, or the stage kernels are faster) */
+int qh_mat_closed_info(const qh_mat *m, int prec, int64_t *bins, int64_t *word_bins, int64_t *launches,
+                       int64_t *slots, int64_t *word_slots);
+
 /* ------------------------------------------------------------------ vectors */
 typedef struct qh_vec qh_vec;
 enum { QH_FP64 = 64, QH_FP32 = 32 };

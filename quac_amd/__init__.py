@@ -183,6 +183,7 @@ def _setup(L):
     sig("qh_mat_get_lanes", i32, vp, P(i32), P(i32))
     sig("qh_mat_layout_info", i32, vp, P(i64), P(i64), P(i64), P(i64), P(i64))
     sig("qh_mat_pair_layout_info", i32, vp, P(i64), P(i64), P(i64), P(i64), P(i64), P(i64), P(i64))
+    sig("qh_mat_closed_info", i32, vp, i32, P(i64), P(i64), P(i64), P(i64), P(i64))
     sig("qh_vec_create", i32, i64, i32, P(vp))
     sig("qh_vec_destroy", i32, vp)
     sig("qh_vec_set", i32, vp, P(dbl))
@@ -387,6 +388,13 @@ class Matrix:
         _qh(lib().qh_mat_pair_layout_info(self.h, *[ctypes.byref(x) for x in v]))
         return dict(zip(("slices", "slots", "stored_pairs", "stored_real_pairs", "meta_bytes", "stored_real_singles",
                          "sep_slots"), [x.value for x in v]))
+
+    def closed_info(self, prec=FP64):
+        """plan of the closed sets of rows for states of a precision: dict(bins, word_bins, launches,
+        slots, word_slots); zeros where rk4 has none"""
+        v = [ctypes.c_int64() for _ in range(5)]
+        _qh(lib().qh_mat_closed_info(self.h, prec, *[ctypes.byref(x) for x in v]))
+        return dict(zip(("bins", "word_bins", "launches", "slots", "word_slots"), [x.value for x in v]))
 
     def __del__(self):
         if getattr(self, "owned", False) and self.h and _lib is not None:

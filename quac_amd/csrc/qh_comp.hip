@@ -794,6 +794,7 @@ struct qh_comp {
   double *trace = nullptr;  // QH_COMP_TRACE doubles for the trace renormalisation
   std::vector<CpClass> classes, brief;  // brief: of a call of up to brief_steps steps
   int64_t brief_steps = 0;
+  int64_t slots_of[2] = {0, 0};  // in registers, as words
   // launches of fewer blocks than CUs run on a stream of their own beside the
   // others (disjoint rows), between two events of the library stream
   hipStream_t side = nullptr;
@@ -914,6 +915,7 @@ int cp_build_small(qh_mat *A, int f32, int *done) {
   CP_HIP(hipGetLastError());
 #undef CP_HIP
   const int S = rows > 1024 ? 2 : 1;
+  c->slots_of[0] = slots;
   c->classes.push_back(CpClass{cp_threads(rows), S, W, false, false, 0, nb, rows + 1});
   c->a = CpArgs{};
   c->a.bins = bins;
@@ -1120,6 +1122,7 @@ int cp_build(qh_mat *A, int f32) {
   c->classes = sh.classes;
   c->brief = sh.brief;
   c->brief_steps = sh.brief_steps;
+  std::copy_n(slots, 2, c->slots_of);
   for (const CpClass &k : c->classes)
     if (k.side && !c->side) {
       CP_HIP(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
@@ -1246,3 +1249,21 @@ int qh_comp_rk4(qh_mat *A, qh_vec *x, double dt, int64_t nsteps) {
 }
 
 double *qh_comp_trace(const qh_mat *A, int prec) { return A->comp[prec == QH_FP32]->trace; }
+
+extern "C" int qh_mat_closed_info(const qh_mat *m, int prec, int64_t *bins, int64_t *word_bins, int64_t *launches,
+                                  int64_t *slots, int64_t *word_slots) {
+  QH_REQUIRE(m && (prec == QH_FP64 || prec == QH_FP32), QH_EINVAL, "qh_mat_closed_info: a matrix and a precision required");
+  const qh_comp *c = m->comp[prec == QH_FP32];
+  int64_t all = 0, words = 0;
+  if (c)
+    for (const CpClass &k : c->classes) {
+      all += k.count;
+      if (k.W == 0) words += k.count;
+    }
+  if (bins) *bins = all;
+  if (word_bins) *word_bins = words;
+  if (launches) *launches = c ? (int64_t)c->classes.size() : 0;
+  if (slots) *slots = c ? c->slots_of[0] : 0;
+  if (word_slots) *word_slots = c ? c->slots_of[1] : 0;
+  return QH_OK;
+}

@@ -55,6 +55,7 @@ def _start(n):
 def _steps(A, x0, prec, dt, steps, **kw):
     v = qa.DeviceVec(len(x0), prec)
     v.set(x0)
+    qa.rk4_prepare(A, v, dt, **kw)  # the plan is formed now, whatever the steps
     qa.rk4_device(A, v, dt, steps, **kw)
     return v.get()
 
@@ -77,6 +78,7 @@ def test_closed_sets_match_oracle(recipe):
             tol = steps * np.abs(x0).max() * (2 * dt * norm + 8) * eps + (2.0 ** -47 if prec == qa.FP32 else 0.0)
             got = _steps(A, x0, prec, dt, steps)
             assert np.abs(got - ref).max() <= tol, (steps, prec)
+            assert A.closed_info(prec)["bins"] > 0 or A.info()[0] <= 800
     A.set_lanes(8, 8)  # the stage kernels
     ref = _steps(A, x0, qa.FP64, dt, 7)
     A.set_lanes(0, 0)
@@ -84,14 +86,15 @@ def test_closed_sets_match_oracle(recipe):
     qs.destroy()
 
 
-def test_entries_read_as_words():
-    """13 slots a row and a component of 2048 rows: the kernel that reads its entries
-    at every stage, beside the ones that hold them"""
+def test_largest_sets_in_registers():
+    """a component of 2048 rows and 11 slots: the most rows and slots of two rows a
+    thread"""
     r = _noisy(11)
     qs, _, _ = build_system(r)
     A = qs.matrix()
     x0 = _start(2048)
     got = _steps(A, x0, qa.FP64, 0.02, 3)
+    assert A.closed_info()["bins"] > 0 and A.closed_info()["word_bins"] == 0
     A.set_lanes(8, 0)
     ref = _steps(A, x0, qa.FP64, 0.02, 3)
     # rows of h A sum to at most 0.02 * 2 * 11 * 0.2 here
@@ -99,26 +102,38 @@ def test_entries_read_as_words():
     qs.destroy()
 
 
-def test_entries_read_as_words_fp32():
-    """components of up to 2280 rows and 13 slots (more than are fetched ahead), enough
-    of them to fill the chip: complex64 stage vectors"""
-    recipe, count, dt, steps = _tc(4, 10), 20, 0.02, 3
+# the largest set of four emitters and a cavity of n levels has 256 n - 280 rows: 2280 for
+# 10 levels, 4584 and 4840 for 19 and 20 (the limit in FP64 is 4800), 7912 and 8168 for 32
+# and 33 (8128 in FP32)
+@pytest.mark.parametrize("levels,count,prec,words", [
+    (10, 20, qa.FP32, True), (10, 20, qa.FP64, True), (19, 12, qa.FP64, True), (20, 12, qa.FP64, False),
+    (32, 12, qa.FP32, True), (33, 12, qa.FP32, False)])
+def test_entries_read_as_words(levels, count, prec, words):
+    """components too large for registers, of up to 13 slots (more than are fetched
+    ahead), enough of them to fill the chip; complex64 stage vectors in FP32"""
+    recipe, dt, steps = _tc(4, levels), 0.02, 3
     systems = [build_system(recipe)[0] for _ in range(count)]
-    b = qa.Batch([s.matrix() for s in systems], [160] * count, prec=qa.FP32)
-    x0 = _start(160)
+    n = 16 * levels
+    b = qa.Batch([s.matrix() for s in systems], [n] * count, prec=prec)
+    x0 = _start(n)
     for i in range(count):
         b.set_state(i, x0 if i % 2 else x0.conj())
+    qa.rk4_prepare(b.matrix(), b.state(), dt)
     b.rk4(dt, steps)
+    info = b.matrix().closed_info(prec)
+    assert (info["word_bins"] > 0) == words and (info["bins"] > 0) == words
     tot, terms = recipes.oracle_terms(recipe)
     m = oracle.construct(tot, terms, dm=True)
     rp, _, val = systems[0].matrix().export()
     norm = np.add.reduceat(np.abs(val), rp[:-1]).max()
-    # per step: h |A| of a state rounded to 32 bits, and the two words' rounding
-    tol = steps * np.abs(x0).max() * (2 * dt * norm * 2.0 ** -24 + 8 * 2.0 ** -48)
-    for i in (0, 7, count - 1):
+    # per step: h |A| of a state rounded to 32 bits, and the two words' rounding; FP64: a
+    # few roundings of the state and of h A times it
+    eps = (2 * dt * norm + 8) * 2.0 ** -53 if prec == qa.FP64 else 2 * dt * norm * 2.0 ** -24 + 8 * 2.0 ** -48
+    for i in (0, count - 1):
         ref = m.rk4(x0 if i % 2 else x0.conj(), dt, steps)
-        assert np.abs(b.get_state(i) - ref).max() <= tol
-    assert np.array_equal(b.get_state(1), b.get_state(count - 1))
+        assert np.abs(b.get_state(i) - ref).max() <= steps * np.abs(x0).max() * eps
+    if words:  # (the order of a row's slots on the sliced layout depends on where its block starts)
+        assert np.array_equal(b.get_state(1), b.get_state(count - 1))
     b.destroy()
     for s in systems:
         s.destroy()
@@ -150,7 +165,9 @@ def test_batch_of_uneven_blocks():
     starts = [_start(t) for t in tots]
     for i, x0 in enumerate(starts):
         b.set_state(i, x0)
+    qa.rk4_prepare(b.matrix(), b.state(), 0.01)
     b.rk4(0.01, 6)
+    assert b.matrix().closed_info()["bins"] > 0
     for i, (s, x0) in enumerate(zip(sizes, starts)):
         tot, terms = recipes.oracle_terms(_tc(*s))
         ref = oracle.construct(tot, terms, dm=True).rk4(x0, 0.01, 6)
@@ -173,8 +190,11 @@ def test_batch_of_shapes_with_no_common_kernel(sizes, prec):
     starts = [_start(t) for t in tots]
     for i, x0 in enumerate(starts):
         b.set_state(i, x0)
+    qa.rk4_prepare(b.matrix(), b.state(), dt)
     b.rk4(dt, 1)
     b.rk4(dt, steps - 1)
+    info = b.matrix().closed_info(prec)
+    assert info["launches"] > 1 and (info["word_bins"] > 0) == (len(sizes) == 3)
     for i, (s, x0) in enumerate(zip(sizes, starts)):
         tot, terms = recipes.oracle_terms(_tc(*s))
         m = oracle.construct(tot, terms, dm=True)
@@ -198,6 +218,7 @@ def test_success_leaves_the_error_text():
     assert qa.lib().qh_mat_set_lanes(A.h, 3, 0) != 0
     text = qa.lib().qh_last_error()
     assert b"lanes" in text
+    qa.rk4_prepare(A, v, 0.01)
     qa.rk4_device(A, v, 0.01, 3)
     assert qa.lib().qh_last_error() == text
     qs.destroy()
