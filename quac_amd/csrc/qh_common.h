@@ -158,6 +158,7 @@ struct qh_mat {
   std::vector<int64_t> blk_off;  // row offsets of the blocks of a block-diagonal matrix (and its row count)
   int comp_state[2] = {0, 0};  // for FP64 and FP32 states: 0 not looked at, 1 plan in comp, -1 not worth it
   qh_comp *comp[2] = {nullptr, nullptr};
+  int64_t comp_seen = 0;  // FP64 steps run on the stage kernels while comp_state is 0
   qh_td_cache *td_cache = nullptr;  // built by the first time-dependent RHS on this matrix
 };
 // variant codes selecting the sliced-ELL kernel: 128 / 129 / 130 process 2 / 4 / 8
@@ -201,12 +202,15 @@ int qh_rk3bs_td_sliced(qh_mat *A, const qh_vec *x, qh_vec *xn, qh_vec *k1, qh_ve
                        qh_vec *y, double h, double atol, double rtol, int have_k1, double *err,
                        const qh_td_ell *td4, int *done);
 
-// RK4 steps of a generator whose rows fall apart into closed sets (qh_comp.hip):
-// *usable = 1 where the plan exists (built on the first call) and beats the stage
-// kernels; nsteps steps of x in place on the library stream; QH_COMP_TRACE doubles
-// of device memory that the trace renormalisation of x may use (kept with the plan)
+// RK4 steps of a generator whose rows fall apart into closed sets (qh_comp.hip).
+// qh_comp_prepare: *usable = 1 where a plan exists that beats the stage kernels; it is
+// built by the call whose nsteps steps, with those that ran before, pay for it (layout:
+// the stage kernels have the layout they need; comp_seen counts steps that ran there), or
+// now where nsteps < 0.  qh_comp_rk4: nsteps steps of x in place on the library stream.
+// qh_comp_trace: QH_COMP_TRACE doubles of device memory that the trace renormalisation
+// of x may use (kept with the plan).
 #define QH_COMP_TRACE 1024
-int qh_comp_prepare(qh_mat *A, int prec, int *usable);
+int qh_comp_prepare(qh_mat *A, int prec, int64_t nsteps, int graph_len, bool layout, int *usable);
 int qh_comp_rk4(qh_mat *A, qh_vec *x, double dt, int64_t nsteps);
 double *qh_comp_trace(const qh_mat *A, int prec);
 

@@ -1181,16 +1181,34 @@ int cp_build(qh_mat *A, int f32) {
   return QH_OK;
 }
 
+// The matrices whose plan was refused, by precision, rows and entries, for the rest of
+// the process, so that of the matrices of a sweep (one structure, other values) one is
+// looked at; the entry decides only the speed.
+struct CpRefused {
+  int prec;
+  int64_t rows, nnz;
+};
+CpRefused g_refused[64];
+unsigned g_nrefused = 0;
+
+bool cp_refused(const qh_mat *A, int prec) {
+  for (unsigned i = 0; i < g_nrefused && i < 64; i++)
+    if (g_refused[i].prec == prec && g_refused[i].rows == A->rows && g_refused[i].nnz == A->nnz) return true;
+  return false;
+}
+
 }  // namespace
 
-int qh_comp_prepare(qh_mat *A, int prec, int *usable) {
+int qh_comp_prepare(qh_mat *A, int prec, int64_t nsteps, int graph_len, bool layout, int *usable) {
   const int f32 = prec == QH_FP32;
   *usable = 0;
-  if (A->comp_state[f32] == 0) {
-    // row and slot numbers are 32-bit
+  if (A->comp_state[f32] == 0 && cp_refused(A, prec)) A->comp_state[f32] = -1;
+  if (A->comp_state[f32] == 0 && (nsteps < 0 || cp_pays(A->rows, A->comp_seen, nsteps, graph_len, layout))) {
     const std::string text = qh_last_error();
+    bool fits = true;
     auto build = [&]() -> int {
       int rc = QH_OK, done = 0;
+      // row and slot numbers are 32-bit
       if (A->rows < 1 || A->rows > (int64_t)1 << 30)
         A->comp_state[f32] = -1;
       else if (A->rows <= CP_SMALL_ROWS)
@@ -1202,9 +1220,11 @@ int qh_comp_prepare(qh_mat *A, int prec, int *usable) {
       (void)hipGetLastError();
       qh_set_error("%s", text.c_str());
       A->comp_state[f32] = -1;  // the stage kernels run without the plan
+      fits = false;
     };
     const int rc = qh_optional(QH_ENOMEM, build, none);
     if (rc) return rc;
+    if (A->comp_state[f32] == -1 && fits) g_refused[g_nrefused++ % 64] = CpRefused{prec, A->rows, A->nnz};
   }
   *usable = A->comp_state[f32] == 1;
   return QH_OK;

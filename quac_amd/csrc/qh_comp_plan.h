@@ -202,6 +202,30 @@ inline CpShapes cp_shapes(const std::vector<CpBin> &bin, bool f32, int cus) {
   return out;
 }
 
+// Time in us that a plan of a matrix of n rows takes to form (one workgroup up to
+// 16 384 rows): measured 55 at 1296 rows, 78 at 4096, 140 at 8464, 200 at 16 384, 258 at
+// 18 496, 370 at 65 536, 1350 at 1 M, 3300 at 4 M; a refused one costs up to that.
+inline double cp_plan_us(int64_t n) {
+  const double r = (double)n;
+  if (n <= 16384) return 45.0 + 0.0105 * r;
+  return 230.0 + 0.0023 * std::min(r, 65536.0) + 0.0008 * std::max(0.0, r - 65536.0);
+}
+
+// Whether a call of nsteps steps forms the plan, seen steps of the matrix having run on
+// the stage kernels: where these steps there would take as long (their part that the
+// plan saves, the captured graph of a call of graph_len steps or more, and the sliced
+// layout where it is still to be built).  So a matrix that is stepped a few times never
+// waits for a plan, and one that is stepped often waits at most twice as long as it must.
+// First call, plan / stage kernels once their variant is known, for 1, 5 and 20 steps:
+// Tavis-Cummings 2^2 x 23 151 / 41, 150 / 90, 166 / 393 us; 2^3 x 17 268 / 51, 283 / 110,
+// 312 / 475 us.
+inline bool cp_pays(int64_t n, int64_t seen, int64_t nsteps, int graph_len, bool layout) {
+  const double step_us = 4.0 * (2.5 + 1.1e-5 * (double)n);
+  const double stage_us = 0.75 * step_us * ((double)seen + (double)nsteps) + (nsteps >= graph_len ? 250.0 : 0.0) +
+                          (layout ? 0.0 : 100.0 + 0.0012 * (double)n);
+  return stage_us >= cp_plan_us(n);
+}
+
 // All launches of a plan: fork() before the first where some run on the side stream,
 // launch(class) each, and join() after them, also when a launch fails: the caller's
 // stream never goes on while the side stream still writes the state.

@@ -1220,6 +1220,22 @@ int lanes_for(qh_mat *A, int prec, int *g) {
   return rc;
 }
 
+// What the FP64 stage kernels of A need before their first launch: nothing, the layout
+// of the chosen variant, or the choice itself
+enum { STAGE_READY = 0, STAGE_LAYOUT = 1, STAGE_CHOICE = 2 };
+int stage_needs(const qh_mat *A) {
+  int g = A->lanes64;
+  for (int i = 0; i < g_ntune && i < 64 && !g; i++)
+    if (g_tune[i].prec == QH_FP64 && g_tune[i].rows == A->rows && g_tune[i].nnz == A->nnz) g = g_tune[i].g;
+  if (!g) return STAGE_CHOICE;
+  return QH_IS_KSELL(g) && A->ks_state == 0 ? STAGE_LAYOUT : STAGE_READY;
+}
+
+// Up to so many rows the few steps of a matrix whose plan does not pay yet run on the
+// CSR kernel with 8 lanes a row without a choice being made, which would time every
+// variant (1.6 to 4 ms)
+#define QH_UNTUNED_ROWS 65536
+
 // ------------------------------------------------------------ trace renorm
 // FP64 trace of a complex64 (hi+lo) density matrix: per-block partial sums,
 // then one block sums them and writes 1/Tr; the scale kernel reads it.
@@ -1805,22 +1821,32 @@ static int rk4_impl(qh_mat *A, qh_vec *x, double dt, int64_t nsteps, int64_t tot
   }
   hipStream_t s = qh_stream();
   // generators that fall apart into small closed sets of rows
+  const int len = graph_len(renorm_every);
+  bool untuned = false;
   if (!timed && !A->lanes_forced) {
     int usable = 0;
-    rc = qh_comp_prepare(A, x->prec, &usable);
+    // (an FP32 state does not wait for the steps that pay for a plan: the plan steps it in
+    // 64 bits, the stage kernels in 32)
+    const int needs = x->prec == QH_FP64 ? stage_needs(A) : STAGE_CHOICE;
+    const bool wait = x->prec == QH_FP64 && (needs != STAGE_CHOICE || A->rows <= QH_UNTUNED_ROWS);
+    rc = qh_comp_prepare(A, x->prec, wait ? nsteps : -1, len, needs != STAGE_LAYOUT, &usable);
     if (rc) return rc;
+    if (wait && A->comp_state[0] == 0) {  // not looked at yet
+      A->comp_seen += nsteps;
+      untuned = needs == STAGE_CHOICE;
+    }
     if (usable) {
-      const int64_t len = renorm_every > 0 ? renorm_every : nsteps;
+      const int64_t run = renorm_every > 0 ? renorm_every : nsteps;
       double *t = qh_comp_trace(A, x->prec);
-      for (int64_t st = 0; st < nsteps && !rc; st += len) {
-        rc = qh_comp_rk4(A, x, dt, std::min<int64_t>(len, nsteps - st));
-        if (!rc && renorm_every > 0 && st + len <= nsteps) rc = renorm_launch(s, x, x->d, tot, 0, t, t + 512);
+      for (int64_t st = 0; st < nsteps && !rc; st += run) {
+        rc = qh_comp_rk4(A, x, dt, std::min<int64_t>(run, nsteps - st));
+        if (!rc && renorm_every > 0 && st + run <= nsteps) rc = renorm_launch(s, x, x->d, tot, 0, t, t + 512);
       }
       return rc;
     }
   }
-  int G = 0;
-  rc = lanes_for(A, x->prec, &G);
+  int G = 8;
+  if (!untuned) rc = lanes_for(A, x->prec, &G);
   if (rc) return rc;
   rc = stepper_prepare(A, x->prec, x->n);
   if (rc) return rc;
@@ -1850,7 +1876,6 @@ static int rk4_impl(qh_mat *A, qh_vec *x, double dt, int64_t nsteps, int64_t tot
   }
 
   // graph path: capture len steps once, replay
-  const int len = graph_len(renorm_every);
   const int64_t full = nsteps / len;
   if (full > 0) {
     rc = graph_prepare(A, x, dt, tot, renorm_every, G, len);
@@ -1888,7 +1913,7 @@ extern "C" int qh_rk4_prepare(qh_mat *A, qh_vec *x, double dt, int64_t tot, int 
   if (A->rows <= QH_SMALL_ROWS && !A->lanes_forced) return QH_OK;  // one-workgroup path: nothing to capture
   if (!A->lanes_forced) {
     int usable = 0;
-    rc = qh_comp_prepare(A, x->prec, &usable);
+    rc = qh_comp_prepare(A, x->prec, -1, 0, true, &usable);
     if (rc || usable) return rc;
   }
   int G = 0;

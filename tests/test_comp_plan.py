@@ -123,6 +123,29 @@ int main() {
     assert out == "ok\n"
 
 
+def test_plan_waits_for_the_steps_that_pay_for_it(run):
+    """few steps never wait for a plan, a graph's worth of them on a small matrix does,
+    and steps in several calls count together"""
+    out = run("pays", CHECK + r"""
+int main() {
+  for (int64_t n : {801, 1296, 4096, 8464, 16384, 16385, 57600, 65536}) {
+    NEED(!cp_pays(n, 0, 0, 8, true) && !cp_pays(n, 0, 1, 8, true) && !cp_pays(n, 0, 4, 8, true));
+    NEED(cp_pays(n, 0, 20, 8, true) && cp_pays(n, 0, 100, 8, true));
+    int64_t k = 0;
+    while (!cp_pays(n, k, 1, 8, true)) k++;
+    NEED(k >= 4 && k <= 40);
+    NEED(!cp_pays(n, 0, k, 1000, true) && cp_pays(n, 0, k + 1, 1000, true));
+    for (int64_t s = 1; s < 100; s++) NEED(cp_pays(n, s, 5, 8, true) || !cp_pays(n, s - 1, 5, 8, true));
+    NEED(!cp_pays(n, 3, 2, 8, true) || cp_pays(n, 3, 2, 8, false));
+  }
+  // 16 M rows: ten steps with the layout still to be built
+  NEED(cp_pays(16777216, 0, 10, 8, false) && !cp_pays(16777216, 0, 10, 8, true));
+  printf("ok\n");
+}
+""")
+    assert out == "ok\n"
+
+
 def test_side_stream_is_joined_when_a_launch_fails(run):
     """the order of fork, launches and join for every launch that may fail"""
     out = run("order", CHECK + r"""

@@ -262,3 +262,55 @@ def test_short_calls_step_the_same_state(recipe, prec):
     tol = 5 * np.abs(x0).max() * (2 * dt * norm + 8) * (2.0 ** -53 if prec == qa.FP64 else 2.0 ** -47)
     assert np.abs(_steps(A, x0, prec, dt, 5) - ref).max() <= tol + (2.0 ** -47 if prec == qa.FP32 else 0.0)
     qs.destroy()
+
+
+@pytest.mark.parametrize("prec", [qa.FP64, qa.FP32])
+def test_plan_is_formed_when_it_pays(prec):
+    """a few FP64 steps run without a plan and without a choice of variant; the plan
+    follows when as many steps have run, and the state goes on from where it is; an FP32
+    state has its plan, which steps it in 64 bits, at once"""
+    recipe, dt = _tc(2, 13), 0.02
+    qs, _, _ = build_system(recipe)
+    A, n = qs.matrix(), qs.total_levels
+    x0 = _start(n)
+    tot, terms = recipes.oracle_terms(recipe)
+    m = oracle.construct(tot, terms, dm=True)
+    rp, _, val = A.export()
+    norm = np.add.reduceat(np.abs(val), rp[:-1]).max()
+    v = qa.DeviceVec(len(x0), prec)
+    v.set(x0)
+    formed = 0
+    for k in range(1, 41):
+        qa.rk4_device(A, v, dt, 1)
+        if not formed and A.closed_info(prec)["bins"]:
+            formed = k
+        if k in (1, 3, 40):
+            # a few roundings of the state and of h A times it a step
+            eps = 2.0 ** -53 if prec == qa.FP64 else 2.0 ** -47
+            assert np.abs(v.get() - m.rk4(x0, dt, k)).max() <= (k + 1) * np.abs(x0).max() * (2 * dt * norm + 8) * eps, k
+    assert (3 <= formed <= 20 if prec == qa.FP64 else formed == 1) and A.lanes() == (0, 0)
+    B, _, _ = build_system(recipe)
+    v.set(x0)
+    qa.rk4_device(B.matrix(), v, dt, 40)  # enough steps in one call
+    assert B.matrix().closed_info(prec)["bins"] > 0
+    for s in (qs, B):
+        s.destroy()
+
+
+def test_refused_plan_is_looked_at_once():
+    """one set of 4096 rows: the stage kernels step it, the second matrix of the size
+    without another look"""
+    recipe = _noisy(6, [("ham", 0.3 + 0.1 * i, [(i, "sx")]) for i in range(6)])
+    x0, dt = _start(64), 0.01
+    tot, terms = recipes.oracle_terms(recipe)
+    m = oracle.construct(tot, terms, dm=True)
+    for steps in (60, 3):
+        qs, _, _ = build_system(recipe)
+        v = qa.DeviceVec(len(x0), qa.FP64)
+        v.set(x0)
+        qa.rk4_device(qs.matrix(), v, dt, steps)
+        assert qs.matrix().closed_info()["bins"] == 0 and qs.matrix().lanes()[0] != 0
+        rp, _, val = qs.matrix().export()
+        norm = np.add.reduceat(np.abs(val), rp[:-1]).max()
+        assert np.abs(v.get() - m.rk4(x0, dt, steps)).max() <= steps * np.abs(x0).max() * (2 * dt * norm + 8) * 2.0 ** -53
+        qs.destroy()
