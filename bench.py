@@ -61,16 +61,17 @@ def rk4_step_bytes(nnz, rows, S):
 
 def kernel_name(variant, real):
     """name of the stage kernel a lanes-per-row variant code selects"""
-    if 128 <= variant <= 136:
-        u, vv, pp, nt = {128: (2, 0, 0, 0), 129: (4, 0, 0, 0), 130: (8, 0, 0, 0), 131: (4, 1, 0, 0),
-                         132: (8, 1, 0, 0), 133: (2, 0, 1, 0), 134: (4, 0, 1, 0), 135: (4, 0, 0, 1),
-                         136: (4, 1, 0, 1)}[variant]
+    if 128 <= variant <= 138:
+        u, vv, pp, rl, nt = {128: (2, 0, 0, 0, 0), 129: (4, 0, 0, 0, 0), 130: (8, 0, 0, 0, 0), 131: (4, 1, 0, 0, 0),
+                             132: (8, 1, 0, 0, 0), 133: (2, 0, 1, 0, 0), 134: (4, 0, 1, 0, 0), 135: (4, 0, 0, 0, 1),
+                             136: (4, 1, 0, 0, 1), 137: (2, 0, 1, 1, 0), 138: (4, 0, 1, 1, 0)}[variant]
         tf = ("false", "true")
-        return f"k_ks_stage<{real}, MODE, {u}, {tf[vv]}, {tf[pp]}, {tf[nt]}> (sliced layout)"
-    if variant in (140, 141, 142, 143, 144):
-        u, w, nt = {140: (2, "false", "false"), 141: (4, "false", "false"), 142: (2, "true", "false"),
-                    143: (2, "false", "true"), 144: (2, "true", "true")}[variant]
-        return f"k_ks2_stage<MODE, {u}, {w}, {nt}> (row-pair sliced layout)"
+        return f"k_ks_stage<{real}, MODE, {u}, {tf[vv]}, {tf[pp]}, {tf[rl]}, {tf[nt]}> (sliced layout)"
+    if 140 <= variant <= 146:
+        u, w, nt, rl = {140: (2, 0, 0, 0), 141: (4, 0, 0, 0), 142: (2, 1, 0, 0), 143: (2, 0, 1, 0), 144: (2, 1, 1, 0),
+                        145: (2, 0, 0, 1), 146: (2, 0, 1, 1)}[variant]
+        tf = ("false", "true")
+        return f"k_ks2_stage<MODE, {u}, {tf[w]}, {tf[nt]}, SEP, TDP, {tf[rl]}> (row-pair sliced layout)"
     return f"k_rk_stage<{real}, {variant}> (CSR, {variant} lanes per row)"
 
 
@@ -93,7 +94,7 @@ def format_step_bytes(A, rows):
     words, K1..K3, and the new high and low words written); and the layout
     statistics"""
     lanes = A.lanes()
-    if lanes[1] in (140, 141, 142, 143, 144):  # row-pair layout: 40-byte slot metadata, values per lane pair
+    if 140 <= lanes[1] <= 146:  # row-pair layout: 40-byte slot metadata, values per lane pair
         layout = dict(A.pair_layout_info(), kind="row-pair (128 rows per wavefront)")
         meta = layout["meta_bytes"]
         vals = layout["stored_pairs"] * 16 + layout["stored_real_pairs"] * 8 + layout["stored_real_singles"] * 4

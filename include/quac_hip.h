@@ -72,14 +72,16 @@ int qh_mat_make_fp32(qh_mat *m);
 /* block-diagonal concatenation of n matrices (batched parameter sweeps) */
 int qh_mat_blockdiag(int n, qh_mat *const *mats, qh_mat **out);
 /* select SpMV variant: lanes per row G in {1,2,4,8,16,32,64} of the CSR kernel,
- * 128..136 = slot-aligned sliced ELL (one wavefront per 64 rows; 2/4/8 slots per
+ * 128..138 = slot-aligned sliced ELL (one wavefront per 64 rows; 2/4/8 slots per
  * pass, 131/132 with vector-loaded uniform values, 133/134 with 2/4 slots per pass
  * and the next pass's loads in flight, 135/136 = 129/131 with the streamed data
- * under the non-temporal cache policy); FP32 only: 140/141/142 = row-pair sliced
+ * under the non-temporal cache policy, 137/138 = 133/134 with a slice's slot
+ * metadata in registers); FP32 only: 140/141/142 = row-pair sliced
  * layout (one wavefront per 128 rows, two rows per lane, 16-byte loads; 2/4/2
  * slots per pass, 142 reading the slots that stay inside each 2048-row window
  * from an LDS copy; 143/144 = 140/142 with the streamed data under the
- * non-temporal cache policy); 0 = autotune */
+ * non-temporal cache policy; 145/146 = 140/143 with a slice's slot metadata in
+ * registers); 0 = autotune */
 int qh_mat_set_lanes(qh_mat *m, int lanes64, int lanes32);
 int qh_mat_get_lanes(const qh_mat *m, int *lanes64, int *lanes32);
 /* sliced layout statistics (built on demand): slices, slots, stored complex
@@ -173,7 +175,7 @@ int qh_rk4_td_steps(qh_mat *A, int ntd, qh_mat *const *Ak, const double *s_re_im
  * 4096, at most 8192; applies from the next merged build), sliced = 1 runs A's
  * part on its sliced layout where it has one (default), 0 the fused CSR kernel;
  * lanes = how the A_k entries join a sliced stage: 0 = summed inside A's stage
- * kernel where its variant allows (128, 134, 136, 140, 142, 143), else as 1; 1 = a
+ * kernel where its variant allows (128, 134, 136, 138, 140, 142, 143, 145, 146), else as 1; 1 = a
  * pass of their own, one thread per row over the sliced (64-row, entry-major)
  * form of the dictionary entries; 4, 8, 16 = a pass with that many lanes per row
  * over their CSR (0 and 1 fall back to 4 or 8 lanes, by the rows' average
@@ -197,7 +199,7 @@ int qh_rk3bs_step(qh_mat *A, const qh_vec *x, qh_vec *xn, qh_vec *k1, qh_vec *k2
  * integrator of time_step_sys with time-dependent terms, qsystem.c:1003-1005,
  * 1288-1330): s4_re_im holds the coefficients of the stage times t, t + h/2,
  * t + 3h/4, t + h (4 x ntd complex; the first unused when have_k1).  Where A has
- * a one-row sliced FP64 variant (128, 134, 136) the merged entries are summed in
+ * a one-row sliced FP64 variant (128, 134, 136, 138) the merged entries are summed in
  * the four stage launches of qh_rk3bs_step; otherwise four qh_spmv_td
  * evaluations and the combinations. */
 int qh_rk3bs_td_step(qh_mat *A, int ntd, qh_mat *const *Ak, const double *s4_re_im, const qh_vec *x, qh_vec *xn,

@@ -164,15 +164,16 @@ struct qh_mat {
 // variant codes selecting the sliced-ELL kernel: 128 / 129 / 130 process 2 / 4 / 8
 // slots per pass; 131 / 132 process 4 / 8 slots per pass and read the uniform
 // slot values with vector loads; 133 / 134 process 2 / 4 slots per pass with the
-// loads of the next pass in flight during the products of the current one and the
-// slice's metadata in registers (slices of at most 64 slots)
+// loads of the next pass in flight during the products of the current one
 #define QH_KSELL 128
 // 135 / 136: 129 / 131 with the streamed data under the non-temporal cache policy
-#define QH_IS_KSELL(g) ((g) >= 128 && (g) <= 136)
+// 137 / 138: 133 / 134 with the slice's metadata in registers (at most 64 slots a slice)
+#define QH_IS_KSELL(g) ((g) >= 128 && (g) <= 138)
 // 140 / 141: the FP32 row-pair sliced layout, 2 / 4 slots per pass (pipelined);
 // 142: 2 slots per pass, the slots inside each 2048-row window read from LDS;
 // 143 / 144: 140 / 142 with the streamed data under the non-temporal cache policy
-#define QH_IS_KS2(g) ((g) >= 140 && (g) <= 144)
+// 145 / 146: 140 / 143 with the slice's metadata in registers
+#define QH_IS_KS2(g) ((g) >= 140 && (g) <= 146)
 
 struct qh_vec {
   int64_t n = 0;
@@ -200,7 +201,7 @@ int ks2_launch(int G, int mode, hipStream_t s, const qh_mat *A, const void *xin,
 // launched (*done = 0)
 int qh_rk3bs_td_sliced(qh_mat *A, const qh_vec *x, qh_vec *xn, qh_vec *k1, qh_vec *k2, qh_vec *k3, qh_vec *k4,
                        qh_vec *y, double h, double atol, double rtol, int have_k1, double *err,
-                       const qh_td_ell *td4, int *done);
+                       int G, const qh_td_ell *td4, int *done);
 
 // RK4 steps of a generator whose rows fall apart into closed sets (qh_comp.hip).
 // qh_comp_prepare: *usable = 1 where a plan exists that beats the stage kernels; it is
@@ -226,7 +227,7 @@ struct qh_td_ell {
   const int32_t *col;
   const uint16_t *idx;
   const double2 *cf;
-  // variant 134, FP64: entries that every row of a uniform slot of A has in the same
+  // variant 138, FP64: entries that every row of a uniform slot of A has in the same
   // place and with the same value are not in the lists but added to the slot's value:
   // their dictionary index per slot of A (-1: none), and the dictionary's size (at
   // most 64); null: all entries are in the lists
@@ -237,7 +238,7 @@ struct qh_td_ell {
 // A's part of the time-dependent RK stages on A's autotuned variant when that is
 // a sliced layout (qh_spmv.hip): *G = the variant, or 0 where A runs on its CSR
 // (a generator of at most 800 rows, or a CSR variant chosen)
-int qh_td_sliced_prepare(qh_mat *A, int prec, int *G);
+int qh_td_sliced_prepare(qh_mat *A, int prec, bool fuse, int *G);
 // one stage of y' = A y on variant G: mode 0 kout = A xin; 1 also ynext = x +
 // cn kout; 2 xout = x + h/6 (k1 + 2 k2 + 2 k3 + A xin) (x and the low word xlo of
 // an FP32 state may be updated in place, xout = x)

@@ -1022,7 +1022,8 @@ int ks2_build(qh_mat *A) {
 
 // One stage launch on the row-pair layout (G = 140 / 141: 2 / 4 slots per pass;
 // 142: 2 slots per pass, window slots read from LDS; 143 / 144: 140 / 142 with
-// the non-temporal cache policy on the streamed data);
+// the non-temporal cache policy on the streamed data; 145 / 146: 140 / 143 with
+// the slice's metadata in registers);
 // mode as in the one-row-per-lane kernels.
 int ks2_launch(int G, int mode, hipStream_t s, const qh_mat *A, const void *xin, void *kout, void *ynext, double cn,
                const void *x, const void *k1, const void *k2, const void *k3, void *xout, double h, float2 *xlo,
@@ -1057,10 +1058,9 @@ int ks2_launch(int G, int mode, hipStream_t s, const qh_mat *A, const void *xin,
     qh_set_error("unsupported row-pair variant %d / mode %d", G, mode);
     return QH_EINVAL;
   }
-  // a slice of more than 64 slots: the metadata read from memory slot by slot
-  const int QH_KS2_LONG = 0;
-  if (A->ks2_maxslots > 64 && !win && !(td && G == 141)) G = QH_KS2_LONG;
-  if (td) {  // the time-dependent entries summed in the same kernel (variants 140, 142, 143)
+  // metadata in registers: one slot a lane
+  if (A->ks2_maxslots > 64) G = G == 145 ? 140 : G == 146 ? 143 : G;
+  if (td) {  // the time-dependent entries summed in the same kernel (variants 140, 142, 143, 145, 146)
 #define QH_LK2D(MM, UU, WW, NN, RR)                                                             \
   do {                                                                                      \
     if (A->ks2_nsep)                                                                        \
@@ -1070,10 +1070,11 @@ int ks2_launch(int G, int mode, hipStream_t s, const qh_mat *A, const void *xin,
   } while (0)
 #define QH_LK2DG(MM)                                                                        \
   switch (G) {                                                                              \
-    case QH_KS2_LONG: QH_LK2D(MM, 2, false, false, false); break;                           \
-    case 140: QH_LK2D(MM, 2, false, false, true); break;                                    \
+    case 140: QH_LK2D(MM, 2, false, false, false); break;                                   \
     case 142: QH_LK2D(MM, 2, true, false, false); break;                                    \
-    case 143: QH_LK2D(MM, 2, false, true, true); break;                                     \
+    case 143: QH_LK2D(MM, 2, false, true, false); break;                                    \
+    case 145: QH_LK2D(MM, 2, false, false, true); break;                                    \
+    case 146: QH_LK2D(MM, 2, false, true, true); break;                                     \
     default:                                                                                \
       qh_set_error("row-pair variant %d has no time-dependent form", G);                    \
       return QH_EINVAL;                                                                     \
@@ -1089,13 +1090,14 @@ int ks2_launch(int G, int mode, hipStream_t s, const qh_mat *A, const void *xin,
 #undef QH_LK2D
     return QH_OK;
   }
-#define QH_LK2G(MM)                      \
-  switch (G) {                           \
-    case QH_KS2_LONG: QH_LK2(MM, 2, false, false, false); break; \
-    case 140: QH_LK2(MM, 2, false, false, true); break; \
-    case 141: QH_LK2(MM, 4, false, false, true); break; \
+#define QH_LK2G(MM)                                      \
+  switch (G) {                                           \
+    case 140: QH_LK2(MM, 2, false, false, false); break; \
+    case 141: QH_LK2(MM, 4, false, false, false); break; \
     case 142: QH_LK2(MM, 2, true, false, false); break;  \
-    case 143: QH_LK2(MM, 2, false, true, true); break;  \
+    case 143: QH_LK2(MM, 2, false, true, false); break;  \
+    case 145: QH_LK2(MM, 2, false, false, true); break;  \
+    case 146: QH_LK2(MM, 2, false, true, true); break;   \
     default: QH_LK2(MM, 2, true, true, false); break;    \
   }
   if (mode == MODE_SPMV) {

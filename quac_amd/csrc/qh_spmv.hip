@@ -520,7 +520,8 @@ __device__ inline void st_nt(typename C2<R>::T *p, int64_t r, typename C2<R>::T 
 // the next stage input keep the default one)
 // TDP: the row also sums its merged A_k entries of a time-dependent RHS (the
 // sliced form over the same 64-row slices), before the epilogue
-template <typename R, int MODE, int U, bool VV, bool PIPE, bool NT = false, bool TDP = false>
+// RL: the slice's metadata in registers (at most 64 slots)
+template <typename R, int MODE, int U, bool VV, bool PIPE, bool RL, bool NT, bool TDP>
 __global__ void __launch_bounds__(256) k_ks_stage(
     int32_t nrows, int32_t nslices, const int32_t *__restrict__ moff, const int32_t *__restrict__ umid,
     const int32_t *__restrict__ cmid, const qh_kmeta *__restrict__ meta, const qh_kmeta32 *__restrict__ meta32,
@@ -544,9 +545,6 @@ __global__ void __launch_bounds__(256) k_ks_stage(
   const uint32_t r8 = (uint32_t)r * (uint32_t)sizeof(T);
   KsAcc acc{0.0, 0.0};
   constexpr int AUX = NT ? 2 : 0;
-  // the pipelined kernels hold the slice's metadata in registers (at most 64
-  // slots: launch_ks chooses another kernel beyond)
-  constexpr bool RL = PIPE;
   if constexpr (sizeof(R) == 4 && !VV && MODE != MODE_LAST) {
     KsRegs<qh_kmeta32> regs;
     if (RL) regs.load(meta32 + k0, kend - k0, lane);
@@ -972,22 +970,24 @@ int launch_ks(int G, hipStream_t s, const qh_mat *A, const void *xin, void *kout
   const dim3 grid(qh_blocks(A->nslices, 4)), blk(256);
   const int32_t n = (int32_t)A->rows, ns = A->nslices;
   const qh_td_ell none{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0};
-  // the pipelined kernels hold a slice's metadata in registers, one slot a lane
-  if (A->ks_maxslots > 64) G = G == 133 ? 128 : G == 134 ? (td ? 128 : 129) : G;
-#define QH_LKT(UU, VV, PP, NN, TT, TD)                                                                             \
-  hipLaunchKernelGGL((k_ks_stage<R, MODE, UU, VV, PP, NN, TT>), grid, blk, 0, s, n, ns, A->ks_moff, A->ks_umid,     \
+  // metadata in registers: one slot a lane
+  if (A->ks_maxslots > 64) G = G == 137 ? 133 : G == 138 ? 134 : G;
+#define QH_LKT(UU, VV, PP, RR, NN, TT, TD)                                                                         \
+  hipLaunchKernelGGL((k_ks_stage<R, MODE, UU, VV, PP, RR, NN, TT>), grid, blk, 0, s, n, ns, A->ks_moff, A->ks_umid,     \
                      A->ks_cmid,                                                                              \
                      A->ks_meta, A->ks_meta32, (int32_t)(A->ks_slots + QH_KS_PAD), (int32_t)A->ks_nval, kv,    \
                      (int32_t)A->ks_nsval, sv, (const T *)xin, (T *)kout, (T *)ynext, cn, (const T *)x,       \
                      (const T *)k1, (const T *)k2, (const T *)k3, (T *)xout, h, xlo, atol, rtol, eacc, TD)
-#define QH_LK(UU, VV, PP, NN) QH_LKT(UU, VV, PP, NN, false, none)
+#define QH_LK(UU, VV, PP, NN) QH_LKT(UU, VV, PP, false, NN, false, none)
+#define QH_LKR(UU) QH_LKT(UU, false, true, true, false, false, none)
   if constexpr (MODE == MODE_SPMV || MODE == MODE_STAGE || MODE == MODE_FINAL ||
                 ((MODE == MODE_BS3 || MODE == MODE_BS3E) && sizeof(R) == 8)) {
-    if (td) {  // the time-dependent entries summed in the same kernel (variants 128, 134, 136)
+    if (td) {  // the time-dependent entries summed in the same kernel (variants 128, 134, 136, 138)
       switch (G) {
-        case 128: QH_LKT(2, false, false, false, true, *td); return QH_OK;
-        case 134: QH_LKT(4, false, true, false, true, *td); return QH_OK;
-        case 136: QH_LKT(4, true, false, true, true, *td); return QH_OK;
+        case 128: QH_LKT(2, false, false, false, false, true, *td); return QH_OK;
+        case 134: QH_LKT(4, false, true, false, false, true, *td); return QH_OK;
+        case 136: QH_LKT(4, true, false, false, true, true, *td); return QH_OK;
+        case 138: QH_LKT(4, false, true, true, false, true, *td); return QH_OK;
         default:
           qh_set_error("variant %d has no time-dependent form", G);
           return QH_EINVAL;
@@ -1007,11 +1007,14 @@ int launch_ks(int G, hipStream_t s, const qh_mat *A, const void *xin, void *kout
     case 134: QH_LK(4, false, true, false); break;
     case 135: QH_LK(4, false, false, true); break;
     case 136: QH_LK(4, true, false, true); break;
+    case 137: QH_LKR(2); break;
+    case 138: QH_LKR(4); break;
     default:
       qh_set_error("unsupported sliced-layout variant %d", G);
       return QH_EINVAL;
   }
 #undef QH_LK
+#undef QH_LKR
 #undef QH_LKT
   return QH_OK;
 }
@@ -1089,6 +1092,7 @@ int rk4_step(hipStream_t s, const qh_mat *A, int G, void *x, float2 *xlo, void *
 }
 
 // ------------------------------------------------------------ autotuner
+#define QH_REGMETA_ROWS (1 << 17)
 // Time each variant (CSR lanes per row, sliced layouts) on the real matrix with
 // whole RK4 steps (the stage epilogues' vector traffic and registers are part of
 // what the stepping runs) and keep the fastest.
@@ -1127,13 +1131,20 @@ int autotune(qh_mat *A, int *out_g) {
     int brc = ks_build(A);
     if (!brc && A->ks_state == 1 && sizeof(R) == 4) brc = ks_make_fp32(A);
     if (brc) return brc;
+    // the metadata in registers pays where it streams (variants 137, 138, 145, 146; FP64
+    // a stage: 10-qubit chain 28.7 -> 24.7 us, 9-qubit chain 7.8 -> 8.7 us, 8-qubit chain
+    // 4.70 -> 4.92 us; FP32: 11-qubit chain 82.7 -> 88.5 us, 12-qubit circuit 154 -> 140
+    // us), so it is tried on large matrices, in FP32 on the row-pair layout only; there
+    // 130 and 132 (8 slots a pass), never the fastest of those measured, make room
+    const bool large = A->rows >= QH_REGMETA_ROWS;
     if (A->ks_state == 1)
-      for (int u = 128; u <= 136; u++) cands.push_back(u);
+      for (int u = 128; u <= (large && sizeof(R) == 8 ? 138 : 136); u++)
+        if (!(large && (u == 130 || u == 132))) cands.push_back(u);
     if (sizeof(R) == 4) {
       brc = ks2_build(A);
       if (brc) return brc;
       if (A->ks2_state == 1)
-        for (int u = 140; u <= 144; u++) cands.push_back(u);
+        for (int u = 140; u <= (large ? 146 : 144); u++) cands.push_back(u);
     }
   }
   // the CSR kernels only when no sliced layout exists or the matrix is small:
@@ -1930,7 +1941,7 @@ extern "C" int qh_mat_set_lanes(qh_mat *m, int l64, int l32) {
     return g == 0 || g == 1 || g == 2 || g == 4 || g == 8 || g == 16 || g == 32 || g == 64 || QH_IS_KSELL(g);
   };
   QH_REQUIRE(ok(l64) && (ok(l32) || QH_IS_KS2(l32)), QH_EINVAL,
-             "lanes per row must be a power of two <= 64, 128..136 (sliced layout), or for FP32 140..144 (row-pair "
+             "lanes per row must be a power of two <= 64, 128..138 (sliced layout), or for FP32 140..146 (row-pair "
              "sliced layout)");
   m->lanes64 = l64;
   m->lanes32 = l32;
@@ -2180,14 +2191,11 @@ extern "C" int qh_rk3bs_step(qh_mat *A, const qh_vec *x, qh_vec *xn, qh_vec *k1,
 
 int qh_rk3bs_td_sliced(qh_mat *A, const qh_vec *x, qh_vec *xn, qh_vec *k1, qh_vec *k2, qh_vec *k3, qh_vec *k4,
                        qh_vec *y, double h, double atol, double rtol, int have_k1, double *err,
-                       const qh_td_ell *td4, int *done) {
+                       int G, const qh_td_ell *td4, int *done) {
   *done = 0;
   int rc = rk3bs_check(A, x, xn, k1, k2, k3, k4, y, err, "qh_rk3bs_td_step");
   if (rc) return rc;
-  int G = 0;
-  rc = qh_td_sliced_prepare(A, QH_FP64, &G);
-  if (rc) return rc;
-  if (!(G == 128 || G == 134 || G == 136) || A->ks_state != 1) return QH_OK;
+  if (!(G == 128 || G == 134 || G == 136 || G == 138) || A->ks_state != 1) return QH_OK;
   *done = 1;
   return rk3bs_ks(G, A, x, xn, k1, k2, k3, k4, y, h, atol, rtol, have_k1, err, td4);
 }
@@ -2434,19 +2442,21 @@ extern "C" qh_mat *qh_batch_matrix(qh_batch *b) { return b ? b->A : nullptr; }
 extern "C" int64_t qh_batch_offset(qh_batch *b, int i) { return (b && i >= 0 && i < b->n) ? b->off[i] : -1; }
 
 // ------------------------------------------------------------ time-dependent stages
-int qh_td_sliced_prepare(qh_mat *A, int prec, int *G) {
+int qh_td_sliced_prepare(qh_mat *A, int prec, bool fuse, int *G) {
   *G = 0;
   if (A->rows <= QH_SMALL_ROWS && !A->lanes_forced) return QH_OK;
   int g = 0;
   const int rc = lanes_for(A, prec, &g);
   if (rc) return rc;
-  // the autotuner's choice holds for A alone; the same layout is read by the
-  // variant that sums the A_k entries in A's kernel, which saves the pass of their
-  // own (10-qubit chain, three drives, FP64: 37 us a stage against 55 us; 31.6 us where
-  // A's slots take them over)
-  if (!A->lanes_forced) {
+  // The autotuner's choice holds for A alone; where the A_k entries can be summed in A's
+  // kernel (fuse), the variant of the same layout that does so saves the pass of their own.
+  // Ten steps with three drives, own pass -> summed: chain of 10 qubits FP64 2270 -> 1370
+  // us (A's slots taking the drives over), 9 qubits FP32 617 -> 460 us, decay and dephasing
+  // of 10 qubits FP64 1910 -> 975 us; three 6-level cavities 300 -> 310 us.
+  if (fuse && !A->lanes_forced) {
     if (g == 135) g = 136;
-    else if (QH_IS_KSELL(g) && g != 128 && g != 136) g = 134;
+    else if (g == 137) g = 138;
+    else if (QH_IS_KSELL(g) && g != 128 && g != 136 && g != 138) g = 134;
     else if (g == 141) g = 140;
     else if (g == 144) g = 142;
   }
@@ -2460,10 +2470,10 @@ int qh_td_sliced_stage(int G, const qh_mat *A, int prec, int mode, const void *x
   hipStream_t s = qh_stream();
   *fused = 0;
   int rc;
-  if (td && prec == QH_FP32 && (G == 140 || G == 142 || G == 143) && A->ks2_state == 1) {
+  if (td && prec == QH_FP32 && QH_IS_KS2(G) && G != 141 && G != 144 && A->ks2_state == 1) {
     *fused = 1;
     rc = ks2_launch(G, mode, s, A, xin, kout, ynext, cn, x, k1, k2, k3, xout, h, xlo, td);
-  } else if (td && (G == 128 || G == 134 || G == 136) && A->ks_state == 1) {
+  } else if (td && (G == 128 || G == 134 || G == 136 || G == 138) && A->ks_state == 1) {
     *fused = 1;
 #define QH_TF(R, M) \
   launch_ks<R, M>(G, s, A, xin, kout, ynext, cn, x, k1, k2, k3, xout, h, xlo, 0.0, 0.0, nullptr, td)

@@ -761,7 +761,7 @@ __global__ void __launch_bounds__(64) k_td_fold(int64_t nrows, const int32_t *__
   }
 }
 
-// builds the lists for variant 134 of A's sliced layout, once per cache (without the
+// builds the lists for variant 138 of A's sliced layout, once per cache (without the
 // memory for them all entries stay in the full lists)
 static int td_fold(const qh_mat *A, qh_td_cache *c) {
   if (c->fold_state) return QH_OK;
@@ -814,7 +814,7 @@ static int td_fold(const qh_mat *A, qh_td_cache *c) {
 // same pass (lanes 0: wherever A's variant has that form), or null
 static const qh_td_ell *td_fusable(const qh_td_cache *c, int G, int prec, const double2 *cf, qh_td_ell *buf) {
   if (!c->soff || g_td_lanes != 0) return nullptr;
-  if (G == 134 && prec == QH_FP64 && c->fold_state == 1)
+  if (G == 138 && prec == QH_FP64 && c->fold_state == 1)
     *buf = qh_td_ell{c->soff, c->fw, c->fcol, c->fidx, cf, c->fslot, (int32_t)c->dv.size()};
   else
     *buf = qh_td_ell{c->soff, c->sw, c->ecol, c->eidx, cf, nullptr, 0};
@@ -833,6 +833,15 @@ extern "C" int qh_td_config(int dict_max, int sliced, int lanes) {
   return QH_OK;
 }
 
+// the variant of A's stages: where its slots take entries over, the one that adds them
+static int td_variant(qh_mat *A, qh_td_cache *c, int prec, int *G) {
+  int rc = qh_td_sliced_prepare(A, prec, c->soff && g_td_lanes == 0, G);
+  if (rc || prec != QH_FP64 || g_td_lanes != 0 || (*G != 134 && *G != 138)) return rc;
+  rc = td_fold(A, c);
+  if (c->fold_state == 1) *G = 138;
+  return rc;
+}
+
 extern "C" int qh_spmv_td(const qh_mat *A, int ntd, qh_mat *const *Ak, const double *s_re_im, const qh_vec *x,
                           qh_vec *y) {
   int rc = qh_ensure_init();
@@ -848,8 +857,7 @@ extern "C" int qh_spmv_td(const qh_mat *A, int ntd, qh_mat *const *Ak, const dou
   if (rc) return rc;
   int G = 0;
   if (g_td_sliced) {
-    rc = qh_td_sliced_prepare(Am, x->prec, &G);
-    if (!rc && G == 134 && x->prec == QH_FP64) rc = td_fold(A, c);
+    rc = td_variant(Am, c, x->prec, &G);
     if (rc) return rc;
   }
   std::vector<double2> hs((size_t)c->stride() + 1);
@@ -881,8 +889,7 @@ extern "C" int qh_rk4_td_step(qh_mat *A, int ntd, qh_mat *const *Ak, const doubl
   if (rc) return rc;
   int G = 0;
   if (g_td_sliced) {
-    rc = qh_td_sliced_prepare(A, x->prec, &G);
-    if (!rc && G == 134 && x->prec == QH_FP64) rc = td_fold(A, c);
+    rc = td_variant(A, c, x->prec, &G);
     if (rc) return rc;
   }
   if (c->prec != x->prec) {
@@ -953,8 +960,7 @@ extern "C" int qh_rk3bs_td_step(qh_mat *A, int ntd, qh_mat *const *Ak, const dou
   if (g_td_sliced && c->soff && g_td_lanes == 0) {
     // the four stage tables in one upload, the entries summed in A's stage kernels
     int G = 0;
-    rc = qh_td_sliced_prepare(A, x->prec, &G);
-    if (!rc && G == 134) rc = td_fold(A, c);
+    rc = td_variant(A, c, x->prec, &G);
     if (rc) return rc;
     const int st = c->stride();
     std::vector<double2> hs((size_t)4 * st);
@@ -963,7 +969,7 @@ extern "C" int qh_rk3bs_td_step(qh_mat *A, int ntd, qh_mat *const *Ak, const dou
     qh_td_ell t4[4];
     for (int j = 0; j < 4; j++) td_fusable(c, G, x->prec, c->s + (size_t)j * st, &t4[j]);
     int done = 0;
-    rc = qh_rk3bs_td_sliced(A, x, xn, k1, k2, k3, k4, y, h, atol, rtol, have_k1, err, t4, &done);
+    rc = qh_rk3bs_td_sliced(A, x, xn, k1, k2, k3, k4, y, h, atol, rtol, have_k1, err, G, t4, &done);
     if (rc || done) return rc;
   }
   // four RHS evaluations and the combinations

@@ -59,3 +59,9 @@ def test_committed_traffic_summary_is_read():
 def test_kernel_names_cover_every_variant_code():
     for g in list(range(128, 137)) + list(range(140, 145)):
         assert "stage" in bench.kernel_name(g, "float")
+
+
+def test_kernel_names_of_metadata_in_registers():
+    for g in (137, 138, 145, 146):
+        assert "stage" in bench.kernel_name(g, "float") and bench.kernel_name(g, "float") != bench.kernel_name(
+            {137: 133, 138: 134, 145: 140, 146: 143}[g], "float")

@@ -2,6 +2,8 @@
 y = x + c A y', qh_spmv.hip / qh_ks2.hip) on every kernel variant, at row counts
 with a remainder in each tile (64-row and 128-row slices, 2048-row windows, an odd
 last row), against the oracle's classic RK4 in FP64."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -58,3 +60,44 @@ def test_nested_rk4_matches_oracle(dims, lanes):
         assert np.abs(v.get() - ref).max() <= tol, (lanes, prec)
     A.set_lanes(0, 0)
     qs.destroy()
+
+
+@pytest.mark.parametrize("dims", [(2, 4, 4), (7, 7)])
+@pytest.mark.parametrize("lanes", [129, 131, 133, 135, 137, 138, 145, 146])
+def test_nested_rk4_other_variants(dims, lanes):
+    """the remaining variants, among them those that hold a slice's slot metadata in
+    registers"""
+    test_nested_rk4_matches_oracle(dims, lanes)
+
+
+@pytest.mark.parametrize("lanes", [133, 134, 137, 138, 140, 143, 145, 146])
+def test_metadata_of_long_slices(lanes):
+    """entries without order, so that nearly every one is a slot of its own and a slice has
+    more than 64: the variants that hold the metadata in registers read it from memory"""
+    n, w, dt = 1100, 4, 0.01
+    rng = np.random.default_rng(4)
+    col = np.sort(np.array([rng.choice(n, w, replace=False) for _ in range(n)]), axis=1).astype(np.int64)
+    val = rng.normal(size=(n, w)) + 1j * rng.normal(size=(n, w))
+    rp = (w * np.arange(n + 1)).astype(np.int64)
+    h = ctypes.c_void_p()
+    assert qa.lib().qh_mat_from_csr(ctypes.c_int64(n), *[a.ctypes.data_as(ctypes.c_void_p) for a in (rp, col, val)],
+                                    ctypes.byref(h)) == 0
+    A = qa.Matrix(h, owned=True)
+    prec = qa.FP32 if lanes >= 140 else qa.FP64
+    lay = A.pair_layout_info() if lanes >= 140 else A.layout_info()
+    assert lay["slots"] > 64 * lay["slices"]
+    A.set_lanes(lanes if lanes < 140 else 8, lanes)
+    x0 = rng.normal(size=n) + 1j * rng.normal(size=n)
+    v = qa.DeviceVec(n, prec)
+    v.set(x0)
+    qa.rk4_device(A, v, dt, 3)
+    ref = x0
+    for _ in range(3):
+        y = ref
+        for c in (dt / 4, dt / 3, dt / 2, dt):
+            y = ref + c * (val * y[col]).sum(axis=1)
+        ref = y
+    norm = np.abs(val).sum(axis=1).max()
+    eps = 2.0 ** -24 if prec == qa.FP32 else 2.0 ** -53
+    tol = 3 * np.abs(x0).max() * (2 * dt * norm * eps + 8 * (2.0 ** -48 if prec == qa.FP32 else eps))
+    assert np.abs(v.get() - ref).max() <= tol

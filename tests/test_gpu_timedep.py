@@ -217,6 +217,13 @@ def test_td_rk4_sliced_variants_vs_oracle(prec, variant):
     _forms_case(prec, "sliced_dict", variant, 12, 100)
 
 
+@pytest.mark.parametrize("prec,variant", [("fp64", 138), ("fp32", 138), ("fp32", 140), ("fp32", 145), ("fp32", 146)])
+def test_td_rk4_metadata_in_registers_vs_oracle(prec, variant):
+    """the variants that hold a slice's slot metadata in registers, and 140, which read it
+    that way before"""
+    _forms_case(prec, "sliced_dict", variant, 12, 100)
+
+
 def test_td_rk4_sliced_autotuned_vs_fused():
     """a 24-level cavity (2 304 rows): the autotuned variant of A (sliced or CSR,
     whichever the tuner picks) against the fused CSR kernel, FP64 and FP32, with
