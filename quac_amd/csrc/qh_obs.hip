@@ -112,42 +112,75 @@ __global__ void __launch_bounds__(256) k_expect_wf(const void *x, const float2 *
   block_sum2(ar, ai, partial);
 }
 
-// Ensemble of M wavefunctions (trajectory e at [e*tot, (e+1)*tot)), a wavefront per
+// Threads of a trajectory of tot amplitudes in the statistics of M trajectories: a
+// wavefront where there are enough of them to fill the chip or the trajectory is short,
+// else a workgroup.  An expectation value, wavefront / workgroup: 100 trajectories of 4096
+// 46.8 / 24.3 us, 8 of 32 768 256 / 38.2 us, 64 of 1024 23.5 / 18.1 us.
+int ens_threads(int64_t M, int64_t tot) { return tot <= 256 || M >= 8192 ? 64 : tot <= 4096 ? 256 : 1024; }
+unsigned ens_blocks(int64_t M, int T) { return (unsigned)(T == 64 ? (M + 3) / 4 : M); }
+
+// the sums of v over the T threads of a trajectory (64: a wavefront of a block of 256; else
+// the block), in every thread of the first wavefront
+template <int T, int K>
+__device__ __forceinline__ void ens_sum(double (&v)[K]) {
+#pragma unroll
+  for (int k = 0; k < K; k++)
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_xor(v[k], o, 64);
+  if constexpr (T > 64) {
+    __shared__ double sh[K][T / 64];
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+      for (int k = 0; k < K; k++) sh[k][threadIdx.x >> 6] = v[k];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+      v[k] = 0.0;
+      for (int w = 0; w < T / 64; w++) v[k] += sh[k][w];
+    }
+  }
+}
+
+// Ensemble of M wavefunctions (trajectory e at [e*tot, (e+1)*tot)), T threads per
 // trajectory: the block's sum over its trajectories of <psi|O|psi> / <psi|psi>
 // (qvec_utilities.c:1353-1420)
-__global__ void __launch_bounds__(256) k_expect_ens(const double2 *x, int64_t M, int64_t tot, ChainArg arg,
-                                                    const qh_op *ops, int nops, const qh_level *tab, double2 *out) {
+template <int T>
+__global__ void __launch_bounds__(T < 256 ? 256 : T) k_expect_ens(const double2 *x, int64_t M, int64_t tot,
+                                                                  ChainArg arg, const qh_op *ops, int nops,
+                                                                  const qh_level *tab, double2 *out) {
   const Chain c = chain_of(arg, ops, nops, tab);
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  constexpr int PER = T == 64 ? 4 : 1;  // trajectories of a block at a time
+  const int own = T == 64 ? threadIdx.x >> 6 : 0, lane = T == 64 ? threadIdx.x & 63 : threadIdx.x;
   double sr = 0.0, si = 0.0;
-  for (int64_t e = (int64_t)blockIdx.x * 4 + wave; e < M; e += (int64_t)gridDim.x * 4) {
+  for (int64_t e = (int64_t)blockIdx.x * PER + own; e < M; e += (int64_t)gridDim.x * PER) {
     const double2 *p = x + e * tot;
-    double ar = 0.0, ai = 0.0, nn = 0.0;
-    for (int64_t i = lane; i < tot; i += 64) {
+    double v[3] = {0.0, 0.0, 0.0};
+    for (int64_t i = lane; i < tot; i += T) {
       const double2 pi = p[i];
-      nn += pi.x * pi.x + pi.y * pi.y;
+      v[2] += pi.x * pi.x + pi.y * pi.y;
       int64_t k;
-      double2 v;
-      if (!chain_ig(c.ops, c.n, c.tab, i, k, v)) continue;
+      double2 a;
+      if (!chain_ig(c.ops, c.n, c.tab, i, k, a)) continue;
       const double2 pk = p[k];
-      const double tr = v.x * pk.x - v.y * pk.y, ti = v.x * pk.y + v.y * pk.x;
-      ar += pi.x * tr + pi.y * ti;
-      ai += pi.x * ti - pi.y * tr;
+      const double tr = a.x * pk.x - a.y * pk.y, ti = a.x * pk.y + a.y * pk.x;
+      v[0] += pi.x * tr + pi.y * ti;
+      v[1] += pi.x * ti - pi.y * tr;
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      ar += __shfl_xor(ar, o, 64);
-      ai += __shfl_xor(ai, o, 64);
-      nn += __shfl_xor(nn, o, 64);
-    }
-    sr += ar / nn;
-    si += ai / nn;
+    ens_sum<T>(v);
+    sr += v[0] / v[2];
+    si += v[1] / v[2];
   }
-  __shared__ double2 sh[4];
-  if (lane == 0) sh[wave] = make_double2(sr, si);
-  __syncthreads();
-  if (threadIdx.x == 0)
-    out[blockIdx.x] = make_double2((sh[0].x + sh[1].x) + (sh[2].x + sh[3].x), (sh[0].y + sh[1].y) + (sh[2].y + sh[3].y));
+  if constexpr (T > 64) {
+    if (threadIdx.x == 0) out[blockIdx.x] = make_double2(sr, si);
+  } else {
+    __shared__ double2 sh[4];
+    if (lane == 0) sh[own] = make_double2(sr, si);
+    __syncthreads();
+    if (threadIdx.x == 0)
+      out[blockIdx.x] =
+          make_double2((sh[0].x + sh[1].x) + (sh[2].x + sh[3].x), (sh[0].y + sh[1].y) + (sh[2].y + sh[3].y));
+  }
 }
 
 __global__ void __launch_bounds__(256) k_trace(const void *x, const float2 *lo, int64_t tot, double2 *partial) {
@@ -426,12 +459,17 @@ extern "C" int qh_ens_expect(const qh_vec *ens, int64_t M, int64_t tot, int nops
   ChainArg arg;
   rc = place_chain(nops, ops, nlev, levels, &arg, &dops, &dlev, 0, nullptr);
   // the blocks write their sums straight into pinned host memory
-  const int nb = (int)std::min<int64_t>((M + 3) / 4, NB);
+  const int T = ens_threads(M, tot), nb = (int)std::min<int64_t>(ens_blocks(M, T), NB);
   double2 *h = nullptr;
   if (!rc) rc = qh_scratch(0, nullptr, sizeof(double2) * (size_t)nb, (void **)&h);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_expect_ens, dim3(nb), dim3(256), 0, qh_stream(), (const double2 *)ens->d, M, tot, arg, dops,
-                     nops, dlev, h);
+  auto run = [&](auto *kernel) {
+    hipLaunchKernelGGL(kernel, dim3(nb), dim3(T < 256 ? 256 : T), 0, qh_stream(), (const double2 *)ens->d, M, tot, arg,
+                       dops, nops, dlev, h);
+  };
+  if (T == 64) run(k_expect_ens<64>);
+  else if (T == 256) run(k_expect_ens<256>);
+  else run(k_expect_ens<1024>);
   QH_HIP(hipGetLastError());
   QH_HIP(hipStreamSynchronize(qh_stream()));
   double sr = 0.0, si = 0.0;
@@ -445,19 +483,23 @@ extern "C" int qh_ens_expect(const qh_vec *ens, int64_t M, int64_t tot, int nops
 namespace {
 const int EP_CHUNKS = 256;            // chunks of trajectories at most
 const int64_t EP_PARTS = 1 << 22;     // and of their partial sums (32 MB of scratch)
+// amplitudes up to which the host forms the probabilities (20 trajectories of 64 levels: 18
+// us, 33 us on the device; 200 of 64: 52 and 35 us)
+const int64_t EP_HOST = 8192;
 
-// one wavefront per trajectory: its squared norm
-__global__ void __launch_bounds__(256) k_ep_norms(const double2 *x, int64_t M, int64_t tot, double *nrm) {
-  const int64_t e = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+// T threads per trajectory: its squared norm
+template <int T>
+__global__ void __launch_bounds__(T < 256 ? 256 : T) k_ep_norms(const double2 *x, int64_t M, int64_t tot, double *nrm) {
+  const int64_t e = T == 64 ? (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;
   if (e >= M) return;  // whole wavefront
-  double s = 0.0;
-  for (int64_t i = threadIdx.x & 63; i < tot; i += 64) {
+  const int lane = T == 64 ? threadIdx.x & 63 : threadIdx.x;
+  double s[1] = {0.0};
+  for (int64_t i = lane; i < tot; i += T) {
     const double2 a = x[e * tot + i];
-    s += a.x * a.x + a.y * a.y;
+    s[0] += a.x * a.x + a.y * a.y;
   }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-  if ((threadIdx.x & 63) == 0) nrm[e] = s;
+  ens_sum<T>(s);
+  if (lane == 0) nrm[e] = s[0];
 }
 
 // Level i of 64 a block, one chunk of the trajectories: the sum of |a_i|^2 / norm, or
@@ -507,6 +549,35 @@ extern "C" int qh_ens_probs(const qh_vec *ens, int64_t M, int64_t tot, double *m
   if (rc) return rc;
   QH_REQUIRE(ens && mean && var && ens->prec == QH_FP64 && M >= 1 && M <= (1 << 30) && tot >= 1 && ens->n == M * tot,
              QH_EINVAL, "qh_ens_probs: FP64 ensemble of M trajectories of dimension tot required");
+  if (M * tot <= EP_HOST) {  // one copy and a loop take less than five launches
+    double2 *a = nullptr;
+    rc = qh_scratch(0, nullptr, sizeof(double2) * (size_t)(M * tot), (void **)&a);
+    if (rc) return rc;
+    QH_HIP(hipMemcpyAsync(a, ens->d, sizeof(double2) * (size_t)(M * tot), hipMemcpyDeviceToHost, qh_stream()));
+    QH_HIP(hipStreamSynchronize(qh_stream()));
+    std::fill_n(mean, tot, 0.0);
+    std::fill_n(var, tot, 0.0);
+    for (int64_t e = 0; e < M; e++) {  // |a_i|^2 / norm, kept in the copy
+      double2 *p = a + e * tot;
+      double n = 0.0;
+      for (int64_t i = 0; i < tot; i++) {
+        p[i].x = p[i].x * p[i].x + p[i].y * p[i].y;
+        n += p[i].x;
+      }
+      for (int64_t i = 0; i < tot; i++) {
+        p[i].x /= n;
+        mean[i] += p[i].x;
+      }
+    }
+    for (int64_t i = 0; i < tot; i++) mean[i] /= (double)M;
+    for (int64_t e = 0; e < M; e++)
+      for (int64_t i = 0; i < tot; i++) {
+        const double d = a[e * tot + i].x - mean[i];
+        var[i] += d * d;
+      }
+    for (int64_t i = 0; i < tot; i++) var[i] /= (double)(M > 1 ? M - 1 : 1);
+    return QH_OK;
+  }
   const int chunks =
       (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(EP_CHUNKS, (M + 3) / 4), EP_PARTS / tot));
   double *d = nullptr, *h = nullptr;
@@ -518,7 +589,13 @@ extern "C" int qh_ens_probs(const qh_vec *ens, int64_t M, int64_t tot, double *m
   const double2 *x = (const double2 *)ens->d;
   const dim3 grid(qh_blocks(tot, 64), chunks);
   const unsigned nb = qh_blocks(tot, 16);
-  hipLaunchKernelGGL(k_ep_norms, dim3(qh_blocks(M, 4)), dim3(256), 0, s, x, M, tot, nrm);
+  const int T = ens_threads(M, tot);
+  auto norms = [&](auto *kernel) {
+    hipLaunchKernelGGL(kernel, dim3(ens_blocks(M, T)), dim3(T < 256 ? 256 : T), 0, s, x, M, tot, nrm);
+  };
+  if (T == 64) norms(k_ep_norms<64>);
+  else if (T == 256) norms(k_ep_norms<256>);
+  else norms(k_ep_norms<1024>);
   hipLaunchKernelGGL(k_ep_sums, grid, dim3(256), 0, s, x, M, tot, nrm, nullptr, part);
   hipLaunchKernelGGL(k_ep_total, dim3(nb), dim3(256), 0, s, part, chunks, tot, (double)M, res);
   hipLaunchKernelGGL(k_ep_sums, grid, dim3(256), 0, s, x, M, tot, nrm, (const double *)res, part);

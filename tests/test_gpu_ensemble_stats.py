@@ -47,3 +47,11 @@ def test_ensemble_statistics(levels, count):
         assert L.qh_ens_expect(v.h, count, levels, 1, ctypes.addressof(op), levels, ctypes.addressof(lev),
                                ctypes.byref(re), ctypes.byref(im)) == 0
         assert abs(re.value + 1j * im.value - ref) <= 4 * tol * max(levels, 1)
+
+
+# a workgroup of 256 and of 1024 threads a trajectory; the most amplitudes that the host
+# sums, and one trajectory more; enough short trajectories for a wavefront each
+@pytest.mark.parametrize("levels,count", [(257, 5), (300, 100), (1000, 9), (4096, 3), (4097, 2), (16384, 4), (513, 600),
+                                          (64, 128), (64, 129), (260, 8192)])
+def test_long_trajectories(levels, count):
+    test_ensemble_statistics(levels, count)
