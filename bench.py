@@ -6,8 +6,9 @@ FP64; SpMV % HBM peak".  One JSON line on stdout.
 Headline (default workload):
   * value: the batched parameter sweep of 512 Tavis-Cummings instances of uneven
     size (seed 2; 100 .. 230 400 superoperator rows), RK4 dt = 0.01, advanced as
-    one FP32 batch (block-diagonal sliced matrix, fused stage kernels, hipGraph
-    replay): instance RK4 steps per second over K timed steps, beside the plain
+    one FP32 batch (block-diagonal matrix, a workgroup per closed set of rows, all
+    steps of a call in a few launches): instance RK4 steps per second over K timed
+    steps, beside the plain
     FP64 path run one instance at a time over the same K steps, with the maximum
     population error of the batch against that FP64 path after the same W + K
     steps.
@@ -105,12 +106,12 @@ def format_step_bytes(A, rows):
     return 4 * (vals + meta) + 20 * rows * 8, layout
 
 
-def read_traffic(path):
-    """HBM bytes per stage launch from a committed rocprofv3 --pmc summary
+def read_traffic(path, per="launch"):
+    """HBM bytes per stage launch (or RK4 step) from a committed rocprofv3 --pmc summary
     (FETCH_SIZE + WRITE_SIZE, each scaled by its copy-kernel factor); None when absent"""
     try:
         for line in open(path):
-            if line.startswith("traffic_bytes_per_launch"):
+            if line.startswith("traffic_bytes_per_" + per):
                 return float(line.split("=", 1)[1]), os.path.relpath(path, ROOT)
     except OSError:
         pass
@@ -152,6 +153,35 @@ def roofline_obj(kname, workload, fmt_bytes, launch_ms, ev_ms, traffic, traffic_
     return out
 
 
+def closed_call_bytes(info, rows, steps):
+    """bytes that a call of `steps` RK4 steps on a closed-set plan has to move for an FP32
+    state: once the state's two words in and out, the diagonal, the row order and the
+    entries held in registers (10 B each), and at every stage the words of the sets that
+    are too large for registers (4 B an entry)"""
+    return rows * (32 + 16 + 4) + info["slots"] * 640 + 4 * steps * info["word_slots"] * 256
+
+
+def closed_roofline_obj(info, rows, steps, ms, workload, traffic_step, traffic_src, csr_step_bytes):
+    """the sweep's calls on its closed-set plan, per RK4 step of the whole batch"""
+    nbytes = closed_call_bytes(info, rows, steps) / steps
+    step_ms = ms / steps
+    out = {"bound": "hbm", "achieved": round(nbytes / (step_ms * 1e-3) / 1e9, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+           "frac": round(nbytes / (step_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4), "traffic": traffic_step,
+           "kernel": f"k_comp_dict<float2, 8> ({info['word_bins']} workgroups) and k_comp_rk4 "
+                     f"({info['bins'] - info['word_bins']}), {info['launches']} launches a call of {steps} steps",
+           "workload": workload, "bytes_per_step": nbytes,
+           "bytes_basis": "words of the large sets at every stage; state, diagonal and the entries held in registers "
+                          "once a call",
+           "step_ms": round(step_ms, 5), "plan": info,
+           "csr_model": {"bytes_per_step": csr_step_bytes,
+                         "gbs": round(csr_step_bytes / (step_ms * 1e-3) / 1e9, 1)}}
+    if traffic_step:
+        tg = traffic_step / (step_ms * 1e-3) / 1e9
+        out.update(traffic_source=traffic_src, traffic_over_format_bytes=round(traffic_step / nbytes, 3),
+                   traffic_gbs=round(tg, 1), traffic_frac=round(tg / HBM_PEAK_GBS, 4))
+    return out
+
+
 # ---------------------------------------------------------------- sweep (value)
 def run_sweep(qa, recipes, build_system, subsystem_layout, K, W, n_inst, renorm):
     from bench_workloads import _pops
@@ -188,11 +218,21 @@ def run_sweep(qa, recipes, build_system, subsystem_layout, K, W, n_inst, renorm)
     qa.synchronize()
     el32 = time.perf_counter() - t
     pops32 = b.populations(subs)
-    lanes = bA.lanes()
-    fmt_step, layout = step_bytes(bA, rows)
-    nprof = min(20, max(K, 1))
-    ev_ms = qa.rk4_device(bA, bx, dt, nprof, timed=True)   # per-launch events (state advanced past the check)
-    launch_ms = tm32.ms / (4 * K) if K > 0 else ev_ms
+    info = bA.closed_info(qa.FP32)
+    workload = f"{n_inst} Tavis-Cummings instances, one block-diagonal batch"
+    if info["bins"]:                            # the closed-set plan stepped the batch
+        traffic, src = read_traffic(os.path.join(ROOT, "profiles", "k_comp_dict_tc512_traffic.txt"), "step")
+        rf = closed_roofline_obj(info, rows, max(K, 1), tm32.ms, workload, traffic, src,
+                                 rk4_step_bytes(nnz, rows, 8)) if K > 0 else None
+        lanes, layout = None, info
+    else:
+        nprof = min(20, max(K, 1))
+        ev_ms = qa.rk4_device(bA, bx, dt, nprof, timed=True)  # per-launch events (state advanced past the check)
+        lanes = bA.lanes()
+        fmt_step, layout = step_bytes(bA, rows)
+        rf = roofline_obj(kernel_name(lanes[1], "float") + " (mean of the 4 fused RK4 stage launches)", workload,
+                          fmt_step / 4, tm32.ms / (4 * K) if K > 0 else ev_ms, ev_ms, None, None,
+                          rk4_step_bytes(nnz, rows, 8) / 4)
 
     el64 = 0.0
     worst = 0.0
@@ -212,10 +252,6 @@ def run_sweep(qa, recipes, build_system, subsystem_layout, K, W, n_inst, renorm)
         qs.destroy()
     v32 = n_inst * K / el32
     v64 = n_inst * K / el64
-    traffic, src = read_traffic(os.path.join(ROOT, "profiles", "k_ks2_stage_tc512_traffic.txt"))
-    rf = roofline_obj(kernel_name(lanes[1], "float") + " (mean of the 4 fused RK4 stage launches)",
-                      f"{n_inst} Tavis-Cummings instances, one block-diagonal batch", fmt_step / 4, launch_ms,
-                      ev_ms, traffic, src, rk4_step_bytes(nnz, rows, 8) / 4)
     return {"v32": v32, "v64": v64, "el32": el32, "el64": el64, "worst": worst, "asm_s": asm_s, "rows": rows,
             "nnz": nnz, "rows_min": min(t * t for t in tots), "rows_max": max(t * t for t in tots), "lanes": lanes,
             "roofline": rf, "layout": layout}
@@ -476,8 +512,8 @@ def main():
     out = {
         "metric": METRIC, "value": value, "unit": unit, "n_gpus": 1, "steps": K, "warmup": W,
         "ms_per_step": round(ms_step, 5), "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
-        "dtype": "fp32 (complex64 matrix values and stage vectors, products and row sums in fp64, hi+lo complex64 "
-                 "state; fp64 trace renormalisation and observables)",
+        "dtype": "fp32 (complex64 stage vectors, hi+lo complex64 state; matrix values complex64, or fp64 where a "
+                 "closed-set plan steps the batch; row sums in fp64; fp64 trace renormalisation and observables)",
         "data": "synthetic", "config": config,
         "roofline": ch["roofline"],
         "cpu_baseline": cpu,

@@ -65,3 +65,16 @@ def test_kernel_names_of_metadata_in_registers():
     for g in (137, 138, 145, 146):
         assert "stage" in bench.kernel_name(g, "float") and bench.kernel_name(g, "float") != bench.kernel_name(
             {137: 133, 138: 134, 145: 140, 146: 143}[g], "float")
+
+
+def test_closed_set_roofline_counts_words_at_every_stage():
+    info = {"bins": 10, "word_bins": 2, "launches": 3, "slots": 7, "word_slots": 11}
+    rows, steps = 1000, 20
+    nbytes = rows * 52 + 7 * 640 + 4 * steps * 11 * 256
+    assert bench.closed_call_bytes(info, rows, steps) == nbytes
+    rf = bench.closed_roofline_obj(info, rows, steps, 1e-3 * steps, "w", 2 * nbytes / steps, "src", 32e6)
+    assert rf["achieved"] == pytest.approx(nbytes / steps / 1e-6 / 1e9, rel=1e-2)
+    assert rf["frac"] == pytest.approx(rf["achieved"] / 8000.0, rel=1e-2, abs=1e-4)
+    assert rf["traffic_over_format_bytes"] == pytest.approx(2.0)
+    t, src = bench.read_traffic(os.path.join(ROOT, "profiles", "k_comp_dict_tc512_traffic.txt"), "step")
+    assert src == os.path.join("profiles", "k_comp_dict_tc512_traffic.txt") and 1e9 < t < 4e9
