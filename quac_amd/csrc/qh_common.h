@@ -185,9 +185,8 @@ struct qh_vec {
 
 // FP32 row-pair sliced layout (qh_ks2.hip): build once per matrix, launch one
 // stage (a MODE of qh_ks.h: SpMV, AXPY, LAST, STAGE, FINAL) with variant G = 140 ..
-// 144; td
-// (may be null): the merged A_k of a time-dependent RHS summed in the same kernel
-// (variants 140, 142, 143)
+// 146; td (may be null): the merged A_k of a time-dependent RHS summed in the same
+// kernel (variants 140, 142, 143, 145, 146)
 struct qh_td_ell;
 int ks2_build(qh_mat *A);
 int ks2_launch(int G, int mode, hipStream_t s, const qh_mat *A, const void *xin, void *kout, void *ynext, double cn,

@@ -9,8 +9,9 @@
 // reads and writes the state once instead of three vector passes and a launch per
 // stage.
 //
-// Plan (once per matrix): connected components of the sparsity pattern (union
-// find), components packed into bins of whole components, rows sorted within a bin.
+// Plan (once per matrix): connected components of the sparsity pattern (the
+// lock-free union find of Anderson & Woll 1991 with the path halving of Tarjan & van
+// Leeuwen 1984), components packed into bins of whole components, rows sorted within a bin.
 // A bin's rows are stored in slices of 64 (one wavefront): the diagonal apart, and
 // every other entry as one or two real entries, first the imaginary parts (an even
 // number of slots a slice), then the real parts, each a value and the 16-bit index
@@ -1272,7 +1273,8 @@ double *qh_comp_trace(const qh_mat *A, int prec) { return A->comp[prec == QH_FP3
 
 extern "C" int qh_mat_closed_info(const qh_mat *m, int prec, int64_t *bins, int64_t *word_bins, int64_t *launches,
                                   int64_t *slots, int64_t *word_slots) {
-  QH_REQUIRE(m && (prec == QH_FP64 || prec == QH_FP32), QH_EINVAL, "qh_mat_closed_info: a matrix and a precision required");
+  QH_REQUIRE(m && (prec == QH_FP64 || prec == QH_FP32), QH_EINVAL,
+             "qh_mat_closed_info: a matrix and a precision required");
   const qh_comp *c = m->comp[prec == QH_FP32];
   int64_t all = 0, words = 0;
   if (c)

@@ -40,10 +40,12 @@ enum { KS_UNI = 0, KS_SCA = 1, KS_CPX = 2, KS_SC1 = 3 };
 // The metadata of a slice's slots held in registers: lane k loads slot k (one
 // trip to memory for the whole slice, at most 64 slots), and a pass reads the slots
 // it needs with v_readlane into scalar registers.  With the metadata behind scalar
-// loads every pass waits for its own before it can issue its gathers; the metadata
-// streams (they miss the scalar cache each time), so those waits were a large part
-// of a wavefront's time.  Per launch: 10-qubit chain FP64 28.2 -> 24.7 us, 12-qubit
-// circuit FP64 243 -> 231 us and FP32 175 -> 138 us, sweep of 512 instances 202 -> 197 us.
+// loads every pass waits for its own before it can issue its gathers; where the
+// metadata streams (they miss the scalar cache each time) those waits are a large part
+// of a wavefront's time, and where the caches hold it the trip ahead of the first pass
+// and the reads of lanes are the longer way.  Per launch, from memory / in registers:
+// 10-qubit chain FP64 28.7 / 24.7 us, 12-qubit circuit FP64 262 / 235 us and FP32 154 /
+// 140 us; 9-qubit chain FP64 7.8 / 8.7 us, three 9-level cavities FP32 12.9 / 13.7 us.
 template <typename M>
 struct KsRegs {
   static constexpr int ND = sizeof(M) / 4;

@@ -1036,15 +1036,15 @@ int ks2_launch(int G, int mode, hipStream_t s, const qh_mat *A, const void *xin,
   const bool win = G == 142 || G == 144;
   const dim3 grid(qh_blocks(ns, win ? KS2_WIN / 128 : 4)), blk(win ? KS2_WIN / 2 : 256);
   const qh_td_ell none{nullptr, nullptr, nullptr, nullptr, nullptr};
-#define QH_LK2T(MM, UU, WW, NN, SS, TT, RR, TD)                                                                      \
-  hipLaunchKernelGGL((k_ks2_stage<MM, UU, WW, NN, SS, TT, RR>), grid, blk, 0, s, n, ns, A->ks2_moff, A->ks2_wmid,       \
-                     A->ks2_smid,                                                                                \
-                     A->ks2_umid, A->ks2_emid, A->ks2_cmid, A->ks2_xmid, A->ks2_sep,                               \
-                     (int32_t)A->ks2_ngh,                                                                        \
-                     A->ks2_gh, MM == MODE_LAST ? (const void *)A->ks2_metad : (const void *)A->ks2_meta, (int32_t)A->ks2_nval, A->ks2_val,                                    \
-                     (int32_t)A->ks2_nsval, A->ks2_sval, (int32_t)A->ks2_nsval1, A->ks2_sval1,                  \
-                     (const float2 *)xin, (float2 *)kout, (float2 *)ynext, cn, (const float2 *)x,                \
-                     (const float2 *)k1, (const float2 *)k2, (const float2 *)k3, (float2 *)xout, h, xlo, TD)
+#define QH_LK2T(MM, UU, WW, NN, SS, TT, RR, TD)                                                                   \
+  hipLaunchKernelGGL((k_ks2_stage<MM, UU, WW, NN, SS, TT, RR>), grid, blk, 0, s, n, ns, A->ks2_moff, A->ks2_wmid, \
+                     A->ks2_smid, A->ks2_umid, A->ks2_emid, A->ks2_cmid, A->ks2_xmid, A->ks2_sep,                 \
+                     (int32_t)A->ks2_ngh, A->ks2_gh,                                                              \
+                     MM == MODE_LAST ? (const void *)A->ks2_metad : (const void *)A->ks2_meta,                    \
+                     (int32_t)A->ks2_nval, A->ks2_val, (int32_t)A->ks2_nsval, A->ks2_sval,                        \
+                     (int32_t)A->ks2_nsval1, A->ks2_sval1, (const float2 *)xin, (float2 *)kout, (float2 *)ynext,  \
+                     cn, (const float2 *)x, (const float2 *)k1, (const float2 *)k2, (const float2 *)k3,           \
+                     (float2 *)xout, h, xlo, TD)
 #define QH_LK2S(MM, UU, WW, NN, SS, RR) QH_LK2T(MM, UU, WW, NN, SS, false, RR, none)
 #define QH_LK2(MM, UU, WW, NN, RR)        \
   do {                                    \
@@ -1053,7 +1053,8 @@ int ks2_launch(int G, int mode, hipStream_t s, const qh_mat *A, const void *xin,
     else                                  \
       QH_LK2S(MM, UU, WW, NN, false, RR); \
   } while (0)
-  const bool known = mode == MODE_SPMV || mode == MODE_STAGE || mode == MODE_FINAL || mode == MODE_AXPY || mode == MODE_LAST;
+  const bool known =
+      mode == MODE_SPMV || mode == MODE_STAGE || mode == MODE_FINAL || mode == MODE_AXPY || mode == MODE_LAST;
   if (!QH_IS_KS2(G) || !known || (td && (mode == MODE_AXPY || mode == MODE_LAST))) {
     qh_set_error("unsupported row-pair variant %d / mode %d", G, mode);
     return QH_EINVAL;
@@ -1061,12 +1062,12 @@ int ks2_launch(int G, int mode, hipStream_t s, const qh_mat *A, const void *xin,
   // metadata in registers: one slot a lane
   if (A->ks2_maxslots > 64) G = G == 145 ? 140 : G == 146 ? 143 : G;
   if (td) {  // the time-dependent entries summed in the same kernel (variants 140, 142, 143, 145, 146)
-#define QH_LK2D(MM, UU, WW, NN, RR)                                                             \
+#define QH_LK2D(MM, UU, WW, NN, RR)                                                         \
   do {                                                                                      \
     if (A->ks2_nsep)                                                                        \
-      QH_LK2T(MM, UU, WW, NN, true, true, RR, *td);                                            \
+      QH_LK2T(MM, UU, WW, NN, true, true, RR, *td);                                         \
     else                                                                                    \
-      QH_LK2T(MM, UU, WW, NN, false, true, RR, *td);                                           \
+      QH_LK2T(MM, UU, WW, NN, false, true, RR, *td);                                        \
   } while (0)
 #define QH_LK2DG(MM)                                                                        \
   switch (G) {                                                                              \

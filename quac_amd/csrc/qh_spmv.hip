@@ -527,9 +527,9 @@ __global__ void __launch_bounds__(256) k_ks_stage(
     const int32_t *__restrict__ cmid, const qh_kmeta *__restrict__ meta, const qh_kmeta32 *__restrict__ meta32,
     int32_t nmeta, int32_t nval, const typename C2<R>::T *__restrict__ val, int32_t nsval,
     const R *__restrict__ sval,
-    const typename C2<R>::T *__restrict__ xin, typename C2<R>::T *__restrict__ kout, typename C2<R>::T *ynext, double cn,
-    const typename C2<R>::T *x, const typename C2<R>::T *__restrict__ k1, const typename C2<R>::T *__restrict__ k2,
-    const typename C2<R>::T *__restrict__ k3, typename C2<R>::T *xout, double h, float2 *__restrict__ xlo, double atol,
+    const typename C2<R>::T *__restrict__ xin, typename C2<R>::T *__restrict__ kout, typename C2<R>::T *ynext,
+    double cn, const typename C2<R>::T *x, const typename C2<R>::T *__restrict__ k1,
+    const typename C2<R>::T *__restrict__ k2, const typename C2<R>::T *__restrict__ k3, typename C2<R>::T *xout, double h, float2 *__restrict__ xlo, double atol,
     double rtol, double *__restrict__ eacc, qh_td_ell td) {
   typedef typename C2<R>::T T;
   const unsigned b = qh_xcd_block(blockIdx.x, gridDim.x);
@@ -962,8 +962,8 @@ int ks_make_fp32(qh_mat *A) {
 // launch the sliced-layout kernel with the slot unroll encoded in the variant code G
 template <typename R, int MODE>
 int launch_ks(int G, hipStream_t s, const qh_mat *A, const void *xin, void *kout, void *ynext, double cn,
-              const void *x, const void *k1, const void *k2, const void *k3, void *xout, double h, float2 *xlo, double atol = 0.0,
-              double rtol = 0.0, double *eacc = nullptr, const qh_td_ell *td = nullptr) {
+              const void *x, const void *k1, const void *k2, const void *k3, void *xout, double h, float2 *xlo,
+              double atol = 0.0, double rtol = 0.0, double *eacc = nullptr, const qh_td_ell *td = nullptr) {
   typedef typename C2<R>::T T;
   const T *kv = sizeof(R) == 8 ? (const T *)A->ks_val : (const T *)A->ks_val32;
   const R *sv = sizeof(R) == 8 ? (const R *)A->ks_sval : (const R *)A->ks_sval32;
@@ -972,12 +972,12 @@ int launch_ks(int G, hipStream_t s, const qh_mat *A, const void *xin, void *kout
   const qh_td_ell none{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0};
   // metadata in registers: one slot a lane
   if (A->ks_maxslots > 64) G = G == 137 ? 133 : G == 138 ? 134 : G;
-#define QH_LKT(UU, VV, PP, RR, NN, TT, TD)                                                                         \
-  hipLaunchKernelGGL((k_ks_stage<R, MODE, UU, VV, PP, RR, NN, TT>), grid, blk, 0, s, n, ns, A->ks_moff, A->ks_umid,     \
-                     A->ks_cmid,                                                                              \
-                     A->ks_meta, A->ks_meta32, (int32_t)(A->ks_slots + QH_KS_PAD), (int32_t)A->ks_nval, kv,    \
-                     (int32_t)A->ks_nsval, sv, (const T *)xin, (T *)kout, (T *)ynext, cn, (const T *)x,       \
-                     (const T *)k1, (const T *)k2, (const T *)k3, (T *)xout, h, xlo, atol, rtol, eacc, TD)
+#define QH_LKT(UU, VV, PP, RR, NN, TT, TD)                                                                  \
+  hipLaunchKernelGGL((k_ks_stage<R, MODE, UU, VV, PP, RR, NN, TT>), grid, blk, 0, s, n, ns, A->ks_moff,     \
+                     A->ks_umid, A->ks_cmid, A->ks_meta, A->ks_meta32, (int32_t)(A->ks_slots + QH_KS_PAD),  \
+                     (int32_t)A->ks_nval, kv, (int32_t)A->ks_nsval, sv, (const T *)xin, (T *)kout,          \
+                     (T *)ynext, cn, (const T *)x, (const T *)k1, (const T *)k2, (const T *)k3, (T *)xout,  \
+                     h, xlo, atol, rtol, eacc, TD)
 #define QH_LK(UU, VV, PP, NN) QH_LKT(UU, VV, PP, false, NN, false, none)
 #define QH_LKR(UU) QH_LKT(UU, false, true, true, false, false, none)
   if constexpr (MODE == MODE_SPMV || MODE == MODE_STAGE || MODE == MODE_FINAL ||
@@ -1413,7 +1413,8 @@ struct SmallRow {
     }
     return c[k];
   }
-  __device__ __forceinline__ void load(int32_t n, int32_t r, const int32_t *rp, const int32_t *col, const double2 *val) {
+  __device__ __forceinline__ void load(int32_t n, int32_t r, const int32_t *rp, const int32_t *col,
+                                       const double2 *val) {
     if (r < n) {
       b = rp[r];
       e = rp[r + 1];

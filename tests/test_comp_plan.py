@@ -21,8 +21,9 @@ def run(tmp_path_factory):
 
     def _run(name, body):
         src, exe = str(d / (name + ".cpp")), str(d / name)
+        heads = ["<array>", "<cstdio>", "<cstdlib>", "<random>", '"qh_comp_plan.h"', '"qh_optional.h"']
         with open(src, "w") as f:
-            f.write('#include <array>\n#include <cstdio>\n#include <cstdlib>\n#include <random>\n#include "qh_comp_plan.h"\n#include "qh_optional.h"\n' + body)
+            f.write("".join(f"#include {h}\n" for h in heads) + body)
         subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-fsanitize=address,undefined", "-I", CSRC, src,
                         "-o", exe], check=True)
         return subprocess.run([exe], check=True, capture_output=True, text=True).stdout
@@ -110,10 +111,11 @@ static std::vector<CpBin> bins(std::vector<std::array<int, 3>> groups) {
 }
 int main() {
   // the bins of decay and dephasing of 8, 10 and 11 qubits
-  const CpShapes s8 = cp_shapes(bins({{9, 256, 8}, {233, 128, 7}, {128, 128, 4}, {266, 64, 6}, {369, 64, 4}}), false, CUS);
-  const CpShapes s10 = cp_shapes(bins({{9, 1024, 10}, {12, 512, 9}, {2156, 512, 7}, {16, 512, 4}, {9, 64, 4}}), false, CUS);
-  const CpShapes s11 = cp_shapes(
-      bins({{9, 2048, 11}, {102, 1024, 10}, {132, 512, 9}, {8458, 512, 8}, {22, 512, 4}, {57, 256, 8}, {13, 64, 8}}), false, CUS);
+  const auto b8 = bins({{9, 256, 8}, {233, 128, 7}, {128, 128, 4}, {266, 64, 6}, {369, 64, 4}});
+  const auto b10 = bins({{9, 1024, 10}, {12, 512, 9}, {2156, 512, 7}, {16, 512, 4}, {9, 64, 4}});
+  const auto b11 = bins(
+      {{9, 2048, 11}, {102, 1024, 10}, {132, 512, 9}, {8458, 512, 8}, {22, 512, 4}, {57, 256, 8}, {13, 64, 8}});
+  const CpShapes s8 = cp_shapes(b8, false, CUS), s10 = cp_shapes(b10, false, CUS), s11 = cp_shapes(b11, false, CUS);
   NEED(s8.classes.size() == 5 && s8.brief.size() == 1 && s8.brief_steps >= 20);
   NEED(s10.brief.size() == 1 && s10.brief_steps >= 2 && s10.brief_steps <= 20);
   NEED(s11.brief.size() == 1 && s11.brief_steps == 0);

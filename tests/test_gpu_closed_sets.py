@@ -312,5 +312,6 @@ def test_refused_plan_is_looked_at_once():
         assert qs.matrix().closed_info()["bins"] == 0 and qs.matrix().lanes()[0] != 0
         rp, _, val = qs.matrix().export()
         norm = np.add.reduceat(np.abs(val), rp[:-1]).max()
-        assert np.abs(v.get() - m.rk4(x0, dt, steps)).max() <= steps * np.abs(x0).max() * (2 * dt * norm + 8) * 2.0 ** -53
+        tol = steps * np.abs(x0).max() * (2 * dt * norm + 8) * 2.0 ** -53
+        assert np.abs(v.get() - m.rk4(x0, dt, steps)).max() <= tol
         qs.destroy()
