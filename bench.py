@@ -222,7 +222,8 @@ def run_sweep(qa, recipes, build_system, subsystem_layout, K, W, n_inst, renorm)
     workload = f"{n_inst} Tavis-Cummings instances, one block-diagonal batch"
     if info["bins"]:                            # the closed-set plan stepped the batch
         traffic, src = read_traffic(os.path.join(ROOT, "profiles", "k_comp_dict_tc512_traffic.txt"), "step")
-        rf = closed_roofline_obj(info, rows, max(K, 1), tm32.ms, workload, traffic, src,
+        per = min(renorm, K) if renorm else K   # steps a call: up to the trace renormalisation
+        rf = closed_roofline_obj(info, rows, per, tm32.ms * per / K, workload, traffic, src,
                                  rk4_step_bytes(nnz, rows, 8)) if K > 0 else None
         lanes, layout = None, info
     else:
